@@ -287,6 +287,7 @@ struct Ctx {
   int m2l_tn = 512;         // targets per M2L tile (512 or 256)
   int m2l_ncell_tiled = 0;  // cells that receive M2L (the tiles' columns)
   Buf<int> m2l_misc, m2l_rs_hist, m2l_scan;
+  Buf<double> m2l_part64;   // FP64 partial locals of the list shares (m2l.hip)
   Buf<float> m2l_part;      // FP32 partial locals of the key slices [slice][cell][P^2]
   // variable-order M2L: order of each (tile, key), parallel to tile_keys
   bool learned = false;
