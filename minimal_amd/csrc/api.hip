@@ -431,7 +431,7 @@ int exafmm_direct(exafmm_ctx *ctx, exafmm_body *targets, int64_t nt, const exafm
     if (!ctx || !targets || !sources || nt < 0 || ns < 0) fail(EXAFMM_ERR_ARG, "bad argument");
     Ctx &c = ctx->c;
     if (on_device) {
-      direct_sum(c.cfg.device, c.s0, targets, nt, sources, ns);
+      direct_sum(c, targets, nt, sources, ns);
       XF_HIP(hipStreamSynchronize(c.s0));
     } else {
       op_p2p(c, targets, nt, sources, ns);

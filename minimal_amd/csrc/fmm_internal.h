@@ -271,6 +271,7 @@ struct Ctx {
   bool capturing = false;
   int graph_locks = 0;
   Buf<double> shift_T;             // scaled M2M / L2L operators per octant
+  Buf<double> direct_part;         // direct sum: partial sums [source share][target][4]
   Buf<double> dipole_part;         // dipole moment: per-workgroup partials, then the sum
   int shift_P = -1;
 
@@ -375,7 +376,7 @@ void m2l_group_launch(const GemmGroupPlan &plan, hipStream_t s);
 void shift_ops(Ctx &c, hipStream_t s);
 void l2l_pass(Ctx &c);
 void l2p_pass(Ctx &c);
-void direct_sum(int device, hipStream_t s, exafmm_body *t, int64_t nt, const exafmm_body *src, int64_t ns);
+void direct_sum(Ctx &c, exafmm_body *t, int64_t nt, const exafmm_body *src, int64_t ns);
 void periodic_far(Ctx &c);
 void dipole_correction(Ctx &c);
 void ewald_sum(Ctx &c, exafmm_body *t, int64_t nt, const exafmm_body *s, int64_t ns, int ksize, double alpha,

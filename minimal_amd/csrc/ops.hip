@@ -113,7 +113,7 @@ __global__ void k_op_l2p(int P, double cx, double cy, double cz, const double2 *
 
 void op_p2p(Ctx &c, exafmm_body *t, int64_t nt, const exafmm_body *s, int64_t ns) {
   DevCopy<exafmm_body> dt(t, nt, c.s0), ds(s, ns, c.s0);
-  direct_sum(c.cfg.device, c.s0, dt.b.p, nt, ds.b.p, ns);
+  direct_sum(c, dt.b.p, nt, ds.b.p, ns);
   dt.back(t, nt, c.s0);
 }
 

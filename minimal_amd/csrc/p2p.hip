@@ -27,6 +27,7 @@
 // lane partials (FP32 sums of at most kP2PFlush terms) are reduced across
 // the lanes and added into Kahan-compensated running sums, one per lane
 // (a lane holds one target's p or force component after the reduction).
+#include <algorithm>
 #include <type_traits>
 
 #include "fmm_internal.h"
@@ -209,21 +210,20 @@ __device__ inline void p2p_round(float4 s, const float (&xt)[TC], const float (&
 // then a butterfly over the lanes that share a target.  Lane l receives
 // component l % kLow (p, F_x, F_y, F_z for 0..3) of target l / kLow, with
 // kLow = 64 / T2 (T2 = TC rounded up to a power of two); other lanes 0.
-template <int TC>
-__device__ inline float p2p_lane_total(const float (&ap)[TC], const float (&ax)[TC], const float (&ay)[TC],
-                                       const float (&az)[TC], int lane) {
+template <int TC, class T>
+__device__ inline T p2p_lane_total(const T (&ap)[TC], const T (&ax)[TC], const T (&ay)[TC], const T (&az)[TC],
+                                   int lane) {
   constexpr int T2 = pow2ceil<TC>();
   constexpr int kLow = kWave / T2;
-  float vp[T2], vx[T2], vy[T2], vz[T2];
+  T vp[T2], vx[T2], vy[T2], vz[T2];
 #pragma unroll
   for (int i = 0; i < T2; i++) {
-    vp[i] = i < TC ? ap[i] : 0.0f;
-    vx[i] = i < TC ? ax[i] : 0.0f;
-    vy[i] = i < TC ? ay[i] : 0.0f;
-    vz[i] = i < TC ? az[i] : 0.0f;
+    vp[i] = i < TC ? ap[i] : T(0);
+    vx[i] = i < TC ? ax[i] : T(0);
+    vy[i] = i < TC ? ay[i] : T(0);
+    vz[i] = i < TC ? az[i] : T(0);
   }
-  float rp = halving<T2>(vp, lane), rx = halving<T2>(vx, lane), ry = halving<T2>(vy, lane),
-        rz = halving<T2>(vz, lane);
+  T rp = halving<T2>(vp, lane), rx = halving<T2>(vx, lane), ry = halving<T2>(vy, lane), rz = halving<T2>(vz, lane);
 #pragma unroll
   for (int m = 1; m < kLow; m <<= 1) {
     rp += __shfl_xor(rp, m);
@@ -232,7 +232,7 @@ __device__ inline float p2p_lane_total(const float (&ap)[TC], const float (&ax)[
     rz += __shfl_xor(rz, m);
   }
   const int comp = lane % kLow;
-  return comp == 0 ? rp : comp == 1 ? rx : comp == 2 ? ry : comp == 3 ? rz : 0.0f;
+  return comp == 0 ? rp : comp == 1 ? rx : comp == 2 ? ry : comp == 3 ? rz : T(0);
 }
 
 // Targets t0 .. t0 + tc - 1 (tc <= TC) of a leaf (a wave) against its whole list.
@@ -399,52 +399,122 @@ __global__ void __launch_bounds__(kP2PWaves *kWave) k_p2p32_grouped(const GroupT
                   t.bodies, lds[w]);
 }
 
-// FP64 path: the reference's arithmetic per interaction (1/R2, q*sqrt, dX
-// scaled by invR2*invR) on absolute FP64 coordinates; one thread per target
-// body, sources in list order.
-__global__ void __launch_bounds__(64) k_p2p64(const int *__restrict__ leaves, const int *__restrict__ nleaves,
-                                              const int *__restrict__ cbeg, const int *__restrict__ ccnt,
-                                              const double4 *__restrict__ xs, const int *__restrict__ lbeg,
-                                              const int *__restrict__ lcnt, const int *__restrict__ list,
-                                              const int *__restrict__ scbeg, const int *__restrict__ sccnt,
-                                              const double4 *__restrict__ sxs, double cycle,
-                                              exafmm_body *__restrict__ bodies,
-                                              const int *__restrict__ list_flags) {
-#pragma clang fp contract(off)
+// One FP64 interaction (3d/kernel.h:135-146): p += q/r, F -= q dX/r^3 (the
+// caller subtracts), pairs at zero distance skipped.  The hardware's 1/sqrt
+// (about 2^-23 relative) takes one third-order step
+//   e = 1 - r^2 y^2,  y += y e (1/2 + 3/8 e)
+// (remainder 5/16 e^3, below 2^-60), five FP64 operations where a divide and
+// a square root expand to about forty.  Squared distances outside
+// [2^-900, 2^900) -- zero, overflow, NaN -- take the plain divide and root.
+__device__ inline void p2p64_pair(double dx, double dy, double dz, double q, double &pot, double &ax, double &ay,
+                                  double &az) {
+  const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
+  double y = __builtin_amdgcn_rsq(r2);
+  const double t = r2 * y;
+  const double e = fma(-t, y, 1.0);
+  y = fma(y * e, fma(e, 0.375, 0.5), y);
+  const unsigned hi = unsigned(__double2hiint(r2));
+  if (hi - (123u << 20) >= (1800u << 20)) y = r2 != 0.0 ? sqrt(1.0 / r2) : 0.0;
+  const double qi = q * y;
+  const double f = qi * (y * y);
+  pot += qi;
+  ax = fma(dx, f, ax);
+  ay = fma(dy, f, ay);
+  az = fma(dz, f, az);
+}
+
+// FP64 P2P: a workgroup per target leaf, its waves taking the leaf's targets
+// in balanced blocks of at most kP2P64TC; as in the FP32 kernel a block's
+// targets are wave-uniform and the lanes take the staged entries' sources,
+// one load per source and block.  FP64 VALU bound (about 25 operations per
+// interaction).  67,984,904 interactions (30,000 bodies): 164 us; 903 us with
+// a thread per target walking its sources one by one through a divide and a
+// square root each.
+constexpr int kP2P64TC = 8;
+
+template <int TC>
+__device__ __attribute__((always_inline)) inline void p2p64_block(int t0, int tc, int tb, int b0, int nl,
+                                                                  const double4 *__restrict__ xs,
+                                                                  const int *__restrict__ list,
+                                                                  const int *__restrict__ scbeg,
+                                                                  const int *__restrict__ sccnt,
+                                                                  const double4 *__restrict__ sxs, double cycle,
+                                                                  exafmm_body *__restrict__ bodies, P2PLds &L) {
+  const int lane = threadIdx.x & (kWave - 1);
+  double xt[TC], yt[TC], zt[TC], ap[TC], ax[TC], ay[TC], az[TC];
+#pragma unroll
+  for (int t = 0; t < TC; t++) {
+    const double4 v = xs[tb + t0 + min(t, tc - 1)];  // wave-uniform address: scalar loads
+    xt[t] = v.x;
+    yt[t] = v.y;
+    zt[t] = v.z;
+    ap[t] = ax[t] = ay[t] = az[t] = 0.0;
+  }
+  for (int seg = 0; seg < nl; seg += kP2PSeg) {
+    const int ne = min(kP2PSeg, nl - seg);
+    int nself = 0;
+    const int total = p2p_stage_entries(L, list, b0, seg, ne, -1, scbeg, sccnt, make_double4(0, 0, 0, 0), cycle,
+                                        lane, &nself);
+    int e = 0;
+    for (int g = lane; g < total; g += kWave) {
+      while (L.pre[e + 1] <= g) e++;
+      const double4 X = sxs[L.beg[e] + g - L.pre[e]];
+      const double sx = X.x + L.dlx[e], sy = X.y + L.dly[e], sz = X.z + L.dlz[e];  // the entry's image shift
+#pragma unroll
+      for (int t = 0; t < TC; t++) p2p64_pair(xt[t] - sx, yt[t] - sy, zt[t] - sz, X.w, ap[t], ax[t], ay[t], az[t]);
+    }
+  }
+  constexpr int kLow = kWave / pow2ceil<TC>();
+  const int t = lane / kLow, comp = lane % kLow;
+  const double v = p2p_lane_total<TC>(ap, ax, ay, az, lane);
+  if (comp < 4 && t < tc) {
+    exafmm_body *ob = bodies + tb + t0 + t;
+    if (comp == 0)
+      ob->p += v;
+    else
+      ob->F[comp - 1] -= v;
+  }
+}
+
+__global__ void __launch_bounds__(kP2PWaves *kWave) k_p2p64(const int *__restrict__ leaves,
+                                                            const int *__restrict__ nleaves,
+                                                            const int *__restrict__ cbeg, const int *__restrict__ ccnt,
+                                                            const double4 *__restrict__ xs,
+                                                            const int *__restrict__ lbeg,
+                                                            const int *__restrict__ lcnt, const int *__restrict__ list,
+                                                            const int *__restrict__ scbeg,
+                                                            const int *__restrict__ sccnt,
+                                                            const double4 *__restrict__ sxs, double cycle,
+                                                            exafmm_body *__restrict__ bodies,
+                                                            const int *__restrict__ list_flags) {
+  __shared__ P2PLds lds[kP2PWaves];
   const int li = blockIdx.x;
   if (li >= *nleaves || p2p_skip(list_flags)) return;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // wave-level syncs only below
   const int c = leaves[li];
   const int tb = cbeg[c], tn = ccnt[c];
   const int b0 = lbeg[c], nl = lcnt[c];
-  for (int i = threadIdx.x; i < tn; i += 64) {
-    const double4 xi = xs[tb + i];
-    double pot = 0, ax = 0, ay = 0, az = 0;
-    for (int s = 0; s < nl; s++) {
-      const int e = list[b0 + s];
-      const int sc = e >> 5, img = e & 31;
-      const double sx = ((img % 3) - 1) * cycle, sy = (((img / 3) % 3) - 1) * cycle, sz = ((img / 9) - 1) * cycle;
-      const int sb = scbeg[sc], sn = sccnt[sc];
-      for (int j = sb; j < sb + sn; j++) {
-        const double4 xj = sxs[j];
-        // 3dp/kernel.h:133: dX = Xi - Xj - iX * cycle
-        double dx = xi.x - xj.x - sx, dy = xi.y - xj.y - sy, dz = xi.z - xj.z - sz;
-        const double R2 = dx * dx + dy * dy + dz * dz;
-        if (R2 != 0) {
-          const double invR2 = 1.0 / R2;
-          const double invR = xj.w * sqrt(invR2);
-          const double f = invR2 * invR;
-          pot += invR;
-          ax += dx * f;
-          ay += dy * f;
-          az += dz * f;
-        }
-      }
+  const int nb = (tn + kP2P64TC - 1) / kP2P64TC;
+  const int per = (tn + nb - 1) / max(nb, 1);
+  for (int t0 = w * per; t0 < tn; t0 += kP2PWaves * per) {
+    const int tc = min(per, tn - t0);
+#define XF_P2P64_BLOCK(N)                                                                          \
+  case N:                                                                                          \
+    p2p64_block<N>(t0, tc, tb, b0, nl, xs, list, scbeg, sccnt, sxs, cycle, bodies, lds[w]);        \
+    break;
+    switch (tc) {
+      XF_P2P64_BLOCK(1)
+      XF_P2P64_BLOCK(2)
+      XF_P2P64_BLOCK(3)
+      XF_P2P64_BLOCK(4)
+      XF_P2P64_BLOCK(5)
+      XF_P2P64_BLOCK(6)
+      XF_P2P64_BLOCK(7)
+      XF_P2P64_BLOCK(8)
+      default:
+        break;
     }
-    exafmm_body *o = bodies + tb + i;
-    o->p += pot;
-    o->F[0] -= ax;
-    o->F[1] -= ay;
-    o->F[2] -= az;
+#undef XF_P2P64_BLOCK
   }
 }
 
@@ -460,7 +530,7 @@ void p2p_apply(Ctx &tc, const Ctx &sc, hipStream_t s, const int *list_flags) {
   const Lists &L = tc.lists;
   const double cycle = tc.cfg.images > 0 ? tc.cfg.cycle : 0.0;
   if (tc.cfg.p2p_precision == EXAFMM_PREC_FP64) {
-    hipLaunchKernelGGL(k_p2p64, dim3(T.nleaves), dim3(64), 0, s, T.leaves.p, T.misc.p + 17, T.cbeg.p, T.ccnt.p,
+    hipLaunchKernelGGL(k_p2p64, dim3(T.nleaves), dim3(kP2PWaves * kWave), 0, s, T.leaves.p, T.misc.p + 17, T.cbeg.p, T.ccnt.p,
                        T.xs.p, L.p2p_beg.p, L.p2p_cnt.p, L.p2p.p, S.cbeg.p, S.ccnt.p, S.xs.p, cycle, tc.bodies,
                        list_flags);
   } else {
@@ -473,50 +543,85 @@ void p2p_apply(Ctx &tc, const Ctx &sc, hipStream_t s, const int *list_flags) {
 }
 
 // ---------------------------------------------------------------- direct sum
-// FP64 oracle on the device: one workgroup per target, threads stride the
-// sources, fixed-order tree reduction (deterministic).
-__global__ void __launch_bounds__(256) k_direct(exafmm_body *__restrict__ t, int64_t nt,
-                                                const exafmm_body *__restrict__ s, int64_t ns) {
-#pragma clang fp contract(off)
-  __shared__ double red[4][256];
-  const int64_t ti = blockIdx.x;
-  if (ti >= nt) return;
-  const double xi = t[ti].X[0], yi = t[ti].X[1], zi = t[ti].X[2];
-  double pot = 0, ax = 0, ay = 0, az = 0;
-  for (int64_t j = threadIdx.x; j < ns; j += 256) {
-    const double dx = xi - s[j].X[0], dy = yi - s[j].X[1], dz = zi - s[j].X[2];
-    const double R2 = dx * dx + dy * dy + dz * dz;
-    if (R2 != 0) {
-      const double invR2 = 1.0 / R2;
-      const double invR = s[j].q * sqrt(invR2);
-      const double f = invR2 * invR;
-      pot += invR;
-      ax += dx * f;
-      ay += dy * f;
-      az += dz * f;
-    }
+// FP64 direct sum.  Lanes take sources, targets are wave-uniform in blocks
+// of kDirectTC, so each loaded source serves kDirectTC interactions and the
+// per-lane sums meet across the lanes once per wave.  The sources are cut
+// into shares; the four waves of a workgroup take four target blocks against
+// the same share (its lines then come from L2 once), or, with fewer than
+// four blocks, quarters of the share.  Each (share, target) partial is
+// stored and k_direct_sum adds a target's partials in a fixed order.  FP64
+// VALU bound.  1,000 targets x 2^20 sources: 0.85 ms; 2.83 ms with a workgroup
+// per target (every target streaming all sources, a divide and a root each).
+constexpr int kDirectTC = 8;
+constexpr int kDirectWaves = 4;
+constexpr int kDirectGroups = 2048;  // workgroups aimed at: eight per CU
+
+__global__ void __launch_bounds__(kDirectWaves *kWave) k_direct(const exafmm_body *__restrict__ t, int64_t nt,
+                                                                const exafmm_body *__restrict__ s, int64_t ns,
+                                                                int wt, double *__restrict__ part) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int ws = kDirectWaves / wt;  // waves that share a target block
+  const int64_t t0 = (int64_t(blockIdx.x) * wt + w % wt) * kDirectTC;
+  if (t0 >= nt) return;
+  const int64_t share = int64_t(blockIdx.y) * ws + w / wt, shares = int64_t(gridDim.y) * ws;
+  const int64_t s0 = share * ns / shares, s1 = (share + 1) * ns / shares;
+  const int tc = int(min(int64_t(kDirectTC), nt - t0));
+  double xt[kDirectTC], yt[kDirectTC], zt[kDirectTC], ap[kDirectTC], ax[kDirectTC], ay[kDirectTC], az[kDirectTC];
+#pragma unroll
+  for (int i = 0; i < kDirectTC; i++) {
+    const exafmm_body *b = t + t0 + min(i, tc - 1);
+    xt[i] = b->X[0];
+    yt[i] = b->X[1];
+    zt[i] = b->X[2];
+    ap[i] = ax[i] = ay[i] = az[i] = 0.0;
   }
-  red[0][threadIdx.x] = pot;
-  red[1][threadIdx.x] = ax;
-  red[2][threadIdx.x] = ay;
-  red[3][threadIdx.x] = az;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o)
-      for (int k = 0; k < 4; k++) red[k][threadIdx.x] += red[k][threadIdx.x + o];
-    __syncthreads();
+  for (int64_t j = s0 + lane; j < s1; j += kWave) {
+    const double sx = s[j].X[0], sy = s[j].X[1], sz = s[j].X[2], q = s[j].q;
+#pragma unroll
+    for (int i = 0; i < kDirectTC; i++) p2p64_pair(xt[i] - sx, yt[i] - sy, zt[i] - sz, q, ap[i], ax[i], ay[i], az[i]);
   }
-  if (threadIdx.x == 0) {
-    t[ti].p += red[0][0];
-    t[ti].F[0] -= red[1][0];
-    t[ti].F[1] -= red[2][0];
-    t[ti].F[2] -= red[3][0];
-  }
+  constexpr int kLow = kWave / kDirectTC;
+  const int i = lane / kLow, comp = lane % kLow;
+  const double v = p2p_lane_total<kDirectTC>(ap, ax, ay, az, lane);
+  if (comp < 4 && i < tc) part[(share * nt + t0 + i) * 4 + comp] = v;
 }
 
-void direct_sum(int, hipStream_t st, exafmm_body *t, int64_t nt, const exafmm_body *s, int64_t ns) {
+// One wave per target: lane (h, comp) = (lane / 4, lane % 4) adds the shares
+// h, h + 16, ..., then the 16 lanes of a component are added by halving.
+__global__ void __launch_bounds__(256) k_direct_sum(exafmm_body *__restrict__ t, int64_t nt, int64_t shares,
+                                                    const double *__restrict__ part) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t i = int64_t(blockIdx.x) * (256 / kWave) + threadIdx.x / kWave;
+  if (i >= nt) return;  // whole wave
+  const int comp = lane & 3;
+  double v = 0.0;
+  for (int64_t h = lane >> 2; h < shares; h += kWave / 4) v += part[(h * nt + i) * 4 + comp];
+#pragma unroll
+  for (int m = 4; m < kWave; m <<= 1) v += __shfl_xor(v, m);
+  if (lane >= 4) return;
+  if (comp == 0)
+    t[i].p += v;
+  else
+    t[i].F[comp - 1] -= v;
+}
+
+void direct_sum(Ctx &c, exafmm_body *t, int64_t nt, const exafmm_body *s, int64_t ns) {
   if (nt <= 0 || ns <= 0) return;
-  hipLaunchKernelGGL(k_direct, dim3(nt), dim3(256), 0, st, t, nt, s, ns);
+  const int64_t blocks = (nt + kDirectTC - 1) / kDirectTC;
+  const int wt = blocks >= 4 ? 4 : blocks >= 2 ? 2 : 1;
+  const int64_t groups = (blocks + wt - 1) / wt;
+  // shares of at least two source rounds per wave, about kDirectGroups workgroups in all
+  const int ws = kDirectWaves / wt;
+  const int64_t gy = std::max<int64_t>(
+      1, std::min<int64_t>((kDirectGroups + groups - 1) / groups, ns / (int64_t(2) * kWave * ws)));
+  const int64_t shares = gy * ws;
+  c.direct_part.ensure(size_t(shares) * nt * 4);
+  hipLaunchKernelGGL(k_direct, dim3(unsigned(groups), unsigned(gy)), dim3(kDirectWaves * kWave), 0, c.s0, t, nt, s, ns,
+                     wt, c.direct_part.p);
+  XF_LAUNCH();
+  hipLaunchKernelGGL(k_direct_sum, dim3(ceil_div(nt, 256 / kWave)), dim3(256), 0, c.s0, t, nt, shares,
+                     c.direct_part.p);
   XF_LAUNCH();
 }
 
