@@ -271,6 +271,7 @@ struct Ctx {
   bool capturing = false;
   int graph_locks = 0;
   Buf<double> shift_T;             // scaled M2M / L2L operators per octant
+  Buf<double> ewald_waves;         // Ewald sum: wave vectors and their structure factors
   Buf<double> direct_part;         // direct sum: partial sums [source share][target][4]
   Buf<double> dipole_part;         // dipole moment: per-workgroup partials, then the sum
   int shift_P = -1;
@@ -406,6 +407,32 @@ void scan_exclusive3(const int *in0, const int *in1, const int *in2, int *out0, 
                      int *running, const int64_t *cap, int *flag, Buf<int> &scratch, hipStream_t s);
 void radix_sort_pairs(unsigned long long *&k, int *&v, unsigned long long *&k2, int *&v2, int n, int lo_bit,
                       int hi_bit, Buf<int> &hist, hipStream_t s);
+
+// ------------------------------------------------------------------ cross-lane sums
+// Sum over the 64 lanes of TC per-lane values by recursive halving: at each
+// step a lane keeps one half of its values and sends the other half to its
+// partner (TC - 1 shuffles instead of 6 TC).  Afterwards lane l holds the
+// partial sum of value l >> (6 - log2 TC) over the lanes that share its low
+// bits; the caller finishes with a butterfly over those bits.
+template <int TC, class T>
+__device__ inline T halving(T (&v)[TC], int lane) {
+  int c = TC;
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    if (c > 1) {
+      const bool up = lane & m;
+#pragma unroll
+      for (int i = 0; i < TC / 2; i++) {
+        if (i < c / 2) {
+          const T lo = v[i], hi = v[i + c / 2];
+          v[i] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, m);
+        }
+      }
+      c >>= 1;
+    }
+  }
+  return v[0];
+}
 
 }  // namespace xf
 

@@ -53,31 +53,6 @@ __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-// Sum over the 64 lanes of TC per-lane values by recursive halving: at each
-// step a lane keeps one half of its values and sends the other half to its
-// partner (TC - 1 shuffles instead of 6 TC).  Afterwards lane l holds the
-// partial sum of value l >> (6 - log2 TC) over the lanes that share its low
-// bits; the caller finishes with a butterfly over those bits.
-template <int TC, class T>
-__device__ inline T halving(T (&v)[TC], int lane) {
-  int c = TC;
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    if (c > 1) {
-      const bool up = lane & m;
-#pragma unroll
-      for (int i = 0; i < TC / 2; i++) {
-        if (i < c / 2) {
-          const T lo = v[i], hi = v[i + c / 2];
-          v[i] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, m);
-        }
-      }
-      c >>= 1;
-    }
-  }
-  return v[0];
-}
-
 template <int N>
 constexpr int pow2ceil() {
   return N <= 1 ? 1 : 2 * pow2ceil<(N + 1) / 2>();
