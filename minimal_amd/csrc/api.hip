@@ -1175,7 +1175,7 @@ int exafmm_graph_gemm_shapes(exafmm_graph *g, int32_t *shapes, int capacity, int
       if (k < capacity) {
         shapes[3 * k] = pl->P;
         shapes[3 * k + 1] = pl->rtb * 16;
-        shapes[3 * k + 2] = pl->kr;
+        shapes[3 * k + 2] = std::max(1, pl->kr / ceil_div(pl->P * pl->P, 32));  // a key has P^2 / 32 units
       }
       k++;
     }

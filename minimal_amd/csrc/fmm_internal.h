@@ -286,7 +286,7 @@ struct Ctx {
   bool m2l_ready = false;
   int m2l_ntiles = 0;
   int m2l_tstride = 0;      // stride of the tile arrays in `tiles` (a bound on the tile count)
-  int m2l_tn = 512;         // targets per M2L tile (512 or 256)
+  bool m2l_by_level = false;  // each tile holds cells of one level
   int m2l_ncell_tiled = 0;  // cells that receive M2L (the tiles' columns)
   Buf<int> m2l_misc, m2l_rs_hist, m2l_scan;
   Buf<double> m2l_part64;   // FP64 partial locals of the list shares (m2l.hip)
@@ -317,6 +317,7 @@ struct Ctx {
   Buf<int> tiles;                  // M2L tile descriptors
   Buf<int> tile_mat;               // per tile [U][kTileN] source indices
   Buf<int> tile_keys;
+  Buf<unsigned long long> tile_mask;  // per (tile, key) slot: column subtiles that hold a pair (m2l_mfma.hip)
   Buf<unsigned> tile_bits;         // per tile: bitmap of its key set (k_tile_count -> k_tile_fill)
   Buf<int> misc;
   // periodic far images
@@ -362,8 +363,9 @@ void p2p_grouped(const GroupTree *g, const int *start, int nprob, int nblocks, h
 // keyed M2L of every problem of one order (BF16x3, fixed order): cast +
 // GEMM, one launch each; the plan holds the device descriptor tables
 struct GemmGroupPlan {
-  int P = 0, rtb = 0, kr = 1, nprob = 0, nblocks = 0, cast_blocks = 0, tn = 512;
+  int P = 0, rtb = 0, kr = 1, nprob = 0, ntiles = 0, groups = 0, cast_blocks = 0;
   size_t lds = 0;
+  Buf<float> seg;  // FP32 partial tiles of the stream-K segments
   Buf<char> desc, cast_desc;
   Buf<int> start, cast_start;
   struct Trial {

@@ -10,12 +10,13 @@
 // per expansion: Re M_n^0, Re/Im M_n^m for m > 0) T is a dense P^2 x P^2
 // matrix, generated once per distinct key in FP64.
 //
-// Targets are grouped in tiles of 256 cells of one level and one octant
-// position (cells with the same position relative to their parent have the
-// same key set away from the domain boundary).  For each key in a tile's
-// key union the 256 source columns are gathered and multiplied by the key's
-// operator; all keys of a tile accumulate into the same MFMA accumulators,
-// so each target's L is written once, without atomics, in a fixed order.
+// Targets are grouped in tiles of 512 cells of one octant position (cells
+// with the same position relative to their parent have the same key set away
+// from the domain boundary and from changes of depth, whatever their level).
+// For each key in a tile's key union the source columns are gathered and
+// multiplied by the key's operator; all keys of a tile accumulate into the
+// same MFMA accumulators, so each target's L is written once, without
+// atomics, in a fixed order.
 //
 // Precision: FP32 uses v_mfma_f32_16x16x4_f32.  BF16X3 splits operator and
 // multipoles into bf16 hi + lo parts and forms hi*hi + hi*lo + lo*hi with
@@ -31,14 +32,24 @@
 namespace xf {
 using namespace xfd;
 
-// GEMM workgroup: 8 waves = column groups of 64 targets x KPAR k-parities
-// (a wave multiplies the k-steps kk = kp, kp + KPAR, ... of its columns):
-// tiles of 512 targets with one parity, 256 with two.
-constexpr int kGemmThreads = 512;
+// GEMM workgroup: 16 waves over a tile of 512 target columns.  The columns
+// form 32 subtiles of 16 (one MFMA column tile each); wave w takes subtiles w
+// and 16 + w.  Neighbouring columns have like key sets, so a key's empty
+// subtiles come in runs, and the interleaving spreads what is left over the
+// waves (they meet at a barrier every round).  Two column tiles per wave keep
+// the accumulators of nine row tiles within 128 registers: four waves per
+// SIMD hide the gathers' latency (with four column tiles and two waves per
+// SIMD they waited half their cycles).
+constexpr int kGemmThreads = 1024;
 constexpr int kGemmWaves = kGemmThreads / 64;
-template <int KPAR>
-constexpr int tile_width() {
-  return 64 * (kGemmWaves / KPAR);
+constexpr int kTileN = 512;
+constexpr int kCT = kTileN / 16 / kGemmWaves;  // column tiles per wave
+// tile column of a wave's column tile ct, lane l
+__device__ inline int tile_col(int w, int ct, int lane) { return (ct * kGemmWaves + w) * 16 + (lane & 15); }
+// Load through the scalar cache: uniform address, data written before the launch.
+template <class T>
+__device__ inline T uniform_load(const T *p) {
+  return *reinterpret_cast<const __attribute__((address_space(4))) T *>(reinterpret_cast<uintptr_t>(p));
 }
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
@@ -77,8 +88,8 @@ __device__ inline unsigned mix32(unsigned h) {
   return h;
 }
 
-// Sort key of a target cell: group (level, octant) in bits 16..23 (255 = no
-// M2L), and with `minhash` the top 16 bits of the minimum hashed key id of
+// Sort key of a target cell: group in bits 16..23 (255 = no M2L) -- the
+// octant, or (level, octant) with `by_level` -- and with `minhash` the top 16 bits of the minimum hashed key id of
 // its list below: cells with similar key sets share that minimum with a
 // probability equal to the sets' Jaccard similarity, so sorting by it packs
 // cells of like key sets into the same tile (fewer empty GEMM slots).
@@ -87,7 +98,7 @@ __device__ inline unsigned mix32(unsigned h) {
 __global__ void __launch_bounds__(256) k_group_keys(int ncells, const double4 *__restrict__ cx,
                                                     const int *__restrict__ cparent, const int *__restrict__ clevel,
                                                     const int *__restrict__ m2l_beg, const int *__restrict__ m2l_cnt,
-                                                    const int2 *__restrict__ list, int minhash, int lmin,
+                                                    const int2 *__restrict__ list, int minhash, int lmin, int by_level,
                                                     unsigned long long *__restrict__ key, int *__restrict__ val) {
   const int lane = threadIdx.x & (kWave - 1);
   const int c = blockIdx.x * (256 / kWave) + int(threadIdx.x / kWave);
@@ -102,7 +113,7 @@ __global__ void __launch_bounds__(256) k_group_keys(int ncells, const double4 *_
       const double4 a = cx[c], b = cx[p];
       o = (a.x > b.x) + ((a.y > b.y) << 1) + ((a.z > b.z) << 2);
     }
-    g = unsigned(min(clevel[c], 30)) * 8 + o;
+    g = (by_level ? unsigned(min(clevel[c], 30)) * 8 : 0u) + o;
     if (minhash) {
       unsigned m = 0xffffffffu;
       const int b0 = m2l_beg[c];
@@ -213,16 +224,21 @@ __global__ void __launch_bounds__(kTileCountThreads) k_tile_count(const int *__r
 // Workgroup (tile, q) owns columns 64q .. 64q + 63: it marks them empty in
 // every key row, then four threads per column walk that column's M2L list
 // (entries i = sub mod 4) and write the source cell into the key's row.
-// The key set comes from k_tile_count's bitmap.
+// The key set comes from k_tile_count's bitmap.  Byte q of a key's mask
+// (tmask, 8 bytes per slot) gets one bit per subtile of 16 columns that holds
+// a pair; a wave fills one subtile.
 __global__ void __launch_bounds__(256) k_tile_fill(const int *__restrict__ tfirst, const int *__restrict__ tcount,
                                                    const int *__restrict__ sorted, const int *__restrict__ beg,
                                                    const int *__restrict__ cnt, const int2 *__restrict__ list,
                                                    int nkeys, const int *__restrict__ tbase,
                                                    const unsigned *__restrict__ tbits, int *__restrict__ tkeys,
-                                                   int tn, int *__restrict__ tmat) {
+                                                   int *__restrict__ tmat, unsigned char *__restrict__ tmask) {
   extern __shared__ unsigned bm[];
+  constexpr int tn = kTileN;
   const int nwords = (nkeys + 31) / 32;
   unsigned *rank = bm + nwords;  // exclusive popcount prefix per word
+  unsigned *hit = rank + nwords;  // [4 subtiles][nwords]: key ranks with a pair in the subtile
+  for (int i = threadIdx.x; i < 4 * nwords; i += blockDim.x) hit[i] = 0;
   const int tile = blockIdx.x, q = blockIdx.y;
   const int *cells = sorted + tfirst[tile];
   const int ncol = tcount[tile];
@@ -285,8 +301,15 @@ __global__ void __launch_bounds__(256) k_tile_fill(const int *__restrict__ tfirs
         const unsigned w = bm[id >> 5];
         const int r = rank[id >> 5] + __popc(w & ((1u << (id & 31)) - 1u));
         tmat[(int64_t(base) + r) * tn + col] = en[k].x >> 5;  // source cell (the image is part of the key)
+        atomicOr(&hit[(threadIdx.x >> 6) * nwords + (r >> 5)], 1u << (r & 31));
       }
     }
+  }
+  __syncthreads();
+  for (int r = threadIdx.x; r < U; r += blockDim.x) {
+    unsigned m = 0;
+    for (int k = 0; k < 4; k++) m |= ((hit[k * nwords + (r >> 5)] >> (r & 31)) & 1u) << k;
+    tmask[(int64_t(base) + r) * 8 + q] = (unsigned char)m;
   }
 }
 
@@ -427,36 +450,32 @@ __global__ void __launch_bounds__(256) k_ops_gen(int P, int fillP, int R, int K4
 }
 
 // ---------------------------------------------------------------- GEMM
-// One workgroup = one tile of up to tile_width<KPAR>() targets and a block
-// of RTB row tiles (blockIdx.y).  8 waves = 8 / KPAR column groups (64
-// targets = 4 column tiles of 16) x KPAR k-parities: wave (g, kp) multiplies
-// the k-steps kk = kp, kp + KPAR, ... of every key for its 64 targets and all
-// RTB row tiles, so each source multipole is fetched once per tile; two
-// parities are added through LDS at the end.  With one parity the tile is
-// 512 targets wide, so each staged operator serves twice the targets (the
-// operator staging is most of the GEMM's fetch).  Per key the block's operator rows are copied
-// global -> LDS (global_load_lds, no register round trip) into the second
-// of two buffers while the first is multiplied; one wait + barrier per key.
-// Each lane's source multipoles for its next k-step are loaded while the
-// current one is multiplied.  All keys of a tile accumulate into the same
-// MFMA accumulators, so each target's L is written once, without atomics.
-constexpr int kGemmMaxRT = 8;  // row tiles per wave (accumulator registers)
+// One workgroup = one tile of up to 512 targets and a block of RTB row
+// tiles (blockIdx.y); a wave holds the accumulators of its column tiles
+// and all RTB row tiles, so each source multipole is fetched once per tile and
+// row block.  The operators are staged global -> LDS (global_load_lds, no
+// register round trip) in rounds, the next round while the current one is
+// multiplied, with one wait and barrier per round; a wave loads its next
+// k-step's source multipoles as soon as it has issued the current one's
+// products.
+constexpr int kGemmMaxRT = 9;     // row tiles per wave (8 accumulator registers each)
+constexpr int kGemmMaxRTF32 = 8;  // the FP32 kernel's
 
 template <int RH>
-__device__ inline void write_locals(int PP, int rbase, int nr, const int *cells, int ncol, int cg,
-                                    const v4f (&acc)[RH][4], int lane, double *L) {
+__device__ inline void write_locals(int PP, int rbase, int nr, const int *cells, int ncol, int w,
+                                    const v4f (&acc)[RH][kCT], int lane, double *L) {
 #pragma unroll
-  for (int ct = 0; ct < 4; ct++) {
-    const int col = cg * 64 + ct * 16 + (lane & 15);
+  for (int ct = 0; ct < kCT; ct++) {
+    const int col = tile_col(w, ct, lane);
     if (col >= ncol) continue;
     double *Lc = L + int64_t(cells[col]) * PP;
 #pragma unroll
     for (int r = 0; r < RH; r++) {
-      if (r >= nr) break;  // row tiles of this block only (another block owns the next ones)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const int row = (rbase + r) * 16 + 4 * (lane >> 4) + i;
-        if (row < PP) Lc[row] += double(acc[r][ct][i]);
+        // row tiles of this block only (another block owns the next ones)
+        if (r < nr && row < PP) Lc[row] += double(acc[r][ct][i]);
       }
     }
   }
@@ -465,20 +484,22 @@ __device__ inline void write_locals(int PP, int rbase, int nr, const int *cells,
 // Split-key variant: this workgroup's share of the locals, stored (each
 // (cell, row) of a tile belongs to one workgroup per key slice).
 template <int RH>
-__device__ inline void write_partial(int PP, int rbase, int nr, const int *cells, int ncol, int cg,
-                                     const v4f (&acc)[RH][4], int lane, float *Lp) {
+__device__ inline void write_partial(int PP, int rbase, int nr, const int *cells, int ncol, int w,
+                                     const v4f (&acc)[RH][kCT], int lane, float *Lp) {
+  // opaque: the row tests and offsets below are then computed here, not hoisted
+  // out of a stream-K workgroup's segment loop into registers it lacks
+  asm volatile("" : "+s"(PP), "+v"(lane));
 #pragma unroll
-  for (int ct = 0; ct < 4; ct++) {
-    const int col = cg * 64 + ct * 16 + (lane & 15);
+  for (int ct = 0; ct < kCT; ct++) {
+    const int col = tile_col(w, ct, lane);
     if (col >= ncol) continue;
     float *Lc = Lp + int64_t(cells ? cells[col] : col) * PP;
 #pragma unroll
     for (int r = 0; r < RH; r++) {
-      if (r >= nr) break;
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const int row = (rbase + r) * 16 + 4 * (lane >> 4) + i;
-        if (row < PP) Lc[row] = acc[r][ct][i];
+        if (r < nr && row < PP) Lc[row] = acc[r][ct][i];
       }
     }
   }
@@ -495,32 +516,10 @@ __global__ void k_combine_slices(int PP, int64_t ncells, int nslice, const int *
   L[int64_t(c) * PP + r] += s;
 }
 
-// Parity 1 hands its accumulators to parity 0 through LDS (the operator
-// buffers are free by then); parity 0 adds them and writes the locals.
-template <int RH, int KPAR>
-__device__ inline void reduce_parities(v4f (&acc)[RH][4], int kp, int cg, int lane, void *lds) {
-  if (KPAR == 1) return;  // one wave per column group: nothing to add
-  v4f *red = reinterpret_cast<v4f *>(lds);
-  __syncthreads();
-  if (kp == 1) {
-#pragma unroll
-    for (int r = 0; r < RH; r++)
-#pragma unroll
-      for (int ct = 0; ct < 4; ct++) red[((cg * RH + r) * 4 + ct) * 64 + lane] = acc[r][ct];
-  }
-  __syncthreads();
-  if (kp == 0) {
-#pragma unroll
-    for (int r = 0; r < RH; r++)
-#pragma unroll
-      for (int ct = 0; ct < 4; ct++) acc[r][ct] += red[((cg * RH + r) * 4 + ct) * 64 + lane];
-  }
-}
-
 // s_waitcnt immediates (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt
 // 6:4, lgkmcnt 11:8) that wait for vmcnt <= N and nothing else.
 constexpr int waitcnt_vm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
-constexpr int kWaitVm0 = waitcnt_vm(0), kWaitVm4 = waitcnt_vm(4), kWaitVm8 = waitcnt_vm(8);
+constexpr int kWaitVm0 = waitcnt_vm(0);
 
 // Row of the full operator layout [kk][row tile][lane] for run c of a
 // block's staged copy (c = kk * nrt + local row tile).
@@ -529,7 +528,7 @@ __device__ inline int op_run(int c, int nrt, int RT, int rt0) {
   return kk * RT + rt0 + rl;
 }
 
-template <int RH, int KPAR>
+template <int RH>
 __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RTB, int K4, int KP,
                                                           const int *__restrict__ tfirst,
                                                           const int *__restrict__ tcount,
@@ -543,11 +542,10 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RT
                                                           int64_t ncells, float *__restrict__ Lpart,
                                                           double *__restrict__ L) {
   extern __shared__ float As[];
-  constexpr int TN = tile_width<KPAR>(), NG = kGemmWaves / KPAR, PARTS = TN / 64;
+  constexpr int TN = kTileN;
   // wave index read through a scalar register: the k-step and key loops
   // below then branch uniformly instead of under execution masks
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int cg = w % NG, kp = w / NG;
   const int tile = blockIdx.x;
   const int ncol = tcount[tile];
   // keys of this workgroup: slice blockIdx.z of gridDim.z of the tile's keys
@@ -557,11 +555,11 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RT
   const int rt0 = blockIdx.y * RTB;
   const int nrt = min(RTB, RT - rt0);
   const int kq = lane >> 4;
-  v4f acc[RH][4];
+  v4f acc[RH][kCT];
 #pragma unroll
   for (int r = 0; r < RH; r++)
 #pragma unroll
-    for (int ct = 0; ct < 4; ct++) acc[r][ct] = v4f{0, 0, 0, 0};
+    for (int ct = 0; ct < kCT; ct++) acc[r][ct] = v4f{0, 0, 0, 0};
   const int64_t per = int64_t(K4) * RT * 64;
   const int NC = K4 * nrt;  // runs of 64 floats per staged block
   const int BUF = NC * 64;  // floats per LDS buffer
@@ -588,34 +586,34 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RT
     };
     auto stage_src = [&](int r) {
       const int nu = min(kr, U - r * kr);
-      for (int j = w; j < PARTS * nu; j += kGemmWaves) {
-        const int ui = j / PARTS, q = j % PARTS;
+      for (int j = w; j < TN / 64 * nu; j += kGemmWaves) {
+        const int ui = j / (TN / 64), q = j % (TN / 64);
         __builtin_amdgcn_global_load_lds(tmat + (int64_t(base) + r * kr + ui) * TN + q * 64 + lane,
                                          Ts + ((r % 3) * kr + ui) * TN + q * 64, 4, 0, 0);
       }
     };
-    auto col_src = [&](int u, int (&sc)[4]) {
-      const int *T = Ts + (((u / kr) % 3) * kr + u % kr) * TN + cg * 64 + (lane & 15);
+    auto col_src = [&](int u, int (&sc)[kCT]) {
+      const int *T = Ts + (((u / kr) % 3) * kr + u % kr) * TN;
 #pragma unroll
-      for (int ct = 0; ct < 4; ct++) sc[ct] = T[ct * 16];
+      for (int ct = 0; ct < kCT; ct++) sc[ct] = T[tile_col(w, ct, lane)];
     };
     // empty slots and k at or past the key's K bound read the zero row
     // (index ncells): unconditional loads stay in flight until used
-    auto load_b = [&](const int (&sc)[4], int kk, int kc, float (&bv)[4]) {
+    auto load_b = [&](const int (&sc)[kCT], int kk, int kc, float (&bv)[kCT]) {
       const int k = kk * 4 + kq;
 #pragma unroll
-      for (int ct = 0; ct < 4; ct++) bv[ct] = mt[int64_t(sc[ct] >= 0 && k < kc ? sc[ct] : ncells) * KP + k];
+      for (int ct = 0; ct < kCT; ct++) bv[ct] = mt[int64_t(sc[ct] >= 0 && k < kc ? sc[ct] : ncells) * KP + k];
     };
     stage_ops(0);
     stage_src(0);
     if (R > 1) stage_src(1);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    int src[4], nsrc[4];
-    float bcur[4], bnext[4];
+    int src[kCT], nsrc[kCT];
+    float bcur[kCT], bnext[kCT];
     col_src(0, src);
     int kc = kcols(0);
-    if (kp < ksteps(kc)) load_b(src, kp, kc, bnext);
+    if (ksteps(kc) > 0) load_b(src, 0, kc, bnext);
     for (int r = 0; r < R; r++) {
       if (r + 1 < R) stage_ops(r + 1);
       if (r + 2 < R) stage_src(r + 2);
@@ -626,16 +624,16 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RT
         const float *Acur = As + size_t((r & 1) * kr + u - u0) * BUF;
         const int ks = ksteps(kc), nr = rtiles(kc);
         const int kc_next = u + 1 < U ? kcols(u + 1) : 0;
-        const bool next = u + 1 < U && kp < ksteps(kc_next);
+        const bool next = u + 1 < U && ksteps(kc_next) > 0;
         if (u + 1 < U) col_src(u + 1, nsrc);
-        for (int kk = kp; kk < ks; kk += KPAR) {
+        for (int kk = 0; kk < ks; kk++) {
 #pragma unroll
-          for (int ct = 0; ct < 4; ct++) bcur[ct] = bnext[ct];
-          if (kk + KPAR < ks) {
-            load_b(src, kk + KPAR, kc, bnext);
+          for (int ct = 0; ct < kCT; ct++) bcur[ct] = bnext[ct];
+          if (kk + 1 < ks) {
+            load_b(src, kk + 1, kc, bnext);
             b_after = true;
           } else if (next) {
-            load_b(nsrc, kp, kc_next, bnext);
+            load_b(nsrc, 0, kc_next, bnext);
             b_after = true;
           }
 #pragma unroll
@@ -643,22 +641,22 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RT
             if (r2 >= nr) break;
             const float a = Acur[(kk * nrt + r2) * 64 + lane];
 #pragma unroll
-            for (int ct = 0; ct < 4; ct++)
+            for (int ct = 0; ct < kCT; ct++)
               acc[r2][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bcur[ct], acc[r2][ct], 0, 0, 0);
           }
         }
-        if (ks <= kp && next) {
-          load_b(nsrc, kp, kc_next, bnext);
+        if (ks <= 0 && next) {
+          load_b(nsrc, 0, kc_next, bnext);
           b_after = true;
         }
 #pragma unroll
-        for (int ct = 0; ct < 4; ct++) src[ct] = nsrc[ct];
+        for (int ct = 0; ct < kCT; ct++) src[ct] = nsrc[ct];
         kc = kc_next;
       }
-      // staging of this round's start landed (only the 4 loads of the last
+      // staging of this round's start landed (only the kCT loads of the last
       // B prefetch are younger); then every wave is done with this round
       if (b_after)
-        __builtin_amdgcn_s_waitcnt(kWaitVm4);
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(kCT));
       else
         __builtin_amdgcn_s_waitcnt(kWaitVm0);
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -667,19 +665,12 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RT
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  reduce_parities<RH, KPAR>(acc, kp, cg, lane, As);
-  if (kp == 0) {
-    if (Lpart)
-      write_partial<RH>(PP, rt0, nrt, sorted + tfirst[tile], ncol, cg, acc, lane,
-                        Lpart + int64_t(blockIdx.z) * ncells * PP);
-    else
-      write_locals<RH>(PP, rt0, nrt, sorted + tfirst[tile], ncol, cg, acc, lane, L);
-  }
+  if (Lpart)
+    write_partial<RH>(PP, rt0, nrt, sorted + tfirst[tile], ncol, w, acc, lane, Lpart + int64_t(blockIdx.z) * ncells * PP);
+  else
+    write_locals<RH>(PP, rt0, nrt, sorted + tfirst[tile], ncol, w, acc, lane, L);
 }
 
-// Keys ub .. ue - 1 of tile bx, row block by.  Output: added into the FP64
-// locals L (Lpart null), or stored as FP32 partial locals, by cell
-// (Lpart + cell * PP, part_local false) or by tile column (Lpart + col * PP).
 // Order of one GEMM launch: pl (k bound pl^2 of every key, unless the
 // per-slot orders tkp are given), the row tiles RTo and k-steps K32o it
 // covers (of the RT x K32 of the operator layout, which holds order
@@ -690,113 +681,158 @@ struct OrderPass {
   const int *perm;
 };
 
-template <int RH, bool SKIP, int KPAR>
-__device__ __attribute__((always_inline)) inline void m2l_bf16x3_body(int bx, int by, int ub, int ue, bool part_local,
-                                       int PP, int RT, int RTB, int K32, int KP, OrderPass op,
-                                       const int *__restrict__ tfirst,
-                                       const int *__restrict__ tcount,
-                                       const int *__restrict__ tbase,
-                                       const int *__restrict__ tU,
-                                       const int *__restrict__ sorted,
-                                       const int *__restrict__ tkeys,
-                                       const int *__restrict__ tmat,
-                                       const v8bf *__restrict__ ophi,
-                                       const v8bf *__restrict__ oplo,
-                                       const __bf16 *__restrict__ mhi,
-                                       const __bf16 *__restrict__ mlo,
-                                       const unsigned char *__restrict__ tkp, int kr,
-                                       int64_t ncells, float *__restrict__ Lpart,
-                                       double *__restrict__ L) {
+// What a BF16x3 GEMM launch reads of one tree: tiles and their keys, sources
+// and subtile masks, operators, cast multipoles.
+struct GemmIn {
+  const int *tfirst, *tcount, *tU, *sorted, *tkeys, *tmat;
+  const unsigned long long *tmask;
+  const v8bf *ophi, *oplo;
+  const __bf16 *mhi, *mlo;
+  int64_t ncells;
+};
+
+// The k-steps of the tile's keys form one sequence of units (key u, k-step
+// kk).  A round is G units (two LDS buffers of G units: a whole key need not
+// fit, a small one takes a fraction of a round); at its start the next
+// round's operators are staged into the other buffer, and the tile-matrix
+// rows of the keys up to kGemmLook past them into a ring, so a wave finds its
+// next key's sources in LDS.
+//
+// A key's subtile masks (tile fill) tell each wave, a block of 64 keys at a
+// time, which keys hold a pair in its columns: the wave skips the others
+// outright and the empty column tiles of the rest, and loads the multipoles
+// of its next non-empty key ahead.  Clustered trees leave most subtiles of a
+// tile's key union empty (200,000 bodies, 90% of them in a Plummer sphere:
+// 56% with 16 columns, 87% with the whole tile).
+//
+// What bounds it: the waits for gathered multipoles and staged operators
+// (MFMA busy a third to a half of the time; the fetch stays near 2 TB/s).
+// Against eight waves of four contiguous column tiles each, whole keys per
+// round, every column multiplied: 1.5M clustered bodies, order 12: 7.1 -> 3.8
+// ms; 10,000 uniform bodies, order 10: 101 -> 37 us; 2^20 uniform: 0.70 -> 0.62
+// ms; 12 problems of a batch graph: 6.5 -> 0.83 ms (with the stream-K launch).
+//
+// The body runs slots first .. first + U - 1 of a tile, row block `by`.
+// Output: added into the FP64 locals L (Lpart null), or stored as FP32
+// partial locals, by cell (Lpart + cell * PP, part_local false) or by tile
+// column (Lpart + col * PP).
+//
+// VAR: learned orders (slot permutation, an order and so K bound and row
+// tiles per slot).  Without it every key has the order op.pl of the operators
+// and all RH row tiles are multiplied (those past a shorter last row block
+// read staged bytes of other rows and are not written).
+constexpr int kGemmLook = 4;
+template <int RH, bool VAR>
+__device__ __attribute__((always_inline)) inline void m2l_bf16x3_body(const GemmIn &g, int tile, int by, int first,
+                                                                      int U, bool part_local, int PP, int RT, int RTB,
+                                                                      int K32, int KP, OrderPass op,
+                                                                      const unsigned char *__restrict__ tkp, int G,
+                                                                      int ring, float *__restrict__ Lpart,
+                                                                      double *__restrict__ L) {
   extern __shared__ v8bf Ab[];
-  constexpr int TN = tile_width<KPAR>(), NG = kGemmWaves / KPAR, PARTS = TN / 64;
-  // wave index read through a scalar register: the k-step and key loops
-  // below then branch uniformly instead of under execution masks
+  constexpr int TN = kTileN;
+  // wave index read through a scalar register: the unit loop below then
+  // branches uniformly instead of under execution masks
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int cg = w % NG, kp = w / NG;
-  const int tile = bx;
-  const int ncol = tcount[tile];
-  // column subtiles of 16 that hold target cells (with SKIP, a partly
-  // filled tile skips the MFMAs of its empty subtiles, whose B operands are
-  // the zero row)
-  const int nct = max(0, min(4, (ncol - cg * 64 + 15) / 16));
-  const int U = ue - ub, base = tbase[tile] + ub;
+  const int ncol = g.tcount[tile];
   // a tile without keys in this launch adds nothing to the locals
   if (U <= 0 && !Lpart) return;
   const int rt0 = by * RTB;
   const int nrt = min(RTB, op.RTo - rt0);
   const int kq = lane >> 4;
-  v4f acc[RH][4];
+  v4f acc[RH][kCT];
 #pragma unroll
   for (int r = 0; r < RH; r++)
 #pragma unroll
-    for (int ct = 0; ct < 4; ct++) acc[r][ct] = v4f{0, 0, 0, 0};
+    for (int ct = 0; ct < kCT; ct++) acc[r][ct] = v4f{0, 0, 0, 0};
   const int64_t per = int64_t(K32) * RT * 64;  // v8bf per key and part
-  const int NC = op.K32o * nrt;                // runs of 64 v8bf per staged part
-  const int E = NC * 64;                       // v8bf per staged part
-  auto slot = [&](int u) { return op.perm ? op.perm[base + u] : base + u; };
+  const int KS = op.K32o;                      // units per key
+  const int UE = nrt * 128;                    // v8bf per staged unit: hi rows, lo rows
+  auto slot = [&](int u) { return VAR && op.perm ? uniform_load(op.perm + first + u) : first + u; };
   // order of key u (tkp: per-key orders of a variable-order evaluation):
   // k-steps and row tiles of this block that it needs, and its K bound
-  auto kcols = [&](int u) { const int p = tkp ? tkp[slot(u)] : op.pl; return p * p; };
-  // a K bound below the operator's order can fall inside a k-group
-  const bool varK = tkp || op.pl * op.pl < PP;
-  auto ksteps = [&](int kc) { return (kc + 31) / 32; };
-  auto rtiles = [&](int kc) { return max(0, min(nrt, (kc + 15) / 16 - rt0)); };
+  auto kcols = [&](int u) {
+    const int p = VAR && tkp ? int(uniform_load(tkp + slot(u))) : op.pl;
+    return p * p;
+  };
+  auto ksteps = [&](int kc) { return VAR ? (kc + 31) / 32 : KS; };
+  auto rtiles = [&](int kc) { return VAR ? max(0, min(nrt, (kc + 15) / 16 - rt0)) : nrt; };
   if (U > 0) {
-    // LDS: operator slots [2 buffers][kr keys][hi, lo][E], then the keys'
-    // column sources (tile matrix rows) [3 buffers][kr keys][TN].  Round r
-    // (keys r kr .. r kr + kr - 1) reads operator buffer r & 1 and source
-    // buffer r % 3; at its start it stages round r + 1's operators and round
-    // r + 2's sources, so the sources of the next round's first key are
-    // already in LDS while this round still runs.
-    int *Ts = reinterpret_cast<int *>(Ab + size_t(4) * kr * E);
-    const int R = (U + kr - 1) / kr;
+    int *Ts = reinterpret_cast<int *>(Ab + size_t(2) * G * UE);
+    const int N = U * KS, R = (N + G - 1) / G;
+    int su = 0, sk = 0;  // the next unit to stage
     auto stage_ops = [&](int r) {
-      for (int u = r * kr; u < min(r * kr + kr, U); u++) {
-        v8bf *dst = Ab + size_t((r & 1) * kr + u - r * kr) * 2 * E;
-        const int kc = kcols(u), ks = ksteps(kc), nr = rtiles(kc);
-        const int64_t k = tkeys[slot(u)];
-        const int n1 = ks * nr;
-        for (int j = w; j < 2 * n1; j += kGemmWaves) {
-          const int part = j >= n1, jj = part ? j - n1 : j;
-          const int kk = jj / nr, rl = jj - kk * nr, cc = kk * nrt + rl;
-          const v8bf *A = (part ? oplo : ophi) + k * per;
-          __builtin_amdgcn_global_load_lds(A + int64_t(op_run(cc, nrt, RT, rt0)) * 64 + lane,
-                                           dst + part * E + cc * 64, 16, 0, 0);
+      const int n = min(G, N - r * G);
+      int off = 0;
+      for (int i = 0; i < n; i++) {
+        const int kc = kcols(su);
+        if (sk < ksteps(kc)) {
+          const int nr = rtiles(kc);
+          const int64_t o = int64_t(uniform_load(g.tkeys + slot(su))) * per + int64_t(sk * RT + rt0) * 64;
+          v8bf *dst = Ab + size_t((r & 1) * G + i) * UE;
+          for (int q = (w - off) & (kGemmWaves - 1); q < 2 * nr; q += kGemmWaves) {
+            const int part = q >= nr, rl = part ? q - nr : q;
+            __builtin_amdgcn_global_load_lds((part ? g.oplo : g.ophi) + o + rl * 64 + lane,
+                                             dst + (part * nrt + rl) * 64, 16, 0, 0);
+          }
+          off += 2 * nr;
+        }
+        if (++sk == KS) {
+          sk = 0;
+          su++;
         }
       }
     };
-    auto stage_src = [&](int r) {
-      const int nu = min(kr, U - r * kr);
-      for (int j = w; j < PARTS * nu; j += kGemmWaves) {
-        const int ui = j / PARTS, q = j % PARTS;
-        __builtin_amdgcn_global_load_lds(tmat + int64_t(slot(r * kr + ui)) * TN + q * 64 + lane,
-                                         Ts + ((r % 3) * kr + ui) * TN + q * 64, 4, 0, 0);
+    // rows of keys a .. b - 1 into the ring (eight waves per key, 64 columns each)
+    auto stage_rows = [&](int a, int b) {
+      constexpr int kRuns = TN / 64;
+      const int q = w % kRuns;
+      for (int u = a + w / kRuns; u < b; u += kGemmWaves / kRuns)
+        __builtin_amdgcn_global_load_lds(g.tmat + int64_t(slot(u)) * TN + q * 64 + lane,
+                                         Ts + (u & (ring - 1)) * TN + q * 64, 4, 0, 0);
+    };
+    // keys whose rows are wanted once the units before (su, sk) are staged
+    auto row_end = [&]() { return min(U, su + (sk > 0) + kGemmLook); };
+    // bit ct of key 64 b + lane: this wave's column tile ct holds a pair
+    auto load_masks = [&](int b) {
+      const int u = b * 64 + lane;
+      const unsigned long long m =
+          (u < U ? g.tmask[VAR && op.perm ? op.perm[first + u] : first + u] : 0ull) >> (8 * (w >> 2) + (w & 3));
+      static_assert(kCT == 2 && kGemmWaves == 16, "bits w and 32 + w of a mask");
+      return int((m & 1) | ((m >> 31) & 2));
+    };
+    // This lane's first element of its columns' source rows, in 16-byte
+    // units (KP is a multiple of 8); empty slots read the zero row (index
+    // ncells), so every load is unconditional and stays in flight until its
+    // k-step: masking at load time would make the wave wait for the data.
+    const unsigned row8 = unsigned(KP) / 8, zero8 = unsigned(g.ncells) * row8;
+    auto col_src = [&](int u, unsigned (&sc)[kCT]) {
+      const int *T = Ts + (u & (ring - 1)) * TN;
+#pragma unroll
+      for (int ct = 0; ct < kCT; ct++) {
+        const int c = T[tile_col(w, ct, lane)];
+        sc[ct] = (c >= 0 ? unsigned(c) * row8 : zero8) + kq;
       }
     };
-    auto col_src = [&](int u, int (&sc)[4]) {
-      const int *T = Ts + (((u / kr) % 3) * kr + u % kr) * TN + cg * 64 + (lane & 15);
+    // k-groups at or past the key's K bound (the last k-step's) read the zero
+    // row; the one vector that straddles a variable order's bound is masked
+    // when it is used (mask_b)
+    auto load_b = [&](const unsigned (&sc)[kCT], int kk, int kc, v8bf (&bh)[kCT], v8bf (&bl)[kCT]) {
+      const v8bf *ph = reinterpret_cast<const v8bf *>(g.mhi) + kk * 4;
+      const v8bf *pl = reinterpret_cast<const v8bf *>(g.mlo) + kk * 4;
+      const bool in = kk * 32 + kq * 8 < kc;
 #pragma unroll
-      for (int ct = 0; ct < 4; ct++) sc[ct] = T[ct * 16];
-    };
-    // Empty slots and k-groups at or past the key's K bound read the zero
-    // row (index ncells), so every load is unconditional and stays in
-    // flight until its k-step: masking at load time would make the wave
-    // wait for the data right away.  The one vector that straddles a
-    // variable order's bound is masked when it is used (mask_b).
-    auto load_b = [&](const int (&sc)[4], int kk, int kc, v8bf (&bh)[4], v8bf (&bl)[4]) {
-      const int k0 = kk * 32 + kq * 8;
-#pragma unroll
-      for (int ct = 0; ct < 4; ct++) {
-        const int64_t o = int64_t(sc[ct] >= 0 && k0 < kc ? sc[ct] : ncells) * KP + k0;
-        bh[ct] = *reinterpret_cast<const v8bf *>(mhi + o);
-        bl[ct] = *reinterpret_cast<const v8bf *>(mlo + o);
+      for (int ct = 0; ct < kCT; ct++) {
+        const unsigned o = in ? sc[ct] : zero8;
+        bh[ct] = ph[o];
+        bl[ct] = pl[o];
       }
     };
-    auto mask_b = [&](int kk, int kc, v8bf (&bh)[4], v8bf (&bl)[4]) {
+    auto mask_b = [&](int kk, int kc, v8bf (&bh)[kCT], v8bf (&bl)[kCT]) {
       const int k0 = kk * 32 + kq * 8;
       if (k0 >= kc || k0 + 8 <= kc) return;
 #pragma unroll
-      for (int ct = 0; ct < 4; ct++)
+      for (int ct = 0; ct < kCT; ct++)
 #pragma unroll
         for (int i = 0; i < 8; i++)
           if (k0 + i >= kc) {
@@ -805,71 +841,91 @@ __device__ __attribute__((always_inline)) inline void m2l_bf16x3_body(int bx, in
           }
     };
     stage_ops(0);
-    stage_src(0);
-    if (R > 1) stage_src(1);
+    int rows = row_end();
+    stage_rows(0, rows);
+    int nib = load_masks(0), nib_next = load_masks(1);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    int src[4], nsrc[4];
-    v8bf bh[4], bl[4], nbh[4], nbl[4];
-    col_src(0, src);
-    int kc = kcols(0);
-    if (kp < ksteps(kc)) load_b(src, kp, kc, nbh, nbl);
+    unsigned long long act = __ballot(nib != 0);
+    unsigned src[kCT];
+    v8bf bh[kCT], bl[kCT];
+    int u = 0, kk = 0, kc = kcols(0);
+    int pu = -1, pk = 0;  // the unit whose multipoles bh, bl hold (or will, once they land)
     for (int r = 0; r < R; r++) {
-      if (r + 1 < R) stage_ops(r + 1);
-      if (r + 2 < R) stage_src(r + 2);
+      const int landed = rows;
+      if (r + 1 < R) {
+        stage_ops(r + 1);
+        const int e = row_end();
+        stage_rows(rows, e);
+        rows = max(rows, e);
+      }
       __builtin_amdgcn_sched_barrier(0);
-      // B prefetches issued after this round's staging: at most the last
-      // one is still in flight when the round ends
+      // B loads issued after this round's staging: at most the last ones are
+      // still in flight when the round ends
       bool b_after = false;
-      const int u0 = r * kr, u1 = min(u0 + kr, U);
-      for (int u = u0; u < u1; u++) {
-        const v8bf *Ahs = Ab + size_t((r & 1) * kr + u - u0) * 2 * E, *Als = Ahs + E;
-        const int ks = ksteps(kc), nr = rtiles(kc);
-        const int kc_next = u + 1 < U ? kcols(u + 1) : 0;
-        const bool next = u + 1 < U && kp < ksteps(kc_next);
-        if (u + 1 < U) col_src(u + 1, nsrc);  // in LDS: round r or r + 1
-        for (int kk = kp; kk < ks; kk += KPAR) {
-#pragma unroll
-          for (int ct = 0; ct < 4; ct++) {
-            bh[ct] = nbh[ct];
-            bl[ct] = nbl[ct];
+      const int n = min(G, N - r * G);
+      for (int i = 0; i < n; i++) {
+        const int m = __builtin_amdgcn_readlane(nib, u & 63);
+        const int ks = ksteps(kc);
+        if (m != 0 && kk < ks) {
+          if (pu != u || pk != kk) {
+            col_src(u, src);
+            load_b(src, kk, kc, bh, bl);
           }
           // only an order below the operator's has a bound inside the padded K range
-          if (varK && kk * 32 + 32 > kc) mask_b(kk, kc, bh, bl);
-          if (kk + KPAR < ks) {
-            load_b(src, kk + KPAR, kc, nbh, nbl);
-            b_after = true;
-          } else if (next) {
-            load_b(nsrc, kp, kc_next, nbh, nbl);
-            b_after = true;
-          }
+          if (VAR && kk * 32 + 32 > kc) mask_b(kk, kc, bh, bl);
+          const v8bf *Ah = Ab + size_t((r & 1) * G + i) * UE + lane, *Al = Ah + nrt * 64;
+          const int nr = rtiles(kc);
 #pragma unroll
           for (int r2 = 0; r2 < RH; r2++) {
-            if (r2 >= nr) break;
-            const int ai = (kk * nrt + r2) * 64 + lane;
-            const v8bf a_hi = Ahs[ai], a_lo = Als[ai];
+            if (!VAR || r2 < nr) {  // uniform, as the subtile bits below
+              const v8bf a_hi = Ah[r2 * 64], a_lo = Al[r2 * 64];
 #pragma unroll
-            for (int ct = 0; ct < 4; ct++) {
-              if (SKIP && ct >= nct) break;
-              acc[r2][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi, bh[ct], acc[r2][ct], 0, 0, 0);
-              acc[r2][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi, bl[ct], acc[r2][ct], 0, 0, 0);
-              acc[r2][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_lo, bh[ct], acc[r2][ct], 0, 0, 0);
+              for (int ct = 0; ct < kCT; ct++) {
+                if (m & (1 << ct)) {
+                  acc[r2][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi, bh[ct], acc[r2][ct], 0, 0, 0);
+                  acc[r2][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi, bl[ct], acc[r2][ct], 0, 0, 0);
+                  acc[r2][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_lo, bh[ct], acc[r2][ct], 0, 0, 0);
+                }
+              }
+            }
+          }
+          // the next unit's multipoles into the same registers: the SIMD's other
+          // waves cover the latency (a second buffer costs the fourth wave)
+          if (kk + 1 < ks) {
+            load_b(src, kk + 1, kc, bh, bl);
+            pu = u;
+            pk = kk + 1;
+            b_after = true;
+          } else {
+            // this wave's next key, if it lies in this block of masks and its row is in LDS
+            const unsigned long long rest = (u & 63) == 63 ? 0ull : act >> ((u & 63) + 1);
+            const int v = u + __ffsll((long long)rest);
+            if (rest && v < landed) {
+              col_src(v, src);
+              load_b(src, 0, kcols(v), bh, bl);
+              pu = v;
+              pk = 0;
+              b_after = true;
             }
           }
         }
-        if (ks <= kp && next) {
-          load_b(nsrc, kp, kc_next, nbh, nbl);
-          b_after = true;
+        if (++kk == KS) {
+          kk = 0;
+          u++;
+          if (u < U) kc = kcols(u);
+          if ((u & 63) == 0) {
+            nib = nib_next;
+            act = __ballot(nib != 0);
+            nib_next = load_masks(u / 64 + 1);
+          }
         }
-#pragma unroll
-        for (int ct = 0; ct < 4; ct++) src[ct] = nsrc[ct];
-        kc = kc_next;
       }
       // the staging issued at this round's start has landed (loads complete
-      // in issue order; only the 8 loads of the last B prefetch are younger),
-      // then every wave is done with this round's buffers
+      // in issue order; only the 2 kCT loads of the last B prefetch are
+      // younger), then every wave is done with this round's buffers
       if (b_after)
-        __builtin_amdgcn_s_waitcnt(kWaitVm8);
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * kCT));
       else
         __builtin_amdgcn_s_waitcnt(kWaitVm0);
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -878,165 +934,182 @@ __device__ __attribute__((always_inline)) inline void m2l_bf16x3_body(int bx, in
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  reduce_parities<RH, KPAR>(acc, kp, cg, lane, Ab);
-  if (kp == 0) {
-    if (Lpart)
-      write_partial<RH>(PP, rt0, nrt, part_local ? nullptr : sorted + tfirst[tile], ncol, cg, acc, lane, Lpart);
-    else
-      write_locals<RH>(PP, rt0, nrt, sorted + tfirst[tile], ncol, cg, acc, lane, L);
-  }
+  if (Lpart)
+    write_partial<RH>(PP, rt0, nrt, part_local ? nullptr : g.sorted + g.tfirst[tile], ncol, w, acc, lane, Lpart);
+  else
+    write_locals<RH>(PP, rt0, nrt, g.sorted + g.tfirst[tile], ncol, w, acc, lane, L);
 }
 
-template <int RH, int KPAR>
-__global__ void __launch_bounds__(kGemmThreads) k_m2l_bf16x3(int PP, int RT, int RTB, int K32, int KP, OrderPass op,
-                                                             const int *__restrict__ tfirst,
-                                                             const int *__restrict__ tcount,
-                                                             const int *__restrict__ tbase,
-                                                             const int *__restrict__ tU,
-                                                             const int *__restrict__ sorted,
-                                                             const int *__restrict__ tkeys,
-                                                             const int *__restrict__ tmat,
-                                                             const v8bf *__restrict__ ophi,
-                                                             const v8bf *__restrict__ oplo,
-                                                             const __bf16 *__restrict__ mhi,
-                                                             const __bf16 *__restrict__ mlo,
-                                                             const unsigned char *__restrict__ tkp, int kr,
-                                                             int64_t ncells, float *__restrict__ Lpart,
-                                                             double *__restrict__ L) {
+template <int RH, bool VAR>
+__global__ void __launch_bounds__(kGemmThreads) k_m2l_bf16x3(GemmIn g, const int *__restrict__ tbase, int PP, int RT,
+                                                             int RTB, int K32, int KP, OrderPass op,
+                                                             const unsigned char *__restrict__ tkp, int G, int ring,
+                                                             float *__restrict__ Lpart, double *__restrict__ L) {
   // keys of this workgroup: slice blockIdx.z of gridDim.z of the tile's keys
-  const int Ut = tU[blockIdx.x];
+  const int Ut = g.tU[blockIdx.x];
   const int ub = int(int64_t(Ut) * blockIdx.z / gridDim.z), ue = int(int64_t(Ut) * (blockIdx.z + 1) / gridDim.z);
-  m2l_bf16x3_body<RH, false, KPAR>(blockIdx.x, blockIdx.y, ub, ue, false, PP, RT, RTB, K32, KP, op, tfirst, tcount, tbase,
-                             tU, sorted, tkeys, tmat, ophi, oplo, mhi, mlo, tkp, kr, ncells,
-                             Lpart ? Lpart + int64_t(blockIdx.z) * ncells * PP : nullptr, L);
+  m2l_bf16x3_body<RH, VAR>(g, blockIdx.x, blockIdx.y, tbase[blockIdx.x] + ub, ue - ub, false, PP, RT, RTB, K32, KP, op, tkp,
+                      G, ring, Lpart ? Lpart + int64_t(blockIdx.z) * g.ncells * PP : nullptr, L);
 }
 
 // Stream-K schedule: the tiles' key slots, in tile order (slot tbase[t] + u
 // is key u of tile t; S slots in all), are split evenly over the gridDim.x
-// workgroups of one persistent launch (one per CU).  Workgroup w takes slots
-// [w S / G, (w + 1) S / G); each tile it touches gives one FP32 partial of the
-// tile's locals, stored by tile column in segment w + t of Lpart, and
-// k_sk_combine adds a tile's segments in workgroup order.  Every workgroup
-// gets the same number of slots, so none waits on a straggler.  A launch of
-// one order of a learned-order evaluation schedules that order's slots:
-// tbase is then the exclusive prefix of their per-tile counts tU, tstart[t]
-// where tile t's run of them starts in the order-grouped slots, and Sdev
-// their total.
-template <int RH, int KPAR>
-__global__ void __launch_bounds__(kGemmThreads) k_m2l_bf16x3_sk(int PP, int RT, int K32, int KP, OrderPass op,
-                                                                int ntiles, int64_t S, const int *__restrict__ Sdev,
-                                                                const int *__restrict__ tfirst,
-                                                                const int *__restrict__ tcount,
-                                                                const int *__restrict__ tbase,
-                                                                const int *__restrict__ tstart,
-                                                                const int *__restrict__ tU,
-                                                                const int *__restrict__ sorted,
-                                                                const int *__restrict__ tkeys,
-                                                                const int *__restrict__ tmat,
-                                                                const v8bf *__restrict__ ophi,
-                                                                const v8bf *__restrict__ oplo,
-                                                                const __bf16 *__restrict__ mhi,
-                                                                const __bf16 *__restrict__ mlo,
-                                                                const unsigned char *__restrict__ tkp, int kr,
-                                                                int64_t ncells, float *__restrict__ Lseg) {
-  const int64_t G = gridDim.x, w = blockIdx.x;
-  if (Sdev) S = *Sdev;  // one order's slot count, summed on the device
-  const int64_t s0 = w * S / G, s1 = (w + 1) * S / G;
-  if (s0 >= s1) return;
-  // first tile holding slot s0: the last t with tbase[t] <= s0
+// workgroups of one persistent launch (one per CU and row block).  Workgroup
+// w takes slots [w S / G, (w + 1) S / G); each tile it touches gives one FP32
+// partial of the tile's locals, stored by tile column in segment w + t of
+// Lseg, and k_sk_combine adds a tile's segments in workgroup order.  Every
+// workgroup gets the same number of slots, so none waits on a straggler.  A
+// launch of one order of a learned-order evaluation schedules that order's
+// slots: tbase is then the exclusive prefix of their per-tile counts tU,
+// tstart[t] where tile t's run of them starts in the order-grouped slots, and
+// Sdev their total.
+//
+// First slot of workgroup w of W (slots are counted in ints), in a scalar
+// register, as is everything the schedule derives from it: the GEMM body has
+// no vector registers to spare.
+__device__ inline int sk_first(int64_t w, int64_t S, int64_t W) { return __builtin_amdgcn_readfirstlane(int(w * S / W)); }
+
+template <class F>
+__device__ __attribute__((always_inline)) inline void sk_segments(int ntiles, int s0, int s1, int off,
+                                                                  const int *tbase, const int *tU, F &&segment) {
+  // first tile holding slot s0 (slots of these tiles start at off): the last t with off + tbase[t] <= s0
   int lo = 0, hi = ntiles - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (tbase[mid] <= s0)
+    if (off + tbase[mid] <= s0)
       lo = mid;
     else
       hi = mid - 1;
   }
-  for (int t = lo; t < ntiles && tbase[t] < s1; t++) {
-    const int64_t b = tbase[t];
-    const int ub = int(max(s0, b) - b), ue = int(min(s1, b + tU[t]) - b);
-    if (ub >= ue) continue;
-    m2l_bf16x3_body<RH, false, KPAR>(t, 0, ub, ue, true, PP, RT, op.RTo, K32, KP, op, tfirst, tcount, tstart, tU, sorted,
-                               tkeys, tmat, ophi, oplo, mhi, mlo, tkp, kr, ncells,
-                               Lseg + (w + t) * int64_t(tile_width<KPAR>()) * PP, nullptr);
+  for (int t = __builtin_amdgcn_readfirstlane(lo); t < ntiles; t++) {
+    const int b = off + tbase[t];
+    if (b >= s1) break;
+    const int ub = __builtin_amdgcn_readfirstlane(max(s0, b) - b);
+    const int n = __builtin_amdgcn_readfirstlane(min(s1, b + tU[t]) - b) - ub;
+    if (n <= 0) continue;
+    segment(t, ub, n);
     __syncthreads();  // the LDS of this segment is free before the next one stages
   }
 }
 
+template <int RH, bool VAR>
+__global__ void __launch_bounds__(kGemmThreads) k_m2l_bf16x3_sk(GemmIn g, const int *__restrict__ tbase,
+                                                                const int *__restrict__ tstart, int PP, int RT, int RTB,
+                                                                int K32, int KP, OrderPass op, int ntiles, int64_t S,
+                                                                const int *__restrict__ Sdev,
+                                                                const unsigned char *__restrict__ tkp, int G, int ring,
+                                                                float *__restrict__ Lseg) {
+  const int W = gridDim.x, w = blockIdx.x;
+  if (Sdev) S = *Sdev;  // one order's slot count, summed on the device
+  const int s0 = sk_first(w, S, W), s1 = sk_first(w + 1, S, W);
+  if (s0 >= s1) return;
+  sk_segments(ntiles, s0, s1, 0, tbase, g.tU, [&](int t, int ub, int n) {
+    m2l_bf16x3_body<RH, VAR>(g, t, blockIdx.y, tstart[t] + ub, n, true, PP, RT, RTB, K32, KP, op, tkp, G, ring,
+                        Lseg + (w + t) * int64_t(kTileN) * PP, nullptr);
+  });
+}
+
 // Sum of a tile's stream-K segments (workgroups wf .. wl in order) into the
-// FP64 locals, rows 0 .. rows - 1 (those the launch computed).  One thread
-// per (tile column, row).
+// FP64 locals: element e = (tile column, row) of tile t, rows 0 .. rows - 1
+// (those the launch computed); slots b .. b + n - 1 of S belong to the tile,
+// its segments start at seg0 + w.
+__device__ inline void sk_combine(int64_t e, int PP, int rows, int ncol, int64_t b, int n, int64_t S, int W,
+                                  int64_t seg0, const int *cells, const float *__restrict__ Lseg,
+                                  double *__restrict__ L) {
+  const int col = int(e / rows), row = int(e % rows);
+  if (col >= ncol || n == 0) return;
+  // workgroup of slot s: the largest w with w S / W <= s
+  auto wg_of = [&](int64_t sl) { return int(((sl + 1) * W - 1) / S); };
+  const int wf = wg_of(b), wl = wg_of(b + n - 1);
+  double acc = 0.0;
+  for (int w = wf; w <= wl; w++) acc += double(Lseg[((w + seg0) * kTileN + col) * PP + row]);
+  L[int64_t(cells[col]) * PP + row] += acc;
+}
+
 __global__ void __launch_bounds__(256) k_sk_combine(int PP, int rows, int ntiles, int64_t S, const int *__restrict__ Sdev,
-                                                    int G, int tn, const int *__restrict__ tfirst,
+                                                    int W, const int *__restrict__ tfirst,
                                                     const int *__restrict__ tcount, const int *__restrict__ tbase,
                                                     const int *__restrict__ tU, const int *__restrict__ sorted,
                                                     const float *__restrict__ Lseg, double *__restrict__ L) {
   const int t = blockIdx.y;
-  const int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  const int col = int(e / rows), row = int(e % rows);
-  if (t >= ntiles || col >= tcount[t] || tU[t] == 0) return;
+  if (t >= ntiles) return;
   if (Sdev) S = *Sdev;
-  // workgroup of slot s: the largest w with w S / G <= s
-  auto wg_of = [&](int64_t sl) { return int(((sl + 1) * G - 1) / S); };
-  const int64_t b = tbase[t];
-  const int wf = wg_of(b), wl = wg_of(b + tU[t] - 1);
-  double acc = 0.0;
-  for (int w = wf; w <= wl; w++) acc += double(Lseg[(int64_t(w + t) * tn + col) * PP + row]);
-  L[int64_t(sorted[tfirst[t] + col]) * PP + row] += acc;
+  sk_combine(int64_t(blockIdx.x) * 256 + threadIdx.x, PP, rows, tcount[t], tbase[t], tU[t], S, W, t,
+             sorted + tfirst[t], Lseg, L);
 }
 
 // One problem of a grouped keyed-GEMM launch (all problems of one order in
 // a batch): its tiles, operators, cast multipoles and locals.
 struct GroupGemm {
-  const int *tfirst, *tcount, *tbase, *tU, *sorted, *tkeys, *tmat;
-  const v8bf *ophi, *oplo;
-  const __bf16 *mhi, *mlo;
+  GemmIn in;
+  const int *tbase;
   double *L;
-  int64_t ncells;
-  int ntiles;
+  int ntiles, tile0;  // tile0: first of its tiles among the launch's
 };
 
-// All problems of one order in one launch: each problem has ntiles x
-// (row blocks) workgroups, one key slice, kr = 1.
-template <int RH, int KPAR>
-__global__ void __launch_bounds__(kGemmThreads) k_m2l_bf16x3_grouped(const GroupGemm *__restrict__ g,
-                                                                     const int *__restrict__ start, int nprob,
-                                                                     int PP, int RT, int RTB, int K32, int KP,
-                                                                     int pl, int kr) {
-  const int b = blockIdx.x, i = group_of(start, nprob, b), lb = b - start[i];
-  const GroupGemm &q = g[i];
-  m2l_bf16x3_body<RH, true, KPAR>(lb % q.ntiles, lb / q.ntiles, 0, q.tU[lb % q.ntiles], false, PP, RT, RTB, K32, KP,
-                            OrderPass{pl, RT, K32, nullptr},
-                            q.tfirst, q.tcount, q.tbase,
-                            q.tU, q.sorted, q.tkeys, q.tmat, q.ophi, q.oplo, q.mhi, q.mlo, nullptr, kr, q.ncells,
-                            nullptr, q.L);
+// All problems of one order in one stream-K launch: the slots of problem i
+// are sstart[i] .. sstart[i + 1] - 1 of S = sstart[nprob], its tiles the
+// launch's tiles tile0 ...  (A workgroup per tile and row block left the
+// chip to the tiles with the most keys: 12 problems of up to 10^5 bodies
+// have 8 tiles each.)
+template <int RH>
+__global__ void __launch_bounds__(kGemmThreads) k_m2l_bf16x3_grouped(const GroupGemm *__restrict__ gr,
+                                                                     const int *__restrict__ sstart, int nprob, int PP,
+                                                                     int RT, int RTB, int K32, int KP, int pl, int G,
+                                                                     int ring, float *__restrict__ Lseg) {
+  const int W = gridDim.x, w = blockIdx.x, S = sstart[nprob];
+  const int s0 = sk_first(w, S, W), s1 = sk_first(w + 1, S, W);
+  if (s0 >= s1) return;
+  const OrderPass op{pl, RT, K32, nullptr};
+  for (int i = __builtin_amdgcn_readfirstlane(group_of(sstart, nprob, s0)); i < nprob && sstart[i] < s1; i++) {
+    const GroupGemm &q = gr[i];
+    sk_segments(q.ntiles, max(s0, sstart[i]), min(s1, sstart[i + 1]), sstart[i], q.tbase, q.in.tU,
+                [&](int t, int ub, int n) {
+                  m2l_bf16x3_body<RH, false>(q.in, t, blockIdx.y, q.tbase[t] + ub, n, true, PP, RT, RTB, K32, KP, op, nullptr,
+                                      G, ring, Lseg + (w + q.tile0 + t) * int64_t(kTileN) * PP, nullptr);
+                });
+  }
 }
 
+__global__ void __launch_bounds__(256) k_sk_combine_grouped(const GroupGemm *__restrict__ gr,
+                                                            const int *__restrict__ sstart,
+                                                            const int *__restrict__ tstart, int nprob, int PP, int W,
+                                                            const float *__restrict__ Lseg) {
+  const int gt = blockIdx.y, i = group_of(tstart, nprob, gt), t = gt - tstart[i];
+  const GroupGemm &q = gr[i];
+  sk_combine(int64_t(blockIdx.x) * 256 + threadIdx.x, PP, PP, q.in.tcount[t], sstart[i] + q.tbase[t], q.in.tU[t],
+             sstart[nprob], W, gt, q.in.sorted + q.in.tfirst[t], Lseg, q.L);
+}
 
-// Row tiles per workgroup: two operator buffers within the LDS budget, at
-// most kGemmMaxRT accumulator row tiles per wave, and room for the parity
-// reduction (4 x RTB x 4 KB).
-static int rows_per_block(const Geom &g, bool bf16, int device, int kr, int tn) {
+// Tile-matrix rows held in LDS for G units of KS per key: two rounds' keys
+// and the look-ahead, a power of two.
+static int gemm_ring(int KS, int G) {
+  int n = 1;
+  while (n < ceil_div(2 * G, KS) + 2 + kGemmLook) n *= 2;
+  return n;
+}
+
+// Row tiles per workgroup for rounds of `kr` (FP32: keys; BF16: units, a key
+// having K32 of them): two operator buffers and the column sources within the
+// LDS budget, at most the accumulators of kGemmMaxRT row tiles per wave.
+static int rows_per_block(const Geom &g, bool bf16, int device, int kr) {
   int max_lds = 0;
   XF_HIP(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
-  const int per_rt = 2 * kr * (bf16 ? g.K32 * 64 * 16 * 2 : g.K4 * 64 * 4);  // both buffers of kr keys
-  const int need = std::max(per_rt, 4 * 4 * 64 * 16);                   // or the reduction
-  const int avail = max_lds - 3 * kr * tn * 4;                           // less the column sources
-  if (need > avail) {
+  const int per_rt = 2 * kr * (bf16 ? 64 * 16 * 2 : g.K4 * 64 * 4);  // both buffers
+  const int avail = max_lds - (bf16 ? gemm_ring(g.K32, kr) : 3 * kr) * kTileN * 4;
+  if (per_rt > avail) {
     if (kr == 1) fail(EXAFMM_ERR_UNSUPPORTED, "expansion order too large for the LDS operator stage");
     return 0;
   }
-  int rtb = std::min({g.R, kGemmMaxRT, avail / need});
+  const int rtb = std::min({g.R, bf16 ? kGemmMaxRT : kGemmMaxRTF32, avail / per_rt});
   // balance the row blocks
   const int nblk = ceil_div(g.R, rtb);
   return ceil_div(g.R, nblk);
 }
 
-static size_t gemm_lds(const Geom &g, bool bf16, int RTB, int kr, int tn) {
-  const size_t ops = size_t(2) * kr * RTB * (bf16 ? g.K32 * 64 * 16 * 2 : g.K4 * 64 * 4) +
-                     size_t(3) * kr * tn * sizeof(int);  // operator slots + column sources
-  const size_t red = size_t(4) * RTB * 4 * 64 * 16;
-  return std::max(ops, red);
+static size_t gemm_lds(const Geom &g, bool bf16, int RTB, int kr) {
+  return size_t(2) * kr * RTB * (bf16 ? 64 * 16 * 2 : g.K4 * 64 * 4) +
+         size_t(bf16 ? gemm_ring(g.K32, kr) : 3 * kr) * kTileN * sizeof(int);
 }
 
 // One order's launch of a learned-order BF16x3 GEMM: order p over the
@@ -1050,41 +1123,23 @@ struct ClassPass {
   const int *pre, *tot;    // per tile: exclusive prefix of the counts; their total (stream-K)
 };
 
-template <int RH, int KPAR>
-static void launch_gemm(Ctx &tc, const Ctx &sc, const Geom &g, int ntiles, bool bf16, int KP, int KPb, int RTB,
-                        int kr, int ksplit, float *Lpart, double *Lout, const ClassPass *cp) {
-  constexpr int TN = tile_width<KPAR>();
-  Ctx &c = tc;
+static GemmIn gemm_in(const Ctx &c, const Ctx &sc, const Geom &g, const ClassPass *cp) {
   const int ts = c.m2l_tstride;
-  const int *tfirst = c.tiles.p, *tcount = c.tiles.p + ts, *tbase = c.tiles.p + 2 * ts, *tU = c.tiles.p + 3 * ts;
-  const int *sorted = c.tiles.p + 4 * ts;
-  const Geom go = cp ? geom(cp->p) : g;  // rows and k-steps this launch covers
-  const dim3 grid(ntiles, ceil_div(go.R, RTB), ksplit);
-  if (bf16) {
-    const v8bf *ophi = reinterpret_cast<const v8bf *>(c.ops32.p);
-    const size_t per = size_t(g.K32) * g.R * 64 * 8;
-    const v8bf *oplo = reinterpret_cast<const v8bf *>(reinterpret_cast<const __bf16 *>(c.ops32.p) +
-                                                      per * c.lists.nkeys);
-    const __bf16 *mhi = reinterpret_cast<const __bf16 *>(sc.mt32.p);
-    const __bf16 *mlo = mhi + bf16_cast_elems(g, sc.t.ncells);
-    const size_t lds = gemm_lds(go, true, RTB, kr, TN);
-    const OrderPass op{go.P, go.R, go.K32, cp ? cp->perm : nullptr};
-    XF_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_m2l_bf16x3<RH, KPAR>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-    hipLaunchKernelGGL((k_m2l_bf16x3<RH, KPAR>), grid, dim3(kGemmThreads), lds, c.s0, g.PP, g.R, RTB, g.K32, KPb, op,
-                       tfirst, tcount, cp ? cp->start : tbase, cp ? cp->cnt : tU, sorted, c.tile_keys.p,
-                       c.tile_mat.p, ophi, oplo, mhi, mlo, (c.learned && (!cp || cp->variable)) ? c.tile_p.p : nullptr, kr,
-                       int64_t(c.t.ncells), ksplit > 1 ? Lpart : nullptr, Lout);
-  } else {
-    const size_t lds = gemm_lds(g, false, RTB, kr, TN);
-    XF_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_m2l_f32<RH, KPAR>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-    hipLaunchKernelGGL((k_m2l_f32<RH, KPAR>), grid, dim3(kGemmThreads), lds, c.s0, g.PP, g.R, RTB, g.K4, KP, tfirst,
-                       tcount, tbase, tU, sorted, c.tile_keys.p, c.tile_mat.p, c.ops32.p, sc.mt32.p,
-                       c.learned ? c.tile_p.p : nullptr, kr, int64_t(c.t.ncells), ksplit > 1 ? Lpart : nullptr,
-                       Lout);
-  }
-  XF_LAUNCH();
+  GemmIn in{};
+  in.tfirst = c.tiles.p;
+  in.tcount = c.tiles.p + ts;
+  in.tU = cp ? cp->cnt : c.tiles.p + 3 * ts;
+  in.sorted = c.tiles.p + 4 * ts;
+  in.tkeys = c.tile_keys.p;
+  in.tmat = c.tile_mat.p;
+  in.tmask = c.tile_mask.p;
+  const size_t per = size_t(g.K32) * g.R * 64 * 8;
+  in.ophi = reinterpret_cast<const v8bf *>(c.ops32.p);
+  in.oplo = reinterpret_cast<const v8bf *>(reinterpret_cast<const __bf16 *>(c.ops32.p) + per * c.lists.nkeys);
+  in.mhi = reinterpret_cast<const __bf16 *>(sc.mt32.p);
+  in.mlo = in.mhi + bf16_cast_elems(g, sc.t.ncells);
+  in.ncells = sc.t.ncells;
+  return in;
 }
 
 struct GemmShape {
@@ -1098,76 +1153,79 @@ static int cu_count(int device) {
   return std::max(n, 1);
 }
 
-// Stream-K launch: all rows per workgroup (R <= kGemmMaxRT), then the
-// fixed-order combine of each tile's segments.
-template <int RH, int KPAR>
-static void launch_gemm_sk(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, int KPb, int kr, double *Lout,
-                           const ClassPass *cp) {
-  constexpr int TN = tile_width<KPAR>();
+// Persistent workgroups per row block of a stream-K launch.
+static int sk_groups(int device, int nblk) { return std::max(1, cu_count(device) / nblk); }
+
+template <class K>
+static void gemm_attr(K *kernel, size_t lds) {
+  XF_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                             int(lds)));
+}
+
+template <int RH>
+static void launch_bf16(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, int KPb, GemmShape sh, float *Lpart,
+                        double *Lout, const ClassPass *cp) {
   const int ts = c.m2l_tstride;
-  const int *tfirst = c.tiles.p, *tcount = c.tiles.p + ts, *tbase = c.tiles.p + 2 * ts, *tU = c.tiles.p + 3 * ts;
-  const int *sorted = c.tiles.p + 4 * ts;
-  const int G = cu_count(c.cfg.device);
-  const int64_t S = c.m2l_totalU;
-  const Geom go = cp ? geom(cp->p) : g;
+  const int *tbase = c.tiles.p + 2 * ts;
+  const Geom go = cp ? geom(cp->p) : g;  // rows and k-steps this launch covers
+  const GemmIn in = gemm_in(c, sc, g, cp);
   const OrderPass op{go.P, go.R, go.K32, cp ? cp->perm : nullptr};
-  c.m2l_part.ensure(size_t(G + ntiles) * TN * g.PP);
-  const v8bf *ophi = reinterpret_cast<const v8bf *>(c.ops32.p);
-  const size_t per = size_t(g.K32) * g.R * 64 * 8;
-  const v8bf *oplo =
-      reinterpret_cast<const v8bf *>(reinterpret_cast<const __bf16 *>(c.ops32.p) + per * c.lists.nkeys);
-  const __bf16 *mhi = reinterpret_cast<const __bf16 *>(sc.mt32.p);
-  const __bf16 *mlo = mhi + bf16_cast_elems(g, sc.t.ncells);
-  const size_t lds = gemm_lds(go, true, go.R, kr, TN);
-  const int *pre = cp ? cp->pre : tbase, *start = cp ? cp->start : tbase, *cnt = cp ? cp->cnt : tU;
+  const unsigned char *tkp = (c.learned && (!cp || cp->variable)) ? c.tile_p.p : nullptr;
+  const int nblk = ceil_div(go.R, sh.rtb), ring = gemm_ring(go.K32, sh.kr);
+  const size_t lds = gemm_lds(go, true, sh.rtb, sh.kr);
+  if (!sh.sk) {
+    auto *k = cp ? &k_m2l_bf16x3<RH, true> : &k_m2l_bf16x3<RH, false>;
+    gemm_attr(k, lds);
+    hipLaunchKernelGGL(k, dim3(ntiles, nblk, sh.ksplit), dim3(kGemmThreads), lds, c.s0, in,
+                       cp ? cp->start : tbase, g.PP, g.R, sh.rtb, g.K32, KPb, op, tkp, sh.kr, ring,
+                       sh.ksplit > 1 ? Lpart : nullptr, Lout);
+    XF_LAUNCH();
+    return;
+  }
+  const int W = sk_groups(c.cfg.device, nblk);
+  const int64_t S = c.m2l_totalU;
+  c.m2l_part.ensure(size_t(W + ntiles) * kTileN * g.PP);
+  const int *pre = cp ? cp->pre : tbase, *start = cp ? cp->start : tbase;
   const int *Sdev = cp ? cp->tot : nullptr;
-  XF_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_m2l_bf16x3_sk<RH, KPAR>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-  hipLaunchKernelGGL((k_m2l_bf16x3_sk<RH, KPAR>), dim3(G), dim3(kGemmThreads), lds, c.s0, g.PP, g.R, g.K32, KPb, op, ntiles,
-                     S, Sdev, tfirst, tcount, pre, start, cnt, sorted, c.tile_keys.p, c.tile_mat.p, ophi, oplo, mhi,
-                     mlo, (c.learned && (!cp || cp->variable)) ? c.tile_p.p : nullptr, kr, int64_t(c.t.ncells), c.m2l_part.p);
+  auto *k = cp ? &k_m2l_bf16x3_sk<RH, true> : &k_m2l_bf16x3_sk<RH, false>;
+  gemm_attr(k, lds);
+  hipLaunchKernelGGL(k, dim3(W, nblk), dim3(kGemmThreads), lds, c.s0, in, pre, start, g.PP, g.R,
+                     sh.rtb, g.K32, KPb, op, ntiles, S, Sdev, tkp, sh.kr, ring, c.m2l_part.p);
   XF_LAUNCH();
   const int rows = std::min(g.PP, 16 * go.R);
-  hipLaunchKernelGGL(k_sk_combine, dim3(ceil_div(int64_t(TN) * rows, 256), ntiles), dim3(256), 0, c.s0, g.PP, rows,
-                     ntiles, S, Sdev, G, TN, tfirst, tcount, pre, cnt, sorted, c.m2l_part.p, Lout);
+  hipLaunchKernelGGL(k_sk_combine, dim3(ceil_div(int64_t(kTileN) * rows, 256), ntiles), dim3(256), 0, c.s0, g.PP, rows,
+                     ntiles, S, Sdev, W, in.tfirst, in.tcount, pre, in.tU, in.sorted, c.m2l_part.p, Lout);
+  XF_LAUNCH();
+}
+
+template <int RH>
+static void launch_f32(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, int KP, GemmShape sh, float *Lpart,
+                       double *Lout) {
+  const int ts = c.m2l_tstride;
+  const int *t = c.tiles.p;
+  const size_t lds = gemm_lds(g, false, sh.rtb, sh.kr);
+  gemm_attr(&k_m2l_f32<RH>, lds);
+  hipLaunchKernelGGL((k_m2l_f32<RH>), dim3(ntiles, ceil_div(g.R, sh.rtb), sh.ksplit), dim3(kGemmThreads), lds, c.s0,
+                     g.PP, g.R, sh.rtb, g.K4, KP, t, t + ts, t + 2 * ts, t + 3 * ts, t + 4 * ts, c.tile_keys.p,
+                     c.tile_mat.p, c.ops32.p, sc.mt32.p, c.learned ? c.tile_p.p : nullptr, sh.kr,
+                     int64_t(c.t.ncells), sh.ksplit > 1 ? Lpart : nullptr, Lout);
   XF_LAUNCH();
 }
 
 static void run_gemm(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, bool bf16, int KP, int KPb, GemmShape sh,
                      double *Lout, const ClassPass *cp = nullptr) {
-  if (sh.sk) {
-    switch (cp ? geom(cp->p).R : g.R) {
-#define XF_GEMM_SK(n)                                                  \
-  case n:                                                              \
-    if (c.m2l_tn == tile_width<1>())                                   \
-      launch_gemm_sk<n, 1>(c, sc, g, ntiles, KPb, sh.kr, Lout, cp);   \
-    else                                                               \
-      launch_gemm_sk<n, 2>(c, sc, g, ntiles, KPb, sh.kr, Lout, cp);   \
-    return;
-      XF_GEMM_SK(1)
-      XF_GEMM_SK(2)
-      XF_GEMM_SK(3)
-      XF_GEMM_SK(4)
-      XF_GEMM_SK(5)
-      XF_GEMM_SK(6)
-      XF_GEMM_SK(7)
-      XF_GEMM_SK(8)
-#undef XF_GEMM_SK
-      default: fail(EXAFMM_ERR_UNSUPPORTED, "stream-K GEMM needs all rows in one workgroup");
-    }
-  }
   float *part = nullptr;
   if (sh.ksplit > 1) {
     c.m2l_part.ensure(size_t(sh.ksplit) * c.t.ncells * g.PP);
     part = c.m2l_part.p;
   }
   switch (sh.rtb) {
-#define XF_GEMM_CASE(n)                                                                          \
-  case n:                                                                                        \
-    if (c.m2l_tn == tile_width<1>())                                                             \
-      launch_gemm<n, 1>(c, sc, g, ntiles, bf16, KP, KPb, sh.rtb, sh.kr, sh.ksplit, part, Lout, cp); \
-    else                                                                                         \
-      launch_gemm<n, 2>(c, sc, g, ntiles, bf16, KP, KPb, sh.rtb, sh.kr, sh.ksplit, part, Lout, cp); \
+#define XF_GEMM_CASE(n)                                                             \
+  case n:                                                                           \
+    if (bf16)                                                                       \
+      launch_bf16<n>(c, sc, g, ntiles, KPb, sh, part, Lout, cp);                    \
+    else                                                                            \
+      launch_f32<n <= kGemmMaxRTF32 ? n : 1>(c, sc, g, ntiles, KP, sh, part, Lout); \
     break;
     XF_GEMM_CASE(1)
     XF_GEMM_CASE(2)
@@ -1177,6 +1235,7 @@ static void run_gemm(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, bool bf16
     XF_GEMM_CASE(6)
     XF_GEMM_CASE(7)
     XF_GEMM_CASE(8)
+    XF_GEMM_CASE(9)
 #undef XF_GEMM_CASE
     default: fail(EXAFMM_ERR_UNSUPPORTED, "expansion order");
   }
@@ -1188,13 +1247,25 @@ static void run_gemm(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, bool bf16
   }
 }
 
-// Autotuner of the GEMM shape: rows of the operator per workgroup (the
-// rows of a tile may be split over several workgroups: more workgroups
-// when tiles are few, more re-reads of the source multipoles), keys per
-// LDS round (more keys per barrier hide the operator-copy latency of short,
-// low-order keys) and key slices per tile (a tile's keys split over
-// several workgroups whose FP32 partial locals a second kernel adds in a
-// fixed order: more parallelism when tiles are few and keys many).  The first time a (order, precision, order policy, tile
+// Rounds the autotuners try, in units of a launch of KS units per key: whole
+// keys as far as two buffers fit, else the most units that do, and half a key.
+static std::vector<int> gemm_rounds(const Geom &go, int device) {
+  std::vector<int> r;
+  for (int n = 1; n <= 4; n++)
+    if (rows_per_block(go, true, device, n * go.K32) >= std::min(go.R, ceil_div(go.R, ceil_div(go.R, kGemmMaxRT))))
+      r.push_back(n * go.K32);
+  for (int G = go.K32 - 1; G > 1 && r.empty(); G--)
+    if (rows_per_block(go, true, device, G) >= ceil_div(go.R, ceil_div(go.R, kGemmMaxRT))) r.push_back(G);
+  if (go.K32 >= 4) r.push_back(go.K32 / 2);
+  if (r.empty()) r.push_back(1);
+  return r;
+}
+
+// Autotuner of the GEMM shape: operator staged per LDS round (more per
+// barrier hides the copy latency of short, low-order keys), stream-K, or a
+// workgroup per tile with key slices (a tile's keys split over several
+// workgroups whose FP32 partial locals a second kernel adds in a fixed order:
+// more parallelism when tiles are few and keys many).  The first time a (order, precision, order policy, tile
 // count class) is seen, every candidate (GEMM and, with key slices, the
 // combining kernel) runs twice into a scratch copy of the locals, alone on
 // the device, timed with HIP events; the fastest run's shape is kept for
@@ -1206,35 +1277,39 @@ static GemmShape gemm_shape(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, bo
   // a learned-order launch of one order is tuned per order (its rows, k-steps and LDS)
   const Geom go = cp ? geom(cp->p) : g;
   const long long key = ((long long)g.P << 24) | ((long long)bf16 << 20) | ((long long)c.learned << 16) |
-                        ((long long)(cp ? cp->p : 0) << 32) | ((long long)(c.m2l_tn == tile_width<1>()) << 40) |
-                        tclass;
+                        ((long long)(cp ? cp->p : 0) << 32) | tclass;
   auto it = c.gemm_tuned.find(key);
   if (it != c.gemm_tuned.end())
     return GemmShape{int(it->second & 255), int((it->second >> 8) & 255), int((it->second >> 16) & 255),
                      int(it->second >> 24)};
   std::vector<GemmShape> cand;
-  // low orders: short keys, so more of them per LDS round
-  const int krmax = go.P <= 10 ? 5 : 3;
-  for (int kr = 1; kr <= krmax; kr++) {
-    const int rmax = rows_per_block(go, bf16, c.cfg.device, kr, c.m2l_tn);
-    if (rmax < 1) continue;
-    int last = -1;
-    for (int nb = ceil_div(go.R, rmax); nb <= ceil_div(go.R, rmax) + 2; nb++) {
-      const int r = ceil_div(go.R, nb);
-      if (r != last && r <= rmax) {
-        cand.push_back(GemmShape{r, kr, 1});
-        // key slices only where the workgroups would not fill the device
-        const int wg = ntiles * nb;
-        for (const int ks : {2, 3, 4, 6, 8})
-          if (wg * ks <= 4096 && c.m2l_totalU >= 8 * ks * ntiles) cand.push_back(GemmShape{r, kr, ks});
+  auto slices = [&](int rtb, int kr, int nb) {
+    cand.push_back(GemmShape{rtb, kr, 1});
+    // key slices only where the workgroups would not fill the device
+    const int wg = ntiles * nb;
+    for (const int ks : {2, 4, 8})
+      if (wg * ks <= 2048 && c.m2l_totalU >= 8 * ks * ntiles) cand.push_back(GemmShape{rtb, kr, ks});
+  };
+  if (bf16) {
+    for (const int G : gemm_rounds(go, c.cfg.device)) {
+      const int r = rows_per_block(go, true, c.cfg.device, G), nb = ceil_div(go.R, r);
+      slices(r, G, nb);
+      if (std::getenv("EXAFMM_GEMM_NO_SK") == nullptr) cand.push_back(GemmShape{r, G, 1, 1});
+    }
+  } else {
+    // low orders: short keys, so more of them per LDS round
+    const int krmax = go.P <= 10 ? 5 : 3;
+    for (int kr = 1; kr <= krmax; kr++) {
+      const int rmax = rows_per_block(go, false, c.cfg.device, kr);
+      if (rmax < 1) continue;
+      int last = -1;
+      for (int nb = ceil_div(go.R, rmax); nb <= ceil_div(go.R, rmax) + 2; nb++) {
+        const int r = ceil_div(go.R, nb);
+        if (r != last && r <= rmax) slices(r, kr, nb);
+        last = r;
       }
-      last = r;
     }
   }
-  // stream-K (BF16x3, all rows per workgroup)
-  if (bf16 && go.R <= kGemmMaxRT && std::getenv("EXAFMM_GEMM_NO_SK") == nullptr)
-    for (int kr = 1; kr <= 3; kr++)
-      if (rows_per_block(go, bf16, c.cfg.device, kr, c.m2l_tn) >= go.R) cand.push_back(GemmShape{go.R, kr, 1, 1});
   GemmShape best = cand[0];
   if (std::getenv("EXAFMM_GEMM_SK_ONLY"))  // the stream-K candidates alone (tests, A/B timing)
     for (const GemmShape &sh : cand)
@@ -1251,7 +1326,7 @@ static GemmShape gemm_shape(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, bo
     c.L_tune.ensure(size_t(c.t.ncells) * c.P * c.P);
     size_t need = 1;
     for (const GemmShape &sh : cand)
-      need = std::max(need, sh.sk ? size_t(cu_count(c.cfg.device) + ntiles) * c.m2l_tn * g.PP
+      need = std::max(need, sh.sk ? size_t(sk_groups(c.cfg.device, ceil_div(go.R, sh.rtb)) + ntiles) * kTileN * g.PP
                                   : size_t(sh.ksplit > 1 ? sh.ksplit : 0) * c.t.ncells * g.PP);
     c.m2l_part.ensure(need);  // no allocation inside the timings
     hipEvent_t e0, e1;
@@ -1294,6 +1369,12 @@ static void ops_remember(Ctx &c, std::vector<unsigned long long> keys, int fillP
   c.ops_cycle = c.cfg.cycle;
 }
 
+// Whether the next keyed GEMM runs learned per-slot orders (a forest has no
+// common root to scale the tolerance by: fixed order).
+static bool learned_orders(const Ctx &c) {
+  return c.cfg.order_policy == EXAFMM_ORDER_LEARNED && c.have_model && c.forest_n == 0;
+}
+
 // Tiles, key lists and operators: depend only on the tree and the lists,
 // so they can be built on a side stream while the upward pass runs.
 void m2l_prepare(Ctx &c, hipStream_t s) {
@@ -1316,9 +1397,15 @@ void m2l_prepare(Ctx &c, hipStream_t s) {
   // (measured 0.50 -> 0.58 on a 2^22-body Plummer set); on uniform trees,
   // where BFS neighbours already share key sets, it changes little.
   const int minhash = 1;
+  // Tiles mix the levels (keys are scale-free: on a clustered set of 200,000
+  // bodies half as many (tile, key) slots as with tiles of one level), unless
+  // the keys carry the level (periodic) or the slots take one learned order
+  // each, chosen for cells of one size.
+  const bool by_level = c.cfg.images > 0 || learned_orders(c);
+  c.m2l_by_level = by_level;
   hipLaunchKernelGGL(k_group_keys, dim3(ceil_div(nc, 256 / kWave)), dim3(256), 0, s, nc, c.t.cx.p, c.t.cparent.p,
                      c.t.clevel.p, c.lists.m2l_beg.p, c.lists.m2l_cnt.p, c.lists.m2l.p, minhash,
-                     m2l_fp64_levels(c), c.t.key.p, c.t.val.p);
+                     m2l_fp64_levels(c), int(by_level), c.t.key.p, c.t.val.p);
   XF_LAUNCH();
   unsigned long long *k1 = c.t.key.p, *k2 = c.t.key2.p;
   int *v1 = c.t.val.p, *v2 = c.t.val2.p;
@@ -1330,12 +1417,7 @@ void m2l_prepare(Ctx &c, hipStream_t s) {
   // tiles of at most tn cells per group, laid out on the device (no host
   // round trip before the per-tile counts); arrays strided by the bound
   // ntmax: [first | count | base | U] x ntmax, then the sorted cells
-  // Tile width: 512 targets halves the operator staging per target where
-  // the tiles fill (a free-space tree's octant groups); periodic trees (image
-  // keys) and forests (many small problems) have more varied key sets, whose
-  // larger per-tile key unions favour 256.
-  c.m2l_tn = (c.cfg.images > 0 || c.forest_n > 0) ? tile_width<2>() : tile_width<1>();
-  const int tn = c.m2l_tn;
+  const int tn = kTileN;
   const int ntmax = ceil_div(nc, tn) + 255;
   c.tiles.ensure(size_t(4) * ntmax + nc);
   int *d_first = c.tiles.p, *d_count = c.tiles.p + ntmax, *d_base = c.tiles.p + 2 * ntmax,
@@ -1369,9 +1451,10 @@ void m2l_prepare(Ctx &c, hipStream_t s) {
   }
   c.tile_keys.ensure(std::max(totalU, 1));
   c.tile_mat.ensure(size_t(std::max(totalU, 1)) * tn);
-  hipLaunchKernelGGL(k_tile_fill, dim3(ntiles, tn / 64), dim3(256), sizeof(unsigned) * 2 * nwords, s, d_first,
+  c.tile_mask.ensure(std::max(totalU, 1));
+  hipLaunchKernelGGL(k_tile_fill, dim3(ntiles, tn / 64), dim3(256), sizeof(unsigned) * 6 * nwords, s, d_first,
                      d_count, d_sorted, c.lists.m2l_beg.p, c.lists.m2l_cnt.p, c.lists.m2l.p, nkeys, d_base,
-                     c.tile_bits.p, c.tile_keys.p, tn, c.tile_mat.p);
+                     c.tile_bits.p, c.tile_keys.p, c.tile_mat.p, reinterpret_cast<unsigned char *>(c.tile_mask.p));
   XF_LAUNCH();
 
   // 2. operators (cached by key set)
@@ -1437,12 +1520,11 @@ void m2l_fast(Ctx &tc, const Ctx &sc) {
     XF_LAUNCH();
   }
 
-  // per-key orders of a learned-order evaluation (need the multipoles)
-  // (a forest has no common root to scale the tolerance by: fixed order)
-  c.learned = c.cfg.order_policy == EXAFMM_ORDER_LEARNED && c.have_model && c.forest_n == 0;
+  // per-key orders of a learned-order evaluation (need the multipoles, and tiles of one level)
+  c.learned = learned_orders(c) && c.m2l_by_level;
   if (c.learned)
     order_select(c, c.tiles.p, c.tiles.p + c.m2l_tstride, c.tiles.p + 2 * c.m2l_tstride,
-                 c.tiles.p + 3 * c.m2l_tstride, c.tiles.p + 4 * c.m2l_tstride, ntiles, c.m2l_totalU, c.m2l_tn, s);
+                 c.tiles.p + 3 * c.m2l_tstride, c.tiles.p + 4 * c.m2l_tstride, ntiles, c.m2l_totalU, kTileN, s);
 
   // 3. GEMM over tiles, shape from the autotuner
   if (c.learned && bf16) {
@@ -1514,19 +1596,13 @@ __global__ void __launch_bounds__(256) k_mt_grouped(const GroupCast *__restrict_
   q.mlo[e] = __bf16(v - float(h));
 }
 
-template <int RH, int KPAR>
-static void group_attr(size_t lds) {
-  XF_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_m2l_bf16x3_grouped<RH, KPAR>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-}
-
 // Descriptor tables of one order's problems (their tiles and operators from
 // m2l_prepare, their cast buffers sized by an earlier evaluation) for one
-// GEMM shape (rows per workgroup, keys per LDS round), the same for every
+// GEMM shape (rows per workgroup, units per LDS round), the same for every
 // problem of the launch.
 static void group_tables(const std::vector<Ctx *> &probs, GemmGroupPlan &plan, int rtb, int kr) {
   plan.nprob = 0;
-  plan.nblocks = plan.cast_blocks = 0;
+  plan.ntiles = plan.cast_blocks = 0;
   if (probs.empty()) return;
   const int P = probs[0]->P;
   const Geom g = geom(P);
@@ -1534,57 +1610,42 @@ static void group_tables(const std::vector<Ctx *> &probs, GemmGroupPlan &plan, i
   plan.P = P;
   plan.rtb = rtb;
   plan.kr = kr;
-  const int nrb = ceil_div(g.R, plan.rtb);
-  plan.tn = probs[0]->m2l_tn;
-  plan.lds = gemm_lds(g, true, plan.rtb, kr, plan.tn);
+  plan.groups = sk_groups(probs[0]->cfg.device, ceil_div(g.R, rtb));
+  plan.lds = gemm_lds(g, true, rtb, kr);
   std::vector<GroupGemm> d;
   std::vector<GroupCast> cd;
-  std::vector<int> st, cst;
-  int64_t acc = 0, cacc = 0;
+  std::vector<int> st, cst;  // st: slot prefix, then tile prefix
+  std::vector<int> tst;
+  int64_t slots = 0, tiles = 0, cacc = 0;
   for (Ctx *cp : probs) {
     Ctx &c = *cp;
     if (c.P != P || c.cfg.m2l_precision != EXAFMM_PREC_BF16X3) fail(EXAFMM_ERR_ARG, "mixed orders in a GEMM group");
-    if (c.m2l_tn != plan.tn) fail(EXAFMM_ERR_ARG, "mixed tile widths in a GEMM group");
     if (!c.m2l_ready) fail(EXAFMM_ERR_STATE, "keyed M2L tiles missing");
-    const int nt = c.m2l_ntiles;
-    if (nt == 0) continue;
+    if (c.m2l_ntiles == 0) continue;
     const int64_t nc = c.t.ncells;
-    const size_t per = size_t(g.K32) * g.R * 64 * 8;
-    const __bf16 *ophi = reinterpret_cast<const __bf16 *>(c.ops32.p);
     const size_t elems = bf16_cast_elems(g, nc);
     c.mt32.ensure(elems + 1);  // two bf16 arrays in a float buffer (set-up time, not under capture)
     __bf16 *mhi = reinterpret_cast<__bf16 *>(c.mt32.p);
-    GroupGemm q;
-    const int ts = c.m2l_tstride;
-    q.tfirst = c.tiles.p;
-    q.tcount = c.tiles.p + ts;
-    q.tbase = c.tiles.p + 2 * ts;
-    q.tU = c.tiles.p + 3 * ts;
-    q.sorted = c.tiles.p + 4 * ts;
-    q.tkeys = c.tile_keys.p;
-    q.tmat = c.tile_mat.p;
-    q.ophi = reinterpret_cast<const v8bf *>(ophi);
-    q.oplo = reinterpret_cast<const v8bf *>(ophi + per * c.lists.nkeys);
-    q.mhi = mhi;
-    q.mlo = mhi + elems;
-    q.L = c.L.p;
-    q.ncells = nc;
-    q.ntiles = nt;
-    d.push_back(q);
-    st.push_back(int(acc));
-    acc += int64_t(nt) * nrb;
-    GroupCast cq{c.M.p, mhi, mhi + elems, nc, g.PP, KPb, int64_t(elems)};
-    cd.push_back(cq);
+    d.push_back(GroupGemm{gemm_in(c, c, g, nullptr), c.tiles.p + 2 * c.m2l_tstride, c.L.p, c.m2l_ntiles, int(tiles)});
+    st.push_back(int(slots));
+    tst.push_back(int(tiles));
+    slots += c.m2l_totalU;
+    tiles += c.m2l_ntiles;
+    cd.push_back(GroupCast{c.M.p, mhi, mhi + elems, nc, g.PP, KPb, int64_t(elems)});
     cst.push_back(int(cacc));
     cacc += ceil_div(int64_t(elems), 256);
   }
-  if (acc > (int64_t(1) << 31) - 1 || cacc > (int64_t(1) << 31) - 1) fail(EXAFMM_ERR_CAPACITY, "batch too large");
+  if (slots > (int64_t(1) << 31) - 1 || tiles > 65535 || cacc > (int64_t(1) << 31) - 1)
+    fail(EXAFMM_ERR_CAPACITY, "batch too large");
   plan.nprob = int(d.size());
-  plan.nblocks = int(acc);
+  plan.ntiles = int(tiles);
   plan.cast_blocks = int(cacc);
   if (!plan.nprob) return;
-  st.push_back(int(acc));
+  st.push_back(int(slots));
+  tst.push_back(int(tiles));
+  st.insert(st.end(), tst.begin(), tst.end());
   cst.push_back(int(cacc));
+  plan.seg.ensure(size_t(plan.groups + tiles) * kTileN * g.PP);
   plan.desc.ensure(sizeof(GroupGemm) * d.size());
   plan.cast_desc.ensure(sizeof(GroupCast) * cd.size());
   plan.start.ensure(st.size());
@@ -1593,47 +1654,26 @@ static void group_tables(const std::vector<Ctx *> &probs, GemmGroupPlan &plan, i
   XF_HIP(hipMemcpy(plan.cast_desc.p, cd.data(), sizeof(GroupCast) * cd.size(), hipMemcpyHostToDevice));
   XF_HIP(hipMemcpy(plan.start.p, st.data(), sizeof(int) * st.size(), hipMemcpyHostToDevice));
   XF_HIP(hipMemcpy(plan.cast_start.p, cst.data(), sizeof(int) * cst.size(), hipMemcpyHostToDevice));
-  switch (plan.rtb) {
-    case 1: plan.tn == tile_width<1>() ? group_attr<1, 1>(plan.lds) : group_attr<1, 2>(plan.lds); break;
-    case 2: plan.tn == tile_width<1>() ? group_attr<2, 1>(plan.lds) : group_attr<2, 2>(plan.lds); break;
-    case 3: plan.tn == tile_width<1>() ? group_attr<3, 1>(plan.lds) : group_attr<3, 2>(plan.lds); break;
-    case 4: plan.tn == tile_width<1>() ? group_attr<4, 1>(plan.lds) : group_attr<4, 2>(plan.lds); break;
-    case 5: plan.tn == tile_width<1>() ? group_attr<5, 1>(plan.lds) : group_attr<5, 2>(plan.lds); break;
-    case 6: plan.tn == tile_width<1>() ? group_attr<6, 1>(plan.lds) : group_attr<6, 2>(plan.lds); break;
-    case 7: plan.tn == tile_width<1>() ? group_attr<7, 1>(plan.lds) : group_attr<7, 2>(plan.lds); break;
-    case 8: plan.tn == tile_width<1>() ? group_attr<8, 1>(plan.lds) : group_attr<8, 2>(plan.lds); break;
-    default: fail(EXAFMM_ERR_UNSUPPORTED, "expansion order");
-  }
 }
 
-// Autotuner of a grouped GEMM: every (rows per workgroup, keys per LDS
-// round) candidate runs on the batch itself (alone on the device, after one
-// untimed launch), timed with HIP events; the fastest shape is kept.  The
-// runs add into the locals, which the graph's prologue clears.
+// Autotuner of a grouped GEMM: every round size runs on the batch itself
+// (alone on the device, after one untimed launch), timed with HIP events; the
+// fastest is kept.  The runs add into the locals, which the graph's prologue
+// clears.
 void m2l_group_setup(const std::vector<Ctx *> &probs, GemmGroupPlan &plan, hipStream_t s, bool tune) {
   if (probs.empty()) return;
   const Geom g = geom(probs[0]->P);
   const int dev = probs[0]->cfg.device;
-  std::vector<std::pair<int, int>> cand;  // (rtb, kr)
-  for (int kr = 1; kr <= 3; kr++) {
-    const int rmax = rows_per_block(g, true, dev, kr, probs[0]->m2l_tn);
-    if (rmax < 1) continue;
-    int last = -1;
-    for (int nb = ceil_div(g.R, rmax); nb <= ceil_div(g.R, rmax) + 1; nb++) {
-      const int r = ceil_div(g.R, nb);
-      if (r != last && r <= rmax) cand.push_back({r, kr});
-      last = r;
-    }
-  }
-  if (cand.empty()) fail(EXAFMM_ERR_UNSUPPORTED, "expansion order too large for the LDS operator stage");
-  std::pair<int, int> best = cand[0];
-  if (tune && cand.size() > 1) {
+  const std::vector<int> rounds = gemm_rounds(g, dev);
+  int best = rounds[0];
+  if (tune && rounds.size() > 1) {
     hipEvent_t e0, e1;
     XF_HIP(hipEventCreate(&e0));
     XF_HIP(hipEventCreate(&e1));
     float bt = 1e30f;
-    for (const auto &c : cand) {
-      group_tables(probs, plan, c.first, c.second);
+    for (const int kr : rounds) {
+      const int rtb = rows_per_block(g, true, dev, kr);
+      group_tables(probs, plan, rtb, kr);
       m2l_group_launch(plan, s);  // untimed
       XF_HIP(hipEventRecord(e0, s));
       m2l_group_launch(plan, s);
@@ -1641,16 +1681,29 @@ void m2l_group_setup(const std::vector<Ctx *> &probs, GemmGroupPlan &plan, hipSt
       XF_HIP(hipEventSynchronize(e1));
       float ms = 0;
       XF_HIP(hipEventElapsedTime(&ms, e0, e1));
-      plan.tuned.push_back({c.first, c.second, ms});
+      plan.tuned.push_back({rtb, kr, ms});
       if (ms < bt) {
         bt = ms;
-        best = c;
+        best = kr;
       }
     }
     XF_HIP(hipEventDestroy(e0));
     XF_HIP(hipEventDestroy(e1));
   }
-  group_tables(probs, plan, best.first, best.second);
+  group_tables(probs, plan, rows_per_block(g, true, dev, best), best);
+}
+
+template <int RH>
+static void launch_group(const GemmGroupPlan &plan, const Geom &g, hipStream_t s) {
+  const GroupGemm *d = reinterpret_cast<const GroupGemm *>(plan.desc.p);
+  gemm_attr(&k_m2l_bf16x3_grouped<RH>, plan.lds);
+  hipLaunchKernelGGL((k_m2l_bf16x3_grouped<RH>), dim3(plan.groups, ceil_div(g.R, plan.rtb)), dim3(kGemmThreads),
+                     plan.lds, s, d, plan.start.p, plan.nprob, g.PP, g.R, plan.rtb, g.K32, bf16_row(g), g.P, plan.kr,
+                     gemm_ring(g.K32, plan.kr), plan.seg.p);
+  XF_LAUNCH();
+  hipLaunchKernelGGL(k_sk_combine_grouped, dim3(ceil_div(int64_t(kTileN) * g.PP, 256), plan.ntiles), dim3(256), 0, s, d,
+                     plan.start.p, plan.start.p + plan.nprob + 1, plan.nprob, g.PP, plan.groups, plan.seg.p);
+  XF_LAUNCH();
 }
 
 void m2l_group_launch(const GemmGroupPlan &plan, hipStream_t s) {
@@ -1659,30 +1712,18 @@ void m2l_group_launch(const GemmGroupPlan &plan, hipStream_t s) {
   const GroupCast *cd = reinterpret_cast<const GroupCast *>(plan.cast_desc.p);
   hipLaunchKernelGGL(k_mt_grouped, dim3(plan.cast_blocks), dim3(256), 0, s, cd, plan.cast_start.p, plan.nprob);
   XF_LAUNCH();
-  const GroupGemm *d = reinterpret_cast<const GroupGemm *>(plan.desc.p);
-  const int KPb = bf16_row(g);
   switch (plan.rtb) {
-#define XF_GROUP_CASE(n)                                                                                         \
-  case n:                                                                                                         \
-    if (plan.tn == tile_width<1>())                                                                              \
-      hipLaunchKernelGGL((k_m2l_bf16x3_grouped<n, 1>), dim3(plan.nblocks), dim3(kGemmThreads), plan.lds, s, d,    \
-                         plan.start.p, plan.nprob, g.PP, g.R, plan.rtb, g.K32, KPb, g.P, plan.kr);                \
-    else                                                                                                          \
-      hipLaunchKernelGGL((k_m2l_bf16x3_grouped<n, 2>), dim3(plan.nblocks), dim3(kGemmThreads), plan.lds, s, d,    \
-                         plan.start.p, plan.nprob, g.PP, g.R, plan.rtb, g.K32, KPb, g.P, plan.kr);                \
-    break;
-    XF_GROUP_CASE(1)
-    XF_GROUP_CASE(2)
-    XF_GROUP_CASE(3)
-    XF_GROUP_CASE(4)
-    XF_GROUP_CASE(5)
-    XF_GROUP_CASE(6)
-    XF_GROUP_CASE(7)
-    XF_GROUP_CASE(8)
-#undef XF_GROUP_CASE
+    case 1: return launch_group<1>(plan, g, s);
+    case 2: return launch_group<2>(plan, g, s);
+    case 3: return launch_group<3>(plan, g, s);
+    case 4: return launch_group<4>(plan, g, s);
+    case 5: return launch_group<5>(plan, g, s);
+    case 6: return launch_group<6>(plan, g, s);
+    case 7: return launch_group<7>(plan, g, s);
+    case 8: return launch_group<8>(plan, g, s);
+    case 9: return launch_group<9>(plan, g, s);
     default: fail(EXAFMM_ERR_UNSUPPORTED, "expansion order");
   }
-  XF_LAUNCH();
 }
 
 }  // namespace xf
