@@ -120,7 +120,7 @@ void do_upward(Ctx &c, hipStream_t s) {
   rec(c, 3, s);
 }
 
-// Interaction lists (geometry only: no multipoles needed).
+// Interaction lists (geometry only: no multipoles needed) and zero locals.
 void do_lists(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels = {}) {
   if (!tc.t.built || !sc.t.built) fail(EXAFMM_ERR_STATE, "horizontal pass before build_tree");
   if (tc.graph_locks) fail(EXAFMM_ERR_STATE, "the context is held by a graph (exafmm_graph_destroy it first)");
@@ -130,8 +130,6 @@ void do_lists(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
   rec(tc, 11, tc.s0);
   traverse(tc, sc, after_kernels);
   rec(tc, 12, tc.s0);
-  tc.L.ensure(size_t(tc.t.ncells) * tc.P * tc.P);
-  XF_HIP(hipMemsetAsync(tc.L.p, 0, sizeof(double) * tc.t.ncells * tc.P * tc.P, tc.s0));
 }
 
 // P2P on the second stream from the current point of the main stream, so it

@@ -131,8 +131,10 @@ constexpr int kPinMisc = 48;      // 19: tree flags and counters
 constexpr int kPinTot = 72;       // 8: list totals and flags
 constexpr int kPinPlan = 80;      // 3: M2L slots, tiles, cells in tiles
 constexpr int kPinInts = 96;
-// traversal flag bits that make the pass repeat: list capacity, key table full
-constexpr int kListRetry = 1 | 8;
+// traversal flag bits that make the pass repeat: list capacity, key table
+// full, small work queue overflow
+constexpr int kListQueue = 64;
+constexpr int kListRetry = 1 | 8 | kListQueue;
 static_assert(kPinLevels + kMaxLevel + 2 <= kPinMisc && kPinMisc + 19 <= kPinTot, "pinned slots overlap");
 
 inline int ceil_div(int64_t a, int64_t b) { return int((a + b - 1) / b); }
@@ -222,14 +224,12 @@ struct Lists {
   Buf<int> tot;               // device totals [m2l, p2p, out], overflow flags
   int64_t cap_m2l = 0, cap_p2p = 0, cap_out = 0;
   int64_t nm2l = 0, np2p = 0;
+  bool large_queue = false;  // a target overflowed the traversal's small queue
   // translation keys
   Buf<unsigned long long> hslots;  // open-addressing key set
   int hcap = 0;
   Buf<int> slot2id;
   Buf<int> scan_tmp;       // device-wide scan partials
-  Buf<int64_t> capd;       // list capacities on the device (scan overflow check)
-  HostBuf<int64_t> caps_pin;
-  int64_t caps_up[3] = {-1, -1, -1};  // capacities last uploaded
   Buf<unsigned long long> keys;    // distinct keys, ascending
   Buf<int> kscratch;
   int nkeys = 0;
@@ -403,10 +403,6 @@ void op_l2p(Ctx &c, const double *C, const double *L, exafmm_body *b, int64_t nb
 void scan_exclusive(const int *in, int *out, int count, int *total, Buf<int> &scratch, hipStream_t s);
 void scan_exclusive_dev(const int *in, int *out, const int *count_dev, int count_bound, int *total,
                         Buf<int> &scratch, hipStream_t s);
-// three arrays at once; running[k] is added to every output and receives the
-// new totals; bit 1 of *flag is raised when a total exceeds cap[k]
-void scan_exclusive3(const int *in0, const int *in1, const int *in2, int *out0, int *out1, int *out2, int count,
-                     int *running, const int64_t *cap, int *flag, Buf<int> &scratch, hipStream_t s);
 void radix_sort_pairs(unsigned long long *&k, int *&v, unsigned long long *&k2, int *&v2, int n, int lo_bit,
                       int hi_bit, Buf<int> &hist, hipStream_t s);
 

@@ -581,15 +581,19 @@ float order_train(Ctx &c, int nsamples, int epochs, float lr, uint64_t seed) {
   XF_HIP(hipMemcpyAsync(beg.data(), c.lists.m2l_beg.p, sizeof(int) * nc, hipMemcpyDeviceToHost, s));
   XF_HIP(hipMemcpyAsync(cnt.data(), c.lists.m2l_cnt.p, sizeof(int) * nc, hipMemcpyDeviceToHost, s));
   XF_HIP(hipStreamSynchronize(s));
-  std::vector<int> owner(nm);
-  for (int t = 0; t < nc; t++)
-    for (int k = 0; k < cnt[t]; k++) owner[beg[t] + k] = t;
+  // entries numbered cell by cell (where a cell's list lies varies)
+  std::vector<int> owner(nm), place(nm);
+  for (int64_t t = 0, e = 0; t < nc; t++)
+    for (int k = 0; k < cnt[t]; k++, e++) {
+      owner[e] = int(t);
+      place[e] = beg[t] + k;
+    }
   std::mt19937_64 rng(seed);
   const int n = int(std::min<int64_t>(nsamples, nm));
   std::vector<int> pt(n), pidx(n);
   for (int i = 0; i < n; i++) {
     const int64_t e = int64_t(rng() % uint64_t(nm));
-    pidx[i] = int(e);
+    pidx[i] = place[e];
     pt[i] = owner[e];
   }
   Buf<int> dpt, didx;

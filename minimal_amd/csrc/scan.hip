@@ -182,12 +182,6 @@ void scan_exclusive_dev(const int *in, int *out, const int *count_dev, int count
   scan_launch<1>(a, 0, count_dev, count_bound, total, nullptr, nullptr, nullptr, scratch, s);
 }
 
-void scan_exclusive3(const int *in0, const int *in1, const int *in2, int *out0, int *out1, int *out2, int count,
-                     int *running, const int64_t *cap, int *flag, Buf<int> &scratch, hipStream_t s) {
-  ScanArrays<3> a{{in0, in1, in2}, {out0, out1, out2}};
-  scan_launch<3>(a, count, nullptr, count, nullptr, running, cap, flag, scratch, s);
-}
-
 // ---------------------------------------------------------------- radix sort
 constexpr int kRsThreads = 256;
 constexpr int kRsItems = 4;

@@ -10,9 +10,12 @@
 // is handed down from c's parent (the parent's pair split on the target
 // side) or b is a child of a pair (c, parent(b)) split on the source side.
 // One wavefront per target cell works through its pairs breadth-first in
-// LDS; every target's lists are therefore built by one wave, in a fixed
-// order, with no atomics.  Each level runs twice: a count pass, an
-// exclusive scan, and a fill pass writing at the scanned offsets.
+// LDS, so every target's lists are built by one wave, in a fixed order.  One
+// launch per level: the entries are staged in LDS, a workgroup reserves room
+// for its targets' lists with one atomic per output array, and the waves copy
+// their entries there (where a list lands varies from run to run, its
+// contents do not).  At 2^20 uniform bodies the lists took 365 us as a count
+// launch, an exclusive scan and a fill launch per level.
 // The MAC is evaluated in FP64 with contraction disabled, so each pair is
 // classified exactly as the reference classifies it.
 //
@@ -20,12 +23,19 @@
 // is visited in its 27 near images; every list entry carries its image
 // index (packed as cell * 32 + image, image = ix+1 + 3(iy+1) + 9(iz+1)) and
 // the MAC uses dX = Xc - Xb - iX * cycle.  Free space uses image 13 (0,0,0).
+#include <algorithm>
+
 #include "fmm_internal.h"
 
 namespace xf {
 
-constexpr int kTravWaves = 4;
-constexpr int kQCap = 2048;
+constexpr int kTravWaves = 8;
+// Pairs per target: the queue that fits beside the staged lists at 16 waves
+// per CU, and the one a pass is repeated with when a target overflows it.
+constexpr int kQSmall = 768, kQCap = 2048;
+// list entries staged per target; a longer list is walked a second time,
+// straight into place
+constexpr int kStageM2L = 256, kStageP2P = 128, kStageOut = 256;
 constexpr unsigned long long kEmpty = ~0ull;
 
 struct TravArgs {
@@ -46,7 +56,7 @@ struct TravArgs {
   int *m2l_cnt, *m2l_beg;
   int2 *m2l;
   int *p2p_cnt, *p2p_beg, *p2p;
-  int *flags;
+  int *flags, *tot;
   int64_t cap_m2l, cap_p2p, cap_out;
   // translation keys
   unsigned long long *hslots;
@@ -119,66 +129,29 @@ __device__ inline int wave_excl_scan(int v, int lane, int &total) {
   return x - v;
 }
 
-template <bool FILL>
-__global__ void __launch_bounds__(kTravWaves *kWave) k_traverse(TravArgs a) {
-  __shared__ int queue[kTravWaves][kQCap];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int w = threadIdx.x / kWave;
-  const int t = blockIdx.x * kTravWaves + w;
-  if (t >= a.lcount) return;
-  const int c = a.lstart + t;
-  int *q = queue[w];
+// The walk of one target's pairs (a wave); q[0 .. tail) holds the initial
+// ones.  emit(kind, position within that kind's list, entry, slot) receives
+// every entry, kind 0 = M2L, 1 = P2P, 2 = handed down to the children.
+// Returns false if the queue overflows.
+template <int QCAP, class F>
+__device__ __attribute__((always_inline)) inline bool walk(const TravArgs &a, int *q, int tail, int lane, double4 Xc,
+                                                           int leafc, int lc, int &nm, int &np, int &no, F &&emit) {
   const unsigned long long lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-
-  // initial pairs: handed down from the parent, or (root, root)
-  int tail;
-  if (a.in) {
-    const int par = a.cparent[c];
-    const int ib = a.in_beg[par];
-    tail = a.in_cnt[par];
-    if (tail > kQCap || int64_t(ib) + tail > a.cap_out) {
-      if (lane == 0) atomicOr(a.flags, 4);
-      return;
-    }
-    for (int i = lane; i < tail; i += kWave) q[i] = a.in[ib + i];
-  } else if (a.self_start) {
-    tail = 1;
-    if (lane == 0) q[0] = (c << 5) | 13;
-  } else if (a.periodic) {
-    tail = 27;
-    if (lane < 27) q[lane] = lane;  // (root, image) for the 27 near images
-  } else {
-    tail = 1;
-    if (lane == 0) q[0] = 13;  // (root, no shift)
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-
-  const double4 Xc = a.cx[c];
-  const int leafc = a.cnch[c] == 0;
-  const int lc = a.clevel[c];
   const double th2 = a.theta;
   int head = 0;
-  int nm = 0, np = 0, no = 0;
-  int bm = 0, bp = 0, bo = 0;
-  if (FILL) {
-    bm = a.m2l_beg[c];
-    bp = a.p2p_beg[c];
-    bo = a.out_beg[c];
-  }
+  nm = np = no = 0;
   while (head < tail) {
     const int k = min(kWave, tail - head);
     int b = -1, kind = -1, nchb = 0, lb = 0;
     double4 Xb;
     int img = 13;
     if (lane < k) {
-      const int e = q[(head + lane) % kQCap];
+      const int e = q[(head + lane) % QCAP];
       b = e >> 5;
       img = e & 31;
       Xb = a.scx[b];
       nchb = a.scnch[b];
-      if (FILL && a.want_keys) lb = a.sclevel[b];  // loaded beside the centre, ahead of the MAC
+      if (a.want_keys) lb = a.sclevel[b];  // loaded beside the centre, ahead of the MAC
       const double sx = ((img % 3) - 1) * a.cycle, sy = (((img / 3) % 3) - 1) * a.cycle,
                    sz = ((img / 9) - 1) * a.cycle;
       bool mac;
@@ -199,25 +172,20 @@ __global__ void __launch_bounds__(kTravWaves *kWave) k_traverse(TravArgs a) {
         kind = 3;
     }
     const unsigned long long mm = __ballot(kind == 0), mp = __ballot(kind == 1), mo = __ballot(kind == 2);
-    if (FILL) {
-      if (kind == 0) {
-        const int pos = bm + nm + __popcll(mm & lt);
-        int slot = 0;
-        if (a.want_keys) {
-          unsigned long long key;
-          if (m2l_key(Xc, lc, Xb, lb, img, a.periodic, key))
-            slot = key_insert(a.hslots, a.hmask, key, a.flags);
-          else
-            atomicOr(a.flags, 16);
-        }
-        if (pos < a.cap_m2l) a.m2l[pos] = make_int2((b << 5) | img, slot);
-      } else if (kind == 1) {
-        const int pos = bp + np + __popcll(mp & lt);
-        if (pos < a.cap_p2p) a.p2p[pos] = (b << 5) | img;
-      } else if (kind == 2) {
-        const int pos = bo + no + __popcll(mo & lt);
-        if (pos < a.cap_out) a.out[pos] = (b << 5) | img;
+    if (kind == 0) {
+      int slot = 0;
+      if (a.want_keys) {
+        unsigned long long key;
+        if (m2l_key(Xc, lc, Xb, lb, img, a.periodic, key))
+          slot = key_insert(a.hslots, a.hmask, key, a.flags);
+        else
+          atomicOr(a.flags, 16);
       }
+      emit(0, nm + __popcll(mm & lt), (b << 5) | img, slot);
+    } else if (kind == 1) {
+      emit(1, np + __popcll(mp & lt), (b << 5) | img, 0);
+    } else if (kind == 2) {
+      emit(2, no + __popcll(mo & lt), (b << 5) | img, 0);
     }
     nm += __popcll(mm);
     np += __popcll(mp);
@@ -226,13 +194,10 @@ __global__ void __launch_bounds__(kTravWaves *kWave) k_traverse(TravArgs a) {
     const int nadd = kind == 3 ? nchb : 0;
     int total;
     const int off = wave_excl_scan(nadd, lane, total);
-    if (tail - head - k + total > kQCap) {
-      if (lane == 0) atomicOr(a.flags, 4);
-      break;
-    }
+    if (tail - head - k + total > QCAP) return false;
     if (nadd) {
       const int first = a.scchild[b];
-      for (int i = 0; i < nadd; i++) q[(tail + off + i) % kQCap] = ((first + i) << 5) | img;
+      for (int i = 0; i < nadd; i++) q[(tail + off + i) % QCAP] = ((first + i) << 5) | img;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
@@ -240,17 +205,133 @@ __global__ void __launch_bounds__(kTravWaves *kWave) k_traverse(TravArgs a) {
     head += k;
     tail += total;
   }
-  if (!FILL && lane == 0) {
-    a.m2l_cnt[c] = nm;
-    a.p2p_cnt[c] = np;
-    a.out_cnt[c] = no;
-  }
+  return true;
 }
 
-// per-level offsets: exclusive scans of the three counts + running totals
-__global__ void k_hash_clear(unsigned long long *slots, int n) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) slots[i] = kEmpty;
+// Initial pairs of target c: handed down from the parent, or (root, root).
+// Returns their number, -1 if they overflow the queue.
+template <int QCAP>
+__device__ inline int start_pairs(const TravArgs &a, int c, int lane, int *q) {
+  int tail;
+  if (a.in) {
+    const int par = a.cparent[c];
+    const int ib = a.in_beg[par];
+    tail = a.in_cnt[par];
+    if (tail > QCAP || int64_t(ib) + tail > a.cap_out) return -1;
+    for (int i = lane; i < tail; i += kWave) q[i] = a.in[ib + i];
+  } else if (a.self_start) {
+    tail = 1;
+    if (lane == 0) q[0] = (c << 5) | 13;
+  } else if (a.periodic) {
+    tail = 27;
+    if (lane < 27) q[lane] = lane;  // (root, image) for the 27 near images
+  } else {
+    tail = 1;
+    if (lane == 0) q[0] = 13;  // (root, no shift)
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  return tail;
+}
+
+template <int QCAP>
+__global__ void __launch_bounds__(kTravWaves *kWave) k_traverse(TravArgs a) {
+  __shared__ int queue[kTravWaves][QCAP];
+  __shared__ int2 sm[kTravWaves][kStageM2L];
+  __shared__ int sp[kTravWaves][kStageP2P], so[kTravWaves][kStageOut];
+  __shared__ int cnt[kTravWaves][3], base[3];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int w = threadIdx.x / kWave;
+  const int t = blockIdx.x * kTravWaves + w;
+  const int c = a.lstart + t;
+  const bool in = t < a.lcount;
+  int *q = queue[w];
+  double4 Xc = make_double4(0, 0, 0, 0);
+  int leafc = 0, lc = 0, nm = 0, np = 0, no = 0;
+  if (in) {
+    Xc = a.cx[c];
+    leafc = a.cnch[c] == 0;
+    lc = a.clevel[c];
+    const int tail = start_pairs<QCAP>(a, c, lane, q);
+    const bool ok = tail >= 0 && walk<QCAP>(a, q, tail, lane, Xc, leafc, lc, nm, np, no,
+                                            [&](int kind, int pos, int entry, int slot) {
+                                              if (kind == 0) {
+                                                if (pos < kStageM2L) sm[w][pos] = make_int2(entry, slot);
+                                              } else if (kind == 1) {
+                                                if (pos < kStageP2P) sp[w][pos] = entry;
+                                              } else if (pos < kStageOut) {
+                                                so[w][pos] = entry;
+                                              }
+                                            });
+    if (!ok) {
+      // a repeated pass with the large queue, or (that one too) an error
+      if (lane == 0) atomicOr(a.flags, QCAP < kQCap ? kListQueue : 4);
+      nm = np = no = 0;
+    }
+  }
+  if (lane == 0) {
+    cnt[w][0] = nm;
+    cnt[w][1] = np;
+    cnt[w][2] = no;
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    int s = 0;
+    for (int i = 0; i < kTravWaves; i++) s += cnt[i][threadIdx.x];
+    const int64_t cap = threadIdx.x == 0 ? a.cap_m2l : threadIdx.x == 1 ? a.cap_p2p : a.cap_out;
+    int b0 = 0;
+    if (s) {
+      b0 = atomicAdd(a.tot + threadIdx.x, s);
+      if (int64_t(b0) + s > cap) atomicOr(a.flags, 1);
+    }
+    base[threadIdx.x] = b0;
+  }
+  __syncthreads();
+  if (!in) return;
+  int bm = base[0], bp = base[1], bo = base[2];
+  for (int i = 0; i < w; i++) {
+    bm += cnt[i][0];
+    bp += cnt[i][1];
+    bo += cnt[i][2];
+  }
+  if (lane == 0) {
+    a.m2l_beg[c] = bm;
+    a.m2l_cnt[c] = nm;
+    a.p2p_beg[c] = bp;
+    a.p2p_cnt[c] = np;
+    a.out_beg[c] = bo;
+    a.out_cnt[c] = no;
+  }
+  auto place = [&](int kind, int pos, int entry, int slot) {
+    if (kind == 0) {
+      if (bm + pos < a.cap_m2l) a.m2l[bm + pos] = make_int2(entry, slot);
+    } else if (kind == 1) {
+      if (bp + pos < a.cap_p2p) a.p2p[bp + pos] = entry;
+    } else if (bo + pos < a.cap_out) {
+      a.out[bo + pos] = entry;
+    }
+  };
+  if (nm > kStageM2L || np > kStageP2P || no > kStageOut) {
+    walk<QCAP>(a, q, start_pairs<QCAP>(a, c, lane, q), lane, Xc, leafc, lc, nm, np, no, place);
+    return;
+  }
+  for (int i = lane; i < nm; i += kWave) place(0, i, sm[w][i].x, sm[w][i].y);
+  for (int i = lane; i < np; i += kWave) place(1, i, sp[w][i], 0);
+  for (int i = lane; i < no; i += kWave) place(2, i, so[w][i], 0);
+}
+
+// Start of a pass: empty key table, zero totals and flags, zero locals, and
+// in a forest empty lists for the cells above the problems' roots.
+__global__ void __launch_bounds__(256) k_lists_init(unsigned long long *__restrict__ slots, int nslots,
+                                                    int *__restrict__ tot, double *__restrict__ L, int64_t nL,
+                                                    TravArgs a, int nv) {
+  const int64_t i0 = int64_t(blockIdx.x) * 256 + threadIdx.x, n = int64_t(gridDim.x) * 256;
+  for (int64_t i = i0; i < nslots; i += n) slots[i] = kEmpty;
+  for (int64_t i = i0; i < nL; i += n) L[i] = 0.0;
+  if (i0 < 8) tot[i0] = 0;
+  for (int64_t i = i0; i < nv; i += n)
+    a.m2l_cnt[i] = a.m2l_beg[i] = a.p2p_cnt[i] = a.p2p_beg[i] = a.out_cnt[i] = a.out_beg[i] = 0;
 }
 
 __global__ void k_hash_collect(const unsigned long long *__restrict__ slots, int n,
@@ -269,36 +350,43 @@ __global__ void k_hash_collect(const unsigned long long *__restrict__ slots, int
 // given) skip a pass that is repeated or ranked by the radix sort instead.
 __global__ void k_entry_ids(int2 *__restrict__ m2l, const int *__restrict__ total, int64_t cap,
                             const int *__restrict__ slot2id, const int *__restrict__ flags) {
-  if (flags && (*flags & (1 | 8 | 32))) return;
+  if (flags && (*flags & (kListRetry | 32))) return;
   const int64_t n = min(int64_t(*total), cap);
   for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256)
     m2l[i].y = slot2id[m2l[i].y];
 }
 
-// Key sort for small key sets (the usual case: hundreds to a few thousand
-// distinct translations): one workgroup, keys in LDS, each key's rank is the
-// number of smaller keys (keys are distinct).  Writes the sorted keys in
-// place and the slot -> rank map.  A larger set raises bit 32 of *flags
-// and is left to the radix sort.
-constexpr int kRankMax = 6144;
-__global__ void __launch_bounds__(1024) k_key_rank(unsigned long long *__restrict__ keys, const int *__restrict__ sl,
-                                                   const int *__restrict__ count, int *__restrict__ slot2id,
+// Key sort for the usual key sets (hundreds to some ten thousand distinct
+// translations): a key's rank is the number of smaller keys.  A workgroup
+// ranks 64 keys, its 16 waves counting over a sixteenth of the set each (the
+// keys they compare with are wave-uniform: scalar loads).  Writes the sorted
+// keys and the slot -> rank map.  A larger set raises bit 32 of *flags and is
+// left to the radix sort.  (One workgroup over the whole set in LDS: 34 us for
+// 1,164 keys, 109 us for 2,180, now 5 - 6 us.)
+constexpr int kRankMax = 12288;
+__global__ void __launch_bounds__(1024) k_key_rank(const unsigned long long *__restrict__ in,
+                                                   const int *__restrict__ sl, const int *__restrict__ count,
+                                                   unsigned long long *__restrict__ keys, int *__restrict__ slot2id,
                                                    int *__restrict__ flags) {
-  __shared__ unsigned long long K[kRankMax];
+  __shared__ int part[16][kWave];
   const int n = *count;
   if (n > kRankMax) {
-    if (threadIdx.x == 0) atomicOr(flags, 32);
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(flags, 32);
     return;
   }
-  for (int i = threadIdx.x; i < n; i += 1024) K[i] = keys[i];
+  const int lane = threadIdx.x & (kWave - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int i = blockIdx.x * kWave + lane;
+  if (int(blockIdx.x) * kWave >= n) return;
+  const unsigned long long k = i < n ? in[i] : 0ull;
+  int r = 0;
+  for (int j = w * n / 16; j < (w + 1) * n / 16; j++) r += in[j] < k;
+  part[w][lane] = r;
   __syncthreads();
-  for (int i = threadIdx.x; i < n; i += 1024) {
-    const unsigned long long k = K[i];
-    int r = 0;
-    for (int j = 0; j < n; j++) r += K[j] < k;
-    keys[r] = k;
-    slot2id[sl[i]] = r;
-  }
+  if (w != 0 || i >= n) return;
+  r = 0;
+  for (int q = 0; q < 16; q++) r += part[q][lane];
+  keys[r] = k;
+  slot2id[sl[i]] = r;
 }
 
 __global__ void k_slot_ids(const int *__restrict__ sl, int n, int *__restrict__ slot2id) {
@@ -321,6 +409,7 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
   Lr.out_beg.ensure(nc);
   Lr.out_cnt.ensure(nc);
   Lr.tot.ensure(8);
+  tc.L.ensure(size_t(nc) * tc.P * tc.P);
   if (Lr.cap_m2l < 200 * nc) Lr.cap_m2l = 200 * nc;
   if (Lr.cap_p2p < 96 * nc) Lr.cap_p2p = 96 * nc;
   if (Lr.cap_out < 96 * nc) Lr.cap_out = 96 * nc;
@@ -328,26 +417,11 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
 
   int tot[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   bool done = false;
-  for (int attempt = 0; attempt < 4; attempt++) {
+  for (int attempt = 0; attempt < 5; attempt++) {
     Lr.m2l.ensure(Lr.cap_m2l);
     Lr.p2p.ensure(Lr.cap_p2p);
     Lr.out.ensure(Lr.cap_out);
-    XF_HIP(hipMemsetAsync(Lr.tot.p, 0, 8 * sizeof(int), s));
-    // capacities on the device, uploaded when they change (from pinned
-    // memory: an asynchronous copy)
-    const int64_t caps[3] = {Lr.cap_m2l, Lr.cap_p2p, Lr.cap_out};
-    if (!Lr.capd.p || !std::equal(caps, caps + 3, Lr.caps_up)) {
-      Lr.capd.ensure(3);
-      Lr.caps_pin.ensure(3);
-      std::copy(caps, caps + 3, Lr.caps_pin.p);
-      XF_HIP(hipMemcpyAsync(Lr.capd.p, Lr.caps_pin.p, sizeof(caps), hipMemcpyHostToDevice, s));
-      std::copy(caps, caps + 3, Lr.caps_up);
-    }
-    if (keys) {
-      Lr.hslots.ensure(Lr.hcap);
-      hipLaunchKernelGGL(k_hash_clear, dim3(ceil_div(Lr.hcap, 256)), dim3(256), 0, s, Lr.hslots.p, Lr.hcap);
-      XF_LAUNCH();
-    }
+    if (keys) Lr.hslots.ensure(Lr.hcap);
     TravArgs a{};
     a.cx = T.cx.p;
     a.cnch = T.cnch.p;
@@ -370,6 +444,7 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
     a.p2p_beg = Lr.p2p_beg.p;
     a.p2p = Lr.p2p.p;
     a.flags = Lr.tot.p + 3;
+    a.tot = Lr.tot.p;
     a.cap_m2l = Lr.cap_m2l;
     a.cap_p2p = Lr.cap_p2p;
     a.cap_out = Lr.cap_out;
@@ -381,11 +456,11 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
     const int l0 = T.lroot;
     if (l0 > 0 && &tc != &sc) fail(EXAFMM_ERR_UNSUPPORTED, "a forest's horizontal pass needs source == target");
     a.self_start = l0 > 0;
-    if (l0 > 0) {
-      const size_t nv = size_t(T.lstart[l0]);
-      for (int *z : {Lr.m2l_cnt.p, Lr.m2l_beg.p, Lr.p2p_cnt.p, Lr.p2p_beg.p, Lr.out_cnt.p, Lr.out_beg.p})
-        XF_HIP(hipMemsetAsync(z, 0, sizeof(int) * nv, s));
-    }
+    const int64_t nL = nc * tc.P * tc.P;
+    hipLaunchKernelGGL(k_lists_init, dim3(int(std::max<int64_t>(64, std::min<int64_t>(ceil_div(nL, 256 * 4), 2048)))),
+                       dim3(256), 0, s, Lr.hslots.p, keys ? Lr.hcap : 0, Lr.tot.p, tc.L.p, nL, a,
+                       l0 > 0 ? T.lstart[l0] : 0);
+    XF_LAUNCH();
     for (int l = l0; l <= T.depth; l++) {
       a.lstart = T.lstart[l];
       a.lcount = T.lstart[l + 1] - T.lstart[l];
@@ -393,12 +468,8 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
       a.in_beg = Lr.out_beg.p;
       a.in_cnt = Lr.out_cnt.p;
       const int g = ceil_div(a.lcount, kTravWaves);
-      hipLaunchKernelGGL(k_traverse<false>, dim3(g), dim3(kTravWaves * kWave), 0, s, a);
-      XF_LAUNCH();
-      scan_exclusive3(Lr.m2l_cnt.p + a.lstart, Lr.p2p_cnt.p + a.lstart, Lr.out_cnt.p + a.lstart,
-                      Lr.m2l_beg.p + a.lstart, Lr.p2p_beg.p + a.lstart, Lr.out_beg.p + a.lstart, a.lcount, Lr.tot.p,
-                      Lr.capd.p, Lr.tot.p + 3, Lr.scan_tmp, s);
-      hipLaunchKernelGGL(k_traverse<true>, dim3(g), dim3(kTravWaves * kWave), 0, s, a);
+      hipLaunchKernelGGL(Lr.large_queue ? k_traverse<kQCap> : k_traverse<kQSmall>, dim3(g), dim3(kTravWaves * kWave), 0,
+                         s, a);
       XF_LAUNCH();
     }
     if (after_kernels) after_kernels();
@@ -409,14 +480,14 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
       Lr.kscratch.ensure(size_t(Lr.hcap) * 2 + 8);
       Lr.slot2id.ensure(Lr.hcap);
       hipLaunchKernelGGL(k_hash_collect, dim3(ceil_div(Lr.hcap, 256)), dim3(256), 0, s, Lr.hslots.p, Lr.hcap,
-                         Lr.keys.p, Lr.kscratch.p, Lr.tot.p + 6);
+                         Lr.keys.p + Lr.hcap, Lr.kscratch.p, Lr.tot.p + 6);
       XF_LAUNCH();
       // The usual small key set is ranked, and the entries renumbered,
       // before the totals are read, so the read overlaps them (counts from
       // the device; a repeated pass redoes it all, a set above kRankMax is
       // flagged and sorted below).
-      hipLaunchKernelGGL(k_key_rank, dim3(1), dim3(1024), 0, s, Lr.keys.p, Lr.kscratch.p, Lr.tot.p + 6,
-                         Lr.slot2id.p, Lr.tot.p + 3);
+      hipLaunchKernelGGL(k_key_rank, dim3(std::min(Lr.hcap, kRankMax) / kWave), dim3(1024), 0, s, Lr.keys.p + Lr.hcap,
+                         Lr.kscratch.p, Lr.tot.p + 6, Lr.keys.p, Lr.slot2id.p, Lr.tot.p + 3);
       XF_LAUNCH();
       hipLaunchKernelGGL(k_entry_ids, dim3(int(std::min<int64_t>(ceil_div(Lr.cap_m2l, 256), 4096))), dim3(256), 0, s,
                          Lr.m2l.p, Lr.tot.p, Lr.cap_m2l, Lr.slot2id.p, Lr.tot.p + 3);
@@ -431,6 +502,10 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
     if (after_kernels && (flags & kListRetry)) stream_wait(tc.s1);
     if (flags & 4) fail(EXAFMM_ERR_CAPACITY, "traversal work queue overflow (pairs per target cell > 2048)");
     if (flags & 16) fail(EXAFMM_ERR_CAPACITY, "M2L offset out of key range");
+    if (flags & kListQueue) {  // from here on with the large queue
+      Lr.large_queue = true;
+      continue;
+    }
     if (flags & 1) {  // list capacity: retry with the exact totals
       Lr.cap_m2l = std::max<int64_t>(Lr.cap_m2l * 2, tot[0]);
       Lr.cap_p2p = std::max<int64_t>(Lr.cap_p2p * 2, tot[1]);
@@ -446,11 +521,11 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
     done = true;
     break;
   }
-  if (!done) fail(EXAFMM_ERR_CAPACITY, "interaction lists or key table still full after 4 passes");
+  if (!done) fail(EXAFMM_ERR_CAPACITY, "interaction lists or key table still full after 5 passes");
   Lr.valid = true;
   Lr.nkeys = 0;
   if (keys) {
-    unsigned long long *k1 = Lr.keys.p, *k2 = Lr.keys.p + Lr.hcap;
+    unsigned long long *k1 = Lr.keys.p + Lr.hcap, *k2 = Lr.keys.p;
     int *v1 = Lr.kscratch.p, *v2 = Lr.kscratch.p + Lr.hcap;
     const int nk = tot[6];
     if (tot[3] & 32) {  // more keys than k_key_rank holds
