@@ -129,7 +129,7 @@ constexpr int kPinLevelMax = 0;   // 9: flags, largest prefix population of leve
 constexpr int kPinLevels = 16;    // kMaxLevel + 2 level sizes
 constexpr int kPinMisc = 48;      // 19: tree flags and counters
 constexpr int kPinTot = 72;       // 8: list totals and flags
-constexpr int kPinPlan = 80;      // 3: M2L slots, tiles, cells in tiles
+constexpr int kPinPlan = 80;      // 4: M2L slots, tiles, cells in tiles, key set differs from the operators'
 constexpr int kPinInts = 96;
 // traversal flag bits that make the pass repeat: list capacity, key table
 // full, small work queue overflow
@@ -243,7 +243,6 @@ struct Ctx {
   std::string last_error;
   HostBuf<int> pin_i;                   // kPin* slots
   HostBuf<double> pin_d;                // root cube
-  HostBuf<unsigned long long> pin_keys; // M2L key set
 
   exafmm_body *bodies = nullptr;   // caller's array (device pointer or our mirror)
   exafmm_body *host_bodies = nullptr;
@@ -281,14 +280,15 @@ struct Ctx {
   // What ops32 holds: operators are pure functions of (key, P, truncation,
   // precision) plus R0 and the cycle for periodic keys, so an unchanged key
   // set is not generated again.
-  std::vector<unsigned long long> ops_keys;
+  Buf<unsigned long long> ops_keys;
+  int ops_nkeys = 0;
   // keyed M2L tiles built by m2l_prepare for the current lists
   bool m2l_ready = false;
   int m2l_ntiles = 0;
   int m2l_tstride = 0;      // stride of the tile arrays in `tiles` (a bound on the tile count)
   bool m2l_by_level = false;  // each tile holds cells of one level
   int m2l_ncell_tiled = 0;  // cells that receive M2L (the tiles' columns)
-  Buf<int> m2l_misc, m2l_rs_hist, m2l_scan;
+  Buf<int> m2l_misc, m2l_rs_hist;
   Buf<double> m2l_part64;   // FP64 partial locals of the list shares (m2l.hip)
   Buf<float> m2l_part;      // FP32 partial locals of the key slices [slice][cell][P^2]
   // variable-order M2L: order of each (tile, key), parallel to tile_keys

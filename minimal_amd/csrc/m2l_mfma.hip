@@ -88,20 +88,30 @@ __device__ inline unsigned mix32(unsigned h) {
   return h;
 }
 
+// Counters of the tile build (m2l_misc): group populations 0..255, then the
+// plan [slots, tiles, cells in tiles, key set differs].
+constexpr int kMiscPlan = 256, kMiscInts = 260;
+
 // Sort key of a target cell: group in bits 16..23 (255 = no M2L) -- the
-// octant, or (level, octant) with `by_level` -- and with `minhash` the top 16 bits of the minimum hashed key id of
-// its list below: cells with similar key sets share that minimum with a
-// probability equal to the sets' Jaccard similarity, so sorting by it packs
-// cells of like key sets into the same tile (fewer empty GEMM slots).
+// octant, or (level, octant) with `by_level` -- and the top 16 bits of the
+// minimum hashed key id of its list below: cells with similar key sets share
+// that minimum with a probability equal to the sets' Jaccard similarity, so
+// sorting by it packs cells of like key sets into the same tile (fewer empty
+// GEMM slots).
 // One wave per cell: the lanes take the list entries in turn and the
 // minimum hash is a wave reduction.
 __global__ void __launch_bounds__(256) k_group_keys(int ncells, const double4 *__restrict__ cx,
                                                     const int *__restrict__ cparent, const int *__restrict__ clevel,
                                                     const int *__restrict__ m2l_beg, const int *__restrict__ m2l_cnt,
-                                                    const int2 *__restrict__ list, int minhash, int lmin, int by_level,
-                                                    unsigned long long *__restrict__ key, int *__restrict__ val) {
+                                                    const int2 *__restrict__ list, int lmin, int by_level,
+                                                    unsigned long long *__restrict__ key, unsigned *__restrict__ key32,
+                                                    int *__restrict__ val, int *__restrict__ misc) {
   const int lane = threadIdx.x & (kWave - 1);
   const int c = blockIdx.x * (256 / kWave) + int(threadIdx.x / kWave);
+  if (blockIdx.x == 0) {  // counters of the launches that follow
+    misc[threadIdx.x] = 0;
+    if (threadIdx.x < kMiscInts - 256) misc[256 + threadIdx.x] = 0;
+  }
   if (c >= ncells) return;  // whole wave
   unsigned g = 255, mh = 0;
   // cells above level lmin take their M2L elsewhere (FP64, per pair)
@@ -114,29 +124,103 @@ __global__ void __launch_bounds__(256) k_group_keys(int ncells, const double4 *_
       o = (a.x > b.x) + ((a.y > b.y) << 1) + ((a.z > b.z) << 2);
     }
     g = (by_level ? unsigned(min(clevel[c], 30)) * 8 : 0u) + o;
-    if (minhash) {
-      unsigned m = 0xffffffffu;
-      const int b0 = m2l_beg[c];
-      for (int i = lane; i < n; i += kWave) m = min(m, mix32(unsigned(list[b0 + i].y)));
+    unsigned m = 0xffffffffu;
+    const int b0 = m2l_beg[c];
+    for (int i = lane; i < n; i += kWave) m = min(m, mix32(unsigned(list[b0 + i].y)));
 #pragma unroll
-      for (int d = 32; d > 0; d >>= 1) m = min(m, unsigned(__shfl_xor(int(m), d)));
-      mh = m >> 16;  // 16 bits: three 8-bit sort passes over the 24-bit key
-    }
+    for (int d = 32; d > 0; d >>= 1) m = min(m, unsigned(__shfl_xor(int(m), d)));
+    mh = m >> 16;  // 16 bits: three 8-bit sort passes over the 24-bit key
   }
   if (lane == 0) {
-    key[c] = (unsigned long long)(g << 16 | mh);
-    val[c] = c;
+    if (key32) {
+      key32[c] = g << 16 | mh;
+    } else {
+      key[c] = (unsigned long long)(g << 16 | mh);
+      val[c] = c;
+    }
   }
 }
 
+// Tiles from the group populations gc[0..254] (group 255 = cells without
+// M2L, not tiled): each group's cells, in sorted order, are cut into tiles
+// of at most kTileN.  Writes each tile's first cell and count, and plan[1] =
+// tiles, plan[2] = cells in tiles.  (Launches of one workgroup like this one
+// and k_tile_scan stay launches: run by the last workgroup of the launch before
+// them, the agent-scope fences of every workgroup of that launch write back
+// and invalidate the L2s under the P2P that runs beside it, which cost more.)
+__global__ void __launch_bounds__(256) k_tile_plan(int *__restrict__ misc, int *__restrict__ tfirst,
+                                                   int *__restrict__ tcount) {
+  __shared__ int wt[4][2];
+  const int gi = threadIdx.x, lane = gi & 63, w = gi >> 6;
+  const int n = gi < 255 ? misc[gi] : 0, nt = (n + kTileN - 1) / kTileN;
+  int it = nt, ic = n;
+  for (int d = 1; d < 64; d <<= 1) {
+    const int x = __shfl_up(it, d), y = __shfl_up(ic, d);
+    if (lane >= d) {
+      it += x;
+      ic += y;
+    }
+  }
+  if (lane == 63) {
+    wt[w][0] = it;
+    wt[w][1] = ic;
+  }
+  __syncthreads();
+  for (int i = 0; i < w; i++) {
+    it += wt[i][0];
+    ic += wt[i][1];
+  }
+  if (gi == 255) {
+    misc[kMiscPlan + 1] = it;
+    misc[kMiscPlan + 2] = ic;
+  }
+  for (int j = 0; j * kTileN < n; j++) {
+    tfirst[it - nt + j] = ic - n + j * kTileN;
+    tcount[it - nt + j] = min(kTileN, n - j * kTileN);
+  }
+}
+
+// The cells in sorted order and the group populations after the radix sort.
 __global__ void __launch_bounds__(256) k_group_hist(int ncells, const unsigned long long *__restrict__ key,
-                                                    int *__restrict__ cnt) {
+                                                    const int *__restrict__ val, int *__restrict__ sorted,
+                                                    int *__restrict__ misc) {
   __shared__ int h[256];
   h[threadIdx.x] = 0;
   __syncthreads();
-  for (int c = blockIdx.x * 256 + threadIdx.x; c < ncells; c += gridDim.x * 256) atomicAdd(&h[int(key[c] >> 16)], 1);
+  for (int c = blockIdx.x * 256 + threadIdx.x; c < ncells; c += gridDim.x * 256) {
+    atomicAdd(&h[int(key[c] >> 16)], 1);
+    sorted[c] = val[c];
+  }
   __syncthreads();
-  if (h[threadIdx.x]) atomicAdd(&cnt[threadIdx.x], h[threadIdx.x]);
+  if (h[threadIdx.x]) atomicAdd(&misc[threadIdx.x], h[threadIdx.x]);
+}
+
+// Small trees: each cell's place is the number of cells that sort before it
+// (lower key, or equal key and lower index).  A workgroup places 64 cells, its
+// 16 waves counting over a sixteenth of the cells each (wave-uniform keys:
+// scalar loads).  Quadratic, and one launch where the radix sort takes nine:
+// at 16,384 cells it costs what they do.
+constexpr int kCellRankMax = 16384;
+__global__ void __launch_bounds__(1024) k_cell_rank(int n, const unsigned *__restrict__ key, int *__restrict__ sorted,
+                                                    int *__restrict__ misc) {
+  __shared__ int part[16][kWave];
+  const int lane = threadIdx.x & (kWave - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int i = blockIdx.x * kWave + lane;
+  const unsigned k = i < n ? key[i] : 0u;
+  const int j0 = w * n / 16, j1 = (w + 1) * n / 16, first = blockIdx.x * kWave;
+  int r = 0;
+  // before this workgroup's cells equal keys count, after them they do not
+  for (int j = j0; j < min(j1, first); j++) r += key[j] <= k;
+  for (int j = max(j0, first); j < min(j1, first + kWave); j++) r += key[j] < k || (key[j] == k && j < i);
+  for (int j = max(j0, first + kWave); j < j1; j++) r += key[j] < k;
+  part[w][lane] = r;
+  __syncthreads();
+  if (w == 0 && i < n) {
+    r = 0;
+    for (int q = 0; q < 16; q++) r += part[q][lane];
+    sorted[r] = i;
+    atomicAdd(&misc[k >> 16], 1);
+  }
 }
 
 // Tile kernels: one thread per target column walks that column's M2L list
@@ -164,60 +248,70 @@ __device__ inline void tile_bitmap(const int *cells, int ncol, const int *beg, c
   __syncthreads();
 }
 
-// Tiles from the group populations gc[0..254] (group 255 = cells without
-// M2L, not tiled): each group's cells, in sorted order, are cut into tiles
-// of at most tn.  Writes each tile's first cell and count, and plan[0] =
-// tiles, plan[1] = cells in tiles.
-__global__ void __launch_bounds__(256) k_tile_plan(const int *__restrict__ gc, int tn, int *__restrict__ tfirst,
-                                                   int *__restrict__ tcount, int *__restrict__ plan) {
-  __shared__ int tb[256], cb[256];
-  const int gi = threadIdx.x;
-  const int n = gi < 255 ? gc[gi] : 0;
-  tb[gi] = (n + tn - 1) / tn;
-  cb[gi] = n;
-  __syncthreads();
-  if (gi == 0) {  // exclusive prefixes of tiles and cells over the groups
-    int t = 0, cc = 0;
-    for (int i = 0; i < 256; i++) {
-      const int a = tb[i], b = cb[i];
-      tb[i] = t;
-      cb[i] = cc;
-      t += a;
-      cc += b;
-    }
-    plan[0] = t;
-    plan[1] = cc;
-  }
-  __syncthreads();
-  for (int j = 0; j * tn < n; j++) {
-    tfirst[tb[gi] + j] = cb[gi] + j * tn;
-    tcount[tb[gi] + j] = min(tn, n - j * tn);
-  }
-}
-
+// Key set and its size per tile (launched over the bound of tiles).  The
+// launch also compares the key set with the one the operators were generated
+// for (old_keys, null if there is none to compare with).
 constexpr int kTileCountThreads = 1024;
-__global__ void __launch_bounds__(kTileCountThreads) k_tile_count(const int *__restrict__ tfirst, const int *__restrict__ tcount,
-                                                    const int *__restrict__ sorted, const int *__restrict__ beg,
-                                                    const int *__restrict__ cnt, const int2 *__restrict__ list,
-                                                    int nkeys, const int *__restrict__ plan, int *__restrict__ tU,
-                                                    unsigned *__restrict__ tbits) {
+__global__ void __launch_bounds__(kTileCountThreads)
+    k_tile_count(const int *__restrict__ tfirst, const int *__restrict__ tcount, const int *__restrict__ sorted,
+                 const int *__restrict__ beg, const int *__restrict__ cnt, const int2 *__restrict__ list, int nkeys,
+                 int *__restrict__ misc, int *__restrict__ tU, unsigned *__restrict__ tbits,
+                 const unsigned long long *__restrict__ keys, const unsigned long long *__restrict__ old_keys) {
   extern __shared__ unsigned bm[];
   __shared__ int tot;
-  if (int(blockIdx.x) >= plan[0]) return;  // launched over the bound of tiles
-  const int nwords = (nkeys + 31) / 32;
-  const int *cells = sorted + tfirst[blockIdx.x];
-  const int ncol = tcount[blockIdx.x];
-  tile_bitmap(cells, ncol, beg, cnt, list, bm, nwords);
-  if (threadIdx.x == 0) tot = 0;
-  __syncthreads();
-  int s = 0;
-  for (int i = threadIdx.x; i < nwords; i += blockDim.x) {
-    s += __popc(bm[i]);
-    tbits[int64_t(blockIdx.x) * nwords + i] = bm[i];  // the key set, for k_tile_fill
+  const int nwords = (nkeys + 31) / 32, ntiles = misc[kMiscPlan + 1];
+  if (int(blockIdx.x) < ntiles) {
+    const int *cells = sorted + tfirst[blockIdx.x];
+    const int ncol = tcount[blockIdx.x];
+    tile_bitmap(cells, ncol, beg, cnt, list, bm, nwords);
+    if (threadIdx.x == 0) tot = 0;
+    __syncthreads();
+    int s = 0;
+    for (int i = threadIdx.x; i < nwords; i += blockDim.x) {
+      s += __popc(bm[i]);
+      tbits[int64_t(blockIdx.x) * nwords + i] = bm[i];  // the key set, for k_tile_fill
+    }
+    atomicAdd(&tot, s);
+    __syncthreads();
+    if (threadIdx.x == 0) tU[blockIdx.x] = tot;
   }
-  atomicAdd(&tot, s);
-  __syncthreads();
-  if (threadIdx.x == 0) tU[blockIdx.x] = tot;
+  if (old_keys)
+    for (int i = blockIdx.x * kTileCountThreads + threadIdx.x; i < nkeys; i += gridDim.x * kTileCountThreads)
+      if (keys[i] != old_keys[i]) atomicOr(&misc[kMiscPlan + 3], 1);
+}
+
+// Tile bases: exclusive scan of the slot counts (one workgroup), and the plan
+// for the host (pinned memory).
+__global__ void __launch_bounds__(kTileCountThreads) k_tile_scan(const int *__restrict__ misc,
+                                                                 const int *__restrict__ tU, int *__restrict__ tbase,
+                                                                 int *host_plan) {
+  __shared__ int wt[kTileCountThreads / kWave];
+  const int ntiles = misc[kMiscPlan + 1];
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  int carry = 0;
+  for (int t0 = 0; t0 < ntiles; t0 += kTileCountThreads) {
+    const int t = t0 + threadIdx.x;
+    const int v = t < ntiles ? tU[t] : 0;
+    int incl = v;
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int x = __shfl_up(incl, d);
+      if (lane >= d) incl += x;
+    }
+    if (lane == kWave - 1) wt[w] = incl;
+    __syncthreads();
+    int before = carry, all = 0;
+    for (int i = 0; i < kTileCountThreads / kWave; i++) {
+      before += i < w ? wt[i] : 0;
+      all += wt[i];
+    }
+    if (t < ntiles) tbase[t] = before + incl - v;
+    carry += all;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    const int plan[4] = {carry, ntiles, misc[kMiscPlan + 2], misc[kMiscPlan + 3]};
+    for (int i = 0; i < 4; i++) __hip_atomic_store(host_plan + i, plan[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 // Key list (ascending) and source matrix [U][tn] (-1 = no pair) of a tile.
@@ -1354,14 +1448,18 @@ static GemmShape gemm_shape(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, bo
   return best;
 }
 
-static bool ops_cached(const Ctx &c, const std::vector<unsigned long long> &keys, int fillP, int bf16) {
+// Whether the operators in ops32 were generated for this configuration and a
+// key set of this size (the keys themselves are compared on the device).
+static bool ops_comparable(const Ctx &c, int nkeys, int fillP, int bf16) {
   const bool periodic = c.cfg.images > 0;
-  return c.ops_P == c.P && c.ops_fill == fillP && c.ops_bf16 == bf16 && c.ops_keys == keys &&
+  return c.ops_P == c.P && c.ops_fill == fillP && c.ops_bf16 == bf16 && c.ops_nkeys == nkeys &&
          (!periodic || (c.ops_R0 == c.t.R0 && c.ops_cycle == c.cfg.cycle));
 }
 
-static void ops_remember(Ctx &c, std::vector<unsigned long long> keys, int fillP, int bf16) {
-  c.ops_keys = std::move(keys);
+static void ops_remember(Ctx &c, int nkeys, int fillP, int bf16, hipStream_t s) {
+  c.ops_keys.ensure(std::max(nkeys, 1));
+  XF_HIP(hipMemcpyAsync(c.ops_keys.p, c.lists.keys.p, sizeof(unsigned long long) * nkeys, hipMemcpyDeviceToDevice, s));
+  c.ops_nkeys = nkeys;
   c.ops_P = c.P;
   c.ops_fill = fillP;
   c.ops_bf16 = bf16;
@@ -1387,34 +1485,21 @@ void m2l_prepare(Ctx &c, hipStream_t s) {
   const int nkeys = c.lists.nkeys;
   if (nkeys > (1 << 16)) fail(EXAFMM_ERR_CAPACITY, "more than 65536 distinct M2L translations");
 
-  // 1. tiles: cells with pairs grouped by (level, octant), then key set
+  // 1. tiles: cells with pairs grouped by octant, then key set
   c.t.key.ensure(nc);
   c.t.key2.ensure(nc);
   c.t.val.ensure(nc);
   c.t.val2.ensure(nc);
-  // cells sorted by (level, octant, min-hash of key set), BFS order within
-  // ties: on adaptive trees this raises the fraction of non-empty GEMM slots
+  // cells sorted by (group, min-hash of key set), BFS order within ties: on adaptive trees this raises the fraction of non-empty GEMM slots
   // (measured 0.50 -> 0.58 on a 2^22-body Plummer set); on uniform trees,
   // where BFS neighbours already share key sets, it changes little.
-  const int minhash = 1;
   // Tiles mix the levels (keys are scale-free: on a clustered set of 200,000
   // bodies half as many (tile, key) slots as with tiles of one level), unless
   // the keys carry the level (periodic) or the slots take one learned order
   // each, chosen for cells of one size.
   const bool by_level = c.cfg.images > 0 || learned_orders(c);
   c.m2l_by_level = by_level;
-  hipLaunchKernelGGL(k_group_keys, dim3(ceil_div(nc, 256 / kWave)), dim3(256), 0, s, nc, c.t.cx.p, c.t.cparent.p,
-                     c.t.clevel.p, c.lists.m2l_beg.p, c.lists.m2l_cnt.p, c.lists.m2l.p, minhash,
-                     m2l_fp64_levels(c), int(by_level), c.t.key.p, c.t.val.p);
-  XF_LAUNCH();
-  unsigned long long *k1 = c.t.key.p, *k2 = c.t.key2.p;
-  int *v1 = c.t.val.p, *v2 = c.t.val2.p;
-  radix_sort_pairs(k1, v1, k2, v2, nc, minhash ? 0 : 16, 24, c.m2l_rs_hist, s);
-  c.m2l_misc.ensure(512);
-  XF_HIP(hipMemsetAsync(c.m2l_misc.p, 0, 256 * sizeof(int), s));
-  hipLaunchKernelGGL(k_group_hist, dim3(std::min(ceil_div(nc, 256), 64)), dim3(256), 0, s, nc, k1, c.m2l_misc.p);
-  XF_LAUNCH();
-  // tiles of at most tn cells per group, laid out on the device (no host
+  // Tiles of at most kTileN cells per group, laid out on the device (no host
   // round trip before the per-tile counts); arrays strided by the bound
   // ntmax: [first | count | base | U] x ntmax, then the sorted cells
   const int tn = kTileN;
@@ -1422,28 +1507,41 @@ void m2l_prepare(Ctx &c, hipStream_t s) {
   c.tiles.ensure(size_t(4) * ntmax + nc);
   int *d_first = c.tiles.p, *d_count = c.tiles.p + ntmax, *d_base = c.tiles.p + 2 * ntmax,
       *d_U = c.tiles.p + 3 * ntmax, *d_sorted = c.tiles.p + 4 * ntmax;
-  int *d_plan = c.m2l_misc.p + 257;  // [ntiles, cells in tiles]
-  hipLaunchKernelGGL(k_tile_plan, dim3(1), dim3(256), 0, s, c.m2l_misc.p, tn, d_first, d_count, d_plan);
+  c.m2l_misc.ensure(kMiscInts);
+  const bool ranked = nc <= kCellRankMax;
+  unsigned *key32 = ranked ? reinterpret_cast<unsigned *>(c.t.key.p) : nullptr;
+  hipLaunchKernelGGL(k_group_keys, dim3(ceil_div(nc, 256 / kWave)), dim3(256), 0, s, nc, c.t.cx.p, c.t.cparent.p,
+                     c.t.clevel.p, c.lists.m2l_beg.p, c.lists.m2l_cnt.p, c.lists.m2l.p, m2l_fp64_levels(c),
+                     int(by_level), c.t.key.p, key32, c.t.val.p, c.m2l_misc.p);
   XF_LAUNCH();
-  XF_HIP(hipMemcpyAsync(d_sorted, v1, sizeof(int) * nc, hipMemcpyDeviceToDevice, s));
+  if (ranked) {
+    hipLaunchKernelGGL(k_cell_rank, dim3(ceil_div(nc, kWave)), dim3(1024), 0, s, nc, key32, d_sorted, c.m2l_misc.p);
+  } else {
+    unsigned long long *k1 = c.t.key.p, *k2 = c.t.key2.p;
+    int *v1 = c.t.val.p, *v2 = c.t.val2.p;
+    radix_sort_pairs(k1, v1, k2, v2, nc, 0, 24, c.m2l_rs_hist, s);
+    hipLaunchKernelGGL(k_group_hist, dim3(std::min(ceil_div(nc, 256), 64)), dim3(256), 0, s, nc, k1, v1, d_sorted,
+                       c.m2l_misc.p);
+  }
+  XF_LAUNCH();
+  hipLaunchKernelGGL(k_tile_plan, dim3(1), dim3(256), 0, s, c.m2l_misc.p, d_first, d_count);
+  XF_LAUNCH();
   const int nwords = (nkeys + 31) / 32;
   c.tile_bits.ensure(size_t(ntmax) * std::max(nwords, 1));
-  hipLaunchKernelGGL(k_tile_count, dim3(ntmax), dim3(kTileCountThreads), sizeof(unsigned) * nwords, s, d_first, d_count,
-                     d_sorted, c.lists.m2l_beg.p, c.lists.m2l_cnt.p, c.lists.m2l.p, nkeys, d_plan, d_U,
-                     c.tile_bits.p);
-  XF_LAUNCH();
-  scan_exclusive_dev(d_U, d_base, d_plan, ntmax, c.m2l_misc.p + 256, c.m2l_scan, s);
-  // one host round trip: tile count, slots, cells in tiles, and the key set
   c.pin_i.ensure(kPinInts);
-  c.pin_keys.ensure(std::max(nkeys, 1));
-  XF_HIP(hipMemcpyAsync(c.pin_i.p + kPinPlan, c.m2l_misc.p + 256, sizeof(int) * 3, hipMemcpyDeviceToHost, s));
-  if (nkeys)
-    XF_HIP(hipMemcpyAsync(c.pin_keys.p, c.lists.keys.p, sizeof(unsigned long long) * nkeys, hipMemcpyDeviceToHost,
-                          s));
+  const bool compare = ops_comparable(c, nkeys, fillP, bf16);
+  hipLaunchKernelGGL(k_tile_count, dim3(ntmax), dim3(kTileCountThreads), sizeof(unsigned) * nwords, s, d_first, d_count,
+                     d_sorted, c.lists.m2l_beg.p, c.lists.m2l_cnt.p, c.lists.m2l.p, nkeys, c.m2l_misc.p, d_U,
+                     c.tile_bits.p, c.lists.keys.p, compare ? c.ops_keys.p : nullptr);
+  XF_LAUNCH();
+  hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(kTileCountThreads), 0, s, c.m2l_misc.p, d_U, d_base,
+                     c.pin_i.p + kPinPlan);
+  XF_LAUNCH();
+  // one host round trip: slots, tiles, cells in tiles, and whether the operators still fit
   stream_wait(s);
   const int *plan = c.pin_i.p + kPinPlan;
-  std::vector<unsigned long long> keys(c.pin_keys.p, c.pin_keys.p + nkeys);
   const int totalU = plan[0], ntiles = plan[1], off = plan[2];
+  const bool cached = compare && plan[3] == 0;
   c.m2l_tstride = ntmax;
   if (ntiles == 0) {
     c.m2l_ready = true;
@@ -1461,22 +1559,22 @@ void m2l_prepare(Ctx &c, hipStream_t s) {
   const double cyc = c.cfg.images > 0 ? c.cfg.cycle : 0.0;
   if (bf16) {
     const size_t per = size_t(g.K32) * g.R * 64 * 8;
-    if (!ops_cached(c, keys, fillP, 1)) {
+    if (!cached) {
       c.ops32.ensure((per * nkeys * 2 + 1) / 2 + 1);
       __bf16 *ophi = reinterpret_cast<__bf16 *>(c.ops32.p);
       hipLaunchKernelGGL(k_ops_gen, dim3(nkeys), dim3(256), 0, s, c.P, fillP, g.R, g.K4, g.K32, c.t.R0, cyc,
                          c.lists.keys.p, (float *)nullptr, ophi, ophi + per * nkeys);
       XF_LAUNCH();
-      ops_remember(c, std::move(keys), fillP, 1);
+      ops_remember(c, nkeys, fillP, 1, s);
     }
   } else {
     const size_t per = size_t(g.K4) * g.R * 64;
-    if (!ops_cached(c, keys, fillP, 0)) {
+    if (!cached) {
       c.ops32.ensure(per * nkeys);
       hipLaunchKernelGGL(k_ops_gen, dim3(nkeys), dim3(256), 0, s, c.P, fillP, g.R, g.K4, g.K32, c.t.R0, cyc,
                          c.lists.keys.p, c.ops32.p, (__bf16 *)nullptr, (__bf16 *)nullptr);
       XF_LAUNCH();
-      ops_remember(c, std::move(keys), fillP, 0);
+      ops_remember(c, nkeys, fillP, 0, s);
     }
   }
   c.m2l_ntiles = ntiles;

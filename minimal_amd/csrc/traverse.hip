@@ -348,8 +348,11 @@ __global__ void k_hash_collect(const unsigned long long *__restrict__ slots, int
 // sorted the slot becomes the key's rank (the id the operators are stored by).
 // The count is the device total, capped at the list capacity; flags (if
 // given) skip a pass that is repeated or ranked by the radix sort instead.
+// host_tot (if given) receives the totals and flags (pinned memory).
 __global__ void k_entry_ids(int2 *__restrict__ m2l, const int *__restrict__ total, int64_t cap,
-                            const int *__restrict__ slot2id, const int *__restrict__ flags) {
+                            const int *__restrict__ slot2id, const int *__restrict__ flags, int *host_tot) {
+  if (host_tot && blockIdx.x == 0 && threadIdx.x < 8)
+    __hip_atomic_store(host_tot + threadIdx.x, total[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   if (flags && (*flags & (kListRetry | 32))) return;
   const int64_t n = min(int64_t(*total), cap);
   for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256)
@@ -409,6 +412,7 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
   Lr.out_beg.ensure(nc);
   Lr.out_cnt.ensure(nc);
   Lr.tot.ensure(8);
+  tc.pin_i.ensure(kPinInts);
   tc.L.ensure(size_t(nc) * tc.P * tc.P);
   if (Lr.cap_m2l < 200 * nc) Lr.cap_m2l = 200 * nc;
   if (Lr.cap_p2p < 96 * nc) Lr.cap_p2p = 96 * nc;
@@ -490,11 +494,10 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
                          Lr.kscratch.p, Lr.tot.p + 6, Lr.keys.p, Lr.slot2id.p, Lr.tot.p + 3);
       XF_LAUNCH();
       hipLaunchKernelGGL(k_entry_ids, dim3(int(std::min<int64_t>(ceil_div(Lr.cap_m2l, 256), 4096))), dim3(256), 0, s,
-                         Lr.m2l.p, Lr.tot.p, Lr.cap_m2l, Lr.slot2id.p, Lr.tot.p + 3);
+                         Lr.m2l.p, Lr.tot.p, Lr.cap_m2l, Lr.slot2id.p, Lr.tot.p + 3, tc.pin_i.p + kPinTot);
       XF_LAUNCH();
     }
-    tc.pin_i.ensure(kPinInts);
-    XF_HIP(hipMemcpyAsync(tc.pin_i.p + kPinTot, Lr.tot.p, sizeof(tot), hipMemcpyDeviceToHost, s));
+    if (!keys) XF_HIP(hipMemcpyAsync(tc.pin_i.p + kPinTot, Lr.tot.p, sizeof(tot), hipMemcpyDeviceToHost, s));
     stream_wait(s);
     std::copy(tc.pin_i.p + kPinTot, tc.pin_i.p + kPinTot + 8, tot);
     const int flags = tot[3];
@@ -536,7 +539,7 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
         XF_HIP(hipMemcpyAsync(Lr.keys.p, k1, sizeof(unsigned long long) * nk, hipMemcpyDeviceToDevice, s));
       if (Lr.nm2l > 0) {
         hipLaunchKernelGGL(k_entry_ids, dim3(std::min(ceil_div(Lr.nm2l, 256), 4096)), dim3(256), 0, s, Lr.m2l.p,
-                           Lr.tot.p, Lr.cap_m2l, Lr.slot2id.p, (const int *)nullptr);
+                           Lr.tot.p, Lr.cap_m2l, Lr.slot2id.p, (const int *)nullptr, (int *)nullptr);
         XF_LAUNCH();
       }
     }
