@@ -206,7 +206,9 @@ struct Tree {
   Buf<int> val, val2;
   Buf<int> hist;       // dense prefix histograms, levels 1..7
   Buf<int> hist_bmax;  // per-block largest populations of levels 3..7
-  Buf<int> lcount, lstart_d, tmp_nch, tmp_off, tmp_bnd, misc;
+  Buf<int> lcount, lstart_d, misc, cursor;
+  Buf<unsigned long long> lookback;  // published prefixes of the level splits (tree.hip)
+  unsigned lookback_tag = 0;
   Buf<double> bounds_part;
   Buf<int> rs_hist;
   Buf<int> scan_tmp;  // device-wide scan partials
@@ -401,8 +403,6 @@ void op_l2p(Ctx &c, const double *C, const double *L, exafmm_body *b, int64_t nb
 
 // generic helpers (scan.hip)
 void scan_exclusive(const int *in, int *out, int count, int *total, Buf<int> &scratch, hipStream_t s);
-void scan_exclusive_dev(const int *in, int *out, const int *count_dev, int count_bound, int *total,
-                        Buf<int> &scratch, hipStream_t s);
 void radix_sort_pairs(unsigned long long *&k, int *&v, unsigned long long *&k2, int *&v2, int n, int lo_bit,
                       int hi_bit, Buf<int> &hist, hipStream_t s);
 

@@ -176,12 +176,6 @@ void scan_exclusive(const int *in, int *out, int count, int *total, Buf<int> &sc
   scan_launch<1>(a, count, nullptr, count, total, nullptr, nullptr, nullptr, scratch, s);
 }
 
-void scan_exclusive_dev(const int *in, int *out, const int *count_dev, int count_bound, int *total,
-                        Buf<int> &scratch, hipStream_t s) {
-  ScanArrays<1> a{{in}, {out}};
-  scan_launch<1>(a, 0, count_dev, count_bound, total, nullptr, nullptr, nullptr, scratch, s);
-}
-
 // ---------------------------------------------------------------- radix sort
 constexpr int kRsThreads = 256;
 constexpr int kRsItems = 4;

@@ -22,11 +22,17 @@ __host__ __device__ constexpr int hist_off(int l) {  // offset of level l (1..7)
   return l <= 1 ? 0 : hist_off(l - 1) + (1 << (3 * (l - 1)));
 }
 constexpr int kHistTotal = hist_off(kHistLevels + 1);
+constexpr int kMiscInts = 64;
 
 // ---------------------------------------------------------------- bounds
+// It also clears the level-7 histogram of the launch after the next.  part:
+// per workgroup [lo, hi, 1 if a coordinate or charge is not finite].
+constexpr int kBoundsBlocks = 256, kBoundsInts = 7;
 __global__ void __launch_bounds__(256) k_bounds_part(const exafmm_body *__restrict__ b, int64_t n,
-                                                     double *__restrict__ part, int *__restrict__ flags) {
+                                                     double *__restrict__ part, int4 *__restrict__ hist7) {
   __shared__ double s[6][256];
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < (1 << (3 * kHistLevels)) / 4; i += gridDim.x * 256)
+    hist7[i] = make_int4(0, 0, 0, 0);
   double lo[3] = {b[0].X[0], b[0].X[1], b[0].X[2]};
   double hi[3] = {lo[0], lo[1], lo[2]};
   int bad = 0;
@@ -39,7 +45,7 @@ __global__ void __launch_bounds__(256) k_bounds_part(const exafmm_body *__restri
     }
     if (!isfinite(b[i].q)) bad = 1;
   }
-  if (bad) atomicOr(flags, 1);
+  bad = __syncthreads_or(bad);
   for (int d = 0; d < 3; d++) {
     s[d][threadIdx.x] = lo[d];
     s[3 + d][threadIdx.x] = hi[d];
@@ -53,21 +59,48 @@ __global__ void __launch_bounds__(256) k_bounds_part(const exafmm_body *__restri
       }
     __syncthreads();
   }
-  if (threadIdx.x < 6) part[blockIdx.x * 6 + threadIdx.x] = s[threadIdx.x][0];
+  if (threadIdx.x < 6) part[blockIdx.x * kBoundsInts + threadIdx.x] = s[threadIdx.x][0];
+  if (threadIdx.x == 6) part[blockIdx.x * kBoundsInts + 6] = bad ? 1.0 : 0.0;
+}
+
+// The root cell and the build's counters.
+struct RootOut {
+  double *root;   // X0, R0
+  int *misc;      // flags and counters (see tree_build)
+  int *lcount, *lstart;
+  double4 *cx;
+  int *cbeg, *ccnt, *cparent, *clevel;
+  int64_t n;
+};
+__device__ inline void write_root(const RootOut &o, double x, double y, double z, double r) {
+  o.root[0] = x;
+  o.root[1] = y;
+  o.root[2] = z;
+  o.root[3] = r;
+  o.cx[0] = make_double4(x, y, z, r);
+  o.cbeg[0] = 0;
+  o.ccnt[0] = int(o.n);
+  o.cparent[0] = -1;
+  o.clevel[0] = 0;
+  o.lcount[0] = 1;
+  o.lstart[0] = 0;
+}
+// (threads 0 .. 255; thread 0 has written misc[0] already)
+__device__ inline void clear_counters(const RootOut &o) {
+  const int t = threadIdx.x;
+  if (t > 0 && t < kMiscInts) o.misc[t] = 0;
+  if (t > 0 && t < kMaxLevel + 2) o.lcount[t] = 0;
 }
 
 // X0 = (max+min)/2, R0 = max half-extent * 1.00001 (3d/build_tree.h:7-21).
-__global__ void __launch_bounds__(256) k_bounds_final(const double *__restrict__ part, int nparts,
-                                                      double *__restrict__ root) {
+__global__ void __launch_bounds__(kBoundsBlocks) k_bounds_final(const double *__restrict__ part, RootOut out) {
   __shared__ double s[6][256];
   const int t = threadIdx.x;
   double v[6];
-  for (int d = 0; d < 6; d++) v[d] = part[d];
-  for (int p = t; p < nparts; p += 256)
-    for (int d = 0; d < 3; d++) {
-      v[d] = fmin(part[p * 6 + d], v[d]);
-      v[3 + d] = fmax(part[p * 6 + 3 + d], v[3 + d]);
-    }
+  for (int d = 0; d < 6; d++) v[d] = part[t * kBoundsInts + d];
+  const int bad = __syncthreads_or(part[t * kBoundsInts + 6] != 0.0);
+  if (t == 0) out.misc[0] = bad ? 1 : 0;
+  clear_counters(out);
   for (int d = 0; d < 6; d++) s[d][t] = v[d];
   __syncthreads();
   for (int o = 128; o > 0; o >>= 1) {
@@ -91,10 +124,20 @@ __global__ void __launch_bounds__(256) k_bounds_final(const double *__restrict__
     R0 = fmax(hi[d] - X0[d], R0);
   }
   R0 *= 1.00001;
-  root[0] = X0[0];
-  root[1] = X0[1];
-  root[2] = X0[2];
-  root[3] = R0;
+  write_root(out, X0[0], X0[1], X0[2], R0);
+}
+
+// Forest: counters, the histogram and the unit root cube of levels 0 ..
+// kForestLevel - 1 (problem-index cells, never paired by the traversal).
+__global__ void __launch_bounds__(256) k_forest_init(RootOut out, int4 *__restrict__ hist7) {
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < (1 << (3 * kHistLevels)) / 4; i += gridDim.x * 256)
+    hist7[i] = make_int4(0, 0, 0, 0);
+  if (blockIdx.x > 0) return;
+  if (threadIdx.x == 0) {
+    out.misc[0] = 0;
+    write_root(out, 0.0, 0.0, 0.0, 1.0);
+  }
+  clear_counters(out);
 }
 
 // Forest: one workgroup per problem (bodies off[p] .. off[p+1] - 1), the
@@ -290,20 +333,17 @@ __global__ void __launch_bounds__(1024) k_hist_pyramid(int *__restrict__ hist, i
 }
 
 // Levels 2 and 1 from level 3, and the largest population of every level
-// (lmax[l], l = 1..7) from the blocks' maxima: one workgroup of 512.
-__global__ void __launch_bounds__(512) k_hist_top(int *__restrict__ hist, const int *__restrict__ bmax,
-                                                  int *__restrict__ lmax) {
-  __shared__ int red[512], s2[64];
-  const int t = threadIdx.x;
-  for (int l = 3; l <= 7; l++) {
-    red[t] = bmax[8 * t + l];
-    __syncthreads();
-    for (int o = 256; o > 0; o >>= 1) {
-      if (t < o) red[t] = max(red[t], red[t + o]);
-      __syncthreads();
+// (lmax[l], l = 1..7) from the blocks' maxima: the first 512 threads of one
+// workgroup (every thread calls it).
+__device__ inline void hist_top(int *hist, const int *__restrict__ bmax, int *lmax) {
+  __shared__ int wmax[5][8], s2[64];
+  const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
+  if (t < 512) {
+    for (int l = 3; l <= 7; l++) {
+      int m = bmax[8 * t + l];
+      for (int o = 1; o < kWave; o <<= 1) m = max(m, __shfl_xor(m, o));
+      if (lane == 0) wmax[l - 3][w] = m;
     }
-    if (t == 0) lmax[l] = red[0];
-    __syncthreads();
   }
   if (t < 64) {
     int s = 0;
@@ -312,6 +352,11 @@ __global__ void __launch_bounds__(512) k_hist_top(int *__restrict__ hist, const 
     hist[hist_off(2) + t] = s;
   }
   __syncthreads();
+  if (t >= 3 && t <= 7) {
+    int m = 0;
+    for (int i = 0; i < 8; i++) m = max(m, wmax[t - 3][i]);
+    lmax[t] = m;
+  }
   if (t == 0) {
     int a2 = 0, a1 = 0;
     for (int i = 0; i < 64; i++) a2 = max(a2, s2[i]);
@@ -324,6 +369,24 @@ __global__ void __launch_bounds__(512) k_hist_top(int *__restrict__ hist, const 
     lmax[2] = a2;
     lmax[1] = a1;
   }
+  __syncthreads();
+}
+__global__ void __launch_bounds__(512) k_hist_top(int *hist, const int *__restrict__ bmax, int *lmax) {
+  hist_top(hist, bmax, lmax);
+}
+
+// Bodies by their level-l prefix (counting sort: cursor holds the prefixes'
+// first places): the order within a prefix is left to k_leaf_gather, which
+// puts every leaf's bodies back into input order.
+__global__ void __launch_bounds__(256) k_place(const unsigned long long *__restrict__ key, int64_t n, int shift,
+                                               int *__restrict__ cursor, unsigned long long *__restrict__ key_out,
+                                               int *__restrict__ val_out) {
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= n) return;
+  const unsigned long long k = key[i];
+  const int pos = atomicAdd(&cursor[int(k >> shift)], 1);
+  key_out[pos] = k;
+  val_out[pos] = int(i);
 }
 
 // ---------------------------------------------------------------- levels
@@ -364,22 +427,6 @@ __device__ inline int split_bounds(int l, int ncrit, int beg, int cnt, const uns
   return k;
 }
 
-__global__ void __launch_bounds__(256) k_split(int l, int ncrit, int lforce, const int *__restrict__ lcount,
-                                               const int *__restrict__ lstart, const int *__restrict__ cbeg,
-                                               const int *__restrict__ ccnt,
-                                               const unsigned long long *__restrict__ key,
-                                               const int *__restrict__ hist, int *__restrict__ nch,
-                                               int *__restrict__ bnd) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= lcount[l]) return;
-  const int c = lstart[l] + t;
-  int b[9];
-  const int k = split_bounds(l, ncrit, cbeg[c], ccnt[c], key, hist, b, lforce);
-  nch[t] = k;
-  if (k == 0) return;
-  for (int o = 0; o < 9; o++) bnd[t * 9 + o] = b[o];
-}
-
 // Writes the non-empty children of level-l cell c (boundaries b) to cells
 // first, first + 1, ... in octant order.
 // r = R_parent / 2 is R0 / 2^(l+1) exactly.  Forest: the cells of level
@@ -411,44 +458,146 @@ __device__ inline void emit_children(int l, int c, int first, const int b[9], co
   }
 }
 
-__global__ void k_level_next(int l, int *__restrict__ lcount, int *__restrict__ lstart, const int *__restrict__ total) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    lcount[l + 1] = *total;
-    lstart[l + 1] = lstart[l] + lcount[l];
+// Exclusive prefix, over the workgroups of a launch, of one count each
+// (decoupled look-back).  A workgroup's number comes from *ticket (zero at
+// the launch), so those before it have started and never wait for it: every
+// wait ends.  A workgroup publishes one word, [tag | state | value] -- state 1
+// its own count, 2 the sum up to and with it -- and no other data is passed, so
+// relaxed atomics are enough.  `tag` differs from that of every earlier launch
+// on the array.  Call with the whole workgroup (at least 64 threads).
+__device__ inline int lookback_ticket(int *ticket) {
+  __shared__ int id;
+  if (threadIdx.x == 0) id = atomicAdd(ticket, 1);
+  __syncthreads();
+  return id;
+}
+__device__ inline int lookback_prefix(int id, int count, unsigned tag, unsigned long long *words) {
+  __shared__ int prefix;
+  if (threadIdx.x < kWave) {
+    const int lane = threadIdx.x;
+    auto word = [&](int state, int v) {
+      return (unsigned long long)tag << 40 | (unsigned long long)state << 32 | unsigned(v);
+    };
+    auto put = [&](int i, unsigned long long v) {
+      __hip_atomic_store(words + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    if (lane == 0) put(id, word(id == 0 ? 2 : 1, count));
+    int sum = 0;
+    for (int top = id - 1; top >= 0; top -= kWave) {  // windows of 64 predecessors, nearest first
+      const int i = top - lane;
+      unsigned long long v = 0;
+      int state = 2;  // before the first: an empty prefix
+      if (i >= 0) {
+        do {
+          v = __hip_atomic_load(words + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } while (unsigned(v >> 40) != tag);
+        state = int(v >> 32) & 3;
+      }
+      const unsigned long long done = __ballot(state == 2);
+      const int last = done ? __ffsll((long long)done) - 1 : kWave - 1;
+      int x = i >= 0 && lane <= last ? int(unsigned(v)) : 0;
+      for (int o = 1; o < kWave; o <<= 1) x += __shfl_xor(x, o);
+      sum += x;
+      if (done) break;
+    }
+    if (lane == 0) {
+      if (id > 0) put(id, word(2, sum + count));
+      prefix = sum;
+    }
   }
+  __syncthreads();
+  return prefix;
 }
 
-// Children of level-l node t, in octant order (3d/build_tree.h:115-132):
-// centre = parent centre + r*(+/-1), r = R0/2^(l+1); R = R0/2^(l+1).
-__global__ void __launch_bounds__(256) k_emit(int l, const int *__restrict__ lcount, const int *__restrict__ lstart,
-                                              const int *__restrict__ nch, const int *__restrict__ off,
-                                              const int *__restrict__ bnd, const double4 *__restrict__ froots,
-                                              const unsigned long long *__restrict__ key,
-                                              double4 *__restrict__ cx, int *__restrict__ cbeg,
-                                              int *__restrict__ ccnt, int *__restrict__ cchild,
-                                              int *__restrict__ cnch, int *__restrict__ cparent,
-                                              int *__restrict__ clevel, int *__restrict__ nsplit) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  const bool in = t < lcount[l];
-  const int k = in ? nch[t] : 0;
+// Exclusive scan of one count per thread over a workgroup of 1024.
+__device__ inline int block_scan(int v, int &total) {
+  __shared__ int wsum[1024 / kWave];
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  int incl = v;
+  for (int d = 1; d < kWave; d <<= 1) {
+    const int x = __shfl_up(incl, d);
+    if (lane >= d) incl += x;
+  }
+  __syncthreads();  // the last use of wsum
+  if (lane == kWave - 1) wsum[w] = incl;
+  __syncthreads();
+  int before = 0;
+  total = 0;
+  for (int i = 0; i < 1024 / kWave; i++) {
+    before += i < w ? wsum[i] : 0;
+    total += wsum[i];
+  }
+  return before + incl - v;
+}
+
+// Splits level l (one cell per thread): child boundaries, the children's
+// places in level l + 1 by a look-back over the workgroups, and the children,
+// in octant order (3d/build_tree.h:115-132): centre = parent centre +
+// r*(+/-1), r = R0/2^(l+1); R = R0/2^(l+1).  One launch per level where split,
+// scan, level sizes and emission took four.
+__global__ void __launch_bounds__(1024) k_split_level(int l, int ncrit, int lforce, int *lcount, int *lstart,
+                                                      const unsigned long long *__restrict__ key,
+                                                      const int *__restrict__ hist, const double4 *__restrict__ froots,
+                                                      double4 *__restrict__ cx, int *cbeg, int *ccnt,
+                                                      int *__restrict__ cchild, int *__restrict__ cnch,
+                                                      int *__restrict__ cparent, int *__restrict__ clevel,
+                                                      int *__restrict__ nsplit, int *__restrict__ ticket, unsigned tag,
+                                                      unsigned long long *__restrict__ words) {
+  const int id = lookback_ticket(ticket);
+  const int count = lcount[l], start = lstart[l], next = start + count;
+  const int t = id * 1024 + threadIdx.x, c = start + t;
+  const bool in = t < count;
+  int b[9];
+  const int k = in ? split_bounds(l, ncrit, cbeg[c], ccnt[c], key, hist, b, lforce) : 0;
   // cells that split, counted per wave (leaves = cells - split cells)
   const unsigned long long sp = __ballot(k > 0);
   if ((threadIdx.x & (kWave - 1)) == 0 && sp) atomicAdd(nsplit, int(__popcll(sp)));
-  if (!in) return;
-  const int c = lstart[l] + t;
-  cnch[c] = k;
-  if (k == 0) {
-    cchild[c] = -1;
-    return;
+  int total;
+  const int off = block_scan(k, total);
+  const int before = lookback_prefix(id, total, tag, words);
+  if (in) {
+    cnch[c] = k;
+    if (k == 0)
+      cchild[c] = -1;
+    else
+      emit_children(l, c, next + before + off, b, froots, key, cx, cbeg, ccnt, cchild, cparent, clevel);
   }
-  int b[9];
-  for (int o = 0; o < 9; o++) b[o] = bnd[t * 9 + o];
-  emit_children(l, c, lstart[l + 1] + off[t], b, froots, key, cx, cbeg, ccnt, cchild, cparent, clevel);
+  if (id == int(gridDim.x) - 1 && threadIdx.x == 0) {
+    lcount[l + 1] = before + total;
+    lstart[l + 1] = next;
+  }
 }
 
-// The top levels, 0 .. lend - 1, split by one workgroup: per level the
-// k_split / exclusive scan / k_level_next / k_emit sequence above, with a
-// workgroup scan and barriers in place of launches.  Level l holds at most
+// The leaves, in breadth-first order, and the cells of the deepest sorted
+// level l, which are leaves: more than ncrit bodies there means the tree needs
+// more levels.
+__global__ void __launch_bounds__(1024) k_leaves(int l, int ncrit, const int *__restrict__ lcount,
+                                                 const int *__restrict__ lstart, const int *__restrict__ ccnt,
+                                                 int *cchild, int *cnch, int *__restrict__ leaves, int *__restrict__ misc,
+                                                 int *__restrict__ ticket, unsigned tag,
+                                                 unsigned long long *__restrict__ words) {
+  const int id = lookback_ticket(ticket);
+  const int last = lstart[l], nc = last + lcount[l];
+  const int c = id * 1024 + threadIdx.x;
+  bool leaf = false;
+  if (c < nc) {
+    leaf = c >= last || cnch[c] == 0;
+    if (c >= last) {
+      cnch[c] = 0;
+      cchild[c] = -1;
+      if (ccnt[c] > ncrit) atomicOr(misc, 2);
+    }
+  }
+  int total;
+  const int off = block_scan(leaf, total);
+  const int before = lookback_prefix(id, total, tag, words);
+  if (leaf) leaves[before + off] = c;
+  if (id == int(gridDim.x) - 1 && threadIdx.x == 0) misc[17] = before + total;
+}
+
+// The top levels, 0 .. lend - 1, split by one workgroup (which also finishes
+// the histogram, hist_top): per level what k_split_level does, with a
+// workgroup scan and barriers.  Level l holds at most
 // 8^l cells, so levels up to kTopLevels - 1 fit kTopPer cells per thread;
 // thread t owns cells kTopPer t .. kTopPer t + kTopPer - 1 of its level.
 // Level 4 (4096 cells) stays on the multi-workgroup kernels: one workgroup
@@ -458,12 +607,13 @@ constexpr int kTopThreads = 1024, kTopPer = 1, kTopLevels = 4;
 static_assert(1 << (3 * (kTopLevels - 1)) <= kTopThreads * kTopPer, "top levels exceed the workgroup");
 __global__ void __launch_bounds__(kTopThreads)
     k_top_levels(int lend, int ncrit, int lforce, int *__restrict__ lcount, int *__restrict__ lstart,
-                 const unsigned long long *__restrict__ key, const int *__restrict__ hist,
-                 const double4 *__restrict__ froots, double4 *__restrict__ cx, int *__restrict__ cbeg,
+                 const unsigned long long *__restrict__ key, int *hist, const int *__restrict__ bmax,
+                 int *__restrict__ lmax, const double4 *__restrict__ froots, double4 *__restrict__ cx, int *__restrict__ cbeg,
                  int *__restrict__ ccnt, int *__restrict__ cchild, int *__restrict__ cnch,
                  int *__restrict__ cparent, int *__restrict__ clevel, int *__restrict__ nsplit) {
   __shared__ int wsum[kTopThreads / kWave];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+  if (bmax) hist_top(hist, bmax, lmax);
   int cnt = lcount[0], start = lstart[0];
   for (int l = 0; l < lend; l++) {
     int b[kTopPer][9], k[kTopPer];
@@ -518,57 +668,38 @@ __global__ void __launch_bounds__(kTopThreads)
   }
 }
 
-__global__ void k_root(int64_t n, const double *__restrict__ root, double4 *__restrict__ cx, int *__restrict__ cbeg,
-                       int *__restrict__ ccnt, int *__restrict__ cparent, int *__restrict__ clevel,
-                       int *__restrict__ lcount, int *__restrict__ lstart) {
-  cx[0] = make_double4(root[0], root[1], root[2], root[3]);
-  cbeg[0] = 0;
-  ccnt[0] = int(n);
-  cparent[0] = -1;
-  clevel[0] = 0;
-  lcount[0] = 1;
-  lstart[0] = 0;
-}
-
-// Cells of the deepest sorted level: leaves; more than ncrit bodies there
-// means the tree needs more than 21 levels.
-__global__ void __launch_bounds__(256) k_last_level(int l, int ncrit, const int *__restrict__ lcount,
-                                                    const int *__restrict__ lstart, const int *__restrict__ ccnt,
-                                                    int *__restrict__ cchild, int *__restrict__ cnch,
-                                                    int *__restrict__ flags) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t == 0) flags[19] = lstart[l] + lcount[l];  // cells in the tree
-  if (t >= lcount[l]) return;
-  const int c = lstart[l] + t;
-  cnch[c] = 0;
-  cchild[c] = -1;
-  if (ccnt[c] > ncrit) atomicOr(flags, 2);
-}
-
-// Leaf flags and the compacted leaf list over the *ncells cells (a device
-// count: grid-stride loops over a grid sized from a host bound).
-__global__ void __launch_bounds__(256) k_leaf_flag(const int *__restrict__ ncells, const int *__restrict__ cnch,
-                                                   int *__restrict__ f) {
-  const int nc = *ncells;
-  for (int c = blockIdx.x * 256 + threadIdx.x; c < nc; c += gridDim.x * 256) f[c] = cnch[c] == 0;
-}
-__global__ void __launch_bounds__(256) k_leaf_compact(const int *__restrict__ ncells, const int *__restrict__ cnch,
-                                                      const int *__restrict__ off, int *__restrict__ leaves) {
-  const int nc = *ncells;
-  for (int c = blockIdx.x * 256 + threadIdx.x; c < nc; c += gridDim.x * 256)
-    if (cnch[c] == 0) leaves[off[c]] = c;
+__global__ void k_root(RootOut out) {
+  out.cx[0] = make_double4(out.root[0], out.root[1], out.root[2], out.root[3]);
+  out.cbeg[0] = 0;
+  out.ccnt[0] = int(out.n);
+  out.cparent[0] = -1;
+  out.clevel[0] = 0;
 }
 
 // One workgroup per leaf: restore input order inside the leaf (rank of
 // each original index among the leaf's), then gather X, q (FP64) and the
-// leaf-relative FP32 copy used by P2P.
+// leaf-relative FP32 copy used by P2P.  The first workgroup also hands the
+// level sizes, the counters and the root to the host (pinned memory).
+struct TreeReport {
+  const int *lcount, *misc;
+  const double *root;
+  int *host_levels, *host_misc;
+  double *host_root;
+};
 __global__ void __launch_bounds__(64) k_leaf_gather(const int *__restrict__ leaves, const int *__restrict__ nleaves,
                                                     const int *__restrict__ cbeg, const int *__restrict__ ccnt,
                                                     const double4 *__restrict__ cx, const int *__restrict__ val,
                                                     const exafmm_body *__restrict__ b, int *__restrict__ perm,
                                                     double4 *__restrict__ xs, float4 *__restrict__ xq,
-                                                    int *__restrict__ body_leaf, int ncrit) {
+                                                    int *__restrict__ body_leaf, int ncrit, TreeReport rep) {
   extern __shared__ int sidx[];  // ncrit ints
+  if (blockIdx.x == 0) {
+    auto put = [](auto *p, auto v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
+    const int t = threadIdx.x;
+    if (t < kMaxLevel + 2) put(rep.host_levels + t, rep.lcount[t]);
+    if (t < 19) put(rep.host_misc + t, rep.misc[t]);
+    if (t < 4) put(rep.host_root + t, rep.root[t]);
+  }
   const int nl = *nleaves;
   for (int li = blockIdx.x; li < nl; li += gridDim.x) {
     const int c = leaves[li];
@@ -630,29 +761,63 @@ void tree_build(Ctx &c) {
   const int ncrit = c.cfg.ncrit;
   if (n > (int64_t(1) << 30)) fail(EXAFMM_ERR_ARG, "N above 2^30 is not supported");
 
-  // misc layout (ints): [0] flags, [1..8] level max, [16] level total,
-  // [17] leaves, [18] cells that split
-  t.misc.ensure(64);
-  t.bounds_part.ensure(256 * 6 + 8);
-  double *root = t.bounds_part.p + 256 * 6;
-  XF_HIP(hipMemsetAsync(t.misc.p, 0, 64 * sizeof(int), s));
+  // misc layout (ints): [0] flags, [1..8] level max, [17] leaves, [18] cells
+  // that split, [24 + l] look-back tickets of level l's split, [46] of k_leaves
+  t.misc.ensure(kMiscInts);
+  t.bounds_part.ensure(kBoundsBlocks * kBoundsInts + 8);
+  double *root = t.bounds_part.p + kBoundsBlocks * kBoundsInts;
+  t.lcount.ensure(kMaxLevel + 2);
+  t.lstart_d.ensure(kMaxLevel + 2);
+  t.hist.ensure(kHistTotal);
+  static_assert(hist_off(kHistLevels) % 4 == 0, "level 7 is cleared 16 bytes at a time");
+  int4 *hist7 = reinterpret_cast<int4 *>(t.hist.p + hist_off(kHistLevels));
+  for (Buf<int> *a : {&t.cbeg, &t.ccnt, &t.cparent, &t.clevel}) a->ensure(1);  // the root; the rest below
+  t.cx.ensure(1);
 
-  // forest: per-problem roots; the root of levels 0 .. kForestLevel - 1
-  // (problem-index cells, never paired by the traversal) is a unit cube
+  // forest: per-problem roots under the problem-index cells
   const bool forest = c.forest_n > 0;
   const double4 *froots = forest ? c.forest_roots.p : nullptr;
   const int lforce = forest ? kForestLevel : 0;
   t.lroot = lforce;
+  // bounds on the cells of each level (a depth of kMaxLevel until Ds is known)
+  const int64_t ub_split = 8 * (n / (ncrit + 1)) + 8;
+  auto level_bound = [&](int l) {
+    int64_t u = std::min<int64_t>(l >= 10 ? n : (int64_t(1) << (3 * l)), n);
+    // nodes of level l are children of level-(l-1) nodes holding > ncrit bodies
+    return l > lforce ? std::min(u, ub_split) : u;  // (a forest's top levels split unconditionally)
+  };
+  auto ensure_cells = [&](int Ds) {
+    int64_t tot = 0;
+    for (int l = 0; l <= Ds; l++) tot += level_bound(l);
+    if (t.cx.cap < size_t(tot) || t.leaves.cap < size_t(tot)) {
+      t.cx.ensure(tot);
+      t.cbeg.ensure(tot);
+      t.ccnt.ensure(tot);
+      t.cchild.ensure(tot);
+      t.cnch.ensure(tot);
+      t.cparent.ensure(tot);
+      t.clevel.ensure(tot);
+      t.leaves.ensure(tot);
+    }
+    return tot;
+  };
+  const bool speculate = t.ds_hint >= 0;
+  int Ds = t.ds_hint;
+  // the root cell is written by the first launches: cells for the largest
+  // depth the build can turn out to have (the histogram's, or the hint's)
+  ensure_cells(speculate ? Ds : kHistLevels);
+  const RootOut rout{root,    t.misc.p, t.lcount.p, t.lstart_d.p, t.cx.p, t.cbeg.p, t.ccnt.p, t.cparent.p,
+                     t.clevel.p, n};
   if (forest) {
+    hipLaunchKernelGGL(k_forest_init, dim3(256), dim3(256), 0, s, rout, hist7);
+    XF_LAUNCH();
     hipLaunchKernelGGL(k_forest_bounds, dim3(c.forest_n), dim3(kFBThreads), 0, s, c.bodies, c.forest_off.p,
                        c.forest_roots.p, t.misc.p);
     XF_LAUNCH();
-    const double unit[4] = {0.0, 0.0, 0.0, 1.0};
-    XF_HIP(hipMemcpyAsync(root, unit, sizeof(unit), hipMemcpyHostToDevice, s));
   } else {
-    hipLaunchKernelGGL(k_bounds_part, dim3(256), dim3(256), 0, s, c.bodies, n, t.bounds_part.p, t.misc.p);
+    hipLaunchKernelGGL(k_bounds_part, dim3(kBoundsBlocks), dim3(256), 0, s, c.bodies, n, t.bounds_part.p, hist7);
     XF_LAUNCH();
-    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(256), 0, s, t.bounds_part.p, 256, root);
+    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBoundsBlocks), 0, s, t.bounds_part.p, rout);
     XF_LAUNCH();
   }
 
@@ -660,8 +825,6 @@ void tree_build(Ctx &c) {
   t.key2.ensure(n);
   t.val.ensure(n);
   t.val2.ensure(n);
-  t.hist.ensure(kHistTotal);
-  XF_HIP(hipMemsetAsync(t.hist.p + hist_off(kHistLevels), 0, sizeof(int) * (1 << (3 * kHistLevels)), s));
   // crowded level-7 prefixes in the last tree: count them per workgroup first
   hipLaunchKernelGGL(t.hist7_max > 64 ? k_keys<true> : k_keys<false>, dim3(ceil_div(n, kKeysThreads)),
                      dim3(kKeysThreads), 0, s, c.bodies, n, root, t.key.p, t.val.p,
@@ -671,8 +834,6 @@ void tree_build(Ctx &c) {
   t.hist_bmax.ensure(8 << (3 * 3));
   hipLaunchKernelGGL(k_hist_pyramid, dim3(1 << (3 * 3)), dim3(1024), 0, s, t.hist.p, t.hist_bmax.p);
   XF_LAUNCH();
-  hipLaunchKernelGGL(k_hist_top, dim3(1), dim3(1 << (3 * 3)), 0, s, t.hist.p, t.hist_bmax.p, t.misc.p);
-  XF_LAUNCH();
 
   // Sort depth Ds: the first level whose most populous prefix holds at
   // most ncrit bodies (kMaxLevel if none of levels 1..7 does).  It needs the
@@ -681,97 +842,80 @@ void tree_build(Ctx &c) {
   // A depth at or above the true one builds the same tree (a cell splits
   // only above ncrit bodies, and each leaf keeps its bodies in input order),
   // so only a smaller one makes the build start over.
-  const bool speculate = t.ds_hint >= 0;
-  int Ds = t.ds_hint;
   c.pin_i.ensure(kPinInts);
   c.pin_d.ensure(4);
   int *hm = c.pin_i.p + kPinLevelMax;
   if (!speculate) {
+    hipLaunchKernelGGL(k_hist_top, dim3(1), dim3(512), 0, s, t.hist.p, t.hist_bmax.p, t.misc.p);
+    XF_LAUNCH();
     XF_HIP(hipMemcpyAsync(hm, t.misc.p, sizeof(int) * 9, hipMemcpyDeviceToHost, s));
     stream_wait(s);
     if (hm[0] & 1) fail(EXAFMM_ERR_ARG, "non-finite body coordinate or charge");
     Ds = sort_depth(hm, n, ncrit, forest, lforce);
   }
 
-  // stable sort by the top Ds octant digits
+  // bodies in the order of their top Ds octant digits: a counting sort on the
+  // histogram up to its depth (2 - 3 launches where the radix sort takes three
+  // per eight bits), the stable radix sort below
   unsigned long long *k1 = t.key.p, *k2 = t.key2.p;
   int *v1 = t.val.p, *v2 = t.val2.p;
-  radix_sort_pairs(k1, v1, k2, v2, int(n), 3 * (kMaxLevel - Ds), 3 * kMaxLevel, t.rs_hist, s);
+  if (Ds <= kHistLevels) {
+    const int Dc = std::max(Ds, 3), bins = 1 << (3 * Dc);  // levels 1 and 2 are summed later
+    t.cursor.ensure(bins);
+    scan_exclusive(t.hist.p + hist_off(Dc), t.cursor.p, bins, nullptr, t.scan_tmp, s);
+    hipLaunchKernelGGL(k_place, dim3(ceil_div(n, 256)), dim3(256), 0, s, k1, n, 3 * (kMaxLevel - Dc), t.cursor.p, k2,
+                       v1);
+    XF_LAUNCH();
+    k1 = k2;
+  } else {
+    radix_sort_pairs(k1, v1, k2, v2, int(n), 3 * (kMaxLevel - Ds), 3 * kMaxLevel, t.rs_hist, s);
+  }
 
   // level-by-level split
-  std::vector<int64_t> ub(Ds + 2);
-  int64_t ubtot = 0;
-  // nodes of level l+1 are children of level-l nodes holding > ncrit bodies
-  const int64_t ub_split = 8 * (n / (ncrit + 1)) + 8;
-  for (int l = 0; l <= Ds; l++) {
-    ub[l] = std::min<int64_t>(l >= 10 ? n : (int64_t(1) << (3 * l)), n);
-    if (l > lforce) ub[l] = std::min(ub[l], ub_split);  // (a forest's top levels split unconditionally)
-    ubtot += ub[l];
+  double4 *const cx0 = t.cx.p;
+  const int64_t ubtot = ensure_cells(Ds);
+  if (t.cx.p != cx0) {  // (a first build deeper than the histogram: the root again)
+    const RootOut again{root,    t.misc.p, t.lcount.p, t.lstart_d.p, t.cx.p, t.cbeg.p, t.ccnt.p, t.cparent.p,
+                        t.clevel.p, n};
+    hipLaunchKernelGGL(k_root, dim3(1), dim3(1), 0, s, again);
+    XF_LAUNCH();
   }
-  t.cx.ensure(ubtot);
-  t.cbeg.ensure(ubtot);
-  t.ccnt.ensure(ubtot);
-  t.cchild.ensure(ubtot);
-  t.cnch.ensure(ubtot);
-  t.cparent.ensure(ubtot);
-  t.clevel.ensure(ubtot);
-  t.lcount.ensure(kMaxLevel + 2);
-  t.lstart_d.ensure(kMaxLevel + 2);
-  XF_HIP(hipMemsetAsync(t.lcount.p, 0, sizeof(int) * (kMaxLevel + 2), s));
-  int64_t ubmax = 1;
-  for (int l = 0; l <= Ds; l++) ubmax = std::max(ubmax, ub[l]);
-  // (the leaf flags and offsets below span all cells: ubtot)
-  t.tmp_nch.ensure(ubtot);
-  t.tmp_off.ensure(ubtot);
-  t.tmp_bnd.ensure(ubmax * 9);
-  t.leaves.ensure(ubtot);
   t.perm.ensure(n);
   t.xs.ensure(n);
   t.xq.ensure(n);
   t.body_leaf.ensure(n);
-  hipLaunchKernelGGL(k_root, dim3(1), dim3(1), 0, s, n, root, t.cx.p, t.cbeg.p, t.ccnt.p, t.cparent.p, t.clevel.p,
-                     t.lcount.p, t.lstart_d.p);
-  XF_LAUNCH();
+  const size_t words = size_t(ceil_div(ubtot, 1024)) + 1;
+  if (t.lookback.cap < words || t.lookback_tag >= (1u << 24) - 64) {  // (a new tag per launch, 24 bits)
+    t.lookback.ensure(words);
+    XF_HIP(hipMemsetAsync(t.lookback.p, 0, sizeof(unsigned long long) * t.lookback.cap, s));
+    t.lookback_tag = 0;
+  }
   const int lfuse = std::min(Ds, kTopLevels);
-  if (lfuse > 0) {
-    hipLaunchKernelGGL(k_top_levels, dim3(1), dim3(kTopThreads), 0, s, lfuse, ncrit, lforce, t.lcount.p,
-                       t.lstart_d.p, k1, t.hist.p, froots, t.cx.p, t.cbeg.p, t.ccnt.p, t.cchild.p, t.cnch.p,
-                       t.cparent.p, t.clevel.p, t.misc.p + 18);
-    XF_LAUNCH();
-  }
-  for (int l = lfuse; l < Ds; l++) {
-    const int g = ceil_div(ub[l], 256);
-    hipLaunchKernelGGL(k_split, dim3(g), dim3(256), 0, s, l, ncrit, lforce, t.lcount.p, t.lstart_d.p, t.cbeg.p,
-                       t.ccnt.p, k1, t.hist.p, t.tmp_nch.p, t.tmp_bnd.p);
-    XF_LAUNCH();
-    scan_exclusive_dev(t.tmp_nch.p, t.tmp_off.p, t.lcount.p + l, int(ub[l]), t.misc.p + 16, t.scan_tmp, s);
-    hipLaunchKernelGGL(k_level_next, dim3(1), dim3(1), 0, s, l, t.lcount.p, t.lstart_d.p, t.misc.p + 16);
-    XF_LAUNCH();
-    hipLaunchKernelGGL(k_emit, dim3(g), dim3(256), 0, s, l, t.lcount.p, t.lstart_d.p, t.tmp_nch.p, t.tmp_off.p,
-                       t.tmp_bnd.p, froots, k1, t.cx.p, t.cbeg.p, t.ccnt.p, t.cchild.p, t.cnch.p, t.cparent.p,
-                       t.clevel.p, t.misc.p + 18);
-    XF_LAUNCH();
-  }
-  hipLaunchKernelGGL(k_last_level, dim3(ceil_div(ub[Ds], 256)), dim3(256), 0, s, Ds, ncrit, t.lcount.p,
-                     t.lstart_d.p, t.ccnt.p, t.cchild.p, t.cnch.p, t.misc.p);
+  // (with a depth of 0 no level is split, but the histogram is still finished)
+  hipLaunchKernelGGL(k_top_levels, dim3(1), dim3(kTopThreads), 0, s, lfuse, ncrit, lforce, t.lcount.p, t.lstart_d.p, k1,
+                     t.hist.p, speculate ? t.hist_bmax.p : nullptr, t.misc.p, froots, t.cx.p, t.cbeg.p, t.ccnt.p,
+                     t.cchild.p, t.cnch.p, t.cparent.p, t.clevel.p, t.misc.p + 18);
   XF_LAUNCH();
+  for (int l = lfuse; l < Ds; l++) {
+    hipLaunchKernelGGL(k_split_level, dim3(ceil_div(level_bound(l), 1024)), dim3(1024), 0, s, l, ncrit, lforce,
+                       t.lcount.p, t.lstart_d.p, k1, t.hist.p, froots, t.cx.p, t.cbeg.p, t.ccnt.p, t.cchild.p, t.cnch.p,
+                       t.cparent.p, t.clevel.p, t.misc.p + 18, t.misc.p + 24 + l, ++t.lookback_tag, t.lookback.p);
+    XF_LAUNCH();
+  }
 
   // Leaves, the gather into tree order and the write-back run before the
-  // level sizes are read, so that read overlaps them: the cell count comes
-  // from the device (misc[19]), the leaf count too (misc[17]), and grids are
-  // sized from the bound ubtot.  A tree the checks below reject or rebuild
-  // (flag bit 1 or 2) leaves the caller's bodies untouched.
-  const int gcells = int(std::min<int64_t>(ceil_div(ubtot, 256), 2048));
-  hipLaunchKernelGGL(k_leaf_flag, dim3(gcells), dim3(256), 0, s, t.misc.p + 19, t.cnch.p, t.tmp_nch.p);
+  // level sizes are read, so that read overlaps them: the counts come from
+  // the device, and grids are sized from the bound ubtot.  A tree the checks
+  // below reject or rebuild (flag bit 1 or 2) leaves the caller's bodies
+  // untouched.
+  hipLaunchKernelGGL(k_leaves, dim3(ceil_div(ubtot, 1024)), dim3(1024), 0, s, Ds, ncrit, t.lcount.p, t.lstart_d.p,
+                     t.ccnt.p, t.cchild.p, t.cnch.p, t.leaves.p, t.misc.p, t.misc.p + 46, ++t.lookback_tag,
+                     t.lookback.p);
   XF_LAUNCH();
-  scan_exclusive_dev(t.tmp_nch.p, t.tmp_off.p, t.misc.p + 19, int(std::min<int64_t>(ubtot, INT32_MAX)), t.misc.p + 17,
-                     t.scan_tmp, s);
-  hipLaunchKernelGGL(k_leaf_compact, dim3(gcells), dim3(256), 0, s, t.misc.p + 19, t.cnch.p, t.tmp_off.p,
-                     t.leaves.p);
-  XF_LAUNCH();
+  const TreeReport rep{t.lcount.p, t.misc.p, root, c.pin_i.p + kPinLevels, c.pin_i.p + kPinMisc, c.pin_d.p};
   hipLaunchKernelGGL(k_leaf_gather, dim3(int(std::min<int64_t>(ubtot, 16384))), dim3(64), sizeof(int) * ncrit, s,
                      t.leaves.p, t.misc.p + 17, t.cbeg.p, t.ccnt.p, t.cx.p, v1, c.bodies, t.perm.p, t.xs.p, t.xq.p,
-                     t.body_leaf.p, ncrit);
+                     t.body_leaf.p, ncrit, rep);
   XF_LAUNCH();
   if (c.defer_writeback)
     c.writeback_pending = true;
@@ -781,10 +925,6 @@ void tree_build(Ctx &c) {
   // level sizes, flags, level maxima, root
   const int *lc = c.pin_i.p + kPinLevels, *fl = c.pin_i.p + kPinMisc;
   const double *rootv = c.pin_d.p;
-  XF_HIP(hipMemcpyAsync(c.pin_i.p + kPinLevels, t.lcount.p, sizeof(int) * (kMaxLevel + 2), hipMemcpyDeviceToHost,
-                        s));
-  XF_HIP(hipMemcpyAsync(c.pin_i.p + kPinMisc, t.misc.p, sizeof(int) * 19, hipMemcpyDeviceToHost, s));
-  XF_HIP(hipMemcpyAsync(c.pin_d.p, root, sizeof(double) * 4, hipMemcpyDeviceToHost, s));
   stream_wait(s);
   if (fl[0] & 1) fail(EXAFMM_ERR_ARG, "non-finite body coordinate or charge");
   // The histogram fixes depths up to kHistLevels; a deeper tree was sorted
