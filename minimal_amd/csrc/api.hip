@@ -172,18 +172,50 @@ void do_downward(Ctx &c) {
   rec(c, 8, c.s0);
 }
 
-// One evaluation over two streams.  P2P needs only the P2P lists: it is
-// launched on s1 as soon as the traversal kernels are enqueued (before the
-// host reads the list totals; a pass that has to be repeated makes it exit
-// at once), and runs beside the rest of the lists, the upward pass and the
-// M2L tile and operator build on s0, its long VALU-bound blocks filling the
-// CUs those latency-bound chains leave idle; the keyed GEMM follows on s0.
-// A periodic tree launches P2P after the lists and the upward pass instead:
-// its far field adds a long latency-bound chain on s0 (the top levels' FP64
-// M2L per pair, the image ladder) that P2P started earlier would starve
-// (N = 2^20, images = 3: 6.5 ms against 6.9).  (Running the upward pass
-// beside the traversal is slower too: its workgroups hold the CUs each
-// short traversal launch waits for.)
+// One evaluation over three streams.  The upward pass needs only the tree: it
+// runs on s2 beside the traversal, whose short launches (one per level) leave
+// the device partly idle.  P2P starts on s1 as soon as the traversal kernels
+// are done (launched before the host reads the list totals; a pass that has
+// to be repeated makes it exit at once).  The rest of the lists and the M2L
+// tile and operator build run on s0 beside them; the keyed GEMM, whose
+// workgroups take every register of a CU and so share none with P2P, follows.
+// A periodic tree launches P2P after the lists are complete: its far field
+// adds a long latency-bound chain on s0 (the top levels' FP64 M2L per pair,
+// the image ladder) that P2P started earlier would starve (N = 2^20, images
+// = 3: 6.5 ms against 6.9).
+void run_passes(Ctx &c) {
+  // P2P on s1 from event 14 (the lists' end on s0)
+  auto launch_p2p = [&c](const int *list_flags) {
+    XF_HIP(hipStreamWaitEvent(c.s1, c.ev[14], 0));
+    rec(c, 5, c.s1);
+    p2p_apply(c, c, c.s1, list_flags);
+    rec(c, 6, c.s1);
+    if (c.writeback_pending) writeback_bodies(c, c.s1);
+    rec(c, 15, c.s1);
+  };
+  // the upward pass on s2, from the tree's end (event 1); joined where the
+  // multipoles are first read (join_upward)
+  auto launch_upward = [&c] {
+    if (c.have_M) return;  // a repeated traversal
+    XF_HIP(hipStreamWaitEvent(c.s2, c.ev[1], 0));
+    do_upward(c, c.s2);
+    c.upward_pending = true;
+  };
+  if (c.cfg.images > 0) {
+    do_lists(c, c, launch_upward);
+    rec(c, 14, c.s0);
+    launch_p2p(nullptr);
+  } else {
+    do_lists(c, c, [&] {
+      rec(c, 14, c.s0);
+      launch_upward();
+      launch_p2p(c.lists.tot.p + 3);
+    });
+  }
+  do_far(c, c);
+  do_downward(c);
+}
+
 void do_passes(Ctx &c) {
   {
     // the bodies' write-back in tree order runs on s1 after P2P, off the
@@ -195,29 +227,15 @@ void do_passes(Ctx &c) {
     c.defer_writeback = true;
     do_build(c);
   }
-  // P2P on s1 from event 14 (the lists' end on s0)
-  auto launch_p2p = [&c](const int *list_flags) {
-    XF_HIP(hipStreamWaitEvent(c.s1, c.ev[14], 0));
-    rec(c, 5, c.s1);
-    p2p_apply(c, c, c.s1, list_flags);
-    rec(c, 6, c.s1);
-    if (c.writeback_pending) writeback_bodies(c, c.s1);
-    rec(c, 15, c.s1);
-  };
-  if (c.cfg.images > 0) {
-    do_lists(c, c);
-    rec(c, 14, c.s0);
-    do_upward(c, c.s0);
-    launch_p2p(nullptr);
-  } else {
-    do_lists(c, c, [&] {
-      rec(c, 14, c.s0);
-      launch_p2p(c.lists.tot.p + 3);
-    });
-    do_upward(c, c.s0);
+  try {
+    run_passes(c);
+  } catch (...) {
+    // what the other streams still run reads this context's tree
+    (void)hipStreamSynchronize(c.s1);
+    (void)hipStreamSynchronize(c.s2);
+    c.upward_pending = false;
+    throw;
   }
-  do_far(c, c);
-  do_downward(c);
 }
 
 }  // namespace
@@ -278,13 +296,13 @@ int exafmm_create(const exafmm_config *cfg, exafmm_ctx **out) {
     c.NT = cfg->P * (cfg->P + 1) / 2;
     try {
       XF_HIP(hipStreamCreateWithFlags(&c.s0, hipStreamNonBlocking));
-      // EXAFMM_SERIAL_STREAMS=1 runs P2P on the main stream (per-kernel
-      // profiles without the P2P / M2L overlap)
+      // EXAFMM_SERIAL_STREAMS=1 runs everything on the main stream (per-kernel
+      // profiles without overlap)
       const char *serial = std::getenv("EXAFMM_SERIAL_STREAMS");
       if (serial && serial[0] == '1')
-        c.s1 = c.s0;
+        c.s1 = c.s2 = c.s0;
       else
-        XF_HIP(hipStreamCreateWithFlags(&c.s1, hipStreamNonBlocking));
+        for (hipStream_t *q : {&c.s1, &c.s2}) XF_HIP(hipStreamCreateWithFlags(q, hipStreamNonBlocking));
       for (auto &e : c.ev) XF_HIP(hipEventCreate(&e));
     } catch (...) {
       delete h;
@@ -311,10 +329,12 @@ int exafmm_destroy(exafmm_ctx *ctx) {
   hipSetDevice(ctx->c.cfg.device);
   if (ctx->c.s0) hipStreamSynchronize(ctx->c.s0);
   if (ctx->c.s1) hipStreamSynchronize(ctx->c.s1);
+  if (ctx->c.s2) hipStreamSynchronize(ctx->c.s2);
   for (auto &e : ctx->c.ev)
     if (e) hipEventDestroy(e);
   if (ctx->c.s0) hipStreamDestroy(ctx->c.s0);
-  if (ctx->c.s1 && ctx->c.s1 != ctx->c.s0) hipStreamDestroy(ctx->c.s1);
+  for (hipStream_t q : {ctx->c.s1, ctx->c.s2})
+    if (q && q != ctx->c.s0) hipStreamDestroy(q);
   delete ctx;
   return EXAFMM_OK;
 }

@@ -240,7 +240,8 @@ struct Lists {
 struct Ctx {
   exafmm_config cfg{};
   int P = 10, NT = 55;
-  hipStream_t s0 = nullptr, s1 = nullptr;
+  // main stream; P2P and the write-back; the upward pass of an evaluation
+  hipStream_t s0 = nullptr, s1 = nullptr, s2 = nullptr;
   hipEvent_t ev[16] = {};
   std::string last_error;
   HostBuf<int> pin_i;                   // kPin* slots
@@ -266,6 +267,7 @@ struct Ctx {
   //   M~ = (Re, Im) M_n^m / R^n,  L~ = (Re, Im) L_j^k R^(j+1)
   Buf<double> M, L;
   bool have_M = false, have_L = false;
+  bool upward_pending = false;  // event 3 on s2 ends an upward pass that s0 has not waited for (join_upward)
   // graph recording (api.hip, exafmm_graph_*): while `capturing`, launches
   // are recorded into a graph (no events, no host waits, no allocation);
   // while a graph holds the context its tree, lists and tiles stay fixed
@@ -340,6 +342,13 @@ void tree_ref_order(Ctx &c, std::vector<int64_t> &bfs2ref, std::vector<int64_t> 
 // with kListRetry bits set is repeated after s1 has drained).
 void traverse(Ctx &tgt, const Ctx &src, const std::function<void()> &after_kernels = {});
 void upward(Ctx &c, hipStream_t s);
+// The main stream waits for an upward pass running on s2: before the first
+// read of the multipoles.
+inline void join_upward(Ctx &c) {
+  if (!c.upward_pending) return;
+  XF_HIP(hipStreamWaitEvent(c.s0, c.ev[3], 0));
+  c.upward_pending = false;
+}
 void m2l_apply(Ctx &tgt, const Ctx &src);
 void m2l_prepare(Ctx &c, hipStream_t s);
 int m2l_fp64_levels(const Ctx &c);  // levels whose M2L runs per pair in FP64 (m2l.hip)

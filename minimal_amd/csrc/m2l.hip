@@ -282,6 +282,7 @@ __global__ void __launch_bounds__(256) k_m2l_fp64_sum(int64_t n, int shares, con
 // (list, cell, harmonics, sums), so below 8,192 cells the lists are shared
 // out over up to 16 workgroups each.
 static void m2l_fp64(Ctx &tc, const Ctx &sc, int ncells, double cycle) {
+  join_upward(tc);
   const int P = tc.P, PP = P * P;
   const int fillP = tc.cfg.m2l_truncation == EXAFMM_M2L_FULL ? 2 * P - 1 : P;
   const M2L64Plan pl = m2l64_plan(P, fillP);

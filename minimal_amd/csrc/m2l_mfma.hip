@@ -1592,6 +1592,7 @@ void m2l_fast(Ctx &tc, const Ctx &sc) {
     m2l_prepare(c, c.s0);
   }
   hipStream_t s = c.s0;
+  join_upward(c);
   const Geom g = geom(c.P);
   const bool bf16 = c.cfg.m2l_precision == EXAFMM_PREC_BF16X3;
   const int nc = int(c.t.ncells);
