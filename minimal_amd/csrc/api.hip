@@ -841,7 +841,8 @@ struct exafmm_graph {
   xf::Buf<xf::GroupTree> gt;
   xf::Buf<xf::GroupLevel> lv;
   xf::Buf<int> starts;
-  Stage pro, p2m, p2p, l2p;
+  Stage pro, p2p, l2p;
+  std::map<int, Stage> p2m;  // by order
   std::vector<Stage> m2m_levels, l2l_levels;  // M2M bottom-up, L2L top-down
   std::vector<std::unique_ptr<xf::GemmGroupPlan>> gemm;  // one per order
   std::vector<int> level_soff_m2m, level_soff_l2l;       // start-array offsets of the level stages
@@ -926,7 +927,13 @@ void grouped_tables(exafmm_graph *g) {
   per_problem(g->pro, [](const Ctx &c) {
     return int64_t(ceil_div(c.t.n, 256)) + ceil_div(c.t.ncells * c.P * c.P, 256);
   });
-  per_problem(g->p2m, [](const Ctx &c) { return int64_t(p2m_group_blocks(c.t.nleaves)); });
+  // one launch per order: the problems of another order have no blocks in it
+  g->p2m.clear();
+  for (const exafmm_ctx *x : g->ctxs) {
+    const int P = x->c.P;
+    if (!g->p2m.count(P))
+      per_problem(g->p2m[P], [P](const Ctx &c) { return c.P == P ? int64_t(p2m_group_blocks(c.t.nleaves)) : 0; });
+  }
   per_problem(g->p2p, [](const Ctx &c) { return int64_t(p2p_group_blocks(c.t.nleaves)); });
   per_problem(g->l2p, [](const Ctx &c) { return int64_t(c.t.nleaves); });
   // per-level stages: the problems that have parents at level l
@@ -997,7 +1004,7 @@ void grouped_record(exafmm_graph *g, hipStream_t sa, hipStream_t sb, hipEvent_t 
   XF_HIP(hipStreamWaitEvent(sb, fork, 0));
   if (g->p2p.blocks) p2p_grouped(g->gt.p, st + g->p2p.off, n, g->p2p.blocks, sb);
   XF_HIP(hipEventRecord(join, sb));
-  if (g->p2m.blocks) p2m_grouped(g->gt.p, st + g->p2m.off, n, g->p2m.blocks, sa);
+  for (const auto &kv : g->p2m) p2m_grouped(kv.first, g->gt.p, st + kv.second.off, n, kv.second.blocks, sa);
   for (size_t k = 0; k < g->m2m_levels.size(); k++) {
     const auto &sg = g->m2m_levels[k];
     if (sg.blocks) m2m_grouped(g->gt.p, g->lv.p + sg.off, st + g->level_soff_m2m[k], sg.n, sg.blocks, sa);

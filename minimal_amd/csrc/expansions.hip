@@ -18,6 +18,8 @@
 // accumulators, with the force from Cartesian ladder identities of the
 // solid harmonics (finite at r = 0 and on the z axis, where the reference's
 // spherical form divides by zero, 3d/kernel.h:31-40).
+#include <type_traits>
+
 #include "fmm_internal.h"
 #include "fmm_ops.h"
 
@@ -35,133 +37,178 @@ struct InvTable {
 };
 static __constant__ InvTable kInv = InvTable();
 
+// f(integral_constant<P>) for the order at run time: kernels whose loops over
+// the degrees unroll are instantiated per order.
+template <class F>
+static void by_order(int P, F &&f) {
+  switch (P) {
+#define XF_ORDER_CASE(n)                          \
+  case n:                                         \
+    return f(std::integral_constant<int, n>());
+    XF_ORDER_CASE(2)
+    XF_ORDER_CASE(3)
+    XF_ORDER_CASE(4)
+    XF_ORDER_CASE(5)
+    XF_ORDER_CASE(6)
+    XF_ORDER_CASE(7)
+    XF_ORDER_CASE(8)
+    XF_ORDER_CASE(9)
+    XF_ORDER_CASE(10)
+    XF_ORDER_CASE(11)
+    XF_ORDER_CASE(12)
+    XF_ORDER_CASE(13)
+    XF_ORDER_CASE(14)
+    XF_ORDER_CASE(15)
+    XF_ORDER_CASE(16)
+#undef XF_ORDER_CASE
+    default:
+      fail(EXAFMM_ERR_UNSUPPORTED, "expansion order");
+  }
+}
+
 // ---------------------------------------------------------------- P2M
-// One wave per leaf: the leaf's bodies are staged in LDS 64 at a time; lane
-// (g, m) = (lane / 16, lane % 16) sums column n = m..P-1 of conj(Y_n^m(u)),
-// u = (x_b - X_c)/R, weighted by q over the bodies b = g mod 4
-// (3d/kernel.h:193 evaluates Y at -beta, i.e. the conjugate); the four body
-// groups are then added with cross-lane shuffles in a fixed order.
+// M~_n^m = sum_b q_b conj(Y_n^m(u_b)), u = (x_b - X_c)/R (3d/kernel.h:193
+// evaluates Y at -beta, i.e. the conjugate).  One wave per leaf.  A column m
+// holds P - m degrees, so a lane takes columns j and P - 1 - j, P + 1 terms
+// whatever j: J = ceil(P / 2) lanes serve a body and G = 64 / J bodies run
+// side by side, with no lane waiting for a longer column.  A term is
+//   Y_n = a z Y_{n-1} + s r^2 Y_{n-2},  s = -1/((n+m)(n-m)),  a = (2n-1) s
+// (n = m + 1: a = -1, s = 0), the factors in registers; where the second
+// column begins they are 0 and its Y_m^m is added.  The G bodies' sums meet
+// in LDS, in body order.  FP64 VALU bound.  (A lane per column and four bodies
+// side by side waited for the longest column: the step of 2^20 uniform bodies,
+// order 10, 3.13 -> 3.04 ms with this, 1.5M clustered, order 12, 8.72 -> 8.56 ms.)
 constexpr int kP2MWaves = 4;
 
-template <int PMAX>
-__device__ __attribute__((always_inline)) inline void p2m_body(int bx, int P, const int *__restrict__ leaves,
-                                const int *__restrict__ nleaves,
-                                const int *__restrict__ cbeg, const int *__restrict__ ccnt,
-                                const double4 *__restrict__ cx,
-                                const double4 *__restrict__ xs, double *__restrict__ M) {
-  static_assert(PMAX <= 16, "16 orders per body group");
-  __shared__ double4 sb[kP2MWaves][kWave];
-  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+template <int P>
+struct P2MShape {
+  static constexpr int J = (P + 1) / 2, G = kWave / J, T = P + 1;
+  static constexpr int S = kWave + J;  // LDS row: lanes reading (term, column) pairs in turn hit distinct banks
+};
+
+template <int P>
+__device__ __attribute__((always_inline)) inline void p2m_body(int bx, const int *__restrict__ leaves,
+                                                               const int *__restrict__ nleaves,
+                                                               const int *__restrict__ cbeg,
+                                                               const int *__restrict__ ccnt,
+                                                               const double4 *__restrict__ cx,
+                                                               const double4 *__restrict__ xs,
+                                                               double *__restrict__ M) {
+  using Sh = P2MShape<P>;
+  constexpr int J = Sh::J, G = Sh::G, T = Sh::T, S = Sh::S;
+  __shared__ double red[kP2MWaves][T * S];
+  const int lane = threadIdx.x % kWave, w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int li = bx * kP2MWaves + w;
-  if (li >= *nleaves) return;
+  if (li >= *nleaves) return;  // whole wave; wave-level syncs only below
   const int c = leaves[li];
   const int beg = cbeg[c], cnt = ccnt[c];
   const double4 C = cx[c];
   const double invR = C.w > 0.0 ? 1.0 / C.w : 0.0;  // R = 0: every body at the centre
-  const int m = lane & 15, g = lane >> 4;
-  // per-lane constants (no divisions per body): 1/(2^m m!) and the
-  // recurrence factors -1/((n+m)(n-m)), n = m+2..P-1
-  double cm = 1.0, sn[PMAX];
-  for (int k = 1; k <= m; k++) cm *= kInv.v[2 * k];
+  const int j = lane % J, g = lane / J, mb = P - 1 - j;
+  const int tb = P - j;  // first term of the second column (none if it is the first: P odd, j = J - 1)
+  double ca = 1.0, cb = mb > j ? 1.0 : 0.0;  // 1/(2^m m!)
+  for (int k = 1; k <= j; k++) ca *= kInv.v[2 * k];
+  for (int k = 1; k <= mb; k++) cb *= kInv.v[2 * k];
+  double fa[T], fs[T], ar[T], ai[T];
 #pragma unroll
-  for (int n = 0; n < PMAX; n++) sn[n] = (n >= m + 2 && n < P) ? -kInv.v[(n + m) * (n - m)] : 0.0;
-  double ar[PMAX], ai[PMAX];
+  for (int t = 0; t < T; t++) {
+    const int m = t < tb ? j : mb, n = t < tb ? j + t : t - 1;
+    const bool in = n > m && !(t >= tb && mb == j);
+    const double s = in ? -kInv.v[(n + m) * (n - m)] : 0.0;
+    fa[t] = in ? (n == m + 1 ? -1.0 : double(2 * n - 1) * s) : 0.0;
+    fs[t] = n == m + 1 ? 0.0 : s;
+    ar[t] = ai[t] = 0.0;
+  }
+  for (int b0 = 0; b0 < cnt; b0 += G) {
+    const int b = b0 + g;
+    const bool valid = g < G && b < cnt;
+    const double4 B = xs[beg + min(b, cnt - 1)];
+    const double q = valid ? B.w : 0.0;
+    const double x = (B.x - C.x) * invR, y = -(B.y - C.y) * invR, z = (B.z - C.z) * invR;  // conjugate
+    const double r2 = x * x + y * y + z * z;
+    // (x + iy)^j, then (x + iy)^(P-1-j) = (x + iy)^j ((x + iy)^2)^(J-1-j) [(x + iy) if P is even]
+    double pr = 1.0, pi = 0.0;
 #pragma unroll
-  for (int n = 0; n < PMAX; n++) ar[n] = ai[n] = 0;
-  for (int b0 = 0; b0 < cnt; b0 += kWave) {
-    const int nb = min(kWave, cnt - b0);
-    if (lane < nb) sb[w][lane] = xs[beg + b0 + lane];
+    for (int k = 1; k < J; k++)
+      if (k <= j) {
+        const double tr = pr * x - pi * y;
+        pi = pr * y + pi * x;
+        pr = tr;
+      }
+    double cr = pr * (q * ca), ci = pi * (q * ca);
+    const double xr = x * x - y * y, xi = 2.0 * (x * y);
+#pragma unroll
+    for (int k = 1; k < J; k++)
+      if (k <= J - 1 - j) {
+        const double tr = pr * xr - pi * xi;
+        pi = pr * xi + pi * xr;
+        pr = tr;
+      }
+    if (P % 2 == 0) {
+      const double tr = pr * x - pi * y;
+      pi = pr * y + pi * x;
+      pr = tr;
+    }
+    const double br = pr * (q * cb), bi = pi * (q * cb);
+    double or_ = 0.0, oi = 0.0;  // the term before
+    ar[0] += cr;
+    ai[0] += ci;
+#pragma unroll
+    for (int t = 1; t < T; t++) {
+      const double az = fa[t] * z, sr = fs[t] * r2;
+      double nr = az * cr + sr * or_, ni = az * ci + sr * oi;
+      if (t >= P - J + 1) {  // the second column may begin here
+        const double sel = t == tb ? 1.0 : 0.0;
+        nr += sel * br;
+        ni += sel * bi;
+      }
+      or_ = cr;
+      oi = ci;
+      cr = nr;
+      ci = ni;
+      ar[t] += cr;
+      ai[t] += ci;
+    }
+  }
+  // sums over the body groups: output o = (term, column pair) by lane o % 64
+  double *R = red[w];
+  double *Mc = M + int64_t(c) * P * P;
+#pragma unroll
+  for (int part = 0; part < 2; part++) {
+#pragma unroll
+    for (int t = 0; t < T; t++) R[t * S + lane] = part ? ai[t] : ar[t];
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (m < P) {
-      // two bodies (bi, bi + 4) per pass: independent recurrence chains
-      // interleave; a missing second body has charge 0 and adds exact zeros
-      for (int bi = g; bi < nb; bi += 8) {
-        const bool two = bi + 4 < nb;
-        const double4 B0 = sb[w][bi], B1 = sb[w][two ? bi + 4 : bi];
-        const double x0 = (B0.x - C.x) * invR, y0 = -(B0.y - C.y) * invR, z0 = (B0.z - C.z) * invR;  // conjugate
-        const double x1 = (B1.x - C.x) * invR, y1 = -(B1.y - C.y) * invR, z1 = (B1.z - C.z) * invR;
-        const double r20 = x0 * x0 + y0 * y0 + z0 * z0, r21 = x1 * x1 + y1 * y1 + z1 * z1;
-        double yr0 = 1.0, yi0 = 0, yr1 = 1.0, yi1 = 0;  // (x + iy)^m
-        for (int k = 1; k <= m; k++) {
-          const double tr0 = yr0 * x0 - yi0 * y0, ti0 = yr0 * y0 + yi0 * x0;
-          const double tr1 = yr1 * x1 - yi1 * y1, ti1 = yr1 * y1 + yi1 * x1;
-          yr0 = tr0;
-          yi0 = ti0;
-          yr1 = tr1;
-          yi1 = ti1;
-        }
-        const double qc0 = B0.w * cm, qc1 = two ? B1.w * cm : 0.0;  // q * Y_m^m = q (x+iy)^m / (2^m m!)
-        double pr0 = 0, pi0 = 0, cr0 = yr0 * qc0, ci0 = yi0 * qc0;
-        double pr1 = 0, pi1 = 0, cr1 = yr1 * qc1, ci1 = yi1 * qc1;
+    for (int o = lane; o < T * J; o += kWave) {
+      const int t = o / J, oj = o % J;
+      const bool second = t >= P - oj;
+      const int m = second ? P - 1 - oj : oj, n = second ? t - 1 : oj + t;
+      double v = 0.0;
 #pragma unroll
-        for (int n = 0; n < PMAX; n++) {
-          if (n < m || n >= P) continue;
-          if (n > m) {
-            double nr0, ni0, nr1, ni1;
-            if (n == m + 1) {
-              nr0 = -z0 * cr0;
-              ni0 = -z0 * ci0;
-              nr1 = -z1 * cr1;
-              ni1 = -z1 * ci1;
-            } else {
-              const double c2 = double(2 * n - 1);
-              nr0 = (c2 * z0 * cr0 + r20 * pr0) * sn[n];
-              ni0 = (c2 * z0 * ci0 + r20 * pi0) * sn[n];
-              nr1 = (c2 * z1 * cr1 + r21 * pr1) * sn[n];
-              ni1 = (c2 * z1 * ci1 + r21 * pi1) * sn[n];
-            }
-            pr0 = cr0;
-            pi0 = ci0;
-            cr0 = nr0;
-            ci0 = ni0;
-            pr1 = cr1;
-            pi1 = ci1;
-            cr1 = nr1;
-            ci1 = ni1;
-          }
-          ar[n] += cr0;
-          ai[n] += ci0;
-          ar[n] += cr1;
-          ai[n] += ci1;
-        }
-      }
+      for (int k = 0; k < G; k++) v += R[t * S + k * J + oj];
+      if (!(second && m == oj) && (part == 0 || m > 0)) Mc[rf(n, m, part)] = v;
     }
     __builtin_amdgcn_wave_barrier();
   }
-#pragma unroll
-  for (int n = 0; n < PMAX; n++) {
-    ar[n] += __shfl_xor(ar[n], 16);
-    ai[n] += __shfl_xor(ai[n], 16);
-    ar[n] += __shfl_xor(ar[n], 32);
-    ai[n] += __shfl_xor(ai[n], 32);
-  }
-  if (g != 0 || m >= P) return;
-  double *Mc = M + int64_t(c) * P * P;
-#pragma unroll
-  for (int n = 0; n < PMAX; n++) {
-    if (n < m || n >= P) continue;
-    Mc[rf(n, m, 0)] = ar[n];
-    if (m > 0) Mc[rf(n, m, 1)] = ai[n];
-  }
 }
 
-template <int PMAX>
-__global__ void __launch_bounds__(kP2MWaves *kWave) k_p2m(int P, const int *__restrict__ leaves,
+template <int P>
+__global__ void __launch_bounds__(kP2MWaves *kWave) k_p2m(const int *__restrict__ leaves,
                                                           const int *__restrict__ nleaves,
                                                           const int *__restrict__ cbeg, const int *__restrict__ ccnt,
                                                           const double4 *__restrict__ cx,
                                                           const double4 *__restrict__ xs, double *__restrict__ M) {
-  p2m_body<PMAX>(blockIdx.x, P, leaves, nleaves, cbeg, ccnt, cx, xs, M);
+  p2m_body<P>(blockIdx.x, leaves, nleaves, cbeg, ccnt, cx, xs, M);
 }
 
-// All problems of a batch in one launch (block -> problem through start[]).
+// The problems of one order of a batch in one launch (block -> problem through start[]).
+template <int P>
 __global__ void __launch_bounds__(kP2MWaves *kWave) k_p2m_grouped(const GroupTree *__restrict__ g,
                                                                   const int *__restrict__ start, int nprob) {
   const int b = blockIdx.x, i = group_of(start, nprob, b);
   const GroupTree &t = g[i];
-  p2m_body<kMaxP>(b - start[i], t.P, t.leaves, t.nleaves, t.cbeg, t.ccnt, t.cx, t.xs, t.M);
+  p2m_body<P>(b - start[i], t.leaves, t.nleaves, t.cbeg, t.ccnt, t.cx, t.xs, t.M);
 }
 
 
@@ -750,8 +797,10 @@ int p2m_group_blocks(int64_t nleaves) { return ceil_div(nleaves, kP2MWaves); }
 int shift_group_rows(int P) { return ceil_div(P * P, 16 * kShiftWaves); }
 int m2m_group_rows(int P) { return ceil_div(P * P, 16); }
 
-void p2m_grouped(const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s) {
-  hipLaunchKernelGGL(k_p2m_grouped, dim3(nblocks), dim3(kP2MWaves * kWave), 0, s, g, start, nprob);
+void p2m_grouped(int P, const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s) {
+  by_order(P, [&](auto p) {
+    hipLaunchKernelGGL((k_p2m_grouped<p()>), dim3(nblocks), dim3(kP2MWaves * kWave), 0, s, g, start, nprob);
+  });
   XF_LAUNCH();
 }
 void m2m_grouped(const GroupTree *g, const GroupLevel *lv, const int *start, int n, int nblocks, hipStream_t s) {
@@ -772,26 +821,10 @@ void upward(Ctx &c, hipStream_t s) {
   const int P = c.P, PP = P * P;
   shift_ops(c, s);
   c.M.ensure(size_t(t.ncells) * PP);
-  const int64_t nl = t.nleaves;
-  // the per-lane degree loop is unrolled to PMAX (masked past P): the
-  // smallest even bound >= P keeps the masked iterations few
-  const dim3 pg(ceil_div(nl, kP2MWaves)), pb(kP2MWaves * kWave);
-  switch (std::max(4, (P + 1) & ~1)) {
-#define XF_P2M_CASE(n)                                                                                      \
-  case n:                                                                                                    \
-    hipLaunchKernelGGL((k_p2m<n>), pg, pb, 0, s, P, t.leaves.p, t.misc.p + 17, t.cbeg.p, t.ccnt.p, t.cx.p, \
-                       t.xs.p, c.M.p);                                                                       \
-    break;
-    XF_P2M_CASE(4)
-    XF_P2M_CASE(6)
-    XF_P2M_CASE(8)
-    XF_P2M_CASE(10)
-    XF_P2M_CASE(12)
-    XF_P2M_CASE(14)
-    XF_P2M_CASE(16)
-#undef XF_P2M_CASE
-    default: fail(EXAFMM_ERR_UNSUPPORTED, "expansion order");
-  }
+  by_order(P, [&](auto p) {
+    hipLaunchKernelGGL((k_p2m<p()>), dim3(ceil_div(t.nleaves, kP2MWaves)), dim3(kP2MWaves * kWave), 0, s, t.leaves.p,
+                       t.misc.p + 17, t.cbeg.p, t.ccnt.p, t.cx.p, t.xs.p, c.M.p);
+  });
   XF_LAUNCH();
   for (int l = t.depth - 1; l >= t.lroot; l--) {  // (a forest stops at its problems' roots)
     const int cnt = t.lstart[l + 1] - t.lstart[l];

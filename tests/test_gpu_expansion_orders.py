@@ -1,0 +1,42 @@
+"""P2M at every order: its loops over the degrees are unrolled per
+order, lanes hold columns in pairs (odd orders leave one alone), and leaves of
+one body, of a few, of a wave's share and of several lie in one tree.
+
+Multipoles are FP64 sums of the same terms in another order: 1e-12 (the bar of
+the parity tests) of the terms' sum, |Y_n^m| <= rho^n / n!, with the distances
+of a leaf's bodies and the half diagonal of a larger cell.
+"""
+import math
+
+import numpy as np
+import pytest
+
+from minimal_amd import fmm
+from minimal_amd.inputs import plummer, uniform_cube
+
+pytestmark = pytest.mark.gpu
+
+
+def _bodies(n, seed):
+    b = uniform_cube(n, seed, "sym")
+    b["X"][: n // 2] = plummer(n // 2, 0.05, 0.5, np.random.default_rng(seed))
+    return b
+
+
+@pytest.mark.parametrize("P", range(2, 17))
+@pytest.mark.parametrize("n,ncrit", [(1, 64), (3000, 100)])
+def test_multipoles(gpu, orc, P, n, ncrit):
+    b, b2 = _bodies(n, 7 * P + n), _bodies(n, 7 * P + n)
+    s = orc.session(P, ncrit, 0.4)
+    s.build_tree(b2)
+    s.upward(b2)
+    f = fmm.FMM(P=P, ncrit=ncrit, theta=0.4)
+    f.build_tree(b)
+    f.upward()
+    cells, diff = f.cells(), np.abs(f.multipoles() - s.M())
+    for i, c in enumerate(cells):
+        mine = b[c["body"]:c["body"] + c["nbody"]]
+        rho = np.linalg.norm(mine["X"] - c["X"], axis=1) if c["nchild"] == 0 else 3 ** 0.5 * c["R"]
+        for k in range(P):
+            bound = np.sum(np.abs(mine["q"]) * rho ** k) / math.factorial(k)
+            assert np.all(diff[i, k * (k + 1) // 2:(k + 1) * (k + 2) // 2] <= 1e-12 * bound), (i, k)
