@@ -590,157 +590,109 @@ __global__ void __launch_bounds__(kShiftWaves *kWave) k_l2l_grouped(const GroupT
 
 
 // ---------------------------------------------------------------- L2P
-// One thread per body.  With u = (x - Xc)/R and
-// Lh_n^m = L_n^m R^n = L~/R, phi = Re sum_{n, m>=0} w_m Lh_n^m Y_n^m(u)
-// (w_0 = 1, w_m = 2, 3d/kernel.h:302-316).  The gradient uses
+// With u = (x - Xc)/R and Lh_n^m = w_m L_n^m R^n = w_m L~/R (w_0 = 1, w_m = 2),
+// phi = Re sum_{n, m>=0} Lh_n^m Y_n^m(u) (3d/kernel.h:302-316).  The gradient uses
 //   dz Y_n^m = -Y_{n-1}^m,  (dx + i dy) Y_n^m = -Y_{n-1}^{m+1},
-//   (dx - i dy) Y_n^m = Y_{n-1}^{m-1} (m >= 1), = -conj(Y_{n-1}^1) (m = 0),
-// collected per harmonic Y_n^m so each column m is generated once.
-// Potential and field of one body at u = (x, y, z) (leaf units) from the
-// leaf's folded coefficients Lh (LDS) and the recurrence factors rec.
-// PC > 0: the order is the compile-time PC and the (n, m) loops unroll, so
-// the LDS offsets and the branches below resolve at compile time.
-template <class T, int PC = 0>
-__device__ __attribute__((always_inline)) inline void l2p_eval(int Prt, T x, T y, T z, const cpx<T> *Lh,
-                                                              const T *rec, T &pot, T &Fx2, T &Fy2, T &Dz) {
-  const int P = PC > 0 ? PC : Prt;
-  const T r2 = x * x + y * y + z * z;
-  T Ar = 0, Ai = 0, Br = 0, Bi = 0;
-  pot = 0;
-  Dz = 0;
-  T ymr = 1, ymi = 0;          // Y_m^m
-  T pr = 0, pi = 0, cr = 0, ci = 0;  // Y_{n-1}^m, Y_n^m
-  auto term = [&](int m, int n) {
-    if (n == m) {
-      if (m > 0) {
-        const T inv = rec[nms(m, m)];
-        const T tr = (ymr * x - ymi * y) * inv, ti = (ymr * y + ymi * x) * inv;
-        ymr = tr;
-        ymi = ti;
-      }
-      pr = 0;
-      pi = 0;
-      cr = ymr;
-      ci = ymi;
-    } else {
-      T nr, ni;
-      if (n == m + 1) {
-        nr = -z * cr;
-        ni = -z * ci;
+//   (dx - i dy) Y_n^m = Y_{n-1}^{m-1} (m >= 1), = -conj(Y_{n-1}^1) (m = 0).
+// Degree by degree, with the harmonics of the last two degrees in registers:
+// every coefficient is read from LDS once and meets Y_{n-1}^{m-1}, Y_{n-1}^m,
+// Y_{n-1}^{m+1} and Y_n^m there.  (Column by column a coefficient was read for
+// each of the four, and orders without an unrolled kernel ran a loop of
+// dependent LDS reads: order 12, 1.5M bodies 223 -> 90 us.)
+template <int P, class T>
+__device__ __attribute__((always_inline)) inline void l2p_eval(T x, T y, T z, const cpx<T> *Lh, T &pot, T &Fx2,
+                                                               T &Fy2, T &Dz) {
+  T r2 = x * x + y * y + z * z;
+  T Ar = 0, Ai = 0, Br = 0, Bi = 0, dz = 0, ph = Lh[0].re;
+  T ar[P], ai[P], br[P], bi[P];  // Y_{n-1}^m, Y_{n-2}^m
+#pragma unroll
+  for (int m = 0; m < P; m++) ar[m] = ai[m] = br[m] = bi[m] = 0;
+  ar[0] = 1;
+  int o = 0;
+#pragma unroll
+  for (int n = 1; n < P; n++) {
+    // opaque position and offset: this degree's harmonics and coefficients are
+    // made here, not all at the front, where they would take every register
+    asm volatile("" : "+v"(o), "+v"(x), "+v"(y), "+v"(z), "+v"(r2), "+v"(ph), "+v"(dz), "+v"(Ar), "+v"(Ai), "+v"(Br),
+                      "+v"(Bi));
+    T cr[P], ci[P];  // Y_n^m
+#pragma unroll
+    for (int m = 0; m <= n; m++) {
+      if (m == n) {
+        const T inv = T(0.5 / n);
+        cr[m] = (ar[n - 1] * x - ai[n - 1] * y) * inv;
+        ci[m] = (ar[n - 1] * y + ai[n - 1] * x) * inv;
+      } else if (m == n - 1) {
+        cr[m] = -z * ar[m];
+        ci[m] = -z * ai[m];
       } else {
-        const T s = rec[nms(n, m)];
-        const T cz = T(2 * n - 1) * z;
-        nr = (cz * cr + r2 * pr) * s;
-        ni = (cz * ci + r2 * pi) * s;
+        const T s = T(-1.0 / double((n + m) * (n - m))), cz = T(2 * n - 1) * z;
+        cr[m] = (cz * ar[m] + r2 * br[m]) * s;
+        ci[m] = m ? (cz * ai[m] + r2 * bi[m]) * s : T(0);
       }
-      pr = cr;
-      pi = ci;
-      cr = nr;
-      ci = ni;
-    }
-    const cpx<T> l0 = Lh[nms(n, m)];
-    pot += l0.re * cr - l0.im * ci;
-    if (n + 1 < P) {
-      const cpx<T> lz = Lh[nms(n + 1, m)];
-      Dz -= lz.re * cr - lz.im * ci;
-      if (m >= 1) {
-        const cpx<T> la = Lh[nms(n + 1, m - 1)];
-        Ar -= la.re * cr - la.im * ci;
-        Ai -= la.re * ci + la.im * cr;
-      }
-      const cpx<T> lb = Lh[nms(n + 1, m + 1)];
-      Br += lb.re * cr - lb.im * ci;
-      Bi += lb.re * ci + lb.im * cr;
-      if (m == 1) {  // the m = 0 terms' (dx - i dy): -Lh_{n+1}^0 conj(Y_n^1)
-        const cpx<T> l00 = Lh[nms(n + 1, 0)];
-        Br -= l00.re * cr + l00.im * ci;
-        Bi -= l00.im * cr - l00.re * ci;
+      const cpx<T> l = Lh[o + nms(n, m)];
+      if (m == 0) {  // real
+        ph += l.re * cr[0];
+        dz -= l.re * ar[0];
+        if (n > 1) {
+          Ar -= T(2) * (l.re * ar[1]);
+          Ai -= T(2) * (l.re * ai[1]);
+        }
+      } else {
+        ph += l.re * cr[m] - l.im * ci[m];
+        if (m < n) dz -= l.re * ar[m] - l.im * ai[m];
+        if (m + 1 < n) {
+          Ar -= l.re * ar[m + 1] - l.im * ai[m + 1];
+          Ai -= l.re * ai[m + 1] + l.im * ar[m + 1];
+        }
+        Br += l.re * ar[m - 1] - l.im * ai[m - 1];
+        Bi += l.re * ai[m - 1] + l.im * ar[m - 1];
       }
     }
-  };
-  if constexpr (PC > 0) {
 #pragma unroll
-    for (int m = 0; m < PC; m++)
-#pragma unroll
-      for (int n = m; n < PC; n++) term(m, n);
-  } else {
-    for (int m = 0; m < P; m++)
-      for (int n = m; n < P; n++) term(m, n);
+    for (int m = 0; m <= n; m++) {
+      br[m] = ar[m];
+      bi[m] = ai[m];
+      ar[m] = cr[m];
+      ai[m] = ci[m];
+    }
   }
+  pot = ph;
+  Dz = dz;
   Fx2 = Ar + Br;  // 2 dphi/dx
   Fy2 = Ai - Bi;  // 2 dphi/dy
 }
 
-// Lh (w_m and L~ -> L R^n folded in) and the recurrence factors of one leaf,
-// entries e = lane, lane + stride, ...
-template <class T>
-__device__ inline void l2p_stage(int P, int e0, int stride, const double *__restrict__ Lc, double invR, cpx<T> *Lh,
-                                 T *rec) {
-  const int NT = P * (P + 1) / 2;
-  for (int e = e0; e < NT; e += stride) {
-    int n, m;
-    jk_of(e, n, m);
-    const double w = (m == 0 ? 1.0 : 2.0) * invR;
-    Lh[e] = {T(Lc[rf(n, m, 0)] * w), T(m ? Lc[rf(n, m, 1)] * w : 0.0)};
-    if (rec) rec[e] = n == m ? T(m ? kInv.v[2 * m] : 0.0) : (n >= m + 2 ? T(-kInv.v[(n + m) * (n - m)]) : T(0));
-  }
-}
-
-template <int MAXP, class T>
-__device__ __attribute__((always_inline)) inline void l2p_body(int bx, int P, const int *__restrict__ leaves, const int *__restrict__ nleaves,
-                                const int *__restrict__ cbeg, const int *__restrict__ ccnt,
-                                const double4 *__restrict__ cx, const double *__restrict__ L,
-                                const double4 *__restrict__ xs, exafmm_body *__restrict__ bodies) {
-  __shared__ cpx<T> Lh[MAXP * (MAXP + 1) / 2];
-  __shared__ T rec[MAXP * (MAXP + 1) / 2];  // 1/(2m) at (m, m), -1/((n+m)(n-m)) at (n, m), n >= m + 2
-  const int li = bx;
-  if (li >= *nleaves) return;
-  const int c = leaves[li];
-  const double4 C = cx[c];
-  const double invR = C.w > 0.0 ? 1.0 / C.w : 0.0;  // R = 0: every body at the centre
-  l2p_stage<T>(P, threadIdx.x, 64, L + int64_t(c) * P * P, invR, Lh, rec);
-  __syncthreads();
-  const int beg = cbeg[c], cnt = ccnt[c];
-  for (int b = beg + threadIdx.x; b < beg + cnt; b += 64) {
-    const double4 B = xs[b];
-    T pot, fx2, fy2, dz;
-    l2p_eval<T>(P, T((B.x - C.x) * invR), T((B.y - C.y) * invR), T((B.z - C.z) * invR), Lh, rec, pot, fx2, fy2, dz);
-    exafmm_body *o = bodies + b;
-    o->p += double(pot);
-    o->F[0] += 0.5 * double(fx2) * invR;
-    o->F[1] += 0.5 * double(fy2) * invR;
-    o->F[2] += double(dz) * invR;
-  }
-}
-
-// FP32 L2P over the bodies in tree order, 64 per wave (full waves whatever
-// the leaf sizes; one wave per leaf leaves half its lanes idle at 32 bodies
-// a leaf).  The wave's bodies fall into runs of equal leaf; up to kL2PSlots
-// runs at a time have their coefficients staged in LDS (one pass for
-// uniform trees, a few when many small leaves share a wave), and each lane
-// evaluates its own body against its run's slot.
+// L2P over the bodies in tree order, 64 per wave (full waves whatever the leaf
+// sizes; one wave per leaf leaves half its lanes idle at 32 bodies a leaf).
+// The wave's bodies fall into runs of equal leaf; up to kL2PSlots runs at a
+// time have their coefficients staged in LDS (one pass for uniform trees, a
+// few when many small leaves share a wave), and each lane evaluates its own
+// body against its run's slot.  T = float, or double in parity mode.
 constexpr int kL2PSlots = 8;
-template <int MAXP, int PC>
-__global__ void __launch_bounds__(64) k_l2p_flat(int P, int64_t n, const int *__restrict__ body_leaf,
-                                                 const double4 *__restrict__ cx, const double *__restrict__ L,
-                                                 const double4 *__restrict__ xs, exafmm_body *__restrict__ bodies) {
-  constexpr int NTM = MAXP * (MAXP + 1) / 2;
-  __shared__ cpx<float> Lh[kL2PSlots][NTM];
-  __shared__ float rec[NTM];
+template <int P, class T>
+__device__ __attribute__((always_inline)) inline void l2p_body(int bx, int64_t n, const int *__restrict__ body_leaf,
+                                                               const double4 *__restrict__ cx,
+                                                               const double *__restrict__ L,
+                                                               const double4 *__restrict__ xs,
+                                                               exafmm_body *__restrict__ bodies) {
+  constexpr int NT = P * (P + 1) / 2, KE = (NT + kWave - 1) / kWave;
+  __shared__ cpx<T> Lh[kL2PSlots][NT | 1];  // odd: the slots' equal entries lie in distinct banks
   __shared__ int sleaf[kL2PSlots];
   const int lane = threadIdx.x;
-  const int64_t b = int64_t(blockIdx.x) * kWave + lane;
+  const int64_t b = int64_t(bx) * kWave + lane;
   const bool valid = b < n;
   const int leaf = valid ? body_leaf[b] : -1;
   const int prev = __shfl_up(leaf, 1);
   const unsigned long long starts = __ballot(valid && (lane == 0 || prev != leaf));
   const int nruns = __popcll(starts);
   const int run = valid ? __popcll(starts & (~0ull >> (63 - lane))) - 1 : -1;
-  const int NT = P * (P + 1) / 2;
-  for (int e = lane; e < NT; e += kWave) {
-    int nn, m;
-    jk_of(e, nn, m);
-    rec[e] = nn == m ? (m ? float(kInv.v[2 * m]) : 0.0f) : (nn >= m + 2 ? float(-kInv.v[(nn + m) * (nn - m)]) : 0.0f);
+  int em[KE], er[KE];  // this lane's coefficients: order m, place of the real part
+#pragma unroll
+  for (int k = 0; k < KE; k++) {
+    int en;
+    jk_of(min(lane + k * kWave, NT - 1), en, em[k]);
+    er[k] = rf(en, em[k], 0);
   }
   double4 C = make_double4(0, 0, 0, 1), B = make_double4(0, 0, 0, 0);
   if (valid) {
@@ -754,18 +706,26 @@ __global__ void __launch_bounds__(64) k_l2p_flat(int P, int64_t n, const int *__
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    for (int e = lane; e < ns * NT; e += kWave) {
-      const int sl = e / NT, k = e - sl * NT, c = sleaf[sl];
-      const double Rc = cx[c].w;
-      l2p_stage<float>(P, k, NT, L + int64_t(c) * P * P, Rc > 0.0 ? 1.0 / Rc : 0.0, Lh[sl], nullptr);
+#pragma unroll 4
+    for (int sl = 0; sl < ns; sl++) {
+      const int c = __builtin_amdgcn_readfirstlane(sleaf[sl]);
+      const double Rc = cx[c].w, w = Rc > 0.0 ? 1.0 / Rc : 0.0;
+      const double *Lc = L + int64_t(c) * P * P;
+#pragma unroll
+      for (int k = 0; k < KE; k++)
+        if (lane + k * kWave < NT) {
+          const double re = Lc[er[k]], im = em[k] ? Lc[er[k] + 1] : 0.0;
+          const double wm = em[k] ? 2.0 * w : w;
+          Lh[sl][lane + k * kWave] = {T(re * wm), T(im * wm)};
+        }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     if (valid && run >= g0 && run < g0 + ns) {
-      float pot, fx2, fy2, dz;
-      l2p_eval<float, PC>(P, float((B.x - C.x) * invR), float((B.y - C.y) * invR), float((B.z - C.z) * invR),
-                          Lh[run - g0], rec, pot, fx2, fy2, dz);
+      T pot, fx2, fy2, dz;
+      l2p_eval<P, T>(T((B.x - C.x) * invR), T((B.y - C.y) * invR), T((B.z - C.z) * invR), Lh[run - g0], pot, fx2, fy2,
+                     dz);
       exafmm_body *o = bodies + b;
       o->p += double(pot);
       o->F[0] += 0.5 * double(fx2) * invR;
@@ -776,19 +736,20 @@ __global__ void __launch_bounds__(64) k_l2p_flat(int P, int64_t n, const int *__
   }
 }
 
-template <int MAXP, class T>
-__global__ void __launch_bounds__(64) k_l2p(int P, const int *__restrict__ leaves, const int *__restrict__ nleaves,
-                                            const int *__restrict__ cbeg, const int *__restrict__ ccnt,
+template <int P, class T>
+__global__ void __launch_bounds__(64) k_l2p(int64_t n, const int *__restrict__ body_leaf,
                                             const double4 *__restrict__ cx, const double *__restrict__ L,
                                             const double4 *__restrict__ xs, exafmm_body *__restrict__ bodies) {
-  l2p_body<MAXP, T>(blockIdx.x, P, leaves, nleaves, cbeg, ccnt, cx, L, xs, bodies);
+  l2p_body<P, T>(blockIdx.x, n, body_leaf, cx, L, xs, bodies);
 }
 
+// The problems of one order of a batch in one launch.
+template <int P>
 __global__ void __launch_bounds__(64) k_l2p_grouped(const GroupTree *__restrict__ g, const int *__restrict__ start,
                                                     int nprob) {
   const int b = blockIdx.x, i = group_of(start, nprob, b);
   const GroupTree &t = g[i];
-  l2p_body<kMaxP, float>(b - start[i], t.P, t.leaves, t.nleaves, t.cbeg, t.ccnt, t.cx, t.L, t.xs, t.bodies);
+  l2p_body<P, float>(b - start[i], t.n, t.body_leaf, t.cx, t.L, t.xs, t.bodies);
 }
 
 
@@ -811,8 +772,10 @@ void l2l_grouped(const GroupTree *g, const GroupLevel *lv, const int *start, int
   hipLaunchKernelGGL(k_l2l_grouped, dim3(nblocks), dim3(kShiftWaves * kWave), 0, s, g, lv, start, n);
   XF_LAUNCH();
 }
-void l2p_grouped(const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s) {
-  hipLaunchKernelGGL(k_l2p_grouped, dim3(nblocks), dim3(64), 0, s, g, start, nprob);
+void l2p_grouped(int P, const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s) {
+  by_order(P, [&](auto p) {
+    hipLaunchKernelGGL((k_l2p_grouped<p()>), dim3(nblocks), dim3(kWave), 0, s, g, start, nprob);
+  });
   XF_LAUNCH();
 }
 
@@ -859,21 +822,12 @@ void l2l_pass(Ctx &c) {
 
 void l2p_pass(Ctx &c) {
   Tree &t = c.t;
-  hipStream_t s = c.s0;
-  const int P = c.P;
   // FP64 evaluation in parity mode, FP32 otherwise
-  if (c.cfg.m2l_precision == EXAFMM_PREC_FP64)
-    hipLaunchKernelGGL((k_l2p<kMaxP, double>), dim3(t.nleaves), dim3(64), 0, s, P, t.leaves.p, t.misc.p + 17,
-                       t.cbeg.p, t.ccnt.p, t.cx.p, c.L.p, t.xs.p, c.bodies);
-  else {
-    // the common orders unrolled at compile time, any other order generic
-    auto flat = k_l2p_flat<kMaxP, 0>;
-    if (P == 6) flat = k_l2p_flat<kMaxP, 6>;
-    if (P == 8) flat = k_l2p_flat<kMaxP, 8>;
-    if (P == 10) flat = k_l2p_flat<kMaxP, 10>;
-    hipLaunchKernelGGL(flat, dim3(ceil_div(t.n, kWave)), dim3(kWave), 0, s, P, t.n, t.body_leaf.p, t.cx.p, c.L.p,
-                       t.xs.p, c.bodies);
-  }
+  by_order(c.P, [&](auto p) {
+    auto k = c.cfg.m2l_precision == EXAFMM_PREC_FP64 ? k_l2p<p(), double> : k_l2p<p(), float>;
+    hipLaunchKernelGGL(k, dim3(ceil_div(t.n, kWave)), dim3(kWave), 0, c.s0, t.n, t.body_leaf.p, t.cx.p, c.L.p, t.xs.p,
+                       c.bodies);
+  });
   XF_LAUNCH();
 }
 

@@ -158,7 +158,7 @@ __device__ inline int group_of(const int *__restrict__ start, int n, int b) {
 // The device arrays of one problem that the charge-dependent passes read
 // and write (its own tree is source and target).
 struct GroupTree {
-  const int *leaves, *nleaves, *cbeg, *ccnt, *cchild, *cnch;
+  const int *leaves, *nleaves, *cbeg, *ccnt, *cchild, *cnch, *body_leaf;
   const double4 *cx, *xs;
   const float4 *xq;
   double4 *xs_w;
@@ -369,7 +369,7 @@ int p2p_group_blocks(int64_t nleaves);
 void p2m_grouped(int P, const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s);
 void m2m_grouped(const GroupTree *g, const GroupLevel *lv, const int *start, int n, int nblocks, hipStream_t s);
 void l2l_grouped(const GroupTree *g, const GroupLevel *lv, const int *start, int n, int nblocks, hipStream_t s);
-void l2p_grouped(const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s);
+void l2p_grouped(int P, const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s);
 void p2p_grouped(const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s);
 // keyed M2L of every problem of one order (BF16x3, fixed order): cast +
 // GEMM, one launch each; the plan holds the device descriptor tables

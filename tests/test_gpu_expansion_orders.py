@@ -1,4 +1,4 @@
-"""P2M at every order: its loops over the degrees are unrolled per
+"""P2M and L2P at every order: their loops over the degrees are unrolled per
 order, lanes hold columns in pairs (odd orders leave one alone), and leaves of
 one body, of a few, of a wave's share and of several lie in one tree.
 
@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 from minimal_amd import fmm
-from minimal_amd.inputs import plummer, uniform_cube
+from minimal_amd.inputs import plummer, rel_l2, uniform_cube
 
 pytestmark = pytest.mark.gpu
 
@@ -40,3 +40,21 @@ def test_multipoles(gpu, orc, P, n, ncrit):
         for k in range(P):
             bound = np.sum(np.abs(mine["q"]) * rho ** k) / math.factorial(k)
             assert np.all(diff[i, k * (k + 1) // 2:(k + 1) * (k + 2) // 2] <= 1e-12 * bound), (i, k)
+
+
+@pytest.mark.parametrize("P", range(2, 17))
+@pytest.mark.parametrize("n,ncrit", [(2000, 2), (3000, 100)])
+def test_field(gpu, orc, P, n, ncrit):
+    """Leaves of one or two bodies (many runs of equal leaf per wave) and of
+    up to a hundred: parity mode against the oracle at its bar, FP32 M2L and
+    L2P within the bar of the FP32 path."""
+    b0 = _bodies(n, 5 * P)
+    ref = b0.copy()
+    orc.fmm(ref, P, ncrit, 0.4, full=True)
+    for prec, bar in ((fmm.PREC_FP64, 1e-11), (fmm.PREC_FP32, 3e-6)):
+        f = fmm.FMM(P=P, ncrit=ncrit, theta=0.4, m2l_precision=prec, p2p_precision=fmm.PREC_FP64,
+                    m2l_truncation=fmm.M2L_FULL)
+        b = b0.copy()
+        f.evaluate(b)
+        for k in ("p", "F"):
+            assert rel_l2(b[k], ref[k]) <= bar, (prec, k)
