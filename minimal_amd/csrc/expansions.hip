@@ -279,9 +279,9 @@ void shift_ops(Ctx &c, hipStream_t s) {
 typedef double v4d __attribute__((ext_vector_type(4)));
 constexpr int kShiftWaves = 4;  // row tiles per workgroup
 constexpr int kShiftBatch = 4;  // k-steps of 4 columns loaded together
-// L2L runs alone on the device (after the GEMM), so it loads deeper: all
-// 25 k-steps of order 10 in two rounds (M2M runs beside P2P, where more
-// registers cost it more than the latency it saves)
+// The batch graph's L2L runs alone on the device (after the GEMM), so it loads
+// deeper: all 25 k-steps of order 10 in two rounds (M2M runs beside P2P, where
+// more registers cost it more than the latency it saves)
 constexpr int kL2LBatch = 13;
 
 __device__ inline int degree_of(int row) {
@@ -380,34 +380,22 @@ __global__ void __launch_bounds__(kM2MWaves *kWave) k_m2m(int P, int lstart, int
   m2m_body(blockIdx.x, blockIdx.y, P, lstart, lcount, cchild, cnch, cx, T, M);
 }
 
-// Row-tile form of M2M and L2L (single tree): one workgroup per 16 parents
-// of a level, wave w = row tile w of the P^2 rows (ceil(P^2/16) waves), each
-// wave looping over the 8 octants.  All 8 x R waves that read a parent
-// tile's operands (the children's multipoles, the parent's locals) run in
-// one workgroup, so those rows come from HBM once and then from that CU's
-// caches (the one-octant-per-workgroup layout fetched them once per XCD
-// and row block).  Operator columns and the B operand are loaded
-// kShiftBatch2 k-steps at a time.
+// Row-tile form of M2M (single tree): one workgroup per 16 parents of a
+// level, wave w = row tile w of the P^2 rows (ceil(P^2/16) waves), each wave
+// looping over the 8 octants.  All waves that read a parent tile's children
+// run in one workgroup, so those rows come from HBM once and then from that
+// CU's caches.  Operator columns and the B operand are loaded kShiftBatch2
+// k-steps at a time.
 constexpr int kShiftBatch2 = 8;
 constexpr int kRowTileMaxWaves = 16;  // P <= 16
-// Levels with fewer parents run the octant-parallel kernels (k_m2m: an
-// octant per wave, k_l2l: an octant per workgroup): their chains of
-// dependent loads are 8x shorter, and few parents leave the cache-sharing
-// of the row-tile form little to share.
+// Levels with fewer parents run the octant-parallel kernel (k_m2m, an octant
+// per wave): its chains of dependent loads are 8x shorter, and few parents
+// leave the cache-sharing of the row-tile form little to share.
 constexpr int kRowTileMinParents = 8192;
 
 // waves of a row-tile workgroup: one per row tile, at least two (filing the
 // children of 16 parents takes 128 threads)
 static int row_tile_waves(int PP) { return std::max(2, ceil_div(PP, 16)); }
-
-__device__ inline void file_children_all(int p0, int lstart, int lcount, const int *__restrict__ cchild,
-                                         const int *__restrict__ cnch, const double4 *__restrict__ cx,
-                                         int (*chl)[16]) {
-  if (threadIdx.x < 128) chl[threadIdx.x / 16][threadIdx.x % 16] = -1;
-  __syncthreads();
-  file_children(threadIdx.x, p0, lstart, lcount, cchild, cnch, cx, -1, chl);
-  __syncthreads();
-}
 
 // M~_parent = sum over octants of T_M2M[octant] M~_child (3d/kernel.h:206),
 // octants added in order into one accumulator per row tile.
@@ -422,7 +410,10 @@ __global__ void __launch_bounds__(kRowTileMaxWaves *kWave) k_m2m_rows(int P, int
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
   const int j16 = lane & 15, kq = lane >> 4;
   const int p0 = blockIdx.x * 16;
-  file_children_all(p0, lstart, lcount, cchild, cnch, cx, chl);
+  if (threadIdx.x < 128) chl[threadIdx.x / 16][threadIdx.x % 16] = -1;
+  __syncthreads();
+  file_children(threadIdx.x, p0, lstart, lcount, cchild, cnch, cx, -1, chl);
+  __syncthreads();
   const int r0 = w * 16;  // blockDim.x = 64 max(2, ceil(PP / 16))
   if (r0 >= PP) return;
   const int jmax = degree_of(min(r0 + 16, PP) - 1);
@@ -459,50 +450,115 @@ __global__ void __launch_bounds__(kRowTileMaxWaves *kWave) k_m2m_rows(int P, int
   }
 }
 
-// L~_child += T_L2L[octant] L~_parent (3d/kernel.h:265-280) for every child
-// of the 16 parents, octant by octant.
-__global__ void __launch_bounds__(kRowTileMaxWaves *kWave) k_l2l_rows(int P, int lstart, int lcount,
-                                                                      const int *__restrict__ cchild,
-                                                                      const int *__restrict__ cnch,
-                                                                      const double4 *__restrict__ cx,
-                                                                      const double *__restrict__ T,
-                                                                      double *__restrict__ L) {
-  __shared__ int chl[8][16];
-  const int PP = P * P;
-  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+// L~_child += T_L2L[octant] L~_parent (3d/kernel.h:265-280) for the cells
+// cell0 .. cell0 + nc - 1 of one level (single tree).  A workgroup keeps one
+// octant's operator in registers -- wave w the row tile w, all its k-steps --
+// and takes the cells of that octant in its range of the level, 16 at a time
+// (grid: (ranges, octants); the octants' workgroups of a range share an XCD and
+// so the parents' rows).  The operator is loaded once per workgroup where the
+// row-tile form above reads it again for every 16 parents, and the waves meet
+// only where a list of cells begins.  Orders above 13 have more row tiles than
+// waves fit beside such registers: two passes over the row tiles.  Bound by the
+// FP64 matrix rate and the cells' rows; the levels of 1.5M clustered bodies,
+// order 12: 650 -> 232 us, of 300,007, order 13: 200 -> 118.
+template <int P>
+struct L2LShape {
+  static constexpr int PP = P * P, RT = (PP + 15) / 16, Passes = RT > 11 ? 2 : 1, W = (RT + Passes - 1) / Passes;
+  static constexpr int KS = (PP + 3) / 4;  // k-steps of a full row tile
+  // k-steps loaded together: 4 to 7, as KS divides best
+  static constexpr int batch() {
+    int best = 7;
+    for (int k = 6; k >= 4; k--)
+      if ((KS + k - 1) / k * k < (KS + best - 1) / best * best) best = k;
+    return best;
+  }
+  static constexpr int B = batch(), NB = (KS + B - 1) / B;
+  static constexpr int PerCU = 2 * W <= 16 ? 2 : 1;  // workgroups a CU has room for
+};
+constexpr int kL2LChunk = 1024;  // cells filtered at a time
+template <int P>
+__global__ void __launch_bounds__(L2LShape<P>::W *kWave) k_l2l_oct(int cell0, int nc,
+                                                                   const unsigned char *__restrict__ coct,
+                                                                   const int *__restrict__ cparent,
+                                                                   const double *__restrict__ T,
+                                                                   double *__restrict__ L) {
+  using Sh = L2LShape<P>;
+  constexpr int PP = Sh::PP, NTH = Sh::W * kWave, B = Sh::B, NB = Sh::NB;
+  __shared__ int cell[kL2LChunk], parent[kL2LChunk];
+  __shared__ int count;
+  const int lane = threadIdx.x % kWave, w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int j16 = lane & 15, kq = lane >> 4;
-  const int p0 = blockIdx.x * 16;
-  file_children_all(p0, lstart, lcount, cchild, cnch, cx, chl);
-  const int r0 = w * 16;
-  if (r0 >= PP) return;
-  const int jmin = degree_of(r0);
-  const int c0 = jmin * jmin;
-  const int ksteps = (PP - c0 + 3) / 4;
-  const int row = min(r0 + j16, PP - 1);
-  const int pl = min(p0 + j16, lcount - 1);
-  const double *Lp = L + int64_t(lstart + pl) * PP;
-  for (int o = 0; o < 8; o++) {
-    const int ch = chl[o][j16];
-    if (!__any(ch >= 0)) continue;
-    const double *To = T + (int64_t(8) + o) * PP * PP;
-    v4d acc = {0, 0, 0, 0};
-    for (int k0 = 0; k0 < ksteps; k0 += kShiftBatch2) {
-      double a[kShiftBatch2], b[kShiftBatch2];
-#pragma unroll
-      for (int s = 0; s < kShiftBatch2; s++) {
-        const int col = c0 + (k0 + s) * 4 + kq;
-        const bool in = col < PP;
-        a[s] = in ? To[int64_t(col) * PP + row] : 0.0;
-        b[s] = (in && ch >= 0) ? Lp[col] : 0.0;
+  const int o = blockIdx.y;
+  const int first = cell0 + int(int64_t(nc) * blockIdx.x / gridDim.x);
+  const int last = cell0 + int(int64_t(nc) * (blockIdx.x + 1) / gridDim.x);
+  const double *To = T + (int64_t(8) + o) * PP * PP;
+  for (int base = first; base < last; base += kL2LChunk) {
+    const int end = min(base + kL2LChunk, last);
+    __syncthreads();  // the last chunk's lists are done with
+    if (threadIdx.x == 0) count = 0;
+    __syncthreads();
+    for (int i0 = base; i0 < end; i0 += NTH) {
+      const int c = i0 + threadIdx.x;
+      const bool mine = c < end && coct[c] == o;
+      const unsigned long long m = __ballot(mine);
+      int at = 0;
+      if (lane == 0 && m) at = atomicAdd(&count, int(__popcll(m)));  // (the order of the list does not matter)
+      at = __shfl(at, 0) + __popcll(m & (lane ? (~0ull >> (64 - lane)) : 0ull));
+      if (mine) {
+        cell[at] = c;
+        parent[at] = cparent[c];
       }
-#pragma unroll
-      for (int s = 0; s < kShiftBatch2; s++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[s], acc, 0, 0, 0);
     }
-    if (ch >= 0) {
+    __syncthreads();
+    const int n = count;
+    if (n == 0) continue;
+    for (int pass = 0; pass < Sh::Passes; pass++) {
+      const int r0 = (pass * Sh::W + w) * 16;
+      if (r0 >= PP) continue;
+      // the row tile's columns c0 .. PP - 1 in nb whole batches that end at the
+      // last column: those before c0 have factors 0
+      const int jmin = degree_of(r0), c0 = jmin * jmin;
+      const int nb = (PP - c0 + 4 * B - 1) / (4 * B), cs = PP - 4 * B * nb + kq;
+      const int row = min(r0 + j16, PP - 1);
+      double a[NB * B];
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int r = r0 + kq + 4 * i;
-        if (r < PP) L[int64_t(ch) * PP + r] += acc[i];
+      for (int s = 0; s < NB * B; s++) {
+        const int col = cs + 4 * s;
+        a[s] = col >= c0 && col < PP ? To[int64_t(col) * PP + row] : 0.0;
+      }
+      for (int g = 0; g < n; g += 16) {
+        const bool in = g + j16 < n;
+        const int at = min(g + j16, n - 1);
+        const double *Lp = L + int64_t(parent[at]) * PP;
+        double *Lc = L + int64_t(cell[at]) * PP;
+        double old[4], b[2][B];
+#pragma unroll
+        for (int s = 0; s < B; s++) b[0][s] = Lp[max(cs + 4 * s, 0)];
+        Lp += cs;
+#pragma unroll
+        for (int i = 0; i < 4; i++) old[i] = Lc[min(r0 + kq + 4 * i, PP - 1)];
+        v4d acc = {0, 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+          if (k < nb) {  // uniform
+            if (k + 1 < nb) {  // the next batch's loads ahead of the products
+#pragma unroll
+              for (int s = 0; s < B; s++) b[(k + 1) & 1][s] = Lp[4 * ((k + 1) * B + s)];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < B; s++)
+              acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k * B + s], b[k & 1][s], acc, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        if (in) {
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int r = r0 + kq + 4 * i;
+            if (r < PP) Lc[r] = old[i] + acc[i];
+          }
+        }
       }
     }
   }
@@ -566,14 +622,6 @@ __device__ __attribute__((always_inline)) inline void l2l_body(int bx, int by, i
     const int r = r0 + kq + 4 * i;
     if (r < PP) L[int64_t(ch) * PP + r] += acc[i];
   }
-}
-
-__global__ void __launch_bounds__(kShiftWaves *kWave) k_l2l(int P, int lstart, int lcount,
-                                                            const int *__restrict__ cchild,
-                                                            const int *__restrict__ cnch,
-                                                            const double4 *__restrict__ cx,
-                                                            const double *__restrict__ T, double *__restrict__ L) {
-  l2l_body(blockIdx.x, blockIdx.y, blockIdx.z, P, lstart, lcount, cchild, cnch, cx, T, L);
 }
 
 // One level of parents of every problem of a batch in one launch (blocks
@@ -805,19 +853,18 @@ void upward(Ctx &c, hipStream_t s) {
 void l2l_pass(Ctx &c) {
   Tree &t = c.t;
   hipStream_t s = c.s0;
-  const int PP = c.P * c.P;
   shift_ops(c, s);
-  for (int l = t.lroot; l < t.depth; l++) {  // parents at level l
-    const int cnt = t.lstart[l + 1] - t.lstart[l];
-    if (cnt >= kRowTileMinParents)
-      hipLaunchKernelGGL(k_l2l_rows, dim3(ceil_div(cnt, 16)), dim3(row_tile_waves(PP) * kWave), 0, s, c.P,
-                         t.lstart[l], cnt, t.cchild.p, t.cnch.p, t.cx.p, c.shift_T.p, c.L.p);
-    else
-      hipLaunchKernelGGL(k_l2l, dim3(ceil_div(cnt, 16), ceil_div(PP, 16 * kShiftWaves), 8),
-                         dim3(kShiftWaves * kWave), 0, s, c.P, t.lstart[l], cnt, t.cchild.p, t.cnch.p, t.cx.p,
-                         c.shift_T.p, c.L.p);
-    XF_LAUNCH();
-  }
+  by_order(c.P, [&](auto p) {
+    using Sh = L2LShape<p()>;
+    for (int l = t.lroot + 1; l <= t.depth; l++) {
+      const int nc = t.lstart[l + 1] - t.lstart[l];
+      // ranges with about 16 cells per octant, until the device is full
+      const int ranges = std::min(std::max(1, nc / 128), 32 * Sh::PerCU);
+      hipLaunchKernelGGL((k_l2l_oct<p()>), dim3(ranges, 8), dim3(Sh::W * kWave), 0, s, t.lstart[l], nc, t.coct.p,
+                         t.cparent.p, c.shift_T.p, c.L.p);
+      XF_LAUNCH();
+    }
+  });
 }
 
 void l2p_pass(Ctx &c) {

@@ -195,6 +195,7 @@ struct Tree {
   Buf<double4> cx;     // centre xyz, radius R
   Buf<int> cbeg, ccnt; // body range in tree order
   Buf<int> cchild, cnch, cparent, clevel;
+  Buf<unsigned char> coct;  // octant within the parent
   Buf<int> leaves;     // leaf cells, BFS order
   Buf<int> perm;       // tree-order position -> caller's body index
   Buf<double4> xs;     // tree-order X, q (FP64)

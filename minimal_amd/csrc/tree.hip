@@ -435,7 +435,8 @@ __device__ inline int split_bounds(int l, int ncrit, int beg, int cnt, const uns
 __device__ inline void emit_children(int l, int c, int first, const int b[9], const double4 *__restrict__ froots,
                                      const unsigned long long *__restrict__ key, double4 *__restrict__ cx,
                                      int *__restrict__ cbeg, int *__restrict__ ccnt, int *__restrict__ cchild,
-                                     int *__restrict__ cparent, int *__restrict__ clevel) {
+                                     int *__restrict__ cparent, int *__restrict__ clevel,
+                                     unsigned char *__restrict__ coct) {
   cchild[c] = first;
   const double4 P = cx[c];
   const double r = P.w * 0.5;
@@ -455,6 +456,7 @@ __device__ inline void emit_children(int l, int c, int first, const int b[9], co
     ccnt[ch] = b1 - b0;
     cparent[ch] = c;
     clevel[ch] = l + 1;
+    coct[ch] = (unsigned char)o;
   }
 }
 
@@ -541,7 +543,7 @@ __global__ void __launch_bounds__(1024) k_split_level(int l, int ncrit, int lfor
                                                       double4 *__restrict__ cx, int *cbeg, int *ccnt,
                                                       int *__restrict__ cchild, int *__restrict__ cnch,
                                                       int *__restrict__ cparent, int *__restrict__ clevel,
-                                                      int *__restrict__ nsplit, int *__restrict__ ticket, unsigned tag,
+                                                      unsigned char *__restrict__ coct, int *__restrict__ nsplit, int *__restrict__ ticket, unsigned tag,
                                                       unsigned long long *__restrict__ words) {
   const int id = lookback_ticket(ticket);
   const int count = lcount[l], start = lstart[l], next = start + count;
@@ -560,7 +562,7 @@ __global__ void __launch_bounds__(1024) k_split_level(int l, int ncrit, int lfor
     if (k == 0)
       cchild[c] = -1;
     else
-      emit_children(l, c, next + before + off, b, froots, key, cx, cbeg, ccnt, cchild, cparent, clevel);
+      emit_children(l, c, next + before + off, b, froots, key, cx, cbeg, ccnt, cchild, cparent, clevel, coct);
   }
   if (id == int(gridDim.x) - 1 && threadIdx.x == 0) {
     lcount[l + 1] = before + total;
@@ -610,7 +612,8 @@ __global__ void __launch_bounds__(kTopThreads)
                  const unsigned long long *__restrict__ key, int *hist, const int *__restrict__ bmax,
                  int *__restrict__ lmax, const double4 *__restrict__ froots, double4 *__restrict__ cx, int *__restrict__ cbeg,
                  int *__restrict__ ccnt, int *__restrict__ cchild, int *__restrict__ cnch,
-                 int *__restrict__ cparent, int *__restrict__ clevel, int *__restrict__ nsplit) {
+                 int *__restrict__ cparent, int *__restrict__ clevel, unsigned char *__restrict__ coct,
+                 int *__restrict__ nsplit) {
   __shared__ int wsum[kTopThreads / kWave];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
   if (bmax) hist_top(hist, bmax, lmax);
@@ -654,7 +657,7 @@ __global__ void __launch_bounds__(kTopThreads)
         if (k[j] == 0)
           cchild[c] = -1;
         else
-          emit_children(l, c, next + off, b[j], froots, key, cx, cbeg, ccnt, cchild, cparent, clevel);
+          emit_children(l, c, next + off, b[j], froots, key, cx, cbeg, ccnt, cchild, cparent, clevel, coct);
         off += k[j];
       }
     }
@@ -797,6 +800,7 @@ void tree_build(Ctx &c) {
       t.cnch.ensure(tot);
       t.cparent.ensure(tot);
       t.clevel.ensure(tot);
+      t.coct.ensure(tot);
       t.leaves.ensure(tot);
     }
     return tot;
@@ -894,12 +898,12 @@ void tree_build(Ctx &c) {
   // (with a depth of 0 no level is split, but the histogram is still finished)
   hipLaunchKernelGGL(k_top_levels, dim3(1), dim3(kTopThreads), 0, s, lfuse, ncrit, lforce, t.lcount.p, t.lstart_d.p, k1,
                      t.hist.p, speculate ? t.hist_bmax.p : nullptr, t.misc.p, froots, t.cx.p, t.cbeg.p, t.ccnt.p,
-                     t.cchild.p, t.cnch.p, t.cparent.p, t.clevel.p, t.misc.p + 18);
+                     t.cchild.p, t.cnch.p, t.cparent.p, t.clevel.p, t.coct.p, t.misc.p + 18);
   XF_LAUNCH();
   for (int l = lfuse; l < Ds; l++) {
     hipLaunchKernelGGL(k_split_level, dim3(ceil_div(level_bound(l), 1024)), dim3(1024), 0, s, l, ncrit, lforce,
                        t.lcount.p, t.lstart_d.p, k1, t.hist.p, froots, t.cx.p, t.cbeg.p, t.ccnt.p, t.cchild.p, t.cnch.p,
-                       t.cparent.p, t.clevel.p, t.misc.p + 18, t.misc.p + 24 + l, ++t.lookback_tag, t.lookback.p);
+                       t.cparent.p, t.clevel.p, t.coct.p, t.misc.p + 18, t.misc.p + 24 + l, ++t.lookback_tag, t.lookback.p);
     XF_LAUNCH();
   }
 

@@ -58,3 +58,20 @@ def test_field(gpu, orc, P, n, ncrit):
         f.evaluate(b)
         for k in ("p", "F"):
             assert rel_l2(b[k], ref[k]) <= bar, (prec, k)
+
+
+@pytest.mark.parametrize("P", [12, 14])
+def test_wide_levels(gpu, P):
+    """Levels of more cells than a workgroup of the L2L pass lists at a time
+    (1,024 in each of 32 ranges; order 14 takes two passes over its row
+    tiles), against the direct sum at the truncation error of the order."""
+    b0 = uniform_cube(60000, P, "sym")
+    f = fmm.FMM(P=P, ncrit=1, theta=0.35)
+    f.evaluate(b0)
+    assert f.num_cells()[0] > 2 * 32768
+    t = b0[:: len(b0) // 2000].copy()
+    fp, fF = t["p"].copy(), t["F"].copy()
+    t["p"], t["F"] = 0, 0
+    f.direct(t, b0)
+    assert rel_l2(fp, t["p"]) <= 1e-5
+    assert rel_l2(fF, t["F"]) <= 1e-5
