@@ -192,85 +192,69 @@ __global__ void __launch_bounds__(kFBThreads) k_forest_bounds(const exafmm_body 
 }
 
 // ---------------------------------------------------------------- keys
-// Octant path of each body through the reference's centre sequence, and
-// the population of its level-7 prefix (dense, 8^7 bins).  With AGG the
-// workgroup first counts its 256 bodies' prefixes in an LDS table and adds
-// one atomic per distinct prefix: clustered inputs (a Plummer core puts
-// most bodies in a few hundred prefixes) would otherwise serialise on the
-// same global counters; spread-out inputs take the direct atomics.
+// Octant path of each body through the reference's centre sequence and, with
+// HIST, the population of its level-7 prefix (dense, 8^7 bins) by atomics.
+// Without it the histogram is taken from the sorted keys (k_hist_sorted):
+// deep trees are sorted by radix anyway, and their crowded prefixes (a Plummer
+// core) make the XCDs' atomics pass the same counters around (1.5M clustered
+// bodies: 243 us, even with each workgroup's bodies counted in LDS first; 32 us
+// without, and 12 for k_hist_sorted).
 constexpr int kKeysThreads = 256;
-constexpr int kKeysSlots = 2 * kKeysThreads;  // load factor <= 1/2: every probe ends
-template <bool AGG>
+template <bool HIST>
 __global__ void __launch_bounds__(kKeysThreads) k_keys(const exafmm_body *__restrict__ b, int64_t n,
                                                        const double *__restrict__ root,
                                                        unsigned long long *__restrict__ key, int *__restrict__ val,
                                                        int *__restrict__ hist7, const double4 *__restrict__ froots,
                                                        const int64_t *__restrict__ off, int nprob) {
-  __shared__ unsigned tbin[AGG ? kKeysSlots : 1];  // prefix + 1 (0: empty)
-  __shared__ int tcnt[AGG ? kKeysSlots : 1];
-  if (AGG) {
-    for (int i = threadIdx.x; i < kKeysSlots; i += kKeysThreads) {
-      tbin[i] = 0u;
-      tcnt[i] = 0;
-    }
-    __syncthreads();
-  }
   const int64_t i = int64_t(blockIdx.x) * kKeysThreads + threadIdx.x;
-  if (i < n) {
-    const double x = b[i].X[0], y = b[i].X[1], z = b[i].X[2];
-    double R0 = root[3], cx = root[0], cy = root[1], cz = root[2];
-    unsigned long long k = 0;
-    int l0 = 0;
-    if (froots) {
-      // forest: the problem's index fills the digits of levels 0 .. kForestLevel - 1,
-      // its own root's octant path the rest
-      int lo = 0, hi = nprob - 1;  // last problem with off[p] <= i
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (off[mid] <= i)
-          lo = mid;
-        else
-          hi = mid - 1;
-      }
-      const double4 Rt = froots[lo];
-      cx = Rt.x;
-      cy = Rt.y;
-      cz = Rt.z;
-      R0 = Rt.w;
-      k = (unsigned long long)lo;
-      l0 = kForestLevel;
+  if (i >= n) return;
+  const double x = b[i].X[0], y = b[i].X[1], z = b[i].X[2];
+  double R0 = root[3], cx = root[0], cy = root[1], cz = root[2];
+  unsigned long long k = 0;
+  int l0 = 0;
+  if (froots) {
+    // forest: the problem's index fills the digits of levels 0 .. kForestLevel - 1,
+    // its own root's octant path the rest
+    int lo = 0, hi = nprob - 1;  // last problem with off[p] <= i
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (off[mid] <= i)
+        lo = mid;
+      else
+        hi = mid - 1;
     }
-    for (int l = l0; l < kMaxLevel; l++) {
-      const int bx = x > cx, by = y > cy, bz = z > cz;
-      const int oct = bx + (by << 1) + (bz << 2);
-      k = (k << 3) | unsigned(oct);
-      const double rr = R0 / (1 << (l - l0 + 1));
-      cx += bx ? rr : -rr;
-      cy += by ? rr : -rr;
-      cz += bz ? rr : -rr;
-    }
-    key[i] = k;
-    val[i] = int(i);
-    const unsigned bin = unsigned(k >> (3 * (kMaxLevel - kHistLevels)));
-    if (!AGG) {
-      atomicAdd(&hist7[bin], 1);
-    } else {
-      unsigned h = ((bin + 1u) * 2654435761u) & unsigned(kKeysSlots - 1);
-      for (;;) {
-        const unsigned prev = atomicCAS(&tbin[h], 0u, bin + 1u);
-        if (prev == 0u || prev == bin + 1u) {
-          atomicAdd(&tcnt[h], 1);
-          break;
-        }
-        h = (h + 1u) & unsigned(kKeysSlots - 1);
-      }
-    }
+    const double4 Rt = froots[lo];
+    cx = Rt.x;
+    cy = Rt.y;
+    cz = Rt.z;
+    R0 = Rt.w;
+    k = (unsigned long long)lo;
+    l0 = kForestLevel;
   }
-  if (AGG) {
-    __syncthreads();
-    for (int j = threadIdx.x; j < kKeysSlots; j += kKeysThreads)
-      if (tcnt[j]) atomicAdd(&hist7[tbin[j] - 1u], tcnt[j]);
+  for (int l = l0; l < kMaxLevel; l++) {
+    const int bx = x > cx, by = y > cy, bz = z > cz;
+    const int oct = bx + (by << 1) + (bz << 2);
+    k = (k << 3) | unsigned(oct);
+    const double rr = R0 / (1 << (l - l0 + 1));
+    cx += bx ? rr : -rr;
+    cy += by ? rr : -rr;
+    cz += bz ? rr : -rr;
   }
+  key[i] = k;
+  val[i] = int(i);
+  if (HIST) atomicAdd(&hist7[unsigned(k >> (3 * (kMaxLevel - kHistLevels)))], 1);
+}
+
+// Level-7 populations from the sorted keys: the ends of a prefix's run add up
+// to its length (two atomics per prefix that occurs).
+__global__ void __launch_bounds__(256) k_hist_sorted(const unsigned long long *__restrict__ key, int64_t n,
+                                                     int *__restrict__ hist7) {
+  constexpr int sh = 3 * (kMaxLevel - kHistLevels);
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= n) return;
+  const unsigned bin = unsigned(key[i] >> sh);
+  if (i == 0 || unsigned(key[i - 1] >> sh) != bin) atomicAdd(&hist7[bin], -int(i));
+  if (i == n - 1 || unsigned(key[i + 1] >> sh) != bin) atomicAdd(&hist7[bin], int(i) + 1);
 }
 
 // Levels 6..3 of the prefix histogram from level 7 (prefixes are in Morton
@@ -829,15 +813,19 @@ void tree_build(Ctx &c) {
   t.key2.ensure(n);
   t.val.ensure(n);
   t.val2.ensure(n);
-  // crowded level-7 prefixes in the last tree: count them per workgroup first
-  hipLaunchKernelGGL(t.hist7_max > 64 ? k_keys<true> : k_keys<false>, dim3(ceil_div(n, kKeysThreads)),
-                     dim3(kKeysThreads), 0, s, c.bodies, n, root, t.key.p, t.val.p,
-                     t.hist.p + hist_off(kHistLevels), froots, forest ? c.forest_off.p : nullptr, c.forest_n);
+  // a tree expected to be deeper than the histogram takes it from the sorted keys
+  const bool sorted_hist = speculate && Ds > kHistLevels;
+  hipLaunchKernelGGL(sorted_hist ? k_keys<false> : k_keys<true>, dim3(ceil_div(n, kKeysThreads)), dim3(kKeysThreads), 0,
+                     s, c.bodies, n, root, t.key.p, t.val.p, t.hist.p + hist_off(kHistLevels), froots,
+                     forest ? c.forest_off.p : nullptr, c.forest_n);
   XF_LAUNCH();
   // one block per level-3 prefix (4096 level-7 bins each)
   t.hist_bmax.ensure(8 << (3 * 3));
-  hipLaunchKernelGGL(k_hist_pyramid, dim3(1 << (3 * 3)), dim3(1024), 0, s, t.hist.p, t.hist_bmax.p);
-  XF_LAUNCH();
+  auto pyramid = [&] {
+    hipLaunchKernelGGL(k_hist_pyramid, dim3(1 << (3 * 3)), dim3(1024), 0, s, t.hist.p, t.hist_bmax.p);
+    XF_LAUNCH();
+  };
+  if (!sorted_hist) pyramid();
 
   // Sort depth Ds: the first level whose most populous prefix holds at
   // most ncrit bodies (kMaxLevel if none of levels 1..7 does).  It needs the
@@ -873,6 +861,12 @@ void tree_build(Ctx &c) {
     k1 = k2;
   } else {
     radix_sort_pairs(k1, v1, k2, v2, int(n), 3 * (kMaxLevel - Ds), 3 * kMaxLevel, t.rs_hist, s);
+    if (sorted_hist) {
+      hipLaunchKernelGGL(k_hist_sorted, dim3(ceil_div(n, 256)), dim3(256), 0, s, k1, n,
+                         t.hist.p + hist_off(kHistLevels));
+      XF_LAUNCH();
+      pyramid();
+    }
   }
 
   // level-by-level split
@@ -953,7 +947,6 @@ void tree_build(Ctx &c) {
   }
   t.depth = depth;
   t.ds_hint = need <= kHistLevels ? need : std::min(kMaxLevel, depth + 1);
-  t.hist7_max = fl[kHistLevels];
   t.ncells = t.lstart.back();
   const int nc = int(t.ncells);
   // every cell either split or is a leaf (the scan above wrote the same
