@@ -88,24 +88,28 @@ __device__ inline unsigned mix32(unsigned h) {
   return h;
 }
 
+constexpr int kMinHashes = 3;
+constexpr int kGroupShift = 48, kSortBits = 56;
+
 // Counters of the tile build (m2l_misc): group populations 0..255, then the
 // plan [slots, tiles, cells in tiles, key set differs].
 constexpr int kMiscPlan = 256, kMiscInts = 260;
 
-// Sort key of a target cell: group in bits 16..23 (255 = no M2L) -- the
-// octant, or (level, octant) with `by_level` -- and the top 16 bits of the
-// minimum hashed key id of its list below: cells with similar key sets share
-// that minimum with a probability equal to the sets' Jaccard similarity, so
-// sorting by it packs cells of like key sets into the same tile (fewer empty
-// GEMM slots).
+// Sort key of a target cell: group in bits 48..55 (255 = no M2L) -- the
+// octant, or (level, octant) with `by_level` -- and below it 16 bits each of the
+// minima of kMinHashes hashes of its key ids: cells with similar key sets share
+// such a minimum with a probability equal to the sets' Jaccard similarity, so
+// sorting by them packs cells of like key sets into the same subtile (fewer
+// empty GEMM columns; with one hash and ties in index order the GEMM of 1.5M
+// clustered bodies took 4.80 ms, with three 4.46, beside P2P).
 // One wave per cell: the lanes take the list entries in turn and the
 // minimum hash is a wave reduction.
 __global__ void __launch_bounds__(256) k_group_keys(int ncells, const double4 *__restrict__ cx,
                                                     const int *__restrict__ cparent, const int *__restrict__ clevel,
                                                     const int *__restrict__ m2l_beg, const int *__restrict__ m2l_cnt,
                                                     const int2 *__restrict__ list, int lmin, int by_level,
-                                                    unsigned long long *__restrict__ key, unsigned *__restrict__ key32,
-                                                    int *__restrict__ val, int *__restrict__ misc) {
+                                                    unsigned long long *__restrict__ key, int *__restrict__ val,
+                                                    int *__restrict__ misc) {
   const int lane = threadIdx.x & (kWave - 1);
   const int c = blockIdx.x * (256 / kWave) + int(threadIdx.x / kWave);
   if (blockIdx.x == 0) {  // counters of the launches that follow
@@ -113,7 +117,8 @@ __global__ void __launch_bounds__(256) k_group_keys(int ncells, const double4 *_
     if (threadIdx.x < kMiscInts - 256) misc[256 + threadIdx.x] = 0;
   }
   if (c >= ncells) return;  // whole wave
-  unsigned g = 255, mh = 0;
+  unsigned g = 255;
+  unsigned long long mh = 0;
   // cells above level lmin take their M2L elsewhere (FP64, per pair)
   const int n = clevel[c] < lmin ? 0 : m2l_cnt[c];
   if (n > 0) {
@@ -124,20 +129,25 @@ __global__ void __launch_bounds__(256) k_group_keys(int ncells, const double4 *_
       o = (a.x > b.x) + ((a.y > b.y) << 1) + ((a.z > b.z) << 2);
     }
     g = (by_level ? unsigned(min(clevel[c], 30)) * 8 : 0u) + o;
-    unsigned m = 0xffffffffu;
-    const int b0 = m2l_beg[c];
-    for (int i = lane; i < n; i += kWave) m = min(m, mix32(unsigned(list[b0 + i].y)));
+    unsigned m[kMinHashes];
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) m = min(m, unsigned(__shfl_xor(int(m), d)));
-    mh = m >> 16;  // 16 bits: three 8-bit sort passes over the 24-bit key
+    for (int h = 0; h < kMinHashes; h++) m[h] = 0xffffffffu;
+    const int b0 = m2l_beg[c];
+    for (int i = lane; i < n; i += kWave) {
+      const unsigned id = unsigned(list[b0 + i].y);
+#pragma unroll
+      for (int h = 0; h < kMinHashes; h++) m[h] = min(m[h], mix32(id + h * 0x9e3779b9u));
+    }
+#pragma unroll
+    for (int h = 0; h < kMinHashes; h++) {
+#pragma unroll
+      for (int d = 32; d > 0; d >>= 1) m[h] = min(m[h], unsigned(__shfl_xor(int(m[h]), d)));
+      mh |= (unsigned long long)(m[h] >> 16) << (kGroupShift - 16 * (h + 1));
+    }
   }
   if (lane == 0) {
-    if (key32) {
-      key32[c] = g << 16 | mh;
-    } else {
-      key[c] = (unsigned long long)(g << 16 | mh);
-      val[c] = c;
-    }
+    key[c] = (unsigned long long)g << kGroupShift | mh;
+    val[c] = c;
   }
 }
 
@@ -188,7 +198,7 @@ __global__ void __launch_bounds__(256) k_group_hist(int ncells, const unsigned l
   h[threadIdx.x] = 0;
   __syncthreads();
   for (int c = blockIdx.x * 256 + threadIdx.x; c < ncells; c += gridDim.x * 256) {
-    atomicAdd(&h[int(key[c] >> 16)], 1);
+    atomicAdd(&h[int(key[c] >> kGroupShift)], 1);
     sorted[c] = val[c];
   }
   __syncthreads();
@@ -201,12 +211,12 @@ __global__ void __launch_bounds__(256) k_group_hist(int ncells, const unsigned l
 // scalar loads).  Quadratic, and one launch where the radix sort takes nine:
 // at 16,384 cells it costs what they do.
 constexpr int kCellRankMax = 16384;
-__global__ void __launch_bounds__(1024) k_cell_rank(int n, const unsigned *__restrict__ key, int *__restrict__ sorted,
+__global__ void __launch_bounds__(1024) k_cell_rank(int n, const unsigned long long *__restrict__ key, int *__restrict__ sorted,
                                                     int *__restrict__ misc) {
   __shared__ int part[16][kWave];
   const int lane = threadIdx.x & (kWave - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int i = blockIdx.x * kWave + lane;
-  const unsigned k = i < n ? key[i] : 0u;
+  const unsigned long long k = i < n ? key[i] : 0ull;
   const int j0 = w * n / 16, j1 = (w + 1) * n / 16, first = blockIdx.x * kWave;
   int r = 0;
   // before this workgroup's cells equal keys count, after them they do not
@@ -219,7 +229,7 @@ __global__ void __launch_bounds__(1024) k_cell_rank(int n, const unsigned *__res
     r = 0;
     for (int q = 0; q < 16; q++) r += part[q][lane];
     sorted[r] = i;
-    atomicAdd(&misc[k >> 16], 1);
+    atomicAdd(&misc[int(k >> kGroupShift)], 1);
   }
 }
 
@@ -1490,9 +1500,9 @@ void m2l_prepare(Ctx &c, hipStream_t s) {
   c.t.key2.ensure(nc);
   c.t.val.ensure(nc);
   c.t.val2.ensure(nc);
-  // cells sorted by (group, min-hash of key set), BFS order within ties: on adaptive trees this raises the fraction of non-empty GEMM slots
-  // (measured 0.50 -> 0.58 on a 2^22-body Plummer set); on uniform trees,
-  // where BFS neighbours already share key sets, it changes little.
+  // cells sorted by (group, min-hashes of the key set), BFS order within ties:
+  // on adaptive trees this raises the fraction of non-empty GEMM slots; on
+  // uniform trees, where BFS neighbours already share key sets, it changes little.
   // Tiles mix the levels (keys are scale-free: on a clustered set of 200,000
   // bodies half as many (tile, key) slots as with tiles of one level), unless
   // the keys carry the level (periodic) or the slots take one learned order
@@ -1509,17 +1519,16 @@ void m2l_prepare(Ctx &c, hipStream_t s) {
       *d_U = c.tiles.p + 3 * ntmax, *d_sorted = c.tiles.p + 4 * ntmax;
   c.m2l_misc.ensure(kMiscInts);
   const bool ranked = nc <= kCellRankMax;
-  unsigned *key32 = ranked ? reinterpret_cast<unsigned *>(c.t.key.p) : nullptr;
   hipLaunchKernelGGL(k_group_keys, dim3(ceil_div(nc, 256 / kWave)), dim3(256), 0, s, nc, c.t.cx.p, c.t.cparent.p,
                      c.t.clevel.p, c.lists.m2l_beg.p, c.lists.m2l_cnt.p, c.lists.m2l.p, m2l_fp64_levels(c),
-                     int(by_level), c.t.key.p, key32, c.t.val.p, c.m2l_misc.p);
+                     int(by_level), c.t.key.p, c.t.val.p, c.m2l_misc.p);
   XF_LAUNCH();
   if (ranked) {
-    hipLaunchKernelGGL(k_cell_rank, dim3(ceil_div(nc, kWave)), dim3(1024), 0, s, nc, key32, d_sorted, c.m2l_misc.p);
+    hipLaunchKernelGGL(k_cell_rank, dim3(ceil_div(nc, kWave)), dim3(1024), 0, s, nc, c.t.key.p, d_sorted, c.m2l_misc.p);
   } else {
     unsigned long long *k1 = c.t.key.p, *k2 = c.t.key2.p;
     int *v1 = c.t.val.p, *v2 = c.t.val2.p;
-    radix_sort_pairs(k1, v1, k2, v2, nc, 0, 24, c.m2l_rs_hist, s);
+    radix_sort_pairs(k1, v1, k2, v2, nc, kGroupShift - 16 * kMinHashes, kSortBits, c.m2l_rs_hist, s);
     hipLaunchKernelGGL(k_group_hist, dim3(std::min(ceil_div(nc, 256), 64)), dim3(256), 0, s, nc, k1, v1, d_sorted,
                        c.m2l_misc.p);
   }
