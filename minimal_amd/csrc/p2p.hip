@@ -379,8 +379,14 @@ __global__ void __launch_bounds__(kP2PWaves *kWave) k_p2p32_grouped(const GroupT
 // (about 2^-23 relative) takes one third-order step
 //   e = 1 - r^2 y^2,  y += y e (1/2 + 3/8 e)
 // (remainder 5/16 e^3, below 2^-60), five FP64 operations where a divide and
-// a square root expand to about forty.  Squared distances outside
-// [2^-900, 2^900) -- zero, overflow, NaN -- take the plain divide and root.
+// a square root expand to about forty.  STEP2: 1/r^2 is y^2 after a Newton
+// step of its own, two operations more; y^2 alone carries twice y's rounding,
+// which shows where few sources are added (1,000 x 1,000 bodies, F against the
+// exact sum: 2.5e-16, with the step 2.1e-16, with a divide and a root 2.2e-16;
+// over more sources the longer chains of additions that lanes over sources
+// replace weigh more).  Squared distances outside [2^-900, 2^900) -- zero,
+// overflow, NaN -- take the plain divide and root.
+template <bool STEP2>
 __device__ inline void p2p64_pair(double dx, double dy, double dz, double q, double &pot, double &ax, double &ay,
                                   double &az) {
   const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
@@ -388,10 +394,15 @@ __device__ inline void p2p64_pair(double dx, double dy, double dz, double q, dou
   const double t = r2 * y;
   const double e = fma(-t, y, 1.0);
   y = fma(y * e, fma(e, 0.375, 0.5), y);
+  double y2 = y * y;
+  if (STEP2) y2 = fma(y2, fma(-r2, y2, 1.0), y2);
   const unsigned hi = unsigned(__double2hiint(r2));
-  if (hi - (123u << 20) >= (1800u << 20)) y = r2 != 0.0 ? sqrt(1.0 / r2) : 0.0;
+  if (hi - (123u << 20) >= (1800u << 20)) {
+    y2 = r2 != 0.0 ? 1.0 / r2 : 0.0;
+    y = sqrt(y2);
+  }
   const double qi = q * y;
-  const double f = qi * (y * y);
+  const double f = qi * y2;
   pot += qi;
   ax = fma(dx, f, ax);
   ay = fma(dy, f, ay);
@@ -436,7 +447,8 @@ __device__ __attribute__((always_inline)) inline void p2p64_block(int t0, int tc
       const double4 X = sxs[L.beg[e] + g - L.pre[e]];
       const double sx = X.x + L.dlx[e], sy = X.y + L.dly[e], sz = X.z + L.dlz[e];  // the entry's image shift
 #pragma unroll
-      for (int t = 0; t < TC; t++) p2p64_pair(xt[t] - sx, yt[t] - sy, zt[t] - sz, X.w, ap[t], ax[t], ay[t], az[t]);
+      for (int t = 0; t < TC; t++)
+        p2p64_pair<false>(xt[t] - sx, yt[t] - sy, zt[t] - sz, X.w, ap[t], ax[t], ay[t], az[t]);
     }
   }
   constexpr int kLow = kWave / pow2ceil<TC>();
@@ -531,6 +543,30 @@ constexpr int kDirectTC = 8;
 constexpr int kDirectWaves = 4;
 constexpr int kDirectGroups = 2048;  // workgroups aimed at: eight per CU
 
+// Sums of targets t0 .. t0 + tc - 1 over the sources first + lane, + stride, ...
+// below s1: component lane % (64 / TC) of target lane / (64 / TC).
+template <int TC, bool STEP2>
+__device__ __attribute__((always_inline)) inline double direct_block(const exafmm_body *__restrict__ t, int tc,
+                                                                     const exafmm_body *__restrict__ s, int64_t s0,
+                                                                     int64_t s1, int64_t stride, int lane) {
+  double xt[TC], yt[TC], zt[TC], ap[TC], ax[TC], ay[TC], az[TC];
+#pragma unroll
+  for (int i = 0; i < TC; i++) {
+    const exafmm_body *b = t + min(i, tc - 1);
+    xt[i] = b->X[0];
+    yt[i] = b->X[1];
+    zt[i] = b->X[2];
+    ap[i] = ax[i] = ay[i] = az[i] = 0.0;
+  }
+  for (int64_t j = s0 + lane; j < s1; j += stride) {
+    const double sx = s[j].X[0], sy = s[j].X[1], sz = s[j].X[2], q = s[j].q;
+#pragma unroll
+    for (int i = 0; i < TC; i++)
+      p2p64_pair<STEP2>(xt[i] - sx, yt[i] - sy, zt[i] - sz, q, ap[i], ax[i], ay[i], az[i]);
+  }
+  return p2p_lane_total<TC>(ap, ax, ay, az, lane);
+}
+
 __global__ void __launch_bounds__(kDirectWaves *kWave) k_direct(const exafmm_body *__restrict__ t, int64_t nt,
                                                                 const exafmm_body *__restrict__ s, int64_t ns,
                                                                 int wt, double *__restrict__ part) {
@@ -542,24 +578,39 @@ __global__ void __launch_bounds__(kDirectWaves *kWave) k_direct(const exafmm_bod
   const int64_t share = int64_t(blockIdx.y) * ws + w / wt, shares = int64_t(gridDim.y) * ws;
   const int64_t s0 = share * ns / shares, s1 = (share + 1) * ns / shares;
   const int tc = int(min(int64_t(kDirectTC), nt - t0));
-  double xt[kDirectTC], yt[kDirectTC], zt[kDirectTC], ap[kDirectTC], ax[kDirectTC], ay[kDirectTC], az[kDirectTC];
-#pragma unroll
-  for (int i = 0; i < kDirectTC; i++) {
-    const exafmm_body *b = t + t0 + min(i, tc - 1);
-    xt[i] = b->X[0];
-    yt[i] = b->X[1];
-    zt[i] = b->X[2];
-    ap[i] = ax[i] = ay[i] = az[i] = 0.0;
-  }
-  for (int64_t j = s0 + lane; j < s1; j += kWave) {
-    const double sx = s[j].X[0], sy = s[j].X[1], sz = s[j].X[2], q = s[j].q;
-#pragma unroll
-    for (int i = 0; i < kDirectTC; i++) p2p64_pair(xt[i] - sx, yt[i] - sy, zt[i] - sz, q, ap[i], ax[i], ay[i], az[i]);
-  }
   constexpr int kLow = kWave / kDirectTC;
   const int i = lane / kLow, comp = lane % kLow;
-  const double v = p2p_lane_total<kDirectTC>(ap, ax, ay, az, lane);
+  const double v = direct_block<kDirectTC, false>(t + t0, tc, s, s0, s1, kWave, lane);
   if (comp < 4 && i < tc) part[(share * nt + t0 + i) * 4 + comp] = v;
+}
+
+// Few sources: a workgroup of 16 waves takes four targets over all of them
+// and adds its waves' sums itself, in one launch.  Up to kDirectOneMax
+// sources a wave has few enough rounds that the launch saved is worth more
+// than the even split: 1,000 x 8,000 in 23 us, 32 in two launches (and 2,000 x
+// 8,000 in 32 against 37); the gap closes beyond.
+constexpr int kDirectOneTC = 4, kDirectOneWaves = 16;
+constexpr int64_t kDirectOneMax = 8192;
+__global__ void __launch_bounds__(kDirectOneWaves *kWave) k_direct_one(exafmm_body *__restrict__ t, int64_t nt,
+                                                                       const exafmm_body *__restrict__ s, int64_t ns) {
+  constexpr int kLow = kWave / kDirectOneTC;
+  __shared__ double red[kDirectOneWaves][kDirectOneTC * 4];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int64_t t0 = int64_t(blockIdx.x) * kDirectOneTC;
+  const int tc = int(min(int64_t(kDirectOneTC), nt - t0));
+  const double v = direct_block<kDirectOneTC, true>(t + t0, tc, s, w * kWave, ns, kDirectOneWaves * kWave, lane);
+  if (lane % kLow < 4) red[w][lane / kLow * 4 + lane % kLow] = v;
+  __syncthreads();
+  const int i = threadIdx.x / 4, comp = threadIdx.x % 4;
+  if (i >= tc) return;
+  double sum = 0.0;
+#pragma unroll
+  for (int k = 0; k < kDirectOneWaves; k++) sum += red[k][threadIdx.x];
+  if (comp == 0)
+    t[t0 + i].p += sum;
+  else
+    t[t0 + i].F[comp - 1] -= sum;
 }
 
 // One wave per target: lane (h, comp) = (lane / 4, lane % 4) adds the shares
@@ -583,6 +634,12 @@ __global__ void __launch_bounds__(256) k_direct_sum(exafmm_body *__restrict__ t,
 
 void direct_sum(Ctx &c, exafmm_body *t, int64_t nt, const exafmm_body *s, int64_t ns) {
   if (nt <= 0 || ns <= 0) return;
+  if (ns <= kDirectOneMax) {
+    hipLaunchKernelGGL(k_direct_one, dim3(ceil_div(nt, kDirectOneTC)), dim3(kDirectOneWaves * kWave), 0, c.s0, t, nt, s,
+                       ns);
+    XF_LAUNCH();
+    return;
+  }
   const int64_t blocks = (nt + kDirectTC - 1) / kDirectTC;
   const int wt = blocks >= 4 ? 4 : blocks >= 2 ? 2 : 1;
   const int64_t groups = (blocks + wt - 1) / wt;

@@ -8,7 +8,7 @@ the same terms in another order: |diff| <= 1e-11 max |oracle|, the bar of the
 parity tests.
 
 Direct sum (k_direct): one target, target blocks that are not full, one to
-four blocks per workgroup, fewer sources than a wave, sources that coincide
+four blocks per workgroup, one launch and two, fewer sources than a wave, sources that coincide
 with targets, and squared distances beyond the range of the fast 1/sqrt
 (zero, denormal, overflowing).  Each interaction carries a few roundings of
 2^-53 and n of them are added: |diff| <= (n + 16) 2^-53 sum |q / r|.
@@ -78,3 +78,9 @@ def test_direct_sum_extreme_distances(gpu):
             assert abs(t["p"][0] - p) <= 8 * 2.0 ** -53 * abs(p), (x[i], t["p"][0], p)
         else:
             assert not np.isfinite(t["p"][0])
+
+
+@pytest.mark.parametrize("ns", [8192, 8193])
+def test_direct_sum_launch_split(gpu, ns):
+    """The most sources that one launch adds, and the fewest of two."""
+    test_direct_sum(gpu, 3, ns)
