@@ -416,28 +416,91 @@ void radix_sort_pairs(unsigned long long *&k, int *&v, unsigned long long *&k2, 
                       int hi_bit, Buf<int> &hist, hipStream_t s);
 
 // ------------------------------------------------------------------ cross-lane sums
+// Value of lane l ^ M (M < 16) by data-parallel-primitive moves inside rows
+// of 16 lanes, one word at a time: no trip through LDS as __shfl_xor takes.
+template <int CTRL, class T>
+__device__ inline T dpp_move(T v) {
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8, "whole words");
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+  } else {
+    struct Words {
+      int w[2];
+    };
+    Words x = __builtin_bit_cast(Words, v);
+    x.w[0] = __builtin_amdgcn_mov_dpp(x.w[0], CTRL, 0xf, 0xf, true);
+    x.w[1] = __builtin_amdgcn_mov_dpp(x.w[1], CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(T, x);
+  }
+}
+template <int M, class T>
+__device__ inline T lane_xor(T v) {
+  static_assert(M == 1 || M == 2 || M == 4 || M == 8, "inside a row");
+  if constexpr (M == 1) return dpp_move<0xB1>(v);                    // quad_perm 1,0,3,2
+  if constexpr (M == 2) return dpp_move<0x4E>(v);                    // quad_perm 2,3,0,1
+  if constexpr (M == 4) return dpp_move<0x1B>(dpp_move<0x141>(v));   // mirror in 8 lanes, then in 4
+  return dpp_move<0x128>(v);                                         // rotate by 8 in 16
+}
+
+// Halves of a and b exchanged between lanes l and l ^ M (M = 16 or 32): lanes
+// without bit M get a's own and partner's values, lanes with it b's.
+template <int M>
+__device__ inline void lane_swap_word(unsigned &a, unsigned &b) {
+  const auto r = M == 32 ? __builtin_amdgcn_permlane32_swap(a, b, false, false)
+                         : __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+template <int M, class T>
+__device__ inline T lane_swap_sum(T a, T b) {
+  struct Words {
+    unsigned w[sizeof(T) / 4];
+  };
+  Words x = __builtin_bit_cast(Words, a), y = __builtin_bit_cast(Words, b);
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(T) / 4; i++) lane_swap_word<M>(x.w[i], y.w[i]);
+  return __builtin_bit_cast(T, x) + __builtin_bit_cast(T, y);
+}
+
+// Sum over the N lanes that differ in their low bits (N = 1, 2, 4, .. 64).
+template <int N, class T>
+__device__ inline T lane_sum(T v) {
+  if constexpr (N > 1) v += lane_xor<1>(v);
+  if constexpr (N > 2) v += lane_xor<2>(v);
+  if constexpr (N > 4) v += lane_xor<4>(v);
+  if constexpr (N > 8) v += lane_xor<8>(v);
+  if constexpr (N > 16) v = lane_swap_sum<16>(v, v);
+  if constexpr (N > 32) v = lane_swap_sum<32>(v, v);
+  return v;
+}
+
 // Sum over the 64 lanes of TC per-lane values by recursive halving: at each
-// step a lane keeps one half of its values and sends the other half to its
-// partner (TC - 1 shuffles instead of 6 TC).  Afterwards lane l holds the
-// partial sum of value l >> (6 - log2 TC) over the lanes that share its low
-// bits; the caller finishes with a butterfly over those bits.
-template <int TC, class T>
-__device__ inline T halving(T (&v)[TC], int lane) {
-  int c = TC;
+// step a lane keeps one half of its values and adds its partner's (TC - 1
+// exchanges instead of 6 TC).  Afterwards lane l holds the partial sum of value
+// l >> (6 - log2 TC) over the lanes that share its low bits; the caller finishes
+// with lane_sum over those bits.
+template <int M, int C, class T>
+__device__ inline void halve(T *v, int lane) {
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    if (c > 1) {
-      const bool up = lane & m;
-#pragma unroll
-      for (int i = 0; i < TC / 2; i++) {
-        if (i < c / 2) {
-          const T lo = v[i], hi = v[i + c / 2];
-          v[i] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, m);
-        }
-      }
-      c >>= 1;
+  for (int i = 0; i < C / 2; i++) {
+    const T lo = v[i], hi = v[i + C / 2];
+    if constexpr (M >= 16) {
+      v[i] = lane_swap_sum<M>(lo, hi);
+    } else {
+      const bool up = lane & M;
+      v[i] = (up ? hi : lo) + lane_xor<M>(up ? lo : hi);
     }
   }
+}
+template <int TC, class T>
+__device__ inline T halving(T (&v)[TC], int lane) {
+  static_assert(TC <= 64 && (TC & (TC - 1)) == 0, "a power of two");
+  if constexpr (TC > 1) halve<32, TC>(v, lane);
+  if constexpr (TC > 2) halve<16, TC / 2>(v, lane);
+  if constexpr (TC > 4) halve<8, TC / 4>(v, lane);
+  if constexpr (TC > 8) halve<4, TC / 8>(v, lane);
+  if constexpr (TC > 16) halve<2, TC / 16>(v, lane);
+  if constexpr (TC > 32) halve<1, TC / 32>(v, lane);
   return v[0];
 }
 

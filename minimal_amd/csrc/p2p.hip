@@ -199,13 +199,10 @@ __device__ inline T p2p_lane_total(const T (&ap)[TC], const T (&ax)[TC], const T
     vz[i] = i < TC ? az[i] : T(0);
   }
   T rp = halving<T2>(vp, lane), rx = halving<T2>(vx, lane), ry = halving<T2>(vy, lane), rz = halving<T2>(vz, lane);
-#pragma unroll
-  for (int m = 1; m < kLow; m <<= 1) {
-    rp += __shfl_xor(rp, m);
-    rx += __shfl_xor(rx, m);
-    ry += __shfl_xor(ry, m);
-    rz += __shfl_xor(rz, m);
-  }
+  rp = lane_sum<kLow>(rp);
+  rx = lane_sum<kLow>(rx);
+  ry = lane_sum<kLow>(ry);
+  rz = lane_sum<kLow>(rz);
   const int comp = lane % kLow;
   return comp == 0 ? rp : comp == 1 ? rx : comp == 2 ? ry : comp == 3 ? rz : T(0);
 }
