@@ -209,7 +209,7 @@ struct Tree {
   Buf<int> lcount, lstart_d, misc, cursor;
   Buf<unsigned long long> lookback;  // published prefixes of the level splits (tree.hip)
   unsigned lookback_tag = 0;
-  Buf<double> bounds_part;
+  Buf<double> bounds_part, forest_part;
   Buf<int> rs_hist;
   Buf<int> scan_tmp;  // device-wide scan partials
   bool built = false;

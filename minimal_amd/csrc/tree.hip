@@ -140,24 +140,23 @@ __global__ void __launch_bounds__(256) k_forest_init(RootOut out, int4 *__restri
   clear_counters(out);
 }
 
-// Forest: one workgroup per problem (bodies off[p] .. off[p+1] - 1), the
-// root of k_bounds_final per problem (min / max are exact, so any reduction
-// order gives the same root).  Empty problems get a unit root.
-constexpr int kFBThreads = 1024;  // one workgroup per problem: up to ~10^5 bodies each
-__global__ void __launch_bounds__(kFBThreads) k_forest_bounds(const exafmm_body *__restrict__ b,
-                                                       const int64_t *__restrict__ off,
-                                                       double4 *__restrict__ roots, int *__restrict__ flags) {
-  __shared__ double s[6][kFBThreads];
-  const int p = blockIdx.x, t = threadIdx.x;
-  const int64_t i0 = off[p], i1 = off[p + 1];
-  if (i1 <= i0) {
-    if (t == 0) roots[p] = make_double4(0.0, 0.0, 0.0, 1.0);
-    return;
-  }
-  double lo[3] = {b[i0].X[0], b[i0].X[1], b[i0].X[2]};
+// Forest: the root of k_bounds_final per problem (min / max are exact, so any
+// reduction order gives the same root).  Empty problems get a unit root.  A
+// problem's bodies are shared by kForestShares workgroups (one alone took 30 -
+// 68 us for 100,000 bodies); part: [problem][share][lo, hi].
+constexpr int kForestShares = 16;
+__global__ void __launch_bounds__(256) k_forest_bounds(const exafmm_body *__restrict__ b,
+                                                       const int64_t *__restrict__ off, double *__restrict__ part,
+                                                       int *__restrict__ flags) {
+  __shared__ double s[256 / kWave][6];
+  const int p = blockIdx.y, t = threadIdx.x, lane = t % kWave, w = t / kWave;
+  const int64_t o0 = off[p], n = off[p + 1] - o0;
+  if (n <= 0) return;
+  const int64_t i0 = o0 + n * blockIdx.x / kForestShares, i1 = o0 + n * (blockIdx.x + 1) / kForestShares;
+  double lo[3] = {b[o0].X[0], b[o0].X[1], b[o0].X[2]};
   double hi[3] = {lo[0], lo[1], lo[2]};
   int bad = 0;
-  for (int64_t i = i0 + t; i < i1; i += kFBThreads) {
+  for (int64_t i = i0 + t; i < i1; i += 256) {
     for (int d = 0; d < 3; d++) {
       const double x = b[i].X[d];
       if (!isfinite(x)) bad = 1;
@@ -167,25 +166,46 @@ __global__ void __launch_bounds__(kFBThreads) k_forest_bounds(const exafmm_body 
     if (!isfinite(b[i].q)) bad = 1;
   }
   if (bad) atomicOr(flags, 1);
-  for (int d = 0; d < 3; d++) {
-    s[d][t] = lo[d];
-    s[3 + d][t] = hi[d];
-  }
+  for (int d = 0; d < 3; d++)
+    for (int o = 1; o < kWave; o <<= 1) {
+      lo[d] = fmin(lo[d], __shfl_xor(lo[d], o));
+      hi[d] = fmax(hi[d], __shfl_xor(hi[d], o));
+    }
+  if (lane == 0)
+    for (int d = 0; d < 3; d++) {
+      s[w][d] = lo[d];
+      s[w][3 + d] = hi[d];
+    }
   __syncthreads();
-  for (int o = kFBThreads / 2; o > 0; o >>= 1) {
-    if (t < o)
-      for (int d = 0; d < 3; d++) {
-        s[d][t] = fmin(s[d][t], s[d][t + o]);
-        s[3 + d][t] = fmax(s[3 + d][t], s[3 + d][t + o]);
-      }
-    __syncthreads();
+  if (t < 6) {
+    double v = s[0][t];
+    for (int k = 1; k < 256 / kWave; k++) v = t < 3 ? fmin(v, s[k][t]) : fmax(v, s[k][t]);
+    part[(int64_t(p) * kForestShares + blockIdx.x) * 6 + t] = v;
   }
-  if (t != 0) return;
-  double X0[3], R0 = 0;
-  for (int d = 0; d < 3; d++) X0[d] = (s[3 + d][0] + s[d][0]) / 2;
+}
+
+__global__ void __launch_bounds__(64) k_forest_roots(const int64_t *__restrict__ off, const double *__restrict__ part,
+                                                     int nprob, double4 *__restrict__ roots) {
+  const int p = blockIdx.x * 64 + threadIdx.x;
+  if (p >= nprob) return;
+  if (off[p + 1] <= off[p]) {
+    roots[p] = make_double4(0.0, 0.0, 0.0, 1.0);
+    return;
+  }
+  const double *q = part + int64_t(p) * kForestShares * 6;
+  double lo[3], hi[3], X0[3], R0 = 0;
   for (int d = 0; d < 3; d++) {
-    R0 = fmax(X0[d] - s[d][0], R0);
-    R0 = fmax(s[3 + d][0] - X0[d], R0);
+    lo[d] = q[d];
+    hi[d] = q[3 + d];
+    for (int k = 1; k < kForestShares; k++) {
+      lo[d] = fmin(lo[d], q[k * 6 + d]);
+      hi[d] = fmax(hi[d], q[k * 6 + 3 + d]);
+    }
+    X0[d] = (hi[d] + lo[d]) / 2;
+  }
+  for (int d = 0; d < 3; d++) {
+    R0 = fmax(X0[d] - lo[d], R0);
+    R0 = fmax(hi[d] - X0[d], R0);
   }
   R0 *= 1.00001;
   roots[p] = make_double4(X0[0], X0[1], X0[2], R0);
@@ -813,8 +833,12 @@ void tree_build(Ctx &c) {
   if (forest) {
     hipLaunchKernelGGL(k_forest_init, dim3(256), dim3(256), 0, s, rout, hist7);
     XF_LAUNCH();
-    hipLaunchKernelGGL(k_forest_bounds, dim3(c.forest_n), dim3(kFBThreads), 0, s, c.bodies, c.forest_off.p,
-                       c.forest_roots.p, t.misc.p);
+    t.forest_part.ensure(size_t(c.forest_n) * kForestShares * 6);
+    hipLaunchKernelGGL(k_forest_bounds, dim3(kForestShares, c.forest_n), dim3(256), 0, s, c.bodies, c.forest_off.p,
+                       t.forest_part.p, t.misc.p);
+    XF_LAUNCH();
+    hipLaunchKernelGGL(k_forest_roots, dim3(ceil_div(c.forest_n, 64)), dim3(64), 0, s, c.forest_off.p, t.forest_part.p,
+                       c.forest_n, c.forest_roots.p);
     XF_LAUNCH();
   } else {
     hipLaunchKernelGGL(k_bounds_part, dim3(kBoundsBlocks), dim3(256), 0, s, c.bodies, n, t.bounds_part.p, hist7);
