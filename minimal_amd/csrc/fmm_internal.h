@@ -301,6 +301,9 @@ struct Ctx {
   int m2l_ntiles_last = 0;  // tiles of the last keyed M2L (statistics)
   std::map<long long, int> gemm_tuned;  // autotuned GEMM shape (rows, keys per round, slices) per class
   Buf<double> L_tune;                   // scratch locals of the autotuning runs
+  // an evaluation beside others does not tune (defer_tuning): it takes a tuned
+  // neighbour's shape and asks for a run of its own
+  bool defer_tuning = false, tuning_wanted = true;
   Buf<unsigned char> tile_p;
   // BF16x3 learned order: each tile's slots grouped by order (tile_perm:
   // permuted slot -> slot; tile_cls: [first | count] x order x tile stride)

@@ -1196,9 +1196,13 @@ static int gemm_ring(int KS, int G) {
 // Row tiles per workgroup for rounds of `kr` (FP32: keys; BF16: units, a key
 // having K32 of them): two operator buffers and the column sources within the
 // LDS budget, at most the accumulators of kGemmMaxRT row tiles per wave.
+static int lds_limit(int device) {
+  int n = 0;
+  XF_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
+  return n;
+}
 static int rows_per_block(const Geom &g, bool bf16, int device, int kr) {
-  int max_lds = 0;
-  XF_HIP(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
+  const int max_lds = lds_limit(device);
   const int per_rt = 2 * kr * (bf16 ? 64 * 16 * 2 : g.K4 * 64 * 4);  // both buffers
   const int avail = max_lds - (bf16 ? gemm_ring(g.K32, kr) : 3 * kr) * kTileN * 4;
   if (per_rt > avail) {
@@ -1260,10 +1264,14 @@ static int cu_count(int device) {
 // Persistent workgroups per row block of a stream-K launch.
 static int sk_groups(int device, int nblk) { return std::max(1, cu_count(device) / nblk); }
 
+// The attribute belongs to the kernel, not to the launch: always the limit, so
+// that contexts on several threads agree on it.
 template <class K>
-static void gemm_attr(K *kernel, size_t lds) {
+static void gemm_attr(K *kernel) {
+  int device = 0;
+  XF_HIP(hipGetDevice(&device));
   XF_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                             int(lds)));
+                             lds_limit(device)));
 }
 
 template <int RH>
@@ -1279,7 +1287,7 @@ static void launch_bf16(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, int KP
   const size_t lds = gemm_lds(go, true, sh.rtb, sh.kr);
   if (!sh.sk) {
     auto *k = cp ? &k_m2l_bf16x3<RH, true> : &k_m2l_bf16x3<RH, false>;
-    gemm_attr(k, lds);
+    gemm_attr(k);
     hipLaunchKernelGGL(k, dim3(ntiles, nblk, sh.ksplit), dim3(kGemmThreads), lds, c.s0, in,
                        cp ? cp->start : tbase, g.PP, g.R, sh.rtb, g.K32, KPb, op, tkp, sh.kr, ring,
                        sh.ksplit > 1 ? Lpart : nullptr, Lout);
@@ -1292,7 +1300,7 @@ static void launch_bf16(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, int KP
   const int *pre = cp ? cp->pre : tbase, *start = cp ? cp->start : tbase;
   const int *Sdev = cp ? cp->tot : nullptr;
   auto *k = cp ? &k_m2l_bf16x3_sk<RH, true> : &k_m2l_bf16x3_sk<RH, false>;
-  gemm_attr(k, lds);
+  gemm_attr(k);
   hipLaunchKernelGGL(k, dim3(W, nblk), dim3(kGemmThreads), lds, c.s0, in, pre, start, g.PP, g.R,
                      sh.rtb, g.K32, KPb, op, ntiles, S, Sdev, tkp, sh.kr, ring, c.m2l_part.p);
   XF_LAUNCH();
@@ -1308,7 +1316,7 @@ static void launch_f32(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, int KP,
   const int ts = c.m2l_tstride;
   const int *t = c.tiles.p;
   const size_t lds = gemm_lds(g, false, sh.rtb, sh.kr);
-  gemm_attr(&k_m2l_f32<RH>, lds);
+  gemm_attr(&k_m2l_f32<RH>);
   hipLaunchKernelGGL((k_m2l_f32<RH>), dim3(ntiles, ceil_div(g.R, sh.rtb), sh.ksplit), dim3(kGemmThreads), lds, c.s0,
                      g.PP, g.R, sh.rtb, g.K4, KP, t, t + ts, t + 2 * ts, t + 3 * ts, t + 4 * ts, c.tile_keys.p,
                      c.tile_mat.p, c.ops32.p, sc.mt32.p, c.learned ? c.tile_p.p : nullptr, sh.kr,
@@ -1383,9 +1391,18 @@ static GemmShape gemm_shape(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, bo
   const long long key = ((long long)g.P << 24) | ((long long)bf16 << 20) | ((long long)c.learned << 16) |
                         ((long long)(cp ? cp->p : 0) << 32) | tclass;
   auto it = c.gemm_tuned.find(key);
-  if (it != c.gemm_tuned.end())
-    return GemmShape{int(it->second & 255), int((it->second >> 8) & 255), int((it->second >> 16) & 255),
-                     int(it->second >> 24)};
+  auto shape = [](int v) { return GemmShape{v & 255, (v >> 8) & 255, (v >> 16) & 255, v >> 24}; };
+  if (it != c.gemm_tuned.end()) return shape(it->second);
+  if (c.defer_tuning && c.cfg.autotune) {
+    // the tuned class nearest in tile count (the low bits of the key), if there is one
+    c.tuning_wanted = true;
+    const std::pair<const long long, int> *near = nullptr;
+    for (const auto &kv : c.gemm_tuned)
+      if ((kv.first >> 16) == (key >> 16) &&
+          (!near || std::llabs(kv.first - key) < std::llabs(near->first - key)))
+        near = &kv;
+    if (near) return shape(near->second);
+  }
   std::vector<GemmShape> cand;
   auto slices = [&](int rtb, int kr, int nb) {
     cand.push_back(GemmShape{rtb, kr, 1});
@@ -1424,6 +1441,7 @@ static GemmShape gemm_shape(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, bo
   if (c.capturing) fail(EXAFMM_ERR_STATE, "GEMM shape not tuned before recording a graph");
   if (std::getenv("EXAFMM_GEMM_SK_ONLY")) cand.erase(std::remove_if(cand.begin(), cand.end(), [](const GemmShape &x) { return !x.sk; }), cand.end());
   if (cand.empty()) fail(EXAFMM_ERR_UNSUPPORTED, "no GEMM shape");
+  if (cand.size() > 1 && c.cfg.autotune && c.defer_tuning) return best;  // (not kept: tuned by the next run)
   if (cand.size() > 1 && c.cfg.autotune) {
     hipStream_t s = c.s0;
     XF_HIP(hipStreamSynchronize(c.s1));  // tune alone on the device
@@ -1804,7 +1822,7 @@ void m2l_group_setup(const std::vector<Ctx *> &probs, GemmGroupPlan &plan, hipSt
 template <int RH>
 static void launch_group(const GemmGroupPlan &plan, const Geom &g, hipStream_t s) {
   const GroupGemm *d = reinterpret_cast<const GroupGemm *>(plan.desc.p);
-  gemm_attr(&k_m2l_bf16x3_grouped<RH>, plan.lds);
+  gemm_attr(&k_m2l_bf16x3_grouped<RH>);
   hipLaunchKernelGGL((k_m2l_bf16x3_grouped<RH>), dim3(plan.groups, ceil_div(g.R, plan.rtb)), dim3(kGemmThreads),
                      plan.lds, s, d, plan.start.p, plan.nprob, g.PP, g.R, plan.rtb, g.K32, bf16_row(g), g.P, plan.kr,
                      gemm_ring(g.K32, plan.kr), plan.seg.p);
