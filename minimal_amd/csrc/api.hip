@@ -843,8 +843,8 @@ struct exafmm_graph {
   xf::Buf<xf::GroupTree> gt;
   xf::Buf<xf::GroupLevel> lv;
   xf::Buf<int> starts;
-  Stage pro, p2p;
-  std::map<int, Stage> p2m, l2p;  // by order
+  Stage pro, p2p, l2p;
+  std::map<int, Stage> p2m;  // by order
   std::vector<Stage> m2m_levels, l2l_levels;  // M2M bottom-up, L2L top-down
   std::vector<std::unique_ptr<xf::GemmGroupPlan>> gemm;  // one per order
   std::vector<int> level_soff_m2m, level_soff_l2l;       // start-array offsets of the level stages
@@ -930,14 +930,13 @@ void grouped_tables(exafmm_graph *g) {
   per_problem(g->pro, [](const Ctx &c) {
     return int64_t(ceil_div(c.t.n, 256)) + ceil_div(c.t.ncells * c.P * c.P, 256);
   });
+  per_problem(g->l2p, [](const Ctx &c) { return int64_t(ceil_div(c.t.n, kWave)); });
   // one launch per order: the problems of another order have no blocks in it
   g->p2m.clear();
-  g->l2p.clear();
   for (const exafmm_ctx *x : g->ctxs) {
     const int P = x->c.P;
     if (g->p2m.count(P)) continue;
     per_problem(g->p2m[P], [P](const Ctx &c) { return c.P == P ? int64_t(p2m_group_blocks(c.t.nleaves)) : 0; });
-    per_problem(g->l2p[P], [P](const Ctx &c) { return c.P == P ? int64_t(ceil_div(c.t.n, kWave)) : 0; });
   }
   per_problem(g->p2p, [](const Ctx &c) { return int64_t(p2p_group_blocks(c.t.nleaves)); });
   // per-level stages: the problems that have parents at level l
@@ -998,7 +997,7 @@ void grouped_tables(exafmm_graph *g) {
 
 // All charge-dependent passes of every problem: one launch per stage (per
 // level for M2M and L2L, per order for the keyed GEMM); P2P on the second
-// stream beside the upward pass and M2L, joined before L2P (a launch per order).
+// stream beside the upward pass and M2L, joined before L2P.
 void grouped_record(exafmm_graph *g, hipStream_t sa, hipStream_t sb, hipEvent_t fork, hipEvent_t join) {
   const int n = int(g->ctxs.size());
   const int *st = g->starts.p;
@@ -1019,19 +1018,7 @@ void grouped_record(exafmm_graph *g, hipStream_t sa, hipStream_t sb, hipEvent_t 
     if (sg.blocks) l2l_grouped(g->gt.p, g->lv.p + sg.off, st + g->level_soff_l2l[k], sg.n, sg.blocks, sa);
   }
   XF_HIP(hipStreamWaitEvent(sa, join, 0));
-  // the orders' launches are short: every other one on the second stream
-  const bool two = g->l2p.size() > 1;
-  if (two) {
-    XF_HIP(hipEventRecord(fork, sa));
-    XF_HIP(hipStreamWaitEvent(sb, fork, 0));
-  }
-  int k = 0;
-  for (const auto &kv : g->l2p)
-    l2p_grouped(kv.first, g->gt.p, st + kv.second.off, n, kv.second.blocks, k++ % 2 ? sb : sa);
-  if (two) {
-    XF_HIP(hipEventRecord(join, sb));
-    XF_HIP(hipStreamWaitEvent(sa, join, 0));
-  }
+  if (g->l2p.blocks) l2p_grouped(g->gt.p, st + g->l2p.off, n, g->l2p.blocks, sa);
 }
 
 }  // namespace

@@ -39,28 +39,17 @@ static __constant__ InvTable kInv = InvTable();
 
 // f(integral_constant<P>) for the order at run time: kernels whose loops over
 // the degrees unroll are instantiated per order.
+#define XF_ORDER_CASE(f, n)                       \
+  case n:                                         \
+    return f(std::integral_constant<int, n>());
+#define XF_ORDER_CASES(f)                                                                                 \
+  XF_ORDER_CASE(f, 2) XF_ORDER_CASE(f, 3) XF_ORDER_CASE(f, 4) XF_ORDER_CASE(f, 5) XF_ORDER_CASE(f, 6)     \
+  XF_ORDER_CASE(f, 7) XF_ORDER_CASE(f, 8) XF_ORDER_CASE(f, 9) XF_ORDER_CASE(f, 10) XF_ORDER_CASE(f, 11)   \
+  XF_ORDER_CASE(f, 12) XF_ORDER_CASE(f, 13) XF_ORDER_CASE(f, 14) XF_ORDER_CASE(f, 15) XF_ORDER_CASE(f, 16)
 template <class F>
 static void by_order(int P, F &&f) {
   switch (P) {
-#define XF_ORDER_CASE(n)                          \
-  case n:                                         \
-    return f(std::integral_constant<int, n>());
-    XF_ORDER_CASE(2)
-    XF_ORDER_CASE(3)
-    XF_ORDER_CASE(4)
-    XF_ORDER_CASE(5)
-    XF_ORDER_CASE(6)
-    XF_ORDER_CASE(7)
-    XF_ORDER_CASE(8)
-    XF_ORDER_CASE(9)
-    XF_ORDER_CASE(10)
-    XF_ORDER_CASE(11)
-    XF_ORDER_CASE(12)
-    XF_ORDER_CASE(13)
-    XF_ORDER_CASE(14)
-    XF_ORDER_CASE(15)
-    XF_ORDER_CASE(16)
-#undef XF_ORDER_CASE
+    XF_ORDER_CASES(f)
     default:
       fail(EXAFMM_ERR_UNSUPPORTED, "expansion order");
   }
@@ -719,14 +708,20 @@ __device__ __attribute__((always_inline)) inline void l2p_eval(T x, T y, T z, co
 // body against its run's slot.  T = float, or double in parity mode.
 constexpr int kL2PSlots = 8;
 template <int P, class T>
+struct L2PLds {
+  cpx<T> Lh[kL2PSlots][(P * (P + 1) / 2) | 1];  // odd: the slots' equal entries lie in distinct banks
+  int leaf[kL2PSlots];
+};
+template <int P, class T>
 __device__ __attribute__((always_inline)) inline void l2p_body(int bx, int64_t n, const int *__restrict__ body_leaf,
                                                                const double4 *__restrict__ cx,
                                                                const double *__restrict__ L,
                                                                const double4 *__restrict__ xs,
-                                                               exafmm_body *__restrict__ bodies) {
+                                                               exafmm_body *__restrict__ bodies,
+                                                               L2PLds<P, T> &lds) {
   constexpr int NT = P * (P + 1) / 2, KE = (NT + kWave - 1) / kWave;
-  __shared__ cpx<T> Lh[kL2PSlots][NT | 1];  // odd: the slots' equal entries lie in distinct banks
-  __shared__ int sleaf[kL2PSlots];
+  auto &Lh = lds.Lh;
+  auto &sleaf = lds.leaf;
   const int lane = threadIdx.x;
   const int64_t b = int64_t(bx) * kWave + lane;
   const bool valid = b < n;
@@ -788,16 +783,24 @@ template <int P, class T>
 __global__ void __launch_bounds__(64) k_l2p(int64_t n, const int *__restrict__ body_leaf,
                                             const double4 *__restrict__ cx, const double *__restrict__ L,
                                             const double4 *__restrict__ xs, exafmm_body *__restrict__ bodies) {
-  l2p_body<P, T>(blockIdx.x, n, body_leaf, cx, L, xs, bodies);
+  __shared__ L2PLds<P, T> lds;
+  l2p_body<P, T>(blockIdx.x, n, body_leaf, cx, L, xs, bodies, lds);
 }
 
-// The problems of one order of a batch in one launch.
-template <int P>
+// All problems of a batch in one launch, each workgroup by its problem's order
+// (a launch per order: 45 us for three orders, their tails one after the other).
 __global__ void __launch_bounds__(64) k_l2p_grouped(const GroupTree *__restrict__ g, const int *__restrict__ start,
                                                     int nprob) {
+  __shared__ L2PLds<kMaxP, float> lds;  // every order's fits
   const int b = blockIdx.x, i = group_of(start, nprob, b);
   const GroupTree &t = g[i];
-  l2p_body<P, float>(b - start[i], t.n, t.body_leaf, t.cx, t.L, t.xs, t.bodies);
+  auto run = [&](auto p) {
+    l2p_body<p(), float>(b - start[i], t.n, t.body_leaf, t.cx, t.L, t.xs, t.bodies,
+                         reinterpret_cast<L2PLds<p(), float> &>(lds));
+  };
+  switch (t.P) {
+    XF_ORDER_CASES(run)
+  }
 }
 
 
@@ -820,10 +823,8 @@ void l2l_grouped(const GroupTree *g, const GroupLevel *lv, const int *start, int
   hipLaunchKernelGGL(k_l2l_grouped, dim3(nblocks), dim3(kShiftWaves * kWave), 0, s, g, lv, start, n);
   XF_LAUNCH();
 }
-void l2p_grouped(int P, const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s) {
-  by_order(P, [&](auto p) {
-    hipLaunchKernelGGL((k_l2p_grouped<p()>), dim3(nblocks), dim3(kWave), 0, s, g, start, nprob);
-  });
+void l2p_grouped(const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s) {
+  hipLaunchKernelGGL(k_l2p_grouped, dim3(nblocks), dim3(kWave), 0, s, g, start, nprob);
   XF_LAUNCH();
 }
 

@@ -372,7 +372,7 @@ int p2p_group_blocks(int64_t nleaves);
 void p2m_grouped(int P, const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s);
 void m2m_grouped(const GroupTree *g, const GroupLevel *lv, const int *start, int n, int nblocks, hipStream_t s);
 void l2l_grouped(const GroupTree *g, const GroupLevel *lv, const int *start, int n, int nblocks, hipStream_t s);
-void l2p_grouped(int P, const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s);
+void l2p_grouped(const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s);
 void p2p_grouped(const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s);
 // keyed M2L of every problem of one order (BF16x3, fixed order): cast +
 // GEMM, one launch each; the plan holds the device descriptor tables
