@@ -105,7 +105,8 @@ void bodies_to_host(Ctx &c) {
 }
 
 // event slots: 0/1 build, 2/3 upward, 11/12 traversal, 9/4 M2L (s0),
-// 5/6 P2P (s1), 15 end of s1's work, 10/8 downward
+// 5/6 P2P (s1), 15 end of s1's work, 10/8 downward, 7 the upward pass's wide
+// part (run_passes)
 void do_build(Ctx &c) {
   if (c.graph_locks) fail(EXAFMM_ERR_STATE, "the context is held by a graph (exafmm_graph_destroy it first)");
   rec(c, 0, c.s0);
@@ -115,10 +116,10 @@ void do_build(Ctx &c) {
   c.lists.valid = false;
 }
 
-void do_upward(Ctx &c, hipStream_t s) {
+void do_upward(Ctx &c, hipStream_t s, hipEvent_t wide = nullptr) {
   if (!c.t.built) fail(EXAFMM_ERR_STATE, "upward pass before build_tree");
   rec(c, 2, s);
-  upward(c, s);
+  upward(c, s, wide);
   rec(c, 3, s);
 }
 
@@ -185,10 +186,21 @@ void do_downward(Ctx &c) {
 // adds a long latency-bound chain on s0 (the top levels' FP64 M2L per pair,
 // the image ladder) that P2P started earlier would starve (N = 2^20, images
 // = 3: 6.5 ms against 6.9).
+//
+// A large tree's upward pass is launched before the traversal (whose first
+// levels leave the device idle), and P2P waits for its wide part: started
+// beside P2P, which leaves no room for their workgroups, the row-tile M2M
+// launches of 1.5M clustered bodies (90,000 cells) ended with it, 1.7 ms after
+// the lists, and the keyed GEMM waited for them (7.55 ms, 7.41 this way).  The
+// M2M of smaller trees is done sooner than that wait costs: 2^20 uniform bodies
+// (37,449 cells) 2.96 ms, 2.99 this way, 300,007 clustered 3.12 and 3.17.
+constexpr int64_t kUpwardFirst = 65536;  // cells
 void run_passes(Ctx &c) {
+  const bool upward_first = c.t.ncells >= kUpwardFirst;
   // P2P on s1 from event 14 (the lists' end on s0)
-  auto launch_p2p = [&c](const int *list_flags) {
+  auto launch_p2p = [&c, upward_first](const int *list_flags) {
     XF_HIP(hipStreamWaitEvent(c.s1, c.ev[14], 0));
+    if (upward_first) XF_HIP(hipStreamWaitEvent(c.s1, c.ev[7], 0));
     rec(c, 5, c.s1);
     p2p_apply(c, c, c.s1, list_flags);
     rec(c, 6, c.s1);
@@ -198,11 +210,12 @@ void run_passes(Ctx &c) {
   // the upward pass on s2, from the tree's end (event 1); joined where the
   // multipoles are first read (join_upward)
   auto launch_upward = [&c] {
-    if (c.have_M) return;  // a repeated traversal
+    if (c.have_M) return;  // launched first, or a repeated traversal
     XF_HIP(hipStreamWaitEvent(c.s2, c.ev[1], 0));
-    do_upward(c, c.s2);
+    do_upward(c, c.s2, c.ev[7]);
     c.upward_pending = true;
   };
+  if (upward_first) launch_upward();
   if (c.cfg.images > 0) {
     do_lists(c, c, launch_upward);
     rec(c, 14, c.s0);

@@ -828,7 +828,7 @@ void l2p_grouped(const GroupTree *g, const int *start, int nprob, int nblocks, h
   XF_LAUNCH();
 }
 
-void upward(Ctx &c, hipStream_t s) {
+void upward(Ctx &c, hipStream_t s, hipEvent_t wide) {
   Tree &t = c.t;
   const int P = c.P, PP = P * P;
   shift_ops(c, s);
@@ -838,6 +838,10 @@ void upward(Ctx &c, hipStream_t s) {
                        t.misc.p + 17, t.cbeg.p, t.ccnt.p, t.cx.p, t.xs.p, c.M.p);
   });
   XF_LAUNCH();
+  int last_wide = t.depth;  // the last level, going up, that fills the device
+  for (int l = t.lroot; l < t.depth && last_wide == t.depth; l++)
+    if (t.lstart[l + 1] - t.lstart[l] >= kRowTileMinParents) last_wide = l;
+  if (wide && last_wide == t.depth) XF_HIP(hipEventRecord(wide, s));
   for (int l = t.depth - 1; l >= t.lroot; l--) {  // (a forest stops at its problems' roots)
     const int cnt = t.lstart[l + 1] - t.lstart[l];
     if (cnt >= kRowTileMinParents)
@@ -847,6 +851,7 @@ void upward(Ctx &c, hipStream_t s) {
       hipLaunchKernelGGL(k_m2m, dim3(ceil_div(cnt, 16), m2m_group_rows(P)), dim3(kM2MWaves * kWave), 0, s, c.P,
                          t.lstart[l], cnt, t.cchild.p, t.cnch.p, t.cx.p, c.shift_T.p, c.M.p);
     XF_LAUNCH();
+    if (wide && l == last_wide) XF_HIP(hipEventRecord(wide, s));
   }
   c.have_M = true;
 }

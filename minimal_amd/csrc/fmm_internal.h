@@ -344,7 +344,8 @@ void tree_ref_order(Ctx &c, std::vector<int64_t> &bfs2ref, std::vector<int64_t> 
 // on s0 and before the host reads the totals (flags in lists.tot[3]; a pass
 // with kListRetry bits set is repeated after s1 has drained).
 void traverse(Ctx &tgt, const Ctx &src, const std::function<void()> &after_kernels = {});
-void upward(Ctx &c, hipStream_t s);
+// wide (if given) is recorded behind the P2M and the levels that fill the device
+void upward(Ctx &c, hipStream_t s, hipEvent_t wide = nullptr);
 // The main stream waits for an upward pass running on s2: before the first
 // read of the multipoles.
 inline void join_upward(Ctx &c) {
