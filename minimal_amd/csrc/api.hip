@@ -1369,6 +1369,9 @@ static void batch_forests(exafmm_ctx *ctx, const exafmm_problem *problems, int c
           failed[gi].msg = e.msg;
         } catch (const std::bad_alloc &) {
           failed[gi].code = EXAFMM_ERR_ALLOC;
+        } catch (const std::exception &e) {
+          failed[gi].code = EXAFMM_ERR_ARG;
+          failed[gi].msg = e.what();
         }
     };
     std::vector<std::thread> threads;
