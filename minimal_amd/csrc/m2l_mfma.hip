@@ -1184,6 +1184,63 @@ __global__ void __launch_bounds__(256) k_sk_combine(int PP, int rows, int ntiles
                   sorted + tfirst[t], Lseg, L);
 }
 
+// The segments of a learned-order evaluation's launches, one per order class,
+// added in one pass over the locals (a pass per class read and wrote them
+// again: over 300,007 bodies' cells at order 13 four passes took 97 us, this 63;
+// over 2^22 bodies' 0.8 ms, 0.4 less).
+constexpr int kMaxClasses = 6;
+struct ClassSum {
+  const int *pre, *cnt, *tot;  // per tile: first slot, slots; all slots (ClassPass)
+  int W, rows;                 // workgroups, rows of the launch
+  int64_t base;                // its segments in the buffer
+};
+struct ClassSums {
+  int n;
+  ClassSum c[kMaxClasses];
+};
+__global__ void __launch_bounds__(256) k_sk_combine_classes(int PP, int rows, int ntiles, ClassSums sums,
+                                                            const int *__restrict__ tfirst,
+                                                            const int *__restrict__ tcount,
+                                                            const int *__restrict__ sorted,
+                                                            const float *__restrict__ Lseg, double *__restrict__ L) {
+  const int t = blockIdx.y;
+  const int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  const int col = int(e / rows), row = int(e % rows);
+  if (t >= ntiles || col >= tcount[t]) return;
+  double *Lc = L + int64_t(sorted[tfirst[t] + col]) * PP + row;
+  // every class's first two segments are loaded before the first is added
+  const int64_t step = int64_t(kTileN) * PP;
+  const float *p[kMaxClasses];
+  int nseg[kMaxClasses];
+  float v[kMaxClasses][2];
+#pragma unroll
+  for (int k = 0; k < kMaxClasses; k++) {
+    const ClassSum &c = sums.c[k];
+    nseg[k] = 0;
+    v[k][0] = v[k][1] = 0.0f;
+    if (k >= sums.n) continue;
+    const int n = c.cnt[t];
+    if (n == 0 || row >= c.rows) continue;
+    const int64_t b = c.pre[t], S = *c.tot;
+    auto wg_of = [&](int64_t sl) { return int(((sl + 1) * c.W - 1) / S); };
+    const int wf = wg_of(b);
+    nseg[k] = wg_of(b + n - 1) - wf + 1;
+    p[k] = Lseg + c.base + (wf + int64_t(t)) * step + int64_t(col) * PP + row;
+    v[k][0] = p[k][0];
+    if (nseg[k] > 1) v[k][1] = p[k][step];
+  }
+  double l = *Lc;
+#pragma unroll
+  for (int k = 0; k < kMaxClasses; k++) {
+    if (nseg[k] == 0) continue;
+    double acc = double(v[k][0]);
+    if (nseg[k] > 1) acc += double(v[k][1]);
+    for (int w = 2; w < nseg[k]; w++) acc += double(p[k][w * step]);
+    l += acc;
+  }
+  *Lc = l;
+}
+
 // One problem of a grouped keyed-GEMM launch (all problems of one order in
 // a batch): its tiles, operators, cast multipoles and locals.
 struct GroupGemm {
@@ -1319,7 +1376,7 @@ static void gemm_attr(K *kernel) {
 
 template <int RH>
 static void launch_bf16(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, int KPb, GemmShape sh, float *Lpart,
-                        double *Lout, const ClassPass *cp) {
+                        double *Lout, const ClassPass *cp, ClassSums *sums) {
   const int ts = c.m2l_tstride;
   const int *tbase = c.tiles.p + 2 * ts;
   const Geom go = cp ? geom(cp->p) : g;  // rows and k-steps this launch covers
@@ -1339,19 +1396,25 @@ static void launch_bf16(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, int KP
   }
   const int W = sk_groups(c.cfg.device, nblk);
   const int64_t S = c.m2l_totalU;
-  c.m2l_part.ensure(size_t(W + ntiles) * kTileN * g.PP);
+  if (!sums) c.m2l_part.ensure(size_t(W + ntiles) * kTileN * g.PP);  // (else sized for every class)
+  float *seg = c.m2l_part.p + (sums ? sums->c[sums->n].base : 0);
   const int *pre = cp ? cp->pre : tbase, *start = cp ? cp->start : tbase;
   const int *Sdev = cp ? cp->tot : nullptr;
   auto *k = cp ? &k_m2l_bf16x3_sk<RH, true> : &k_m2l_bf16x3_sk<RH, false>;
   gemm_attr(k);
   hipLaunchKernelGGL(k, dim3(W, nblk), dim3(kGemmThreads), lds, c.s0, in, pre, start, g.PP, g.R,
-                     sh.rtb, g.K32, KPb, op, ntiles, S, Sdev, tkp, sh.kr, ring, c.m2l_part.p);
+                     sh.rtb, g.K32, KPb, op, ntiles, S, Sdev, tkp, sh.kr, ring, seg);
   XF_LAUNCH();
   const int rows = std::min(g.PP, 16 * go.R);
+  if (sums) {  // added with the other classes' by m2l_fast
+    ClassSum &k = sums->c[sums->n++];
+    k = ClassSum{pre, in.tU, Sdev, W, rows, k.base};
+    return;
+  }
   const int vec = sk_combine_vec(g.PP, rows);
   hipLaunchKernelGGL(vec == 4 ? k_sk_combine<4> : k_sk_combine<1>,
                      dim3(ceil_div(int64_t(kTileN) * rows / vec, 256), ntiles), dim3(256), 0, c.s0, g.PP, rows,
-                     ntiles, S, Sdev, W, in.tfirst, in.tcount, pre, in.tU, in.sorted, c.m2l_part.p, Lout);
+                     ntiles, S, Sdev, W, in.tfirst, in.tcount, pre, in.tU, in.sorted, seg, Lout);
   XF_LAUNCH();
 }
 
@@ -1370,7 +1433,7 @@ static void launch_f32(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, int KP,
 }
 
 static void run_gemm(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, bool bf16, int KP, int KPb, GemmShape sh,
-                     double *Lout, const ClassPass *cp = nullptr) {
+                     double *Lout, const ClassPass *cp = nullptr, ClassSums *sums = nullptr) {
   float *part = nullptr;
   if (sh.ksplit > 1) {
     c.m2l_part.ensure(size_t(sh.ksplit) * c.t.ncells * g.PP);
@@ -1380,7 +1443,7 @@ static void run_gemm(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, bool bf16
 #define XF_GEMM_CASE(n)                                                             \
   case n:                                                                           \
     if (bf16)                                                                       \
-      launch_bf16<n>(c, sc, g, ntiles, KPb, sh, part, Lout, cp);                    \
+      launch_bf16<n>(c, sc, g, ntiles, KPb, sh, part, Lout, cp, sums);              \
     else                                                                            \
       launch_f32<n <= kGemmMaxRTF32 ? n : 1>(c, sc, g, ntiles, KP, sh, part, Lout); \
     break;
@@ -1724,15 +1787,36 @@ void m2l_fast(Ctx &tc, const Ctx &sc) {
     hipLaunchKernelGGL(k_order_prefix, dim3(1), dim3(64 * ncls), 0, s, ntiles, ts, ncls, c.tile_cls.p);
     XF_LAUNCH();
     if (!c.capturing) XF_HIP(hipEventRecord(c.ev[13], s));
+    std::vector<ClassPass> pass;
+    std::vector<GemmShape> shape;
+    bool all_sk = ncls <= kMaxClasses;
     for (int o = ncls - 1; o >= 0; o--) {
       const int *cls = c.tile_cls.p;
       int lo = kMaxP;
       for (int p = kMlpPmin; p <= c.P; p++)
         if (oc.of[p] == o) lo = std::min(lo, p);
-      const ClassPass cp{oc.hi[o], lo < oc.hi[o], c.tile_perm.p, cls + size_t(o) * ts, cls + size_t(ncls + o) * ts,
-                         cls + size_t(2 * ncls + o) * ts, cls + size_t(3 * ncls) * ts + o};
-      const GemmShape sh = gemm_shape(c, sc, g, ntiles, bf16, KP, KPb, &cp);
-      run_gemm(c, sc, g, ntiles, bf16, KP, KPb, sh, c.L.p, &cp);
+      pass.push_back(ClassPass{oc.hi[o], lo < oc.hi[o], c.tile_perm.p, cls + size_t(o) * ts, cls + size_t(ncls + o) * ts,
+                               cls + size_t(2 * ncls + o) * ts, cls + size_t(3 * ncls) * ts + o});
+      shape.push_back(gemm_shape(c, sc, g, ntiles, bf16, KP, KPb, &pass.back()));
+      all_sk = all_sk && shape.back().sk;
+    }
+    // stream-K launches leave their segments for one sum over the classes
+    ClassSums sums{};
+    int rows = 0;
+    int64_t seg = 0;
+    for (size_t k = 0; all_sk && k < pass.size(); k++) {
+      const Geom go = geom(pass[k].p);
+      sums.c[k].base = seg;
+      seg += int64_t(sk_groups(c.cfg.device, ceil_div(go.R, shape[k].rtb)) + ntiles) * kTileN * g.PP;
+      rows = std::max(rows, std::min(g.PP, 16 * go.R));
+    }
+    if (all_sk) c.m2l_part.ensure(size_t(seg));
+    for (size_t k = 0; k < pass.size(); k++)
+      run_gemm(c, sc, g, ntiles, bf16, KP, KPb, shape[k], c.L.p, &pass[k], all_sk ? &sums : nullptr);
+    if (all_sk) {
+      hipLaunchKernelGGL(k_sk_combine_classes, dim3(ceil_div(int64_t(kTileN) * rows, 256), ntiles), dim3(256), 0, s,
+                         g.PP, rows, ntiles, sums, c.tiles.p, c.tiles.p + ts, c.tiles.p + 4 * ts, c.m2l_part.p, c.L.p);
+      XF_LAUNCH();
     }
     return;
   }
