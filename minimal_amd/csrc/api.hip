@@ -211,6 +211,8 @@ void run_passes(Ctx &c) {
   // multipoles are first read (join_upward)
   auto launch_upward = [&c] {
     if (c.have_M) return;  // launched first, or a repeated traversal
+    // created by the first evaluation: a context for sums alone never needs it
+    if (!c.s2) XF_HIP(hipStreamCreateWithFlags(&c.s2, hipStreamNonBlocking));
     XF_HIP(hipStreamWaitEvent(c.s2, c.ev[1], 0));
     do_upward(c, c.s2, c.ev[7]);
     c.upward_pending = true;
@@ -247,7 +249,7 @@ void do_passes(Ctx &c) {
   } catch (...) {
     // what the other streams still run reads this context's tree
     (void)hipStreamSynchronize(c.s1);
-    (void)hipStreamSynchronize(c.s2);
+    if (c.s2) (void)hipStreamSynchronize(c.s2);
     c.upward_pending = false;
     throw;
   }
@@ -317,7 +319,7 @@ int exafmm_create(const exafmm_config *cfg, exafmm_ctx **out) {
       if (serial && serial[0] == '1')
         c.s1 = c.s2 = c.s0;
       else
-        for (hipStream_t *q : {&c.s1, &c.s2}) XF_HIP(hipStreamCreateWithFlags(q, hipStreamNonBlocking));
+        XF_HIP(hipStreamCreateWithFlags(&c.s1, hipStreamNonBlocking));
       for (auto &e : c.ev) XF_HIP(hipEventCreate(&e));
     } catch (...) {
       delete h;

@@ -240,7 +240,7 @@ struct Lists {
 struct Ctx {
   exafmm_config cfg{};
   int P = 10, NT = 55;
-  // main stream; P2P and the write-back; the upward pass of an evaluation
+  // main stream; P2P and the write-back; the upward pass of an evaluation (created by the first)
   hipStream_t s0 = nullptr, s1 = nullptr, s2 = nullptr;
   hipEvent_t ev[16] = {};
   std::string last_error;
