@@ -28,6 +28,7 @@
 
 #include "fmm_internal.h"
 #include "fmm_ops.h"
+#include "sk_schedule.h"
 
 namespace xf {
 using namespace xfd;
@@ -1074,9 +1075,10 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_bf16x3(GemmIn g, const int
 }
 
 // Stream-K schedule: the tiles' key slots, in tile order (slot tbase[t] + u
-// is key u of tile t; S slots in all), are split evenly over the gridDim.x
-// workgroups of one persistent launch (one per CU and row block).  Workgroup
-// w takes slots [w S / G, (w + 1) S / G); each tile it touches gives one FP32
+// is key u of tile t; S slots in all), are split evenly over the W = min(gridDim.x,
+// S) active workgroups of one persistent launch (one per CU and row block;
+// sk_schedule.h).  Workgroup w takes slots [w S / W, (w + 1) S / W), at least
+// one, and the others return; each tile it touches gives one FP32
 // partial of the tile's locals, stored by tile column in segment w + t of
 // Lseg, and k_sk_combine adds a tile's segments in workgroup order.  Every
 // workgroup gets the same number of slots, so none waits on a straggler.  A
@@ -1085,10 +1087,12 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_bf16x3(GemmIn g, const int
 // tstart[t] where tile t's run of them starts in the order-grouped slots, and
 // Sdev their total.
 //
-// First slot of workgroup w of W (slots are counted in ints), in a scalar
+// First slot of active workgroup w (slots are counted in ints), in a scalar
 // register, as is everything the schedule derives from it: the GEMM body has
 // no vector registers to spare.
-__device__ inline int sk_first(int64_t w, int64_t S, int64_t W) { return __builtin_amdgcn_readfirstlane(int(w * S / W)); }
+__device__ inline int sk_first(int64_t w, int64_t S, int64_t W) {
+  return __builtin_amdgcn_readfirstlane(int(sk_slot(w, S, W)));
+}
 
 template <class F>
 __device__ __attribute__((always_inline)) inline void sk_segments(int ntiles, int s0, int s1, int off,
@@ -1120,10 +1124,10 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_bf16x3_sk(GemmIn g, const 
                                                                 const int *__restrict__ Sdev,
                                                                 const unsigned char *__restrict__ tkp, int G, int ring,
                                                                 float *__restrict__ Lseg) {
-  const int W = gridDim.x, w = blockIdx.x;
   if (Sdev) S = *Sdev;  // one order's slot count, summed on the device
+  const int W = sk_active(gridDim.x, S), w = blockIdx.x;
+  if (w >= W) return;
   const int s0 = sk_first(w, S, W), s1 = sk_first(w + 1, S, W);
-  if (s0 >= s1) return;
   sk_segments(ntiles, s0, s1, 0, tbase, g.tU, [&](int t, int ub, int n) {
     m2l_bf16x3_body<RH, VAR>(g, t, blockIdx.y, tstart[t] + ub, n, true, PP, RT, RTB, K32, KP, op, tkp, G, ring,
                         Lseg + (w + t) * int64_t(kTileN) * PP, nullptr);
@@ -1143,9 +1147,8 @@ __device__ inline void sk_combine(int64_t e, int PP, int rows, int ncol, int64_t
                                   double *__restrict__ L) {
   const int per = rows / VEC, col = int(e / per), row = int(e % per) * VEC;
   if (col >= ncol || n == 0) return;
-  // workgroup of slot s: the largest w with w S / W <= s
-  auto wg_of = [&](int64_t sl) { return int(((sl + 1) * W - 1) / S); };
-  const int wf = wg_of(b), wl = wg_of(b + n - 1);
+  W = sk_active(W, S);
+  const int wf = sk_owner(b, S, W), wl = sk_owner(b + n - 1, S, W);
   typedef float vec __attribute__((ext_vector_type(VEC)));
   const int64_t step = int64_t(kTileN) * PP;
   const float *p = Lseg + (wf + seg0) * step + int64_t(col) * PP + row;
@@ -1222,9 +1225,8 @@ __global__ void __launch_bounds__(256) k_sk_combine_classes(int PP, int rows, in
     const int n = c.cnt[t];
     if (n == 0 || row >= c.rows) continue;
     const int64_t b = c.pre[t], S = *c.tot;
-    auto wg_of = [&](int64_t sl) { return int(((sl + 1) * c.W - 1) / S); };
-    const int wf = wg_of(b);
-    nseg[k] = wg_of(b + n - 1) - wf + 1;
+    const int W = sk_active(c.W, S), wf = sk_owner(b, S, W);
+    nseg[k] = sk_owner(b + n - 1, S, W) - wf + 1;
     p[k] = Lseg + c.base + (wf + int64_t(t)) * step + int64_t(col) * PP + row;
     v[k][0] = p[k][0];
     if (nseg[k] > 1) v[k][1] = p[k][step];
@@ -1260,9 +1262,9 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_bf16x3_grouped(const Group
                                                                      const int *__restrict__ sstart, int nprob, int PP,
                                                                      int RT, int RTB, int K32, int KP, int pl, int G,
                                                                      int ring, float *__restrict__ Lseg) {
-  const int W = gridDim.x, w = blockIdx.x, S = sstart[nprob];
+  const int S = sstart[nprob], W = sk_active(gridDim.x, S), w = blockIdx.x;
+  if (w >= W) return;
   const int s0 = sk_first(w, S, W), s1 = sk_first(w + 1, S, W);
-  if (s0 >= s1) return;
   const OrderPass op{pl, RT, K32, nullptr};
   for (int i = __builtin_amdgcn_readfirstlane(group_of(sstart, nprob, s0)); i < nprob && sstart[i] < s1; i++) {
     const GroupGemm &q = gr[i];
