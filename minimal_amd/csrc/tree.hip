@@ -14,6 +14,7 @@
 #include <algorithm>
 
 #include "fmm_internal.h"
+#include "grow.h"
 
 namespace xf {
 
@@ -792,8 +793,6 @@ void tree_build(Ctx &c) {
   t.hist.ensure(kHistTotal);
   static_assert(hist_off(kHistLevels) % 4 == 0, "level 7 is cleared 16 bytes at a time");
   int4 *hist7 = reinterpret_cast<int4 *>(t.hist.p + hist_off(kHistLevels));
-  for (Buf<int> *a : {&t.cbeg, &t.ccnt, &t.cparent, &t.clevel}) a->ensure(1);  // the root; the rest below
-  t.cx.ensure(1);
 
   // forest: per-problem roots under the problem-index cells
   const bool forest = c.forest_n > 0;
@@ -807,21 +806,15 @@ void tree_build(Ctx &c) {
     // nodes of level l are children of level-(l-1) nodes holding > ncrit bodies
     return l > lforce ? std::min(u, ub_split) : u;  // (a forest's top levels split unconditionally)
   };
-  auto ensure_cells = [&](int Ds) {
+  auto cells_bound = [&](int Ds) {
     int64_t tot = 0;
     for (int l = 0; l <= Ds; l++) tot += level_bound(l);
-    if (t.cx.cap < size_t(tot) || t.leaves.cap < size_t(tot)) {
-      t.cx.ensure(tot);
-      t.cbeg.ensure(tot);
-      t.ccnt.ensure(tot);
-      t.cchild.ensure(tot);
-      t.cnch.ensure(tot);
-      t.cparent.ensure(tot);
-      t.clevel.ensure(tot);
-      t.coct.ensure(tot);
-      t.leaves.ensure(tot);
-    }
     return tot;
+  };
+  // (true if an array was allocated again: the root cell in it is lost)
+  auto ensure_cells = [&](int Ds) {
+    return ensure_all(size_t(cells_bound(Ds)), t.cx, t.cbeg, t.ccnt, t.cchild, t.cnch, t.cparent, t.clevel, t.coct,
+                      t.leaves);
   };
   const bool speculate = t.ds_hint >= 0;
   int Ds = t.ds_hint;
@@ -908,9 +901,8 @@ void tree_build(Ctx &c) {
   }
 
   // level-by-level split
-  double4 *const cx0 = t.cx.p;
-  const int64_t ubtot = ensure_cells(Ds);
-  if (t.cx.p != cx0) {  // (a first build deeper than the histogram: the root again)
+  const int64_t ubtot = cells_bound(Ds);
+  if (ensure_cells(Ds)) {  // (a first build deeper than the histogram: the root again)
     const RootOut again{root,    t.misc.p, t.lcount.p, t.lstart_d.p, t.cx.p, t.cbeg.p, t.ccnt.p, t.cparent.p,
                         t.clevel.p, n};
     hipLaunchKernelGGL(k_root, dim3(1), dim3(1), 0, s, again);
