@@ -83,6 +83,9 @@ float elapsed(Ctx &c, int a, int b) {
 void set_bodies(Ctx &c, exafmm_body *b, int64_t n, int on_device) {
   if (c.graph_locks) fail(EXAFMM_ERR_STATE, "the context is held by a graph (exafmm_graph_destroy it first)");
   if (!b || n < 1) fail(EXAFMM_ERR_ARG, "need at least one body");
+  // From here on the last tree's arrays change: if this call fails, the later
+  // passes find no tree instead of sizes and arrays of two different sets.
+  c.t.built = c.have_M = c.have_L = c.lists.valid = false;
   c.t.n = n;
   c.forest_n = 0;  // one problem unless exafmm_evaluate_forest says otherwise
   if (on_device) {
@@ -112,8 +115,6 @@ void do_build(Ctx &c) {
   rec(c, 0, c.s0);
   tree_build(c);
   rec(c, 1, c.s0);
-  c.have_M = c.have_L = false;
-  c.lists.valid = false;
 }
 
 void do_upward(Ctx &c, hipStream_t s, hipEvent_t wide = nullptr) {
@@ -130,6 +131,7 @@ void do_lists(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
   if (tc.P != sc.P) fail(EXAFMM_ERR_ARG, "target and source contexts differ in P");
   if (tc.cfg.images != sc.cfg.images || (tc.cfg.images > 0 && &tc != &sc))
     fail(EXAFMM_ERR_UNSUPPORTED, "a periodic horizontal pass needs source == target");
+  tc.lists.valid = tc.have_L = false;  // until this pass has made them
   rec(tc, 11, tc.s0);
   traverse(tc, sc, after_kernels);
   rec(tc, 12, tc.s0);
