@@ -228,7 +228,7 @@ void run_passes(Ctx &c) {
     do_lists(c, c, [&] {
       rec(c, 14, c.s0);
       launch_upward();
-      launch_p2p(c.lists.tot.p + 3);
+      launch_p2p(c.lists.tot.p + kTotFlags);
     });
   }
   do_far(c, c);

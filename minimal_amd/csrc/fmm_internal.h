@@ -128,13 +128,16 @@ struct HostBuf {
 constexpr int kPinLevelMax = 0;   // 9: flags, largest prefix population of levels 1..8
 constexpr int kPinLevels = 16;    // kMaxLevel + 2 level sizes
 constexpr int kPinMisc = 48;      // 19: tree flags and counters
-constexpr int kPinTot = 72;       // 8: list totals and flags
+constexpr int kPinTot = 72;       // 8: list totals, key count and flags (Lists::tot)
 constexpr int kPinPlan = 80;      // 4: M2L slots, tiles, cells in tiles, key set differs from the operators'
 constexpr int kPinInts = 96;
 // traversal flag bits that make the pass repeat: list capacity, key table
 // full, small work queue overflow
 constexpr int kListQueue = 64;
 constexpr int kListRetry = 1 | 8 | kListQueue;
+// ints of Lists::tot behind the three 64-bit totals
+constexpr int kTotKeys = 6, kTotFlags = 7;
+static_assert(kPinTot % 2 == 0, "64-bit totals");
 static_assert(kPinLevels + kMaxLevel + 2 <= kPinMisc && kPinMisc + 19 <= kPinTot, "pinned slots overlap");
 
 inline int ceil_div(int64_t a, int64_t b) { return int((a + b - 1) / b); }
@@ -223,7 +226,7 @@ struct Lists {
   Buf<int> p2p;               // source cell
   Buf<int> out_beg, out_cnt;  // traversal hand-down lists
   Buf<int> out;
-  Buf<int> tot;               // device totals [m2l, p2p, out], overflow flags
+  Buf<int> tot;               // three 64-bit totals [m2l, p2p, out], then keys and flags (kTot*)
   int64_t cap_m2l = 0, cap_p2p = 0, cap_out = 0;
   int64_t nm2l = 0, np2p = 0;
   bool large_queue = false;  // a target overflowed the traversal's small queue
@@ -341,7 +344,7 @@ void tree_export_cells(Ctx &c, exafmm_cell *out);     // reference numbering
 void tree_ref_order(Ctx &c, std::vector<int64_t> &bfs2ref, std::vector<int64_t> &ref2bfs);
 // Dual-tree traversal into the interaction lists.  after_kernels (if set)
 // runs once per pass, right after the pass's traversal kernels are enqueued
-// on s0 and before the host reads the totals (flags in lists.tot[3]; a pass
+// on s0 and before the host reads the totals (flags in lists.tot[kTotFlags]; a pass
 // with kListRetry bits set is repeated after s1 has drained).
 void traverse(Ctx &tgt, const Ctx &src, const std::function<void()> &after_kernels = {});
 // wide (if given) is recorded behind the P2M and the levels that fill the device

@@ -26,6 +26,7 @@
 #include <algorithm>
 
 #include "fmm_internal.h"
+#include "list_capacity.h"
 
 namespace xf {
 
@@ -56,7 +57,8 @@ struct TravArgs {
   int *m2l_cnt, *m2l_beg;
   int2 *m2l;
   int *p2p_cnt, *p2p_beg, *p2p;
-  int *flags, *tot;
+  int *flags;
+  unsigned long long *tot;
   int64_t cap_m2l, cap_p2p, cap_out;
   // translation keys
   unsigned long long *hslots;
@@ -247,7 +249,8 @@ template <int QCAP>
 __global__ void __launch_bounds__(kTravWaves *kWave) k_traverse(TravArgs a) {
   __shared__ int queue[kTravWaves][QCAP];
   __shared__ int sm[kTravWaves][kStageM2L], sp[kTravWaves][kStageP2P], so[kTravWaves][kStageOut];
-  __shared__ int cnt[kTravWaves][3], base[3];
+  __shared__ int cnt[kTravWaves][3];
+  __shared__ long long base[3];
   const int lane = threadIdx.x & (kWave - 1);
   const int w = threadIdx.x / kWave;
   const int t = blockIdx.x * kTravWaves + w;
@@ -288,26 +291,27 @@ __global__ void __launch_bounds__(kTravWaves *kWave) k_traverse(TravArgs a) {
     for (int i = 0; i < kTravWaves; i++) s += cnt[i][threadIdx.x];
     const int64_t cap = threadIdx.x == 0 ? a.cap_m2l : threadIdx.x == 1 ? a.cap_p2p : a.cap_out;
     int b0 = 0;
-    if (s) {
-      b0 = atomicAdd(a.tot + threadIdx.x, s);
-      if (int64_t(b0) + s > cap) atomicOr(a.flags, 1);
+    if (s) {  // counted in 64 bits: a total past 2^31 entries raises the flag too
+      const unsigned long long first = atomicAdd(a.tot + threadIdx.x, (unsigned long long)s);
+      if (list_overflows(first, s, cap)) atomicOr(a.flags, 1);
+      b0 = list_place(first, cap);
     }
     base[threadIdx.x] = b0;
   }
   __syncthreads();
   if (!in) return;
-  int bm = base[0], bp = base[1], bo = base[2];
+  long long bm = base[0], bp = base[1], bo = base[2];
   for (int i = 0; i < w; i++) {
     bm += cnt[i][0];
     bp += cnt[i][1];
     bo += cnt[i][2];
   }
   if (lane == 0) {
-    a.m2l_beg[c] = bm;
+    a.m2l_beg[c] = list_place(bm, a.cap_m2l);
     a.m2l_cnt[c] = nm;
-    a.p2p_beg[c] = bp;
+    a.p2p_beg[c] = list_place(bp, a.cap_p2p);
     a.p2p_cnt[c] = np;
-    a.out_beg[c] = bo;
+    a.out_beg[c] = list_place(bo, a.cap_out);
     a.out_cnt[c] = no;
   }
   auto place = [&](int kind, int pos, int entry) {
@@ -354,15 +358,15 @@ __global__ void k_hash_collect(const unsigned long long *__restrict__ slots, int
 
 // M2L entries carry their hash slot out of the traversal; after the keys are
 // sorted the slot becomes the key's rank (the id the operators are stored by).
-// The count is the device total, capped at the list capacity; flags (if
-// given) skip a pass that is repeated or ranked by the radix sort instead.
-// host_tot (if given) receives the totals and flags (pinned memory).
-__global__ void k_entry_ids(int2 *__restrict__ m2l, const int *__restrict__ total, int64_t cap,
+// The count is the device total (tot: Lists::tot), capped at the list
+// capacity; flags (if given) skip a pass that is repeated or ranked by the radix
+// sort instead.  host_tot (if given) receives the totals and flags (pinned memory).
+__global__ void k_entry_ids(int2 *__restrict__ m2l, const int *__restrict__ tot, int64_t cap,
                             const int *__restrict__ slot2id, const int *__restrict__ flags, int *host_tot) {
   if (host_tot && blockIdx.x == 0 && threadIdx.x < 8)
-    __hip_atomic_store(host_tot + threadIdx.x, total[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(host_tot + threadIdx.x, tot[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   if (flags && (*flags & (kListRetry | 32))) return;
-  const int64_t n = min(int64_t(*total), cap);
+  const int64_t n = min(*reinterpret_cast<const int64_t *>(tot), cap);
   for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256)
     m2l[i].y = slot2id[m2l[i].y];
 }
@@ -422,12 +426,13 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
   Lr.tot.ensure(8);
   tc.pin_i.ensure(kPinInts);
   tc.L.ensure(size_t(nc) * tc.P * tc.P);
-  if (Lr.cap_m2l < 200 * nc) Lr.cap_m2l = 200 * nc;
-  if (Lr.cap_p2p < 96 * nc) Lr.cap_p2p = 96 * nc;
-  if (Lr.cap_out < 96 * nc) Lr.cap_out = 96 * nc;
+  Lr.cap_m2l = std::max(Lr.cap_m2l, list_capacity(nc, 200));
+  Lr.cap_p2p = std::max(Lr.cap_p2p, list_capacity(nc, 96));
+  Lr.cap_out = std::max(Lr.cap_out, list_capacity(nc, 96));
   if (keys && Lr.hcap == 0) Lr.hcap = 1 << 16;
 
   int tot[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  uint64_t total[3] = {0, 0, 0};
   bool done = false;
   for (int attempt = 0; attempt < 5; attempt++) {
     Lr.m2l.ensure(Lr.cap_m2l);
@@ -455,8 +460,8 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
     a.p2p_cnt = Lr.p2p_cnt.p;
     a.p2p_beg = Lr.p2p_beg.p;
     a.p2p = Lr.p2p.p;
-    a.flags = Lr.tot.p + 3;
-    a.tot = Lr.tot.p;
+    a.flags = Lr.tot.p + kTotFlags;
+    a.tot = reinterpret_cast<unsigned long long *>(Lr.tot.p);
     a.cap_m2l = Lr.cap_m2l;
     a.cap_p2p = Lr.cap_p2p;
     a.cap_out = Lr.cap_out;
@@ -487,28 +492,29 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
     if (after_kernels) after_kernels();
     if (keys) {
       // distinct translation keys out of the hash table (discarded if the
-      // pass has to be repeated), counted into tot[6]
+      // pass has to be repeated), counted into tot[kTotKeys]
       Lr.keys.ensure(size_t(Lr.hcap) * 2);
       Lr.kscratch.ensure(size_t(Lr.hcap) * 2 + 8);
       Lr.slot2id.ensure(Lr.hcap);
       hipLaunchKernelGGL(k_hash_collect, dim3(ceil_div(Lr.hcap, 256)), dim3(256), 0, s, Lr.hslots.p, Lr.hcap,
-                         Lr.keys.p + Lr.hcap, Lr.kscratch.p, Lr.tot.p + 6);
+                         Lr.keys.p + Lr.hcap, Lr.kscratch.p, Lr.tot.p + kTotKeys);
       XF_LAUNCH();
       // The usual small key set is ranked, and the entries renumbered,
       // before the totals are read, so the read overlaps them (counts from
       // the device; a repeated pass redoes it all, a set above kRankMax is
       // flagged and sorted below).
       hipLaunchKernelGGL(k_key_rank, dim3(std::min(Lr.hcap, kRankMax) / kWave), dim3(1024), 0, s, Lr.keys.p + Lr.hcap,
-                         Lr.kscratch.p, Lr.tot.p + 6, Lr.keys.p, Lr.slot2id.p, Lr.tot.p + 3);
+                         Lr.kscratch.p, Lr.tot.p + kTotKeys, Lr.keys.p, Lr.slot2id.p, Lr.tot.p + kTotFlags);
       XF_LAUNCH();
       hipLaunchKernelGGL(k_entry_ids, dim3(int(std::min<int64_t>(ceil_div(Lr.cap_m2l, 256), 4096))), dim3(256), 0, s,
-                         Lr.m2l.p, Lr.tot.p, Lr.cap_m2l, Lr.slot2id.p, Lr.tot.p + 3, tc.pin_i.p + kPinTot);
+                         Lr.m2l.p, Lr.tot.p, Lr.cap_m2l, Lr.slot2id.p, Lr.tot.p + kTotFlags, tc.pin_i.p + kPinTot);
       XF_LAUNCH();
     }
     if (!keys) XF_HIP(hipMemcpyAsync(tc.pin_i.p + kPinTot, Lr.tot.p, sizeof(tot), hipMemcpyDeviceToHost, s));
     stream_wait(s);
     std::copy(tc.pin_i.p + kPinTot, tc.pin_i.p + kPinTot + 8, tot);
-    const int flags = tot[3];
+    std::memcpy(total, tot, sizeof(total));
+    const int flags = tot[kTotFlags];
     // work started by after_kernels ends before a repeated pass resets the flags
     if (after_kernels && (flags & kListRetry)) stream_wait(tc.s1);
     if (flags & 4) fail(EXAFMM_ERR_CAPACITY, "traversal work queue overflow (pairs per target cell > 2048)");
@@ -517,18 +523,21 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
       Lr.large_queue = true;
       continue;
     }
-    if (flags & 1) {  // list capacity: retry with the exact totals
-      Lr.cap_m2l = std::max<int64_t>(Lr.cap_m2l * 2, tot[0]);
-      Lr.cap_p2p = std::max<int64_t>(Lr.cap_p2p * 2, tot[1]);
-      Lr.cap_out = std::max<int64_t>(Lr.cap_out * 2, tot[2]);
+    if (flags & 1) {  // list capacity
+      int64_t *const cap[3] = {&Lr.cap_m2l, &Lr.cap_p2p, &Lr.cap_out};
+      for (int k = 0; k < 3; k++) {
+        const int64_t n = list_grow(*cap[k], total[k]);
+        if (!n) fail(EXAFMM_ERR_CAPACITY, "more than 2^31 - 1 entries of one kind of interaction list");
+        *cap[k] = n;
+      }
       continue;
     }
     if (flags & 8) {  // key table full
       Lr.hcap *= 4;
       continue;
     }
-    Lr.nm2l = tot[0];
-    Lr.np2p = tot[1];
+    Lr.nm2l = int64_t(total[0]);
+    Lr.np2p = int64_t(total[1]);
     done = true;
     break;
   }
@@ -538,8 +547,8 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
   if (keys) {
     unsigned long long *k1 = Lr.keys.p + Lr.hcap, *k2 = Lr.keys.p;
     int *v1 = Lr.kscratch.p, *v2 = Lr.kscratch.p + Lr.hcap;
-    const int nk = tot[6];
-    if (tot[3] & 32) {  // more keys than k_key_rank holds
+    const int nk = tot[kTotKeys];
+    if (tot[kTotFlags] & 32) {  // more keys than k_key_rank holds
       radix_sort_pairs(k1, v1, k2, v2, nk, 0, 64, T.rs_hist, s);
       hipLaunchKernelGGL(k_slot_ids, dim3(ceil_div(std::max(nk, 1), 256)), dim3(256), 0, s, v1, nk, Lr.slot2id.p);
       XF_LAUNCH();
