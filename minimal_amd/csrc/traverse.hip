@@ -37,6 +37,10 @@ constexpr int kQSmall = 768, kQCap = 2048;
 // list entries staged per target; a longer list is walked a second time,
 // straight into place
 constexpr int kStageM2L = 256, kStageP2P = 128, kStageOut = 256;
+// Passes at most: lists that are cut short at every level double the hand-down
+// list's room each time (96 entries per cell; a target hands down fewer than
+// kQCap), and the large queue and a larger key table may take one each.
+constexpr int kListPasses = 16;
 constexpr unsigned long long kEmpty = ~0ull;
 
 struct TravArgs {
@@ -219,7 +223,8 @@ __device__ __attribute__((always_inline)) inline bool walk(const TravArgs &a, in
 }
 
 // Initial pairs of target c: handed down from the parent, or (root, root).
-// Returns their number, -1 if they overflow the queue.
+// Returns their number, -1 if they overflow the queue; 0 if the parent's list
+// did not fit (its launch raised the flag that repeats the pass with more room).
 template <int QCAP>
 __device__ inline int start_pairs(const TravArgs &a, int c, int lane, int *q) {
   int tail;
@@ -227,7 +232,8 @@ __device__ inline int start_pairs(const TravArgs &a, int c, int lane, int *q) {
     const int par = a.cparent[c];
     const int ib = a.in_beg[par];
     tail = a.in_cnt[par];
-    if (tail > QCAP || int64_t(ib) + tail > a.cap_out) return -1;
+    if (int64_t(ib) + tail > a.cap_out) return 0;
+    if (tail > QCAP) return -1;
     for (int i = lane; i < tail; i += kWave) q[i] = a.in[ib + i];
   } else if (a.self_start) {
     tail = 1;
@@ -434,7 +440,7 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
   int tot[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   uint64_t total[3] = {0, 0, 0};
   bool done = false;
-  for (int attempt = 0; attempt < 5; attempt++) {
+  for (int attempt = 0; attempt < kListPasses; attempt++) {
     Lr.m2l.ensure(Lr.cap_m2l);
     Lr.p2p.ensure(Lr.cap_p2p);
     Lr.out.ensure(Lr.cap_out);
@@ -519,29 +525,27 @@ void traverse(Ctx &tc, const Ctx &sc, const std::function<void()> &after_kernels
     if (after_kernels && (flags & kListRetry)) stream_wait(tc.s1);
     if (flags & 4) fail(EXAFMM_ERR_CAPACITY, "traversal work queue overflow (pairs per target cell > 2048)");
     if (flags & 16) fail(EXAFMM_ERR_CAPACITY, "M2L offset out of key range");
-    if (flags & kListQueue) {  // from here on with the large queue
-      Lr.large_queue = true;
-      continue;
-    }
-    if (flags & 1) {  // list capacity
+    // what the next pass needs more of (a pass cut short shows lower bounds)
+    if (flags & kListQueue) Lr.large_queue = true;
+    if (flags & 1) {
       int64_t *const cap[3] = {&Lr.cap_m2l, &Lr.cap_p2p, &Lr.cap_out};
       for (int k = 0; k < 3; k++) {
         const int64_t n = list_grow(*cap[k], total[k]);
         if (!n) fail(EXAFMM_ERR_CAPACITY, "more than 2^31 - 1 entries of one kind of interaction list");
         *cap[k] = n;
       }
-      continue;
     }
-    if (flags & 8) {  // key table full
+    if (flags & 8) {
+      if (Lr.hcap >= 1 << 24) fail(EXAFMM_ERR_CAPACITY, "more than 2^23 distinct M2L translations");
       Lr.hcap *= 4;
-      continue;
     }
+    if (flags & kListRetry) continue;
     Lr.nm2l = int64_t(total[0]);
     Lr.np2p = int64_t(total[1]);
     done = true;
     break;
   }
-  if (!done) fail(EXAFMM_ERR_CAPACITY, "interaction lists or key table still full after 5 passes");
+  if (!done) fail(EXAFMM_ERR_CAPACITY, "interaction lists or key table still full");
   Lr.valid = true;
   Lr.nkeys = 0;
   if (keys) {
