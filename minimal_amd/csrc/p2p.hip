@@ -375,15 +375,12 @@ __global__ void __launch_bounds__(kP2PWaves *kWave) k_p2p32_grouped(const GroupT
 // caller subtracts), pairs at zero distance skipped.  The hardware's 1/sqrt
 // (about 2^-23 relative) takes one third-order step
 //   e = 1 - r^2 y^2,  y += y e (1/2 + 3/8 e)
-// (remainder 5/16 e^3, below 2^-60), five FP64 operations where a divide and
-// a square root expand to about forty.  STEP2: 1/r^2 is y^2 after a Newton
-// step of its own, two operations more; y^2 alone carries twice y's rounding,
-// which shows where few sources are added (1,000 x 1,000 bodies, F against the
-// exact sum: 2.5e-16, with the step 2.1e-16, with a divide and a root 2.2e-16;
-// over more sources the longer chains of additions that lanes over sources
-// replace weigh more).  Squared distances outside [2^-900, 2^900) -- zero,
+// (remainder 5/16 e^3, below 2^-60), and 1/r^2 is y^2 after a Newton step of its
+// own: seven FP64 operations where a divide and a square root expand to about
+// forty.  The rounding is that of the divide and the root: in units of 2^-53, rms,
+// 1/r 0.46 (0.46 with them), 1/r^2 0.44 (0.44; 1.03 without its step), 1/r^3 0.77
+// (0.88; 1.52 without).  Squared distances outside [2^-900, 2^900) -- zero,
 // overflow, NaN -- take the plain divide and root.
-template <bool STEP2>
 __device__ inline void p2p64_pair(double dx, double dy, double dz, double q, double &pot, double &ax, double &ay,
                                   double &az) {
   const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
@@ -392,7 +389,7 @@ __device__ inline void p2p64_pair(double dx, double dy, double dz, double q, dou
   const double e = fma(-t, y, 1.0);
   y = fma(y * e, fma(e, 0.375, 0.5), y);
   double y2 = y * y;
-  if (STEP2) y2 = fma(y2, fma(-r2, y2, 1.0), y2);
+  y2 = fma(y2, fma(-r2, y2, 1.0), y2);
   const unsigned hi = unsigned(__double2hiint(r2));
   if (hi - (123u << 20) >= (1800u << 20)) {
     y2 = r2 != 0.0 ? 1.0 / r2 : 0.0;
@@ -445,7 +442,7 @@ __device__ __attribute__((always_inline)) inline void p2p64_block(int t0, int tc
       const double sx = X.x + L.dlx[e], sy = X.y + L.dly[e], sz = X.z + L.dlz[e];  // the entry's image shift
 #pragma unroll
       for (int t = 0; t < TC; t++)
-        p2p64_pair<false>(xt[t] - sx, yt[t] - sy, zt[t] - sz, X.w, ap[t], ax[t], ay[t], az[t]);
+        p2p64_pair(xt[t] - sx, yt[t] - sy, zt[t] - sz, X.w, ap[t], ax[t], ay[t], az[t]);
     }
   }
   constexpr int kLow = kWave / pow2ceil<TC>();
@@ -542,7 +539,7 @@ constexpr int kDirectGroups = 2048;  // workgroups aimed at: eight per CU
 
 // Sums of targets t0 .. t0 + tc - 1 over the sources first + lane, + stride, ...
 // below s1: component lane % (64 / TC) of target lane / (64 / TC).
-template <int TC, bool STEP2>
+template <int TC>
 __device__ __attribute__((always_inline)) inline double direct_block(const exafmm_body *__restrict__ t, int tc,
                                                                      const exafmm_body *__restrict__ s, int64_t s0,
                                                                      int64_t s1, int64_t stride, int lane) {
@@ -559,7 +556,7 @@ __device__ __attribute__((always_inline)) inline double direct_block(const exafm
     const double sx = s[j].X[0], sy = s[j].X[1], sz = s[j].X[2], q = s[j].q;
 #pragma unroll
     for (int i = 0; i < TC; i++)
-      p2p64_pair<STEP2>(xt[i] - sx, yt[i] - sy, zt[i] - sz, q, ap[i], ax[i], ay[i], az[i]);
+      p2p64_pair(xt[i] - sx, yt[i] - sy, zt[i] - sz, q, ap[i], ax[i], ay[i], az[i]);
   }
   return p2p_lane_total<TC>(ap, ax, ay, az, lane);
 }
@@ -577,7 +574,7 @@ __global__ void __launch_bounds__(kDirectWaves *kWave) k_direct(const exafmm_bod
   const int tc = int(min(int64_t(kDirectTC), nt - t0));
   constexpr int kLow = kWave / kDirectTC;
   const int i = lane / kLow, comp = lane % kLow;
-  const double v = direct_block<kDirectTC, false>(t + t0, tc, s, s0, s1, kWave, lane);
+  const double v = direct_block<kDirectTC>(t + t0, tc, s, s0, s1, kWave, lane);
   if (comp < 4 && i < tc) part[(share * nt + t0 + i) * 4 + comp] = v;
 }
 
@@ -596,7 +593,7 @@ __global__ void __launch_bounds__(kDirectOneWaves *kWave) k_direct_one(exafmm_bo
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int64_t t0 = int64_t(blockIdx.x) * kDirectOneTC;
   const int tc = int(min(int64_t(kDirectOneTC), nt - t0));
-  const double v = direct_block<kDirectOneTC, true>(t + t0, tc, s, w * kWave, ns, kDirectOneWaves * kWave, lane);
+  const double v = direct_block<kDirectOneTC>(t + t0, tc, s, w * kWave, ns, kDirectOneWaves * kWave, lane);
   if (lane % kLow < 4) red[w][lane / kLow * 4 + lane % kLow] = v;
   __syncthreads();
   const int i = threadIdx.x / 4, comp = threadIdx.x % 4;

@@ -1,0 +1,52 @@
+"""Rounding of one FP64 interaction, in the FP64 P2P and in both forms of the
+direct sum (8,192 sources and fewer, more): one charged source at the origin
+among sources without charge, which add exact zeros, and targets on an axis at
+distances of 20 bits, so that dX and r^2 are exact.
+
+Bars, rms over the targets in units of 2^-53 relative to the exact value.  A
+correctly rounded operation leaves 0.5 at most, about 0.4 rms; 1/r comes from a
+divide and a root (or a step as exact), F = dX q/r^3 from that, 1/r^2 and two
+products.  p: sqrt(2) x 0.5 = 0.71.  F: sqrt(0.5 + 2 x 0.25 + 0.25) = 1.12 with
+the root's and the divide's errors independent, five operations in all.
+"""
+import numpy as np
+import pytest
+
+from minimal_amd import fmm
+from minimal_amd.inputs import BODY_DTYPE
+
+pytestmark = pytest.mark.gpu
+
+
+def _axis(n, seed):
+    rng = np.random.default_rng(seed)
+    b = np.zeros(n, BODY_DTYPE)
+    x = rng.permutation(np.arange(1 << 18, 1 << 20))[:n] * 2.0 ** -20
+    b["X"][:, 0] = x
+    return b
+
+
+def _check(b):
+    x = b["X"][:, 0].astype(np.longdouble)
+    for v, ex, bar in ((b["p"], 1 / x, 0.71), (b["F"][:, 0], -1 / (x * x), 1.12)):
+        e = ((v - ex) / ex * 2.0 ** 53).astype(float)
+        assert np.sqrt(np.mean(e * e)) <= bar, (np.sqrt(np.mean(e * e)), bar)
+
+
+@pytest.mark.parametrize("ns", [100, 8192, 8193, 30000])
+def test_direct(gpu, ns):
+    t = _axis(2000, ns)
+    s = np.zeros(ns, BODY_DTYPE)
+    s["X"][1:, 1] = 0.5 + np.arange(ns - 1) * 2.0 ** -20
+    s["q"][0] = 1.0
+    fmm.FMM().direct(t, s)
+    _check(t)
+
+
+def test_p2p(gpu):
+    b = _axis(1001, 1)
+    b["X"][0] = 0.0
+    b["q"][0] = 1.0
+    f = fmm.FMM(P=4, ncrit=1024, m2l_precision=fmm.PREC_FP64, p2p_precision=fmm.PREC_FP64)
+    f.evaluate(b)
+    _check(b[b["q"] == 0])
