@@ -598,9 +598,16 @@ __global__ void __launch_bounds__(kDirectOneWaves *kWave) k_direct_one(exafmm_bo
   __syncthreads();
   const int i = threadIdx.x / 4, comp = threadIdx.x % 4;
   if (i >= tc) return;
-  double sum = 0.0;
+  // the waves' sums pairwise: one after the other their roundings add up (500 to
+  // 8,192 sources of one sign: p off by 1.0 - 1.2e-16 rms, 0.7 this way)
+  double v16[kDirectOneWaves];
 #pragma unroll
-  for (int k = 0; k < kDirectOneWaves; k++) sum += red[k][threadIdx.x];
+  for (int k = 0; k < kDirectOneWaves; k++) v16[k] = red[k][threadIdx.x];
+#pragma unroll
+  for (int o = kDirectOneWaves / 2; o > 0; o /= 2)
+#pragma unroll
+    for (int k = 0; k < o; k++) v16[k] += v16[k + o];
+  const double sum = v16[0];
   if (comp == 0)
     t[t0 + i].p += sum;
   else

@@ -8,12 +8,19 @@ correctly rounded operation leaves 0.5 at most, about 0.4 rms; 1/r comes from a
 divide and a root (or a step as exact), F = dX q/r^3 from that, 1/r^2 and two
 products.  p: sqrt(2) x 0.5 = 0.71.  F: sqrt(0.5 + 2 x 0.25 + 0.25) = 1.12 with
 the root's and the divide's errors independent, five operations in all.
+
+Sums of one sign: the terms are added per lane, the lanes and waves pairwise, so
+that log2(1,024) = 10 levels of additions of like size remain, whose rounding
+(0.3 rms each of the partial's share, halving with every level below the last)
+sums to less than 0.3 sqrt(1 + 1/2 + 1/4 + ...) = 0.42 units of 2^-53, with those
+of the lanes' chains of at most eight terms and of the final addition below 0.9
+(1e-16).
 """
 import numpy as np
 import pytest
 
 from minimal_amd import fmm
-from minimal_amd.inputs import BODY_DTYPE
+from minimal_amd.inputs import BODY_DTYPE, uniform_cube
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +57,17 @@ def test_p2p(gpu):
     f = fmm.FMM(P=4, ncrit=1024, m2l_precision=fmm.PREC_FP64, p2p_precision=fmm.PREC_FP64)
     f.evaluate(b)
     _check(b[b["q"] == 0])
+
+
+@pytest.mark.parametrize("ns", [1000, 4000, 8192])
+def test_sum_of_one_sign(gpu, ns):
+    f = fmm.FMM()
+    e2 = []
+    for seed in range(8):
+        s = uniform_cube(ns, 100 + seed, "unit_over_n")
+        t = uniform_cube(64, 7 + seed, "sym")
+        f.direct(t, s)
+        d = t["X"][:, None].astype(np.longdouble) - s["X"][None].astype(np.longdouble)
+        p = (s["q"] / np.sqrt((d * d).sum(2))).sum(1)
+        e2.append((((t["p"] - p) / p).astype(float) ** 2).mean())
+    assert np.sqrt(np.mean(e2)) * 2.0 ** 53 <= 0.9
