@@ -412,7 +412,7 @@ __device__ inline void p2p64_pair(double dx, double dy, double dz, double q, dou
 // square root each.
 constexpr int kP2P64TC = 8;
 
-template <int TC>
+template <int TC, bool PERIODIC>
 __device__ __attribute__((always_inline)) inline void p2p64_block(int t0, int tc, int tb, int b0, int nl,
                                                                   const double4 *__restrict__ xs,
                                                                   const int *__restrict__ list,
@@ -435,14 +435,22 @@ __device__ __attribute__((always_inline)) inline void p2p64_block(int t0, int tc
     int nself = 0;
     const int total = p2p_stage_entries(L, list, b0, seg, ne, -1, scbeg, sccnt, make_double4(0, 0, 0, 0), cycle,
                                         lane, &nself);
+    // 3dp/kernel.h:133: dX = Xi - Xj - iX * cycle, the image shift last: bodies
+    // that meet through an image meet exactly as they do there
     int e = 0;
     for (int g = lane; g < total; g += kWave) {
       while (L.pre[e + 1] <= g) e++;
       const double4 X = sxs[L.beg[e] + g - L.pre[e]];
-      const double sx = X.x + L.dlx[e], sy = X.y + L.dly[e], sz = X.z + L.dlz[e];  // the entry's image shift
 #pragma unroll
-      for (int t = 0; t < TC; t++)
-        p2p64_pair(xt[t] - sx, yt[t] - sy, zt[t] - sz, X.w, ap[t], ax[t], ay[t], az[t]);
+      for (int t = 0; t < TC; t++) {
+        double dx = xt[t] - X.x, dy = yt[t] - X.y, dz = zt[t] - X.z;
+        if (PERIODIC) {
+          dx -= L.dlx[e];
+          dy -= L.dly[e];
+          dz -= L.dlz[e];
+        }
+        p2p64_pair(dx, dy, dz, X.w, ap[t], ax[t], ay[t], az[t]);
+      }
     }
   }
   constexpr int kLow = kWave / pow2ceil<TC>();
@@ -457,6 +465,7 @@ __device__ __attribute__((always_inline)) inline void p2p64_block(int t0, int tc
   }
 }
 
+template <bool PERIODIC>
 __global__ void __launch_bounds__(kP2PWaves *kWave) k_p2p64(const int *__restrict__ leaves,
                                                             const int *__restrict__ nleaves,
                                                             const int *__restrict__ cbeg, const int *__restrict__ ccnt,
@@ -481,7 +490,7 @@ __global__ void __launch_bounds__(kP2PWaves *kWave) k_p2p64(const int *__restric
     const int tc = min(per, tn - t0);
 #define XF_P2P64_BLOCK(N)                                                                          \
   case N:                                                                                          \
-    p2p64_block<N>(t0, tc, tb, b0, nl, xs, list, scbeg, sccnt, sxs, cycle, bodies, lds[w]);        \
+    p2p64_block<N, PERIODIC>(t0, tc, tb, b0, nl, xs, list, scbeg, sccnt, sxs, cycle, bodies, lds[w]);        \
     break;
     switch (tc) {
       XF_P2P64_BLOCK(1)
@@ -511,9 +520,10 @@ void p2p_apply(Ctx &tc, const Ctx &sc, hipStream_t s, const int *list_flags) {
   const Lists &L = tc.lists;
   const double cycle = tc.cfg.images > 0 ? tc.cfg.cycle : 0.0;
   if (tc.cfg.p2p_precision == EXAFMM_PREC_FP64) {
-    hipLaunchKernelGGL(k_p2p64, dim3(T.nleaves), dim3(kP2PWaves * kWave), 0, s, T.leaves.p, T.misc.p + 17, T.cbeg.p, T.ccnt.p,
-                       T.xs.p, L.p2p_beg.p, L.p2p_cnt.p, L.p2p.p, S.cbeg.p, S.ccnt.p, S.xs.p, cycle, tc.bodies,
-                       list_flags);
+    auto *k = cycle != 0.0 ? k_p2p64<true> : k_p2p64<false>;
+    hipLaunchKernelGGL(k, dim3(T.nleaves), dim3(kP2PWaves * kWave), 0, s, T.leaves.p, T.misc.p + 17, T.cbeg.p,
+                       T.ccnt.p, T.xs.p, L.p2p_beg.p, L.p2p_cnt.p, L.p2p.p, S.cbeg.p, S.ccnt.p, S.xs.p, cycle,
+                       tc.bodies, list_flags);
   } else {
     auto *k = tc.cfg.p2p_precision == EXAFMM_PREC_FP32_NEWTON ? k_p2p32<true> : k_p2p32<false>;
     hipLaunchKernelGGL(k, dim3(ceil_div(T.nleaves, kP2PWaves)), dim3(kP2PWaves * kWave), 0, s, T.leaves.p,
