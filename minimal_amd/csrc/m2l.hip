@@ -13,6 +13,7 @@
 // harmonic table is zero above degree P-1, so j+n <= P-1); "full" keeps
 // every j+n <= 2P-2.
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 #include "fmm_internal.h"
@@ -40,12 +41,22 @@ using namespace xfd;
 // like degree (m2l64_plan): the low degrees, a handful of long sums, run many
 // pairs at once.  The bound is the LDS reads (two 16-byte reads per eight
 // FP64 FMAs) and, for short lists, the chain of the harmonics.
+// WIDE (trees of very different size): the powers (Rs/Rc)^n and the harmonics of
+// d/Rc leave the range of double while their products stay small.  A pair whose
+// source is the larger cell then takes d in units of Rs:
+//   L~_j^k = (-1)^(j+k) (Rc/Rs)^(j+1) sum M~_n^m I_{j+n}^{m-k}(d/Rs),
+// all factors at most 1; the sum of each pair is scaled by (Rc/Rs)^j as it is
+// added.
 // 118,396 pairs (P = 10, reference truncation): 218 us; the periodic top
 // levels of 131,072 bodies: 154 us.  (A wave per cell, one pair after
 // another, a lane per output with the sign cases and powers in the inner
 // loop: 3,382 and 2,469 us.)
 constexpr int kM2L64Threads = 256, kM2L64Waves = kM2L64Threads / kWave;
 constexpr int kM2L64Lds = 40 * 1024;  // three to four workgroups per CU
+// Largest ratio of a source cell's radius to a target cell's without WIDE: its
+// 15th power is 2^480, and harmonics of degree 30 of a distance as many times
+// the target's radius are above 2^-1000.
+constexpr double kM2L64Wide = 4294967296.0;
 
 struct M2L64Plan {
   int batch;                 // pairs in LDS at a time
@@ -105,7 +116,7 @@ static M2L64Plan m2l64_plan(int P, int fillP) {
 // grid: (cells, shares of a cell's list).  part: partial locals [share][cell]
 // [P^2], added in share order by k_m2l_fp64_sum; null with one share (the
 // sums go straight into L).
-template <int P>
+template <int P, bool WIDE>
 __global__ void __launch_bounds__(kM2L64Threads)
     k_m2l_fp64(int fillP, int ncells, M2L64Plan pl, const double4 *__restrict__ cx,
                const double4 *__restrict__ scx, const int *__restrict__ beg, const int *__restrict__ cnt,
@@ -122,6 +133,7 @@ __global__ void __launch_bounds__(kM2L64Threads)
   double *out = part ? part + (int64_t(blockIdx.y) * ncells + c) * PP : L + int64_t(c) * PP;
   double2 *Is = sm;                      // [batch][IS], element (l, o) at l^2 + l + o
   double2 *Ms = sm + pl.batch * IS;      // [batch][MS]
+  __shared__ double ratio[WIDE ? kM2L64Threads : 1];  // per pair of the batch: min(1, Rc/Rs)
   const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
   // this wave's outputs (a range of degrees), and this lane's output and pair slot
   int j0 = 0, j1 = 0;
@@ -159,12 +171,15 @@ __global__ void __launch_bounds__(kM2L64Threads)
         const int img = e.x & 31;
         const double4 Xs = scx[e.x >> 5];
         // 3dp/kernel.h:200: dX = Xi - Xj - iX * cycle
-        const double dx = (Xc.x - Xs.x - ((img % 3) - 1) * cycle) * inv;
-        const double dy = (Xc.y - Xs.y - (((img / 3) % 3) - 1) * cycle) * inv;
-        const double dz = (Xc.z - Xs.z - ((img / 9) - 1) * cycle) * inv;
+        const double unit = WIDE && Xs.w > Xc.w ? 1.0 / Xs.w : inv;
+        const double dx = (Xc.x - Xs.x - ((img % 3) - 1) * cycle) * unit;
+        const double dy = (Xc.y - Xs.y - (((img / 3) % 3) - 1) * cycle) * unit;
+        const double dz = (Xc.z - Xs.z - ((img / 9) - 1) * cycle) * unit;
         const double r2 = dx * dx + dy * dy + dz * dz;
         const double ir2 = 1.0 / r2;
         double ar = sqrt(ir2), ai = 0.0;
+        if (WIDE && Xs.w > Xc.w) ar *= Xc.w * unit;
+        if (WIDE && m == 0) ratio[b] = Xs.w > Xc.w ? Xc.w * unit : 1.0;
         for (int k = 1; k <= m; k++) {
           const double f = double(2 * k - 1) * ir2;
           const double tr = (ar * dx - ai * dy) * f, ti = (ar * dy + ai * dx) * f;
@@ -193,7 +208,7 @@ __global__ void __launch_bounds__(kM2L64Threads)
       if (bm < kPairs)
         for (int b = bm; b < nb; b += kPairs) {
           const int src = list[b0 + q0 + b].x >> 5;
-          const double x = scx[src].w * inv, x2 = x * x, x4 = x2 * x2;
+          const double Rs = scx[src].w, x = WIDE && Rs > Xc.w ? 1.0 : Rs * inv, x2 = x * x, x4 = x2 * x2;
           double v = M[int64_t(src) * PP + im];
           v *= (nm & 1) ? x : 1.0;
           v *= (nm & 2) ? x2 : 1.0;
@@ -215,6 +230,8 @@ __global__ void __launch_bounds__(kM2L64Threads)
       const int nmax = min(P, fillP - j);
       for (int b = slot; b < nb; b += side) {
         const double2 *Ib = Is + b * IS;
+        const double before[4] = {r0, i0, r1, i1};
+        if (WIDE) r0 = i0 = r1 = i1 = 0.0;
 #pragma unroll
         for (int n = 0; n < P; n++) {
           if (n >= nmax) break;
@@ -234,6 +251,14 @@ __global__ void __launch_bounds__(kM2L64Threads)
             i1 = fma(a.y, y1.x, i1);
             y1 = y0;
           }
+        }
+        if (WIDE) {
+          double f = 1.0;
+          for (int q = 0; q < j; q++) f *= ratio[b];
+          r0 = fma(r0, f, before[0]);
+          i0 = fma(i0, f, before[1]);
+          r1 = fma(r1, f, before[2]);
+          i1 = fma(i1, f, before[3]);
         }
       }
     }
@@ -294,10 +319,12 @@ static void m2l_fp64(Ctx &tc, const Ctx &sc, int ncells, double cycle) {
     tc.m2l_part64.ensure(size_t(shares) * ncells * PP);
     part = tc.m2l_part64.p;
   }
+  // (one tree's cells differ by 2^21 at most)
+  const bool wide = sc.t.R0 > kM2L64Wide * std::ldexp(tc.t.R0, -tc.t.depth);
   switch (P) {
 #define XF_M2L64_CASE(n)                                                                                           \
   case n:                                                                                                          \
-    hipLaunchKernelGGL(k_m2l_fp64<n>, dim3(ncells, shares), dim3(kM2L64Threads), lds, tc.s0, fillP, ncells, pl,    \
+    hipLaunchKernelGGL((wide ? k_m2l_fp64<n, true> : k_m2l_fp64<n, false>), dim3(ncells, shares), dim3(kM2L64Threads), lds, tc.s0, fillP, ncells, pl,    \
                        tc.t.cx.p, sc.t.cx.p, tc.lists.m2l_beg.p, tc.lists.m2l_cnt.p, tc.lists.m2l.p, sc.M.p, tc.L.p, \
                        part, cycle);                                                                               \
     break;
