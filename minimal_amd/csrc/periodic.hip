@@ -333,9 +333,12 @@ __device__ inline void ewald_pair(double x2, double &pot, double &grad) {
   double y = __builtin_amdgcn_rsq(x2);
   const double e = fma(-(x2 * y), y, 1.0);
   y = fma(y * e, fma(e, 0.375, 0.5), y);
+  double x = x2 * y;
   const unsigned hi = unsigned(__double2hiint(x2));
-  if (hi - (123u << 20) >= (1800u << 20)) y = sqrt(1.0 / x2);  // outside the step's exponent range
-  const double x = x2 * y;
+  if (hi - (123u << 20) >= (1800u << 20)) {  // outside the step's exponent range, denormals and infinity among it
+    y = 1.0 / sqrt(x2);
+    x = fmin(x2 * y, 1e6);  // (exp(-x^2) is 0 there, and the products below stay finite)
+  }
   const double xk = x + kErfcxK, w = fma(2.0, x, 1.0), dd = xk * w;
   double r = __builtin_amdgcn_rcp(dd);
   const double f = fma(-dd, r, 1.0);
