@@ -1307,8 +1307,9 @@ static void batch_forests(exafmm_ctx *ctx, const exafmm_problem *problems, int c
   for (size_t gi = 0; gi < groups.size(); gi++) {
     const std::vector<int> &g = groups[gi];
     const int P = problems[g[0]].P;
-    if (ctx->forests[gi]->c.P != P) {  // another order in this slot: a new context
-      exafmm_destroy(ctx->forests[gi]);
+    exafmm_ctx *const old = ctx->forests[gi];  // null if its last creation failed
+    if (!old || old->c.P != P) {  // another order in this slot: a new context
+      if (old) exafmm_destroy(old);
       exafmm_config cfg = ctx->c.cfg;
       cfg.P = P;
       ctx->forests[gi] = nullptr;
@@ -1349,6 +1350,17 @@ static void batch_forests(exafmm_ctx *ctx, const exafmm_problem *problems, int c
         XF_HIP(hipMemcpyAsync(q.bodies, buf.p + off[k], sizeof(exafmm_body) * q.n, hipMemcpyDeviceToHost, fc.s0));
     }
   };
+  // The call returns when every forest's work has ended, whatever it returns: a
+  // forest that fails leaves the others copying into the callers' bodies.
+  struct Drain {
+    std::vector<exafmm_ctx *> &forests;
+    ~Drain() {
+      for (exafmm_ctx *f : forests)
+        if (f)
+          for (hipStream_t s : {f->c.s2, f->c.s1, f->c.s0})
+            if (s) (void)hipStreamSynchronize(s);
+    }
+  } drain{ctx->forests};
   // A forest waits for the host a few times, and its tree and lists are chains
   // of short launches: several forests run side by side, a host thread each
   // (48 problems of up to 100,000 bodies, three orders: 5.3 -> 4.7 ms; 20 of up
@@ -1390,6 +1402,7 @@ static void batch_forests(exafmm_ctx *ctx, const exafmm_problem *problems, int c
       if (e.code != EXAFMM_OK) throw Failure{e.code, e.msg.empty() ? "host allocation failed" : e.msg};
   }
   for (exafmm_ctx *f : ctx->forests) {
+    if (!f) continue;  // (a slot beyond this call's groups)
     XF_HIP(hipStreamSynchronize(f->c.s1));
     XF_HIP(hipStreamSynchronize(f->c.s0));
   }
