@@ -309,7 +309,10 @@ typedef struct exafmm_problem {
 /* EXAFMM_BATCH_FOREST: the problems of each order are gathered into one
  * array and evaluated as one forest (exafmm_evaluate_forest), then copied
  * back: every call builds the trees and lists of all problems afresh, with
- * one launch per pass over all problems of an order. */
+ * one launch per pass over all problems of an order.  The forests of
+ * different orders run side by side; where two problems' bodies overlap in
+ * memory they run one after the other instead, lowest order first, each adding
+ * to the results of the one before.  Problems of one order must not overlap. */
 #define EXAFMM_BATCH_FOREST 2
 int exafmm_evaluate_batch(exafmm_ctx *ctx, const exafmm_problem *problems, int count, int flags);
 

@@ -1279,6 +1279,21 @@ __global__ void __launch_bounds__(256) k_forest_copy(const ForestPart *__restric
 // evaluated as one forest (exafmm_evaluate_forest: one tree build, one
 // traversal and one launch per pass over all of them), then copied back.
 constexpr int kForestThreads = 4;  // forests evaluated side by side
+
+// Whether two problems' bodies overlap in memory (one body set evaluated at
+// several orders): their forests then run one after the other, lowest order
+// first, each on the results of the one before.
+static bool problems_overlap(const exafmm_problem *problems, int count) {
+  std::vector<std::pair<uintptr_t, uintptr_t>> r(count);
+  for (int i = 0; i < count; i++) {
+    const uintptr_t b = reinterpret_cast<uintptr_t>(problems[i].bodies);
+    r[i] = {b, b + sizeof(exafmm_body) * size_t(problems[i].n)};
+  }
+  std::sort(r.begin(), r.end());
+  for (int i = 1; i < count; i++)
+    if (r[i].first < r[i - 1].second) return true;
+  return false;
+}
 static void batch_forests(exafmm_ctx *ctx, const exafmm_problem *problems, int count) {
   using namespace xf;
   std::vector<std::vector<int>> groups;  // problem indices, by order, chunks of kForestMax
@@ -1372,8 +1387,12 @@ static void batch_forests(exafmm_ctx *ctx, const exafmm_problem *problems, int c
     ctx->forests[gi]->c.defer_tuning = tuned;
     ctx->forests[gi]->c.tuning_wanted = false;
   }
-  if (!tuned || groups.size() == 1) {
-    for (size_t gi = 0; gi < groups.size(); gi++) evaluate(gi);
+  const bool shared = problems_overlap(problems, count);
+  if (!tuned || shared || groups.size() == 1) {
+    for (size_t gi = 0; gi < groups.size(); gi++) {
+      evaluate(gi);
+      if (shared) XF_HIP(hipStreamSynchronize(ctx->forests[gi]->c.s0));  // its results are the next one's input
+    }
   } else {
     std::vector<Failure> failed(groups.size(), Failure{EXAFMM_OK, {}});
     std::atomic<size_t> next{0};
