@@ -312,7 +312,10 @@ typedef struct exafmm_problem {
  * one launch per pass over all problems of an order.  The forests of
  * different orders run side by side; where two problems' bodies overlap in
  * memory they run one after the other instead, lowest order first, each adding
- * to the results of the one before.  Problems of one order must not overlap. */
+ * to the results of the one before.  Problems of one order must not overlap.
+ * Side by side means a host thread per forest that polls its stream: at most
+ * four, at most the CPUs the calling thread may run on, and at most
+ * EXAFMM_FOREST_THREADS (environment) where that is set. */
 #define EXAFMM_BATCH_FOREST 2
 int exafmm_evaluate_batch(exafmm_ctx *ctx, const exafmm_problem *problems, int count, int flags);
 

@@ -2,6 +2,8 @@
 // pass-level drop-in for buildTree / upwardPass / horizontalPass /
 // downwardPass / direct, exports in the reference's numbering, and stage
 // timing with HIP events.
+#include <sched.h>
+
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -1278,7 +1280,18 @@ __global__ void __launch_bounds__(256) k_forest_copy(const ForestPart *__restric
 // at most kForestMax per forest, are gathered into one device array and
 // evaluated as one forest (exafmm_evaluate_forest: one tree build, one
 // traversal and one launch per pass over all of them), then copied back.
-constexpr int kForestThreads = 4;  // forests evaluated side by side
+// Forests evaluated side by side.  Each has a host thread that polls its
+// stream, so no more than the CPUs the calling thread may run on (a program that
+// pins one rank to a core gets no second thread), and fewer on request
+// (EXAFMM_FOREST_THREADS=1: one after the other).
+constexpr int kForestThreads = 4;
+static int forest_threads() {
+  int n = kForestThreads;
+  cpu_set_t set;
+  if (sched_getaffinity(0, sizeof(set), &set) == 0) n = std::min(n, CPU_COUNT(&set));
+  if (const char *e = std::getenv("EXAFMM_FOREST_THREADS")) n = std::min(n, std::atoi(e));
+  return std::max(n, 1);
+}
 
 // Whether two problems' bodies overlap in memory (one body set evaluated at
 // several orders): their forests then run one after the other, lowest order
@@ -1388,7 +1401,8 @@ static void batch_forests(exafmm_ctx *ctx, const exafmm_problem *problems, int c
     ctx->forests[gi]->c.tuning_wanted = false;
   }
   const bool shared = problems_overlap(problems, count);
-  if (!tuned || shared || groups.size() == 1) {
+  const size_t nthreads = std::min(groups.size(), size_t(forest_threads()));
+  if (!tuned || shared || nthreads == 1) {
     for (size_t gi = 0; gi < groups.size(); gi++) {
       evaluate(gi);
       if (shared) XF_HIP(hipStreamSynchronize(ctx->forests[gi]->c.s0));  // its results are the next one's input
@@ -1410,7 +1424,7 @@ static void batch_forests(exafmm_ctx *ctx, const exafmm_problem *problems, int c
         }
     };
     std::vector<std::thread> threads;
-    for (size_t k = 1; k < std::min(groups.size(), size_t(kForestThreads)); k++) try {
+    for (size_t k = 1; k < nthreads; k++) try {
         threads.emplace_back(work);
       } catch (const std::exception &) {
         break;  // no thread to be had: the others take its forests
