@@ -1791,7 +1791,9 @@ void m2l_fast(Ctx &tc, const Ctx &sc) {
     if (!c.capturing) XF_HIP(hipEventRecord(c.ev[13], s));
     std::vector<ClassPass> pass;
     std::vector<GemmShape> shape;
-    bool all_sk = ncls <= kMaxClasses;
+    // EXAFMM_GEMM_SK_ONLY=class: a sum per class (tests)
+    const char *only = std::getenv("EXAFMM_GEMM_SK_ONLY");
+    bool all_sk = ncls <= kMaxClasses && !(only && std::strcmp(only, "class") == 0);
     for (int o = ncls - 1; o >= 0; o--) {
       const int *cls = c.tile_cls.p;
       int lo = kMaxP;
@@ -1802,7 +1804,10 @@ void m2l_fast(Ctx &tc, const Ctx &sc) {
       shape.push_back(gemm_shape(c, sc, g, ntiles, bf16, KP, KPb, &pass.back()));
       all_sk = all_sk && shape.back().sk;
     }
-    // stream-K launches leave their segments for one sum over the classes
+    // Stream-K launches leave their segments for one sum over the classes: (CUs +
+    // tiles) x 512 x P^2 floats for every class at once (300,007 clustered bodies,
+    // order 13: 4 x 114 MB; 2^22, order 14: 4 x 315 MB).  Where that much is not to
+    // be had, a sum per class in one class's segments.
     ClassSums sums{};
     int rows = 0;
     int64_t seg = 0;
@@ -1812,7 +1817,12 @@ void m2l_fast(Ctx &tc, const Ctx &sc) {
       seg += int64_t(sk_groups(c.cfg.device, ceil_div(go.R, shape[k].rtb)) + ntiles) * kTileN * g.PP;
       rows = std::max(rows, std::min(g.PP, 16 * go.R));
     }
-    if (all_sk) c.m2l_part.ensure(size_t(seg));
+    if (all_sk) try {
+        c.m2l_part.ensure(size_t(seg));
+      } catch (const Failure &e) {
+        if (e.code != EXAFMM_ERR_ALLOC) throw;
+        all_sk = false;
+      }
     for (size_t k = 0; k < pass.size(); k++)
       run_gemm(c, sc, g, ntiles, bf16, KP, KPb, shape[k], c.L.p, &pass[k], all_sk ? &sums : nullptr);
     if (all_sk) {

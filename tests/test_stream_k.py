@@ -125,9 +125,10 @@ def test_few_slots_learned(gpu, monkeypatch):
     orders = set()
     for tol in (-3.0, -4.5, -6.0):
         out = []
-        for env in ("EXAFMM_GEMM_SK_ONLY", "EXAFMM_GEMM_NO_SK"):
+        # one sum over all classes, a sum per class, no stream-K
+        for env, how in (("EXAFMM_GEMM_SK_ONLY", "1"), ("EXAFMM_GEMM_SK_ONLY", "class"), ("EXAFMM_GEMM_NO_SK", "1")):
             with monkeypatch.context() as m:
-                m.setenv(env, "1")
+                m.setenv(env, how)
                 f = fmm.FMM(P=14, ncrit=40, theta=0.4, order_policy=fmm.ORDER_LEARNED)
                 f.set_order_model(w, tol)
                 d = _dirty()
@@ -137,5 +138,6 @@ def test_few_slots_learned(gpu, monkeypatch):
                 orders |= set(np.nonzero(f.order_stats())[0])
                 f.close()
             out.append(b)
-        _close(*out)
+        _close(out[0], out[2])
+        _close(out[1], out[2])
     assert len(orders) > 1
