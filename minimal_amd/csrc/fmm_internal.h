@@ -234,7 +234,6 @@ struct Lists {
   Buf<unsigned long long> hslots;  // open-addressing key set
   int hcap = 0;
   Buf<int> slot2id;
-  Buf<int> scan_tmp;       // device-wide scan partials
   Buf<unsigned long long> keys;    // distinct keys, ascending
   Buf<int> kscratch;
   int nkeys = 0;
@@ -418,7 +417,7 @@ void op_l2l(Ctx &c, const double *Cp, const double *Lp, const double *Cc, double
 void op_l2p(Ctx &c, const double *C, const double *L, exafmm_body *b, int64_t nb);
 
 // generic helpers (scan.hip)
-void scan_exclusive(const int *in, int *out, int count, int *total, Buf<int> &scratch, hipStream_t s);
+void scan_exclusive(const int *in, int *out, int count, Buf<int> &scratch, hipStream_t s);
 void radix_sort_pairs(unsigned long long *&k, int *&v, unsigned long long *&k2, int *&v2, int n, int lo_bit,
                       int hi_bit, Buf<int> &hist, hipStream_t s);
 

@@ -5,21 +5,12 @@
 
 namespace xf {
 
-// Device-wide exclusive scan of NA int arrays of the same length in two
-// launches: each of G workgroups reduces a contiguous range (coalesced
-// 1024-element tiles), then each rescans its range starting from the sum of
-// the ranges before it.  The length may live on the device (n_dev); the
-// grid is sized from a host upper bound and idle workgroups exit.  base
-// (optional) is added to every output and receives the totals; cap/flag
-// (optional) raise bit 1 of *flag when a total exceeds cap[k].
+// Device-wide exclusive scan of an int array in two launches: each of G
+// workgroups reduces a contiguous range (coalesced tiles), then each rescans its
+// range starting from the sum of the ranges before it.  A short array takes one
+// workgroup and one launch.
 constexpr int kScanThreads = 1024;
 constexpr int kScanMaxBlocks = 64;
-
-template <int NA>
-struct ScanArrays {
-  const int *in[NA];
-  int *out[NA];
-};
 
 __device__ inline int block_sum(int v, int *red) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -52,128 +43,97 @@ constexpr int kScanTile = kScanThreads * kScanItems;
 static_assert(kScanTile == kScanChunk, "a workgroup range is a whole number of tiles");
 __device__ inline int scan_pad(int i) { return i + (i >> 5); }
 
-template <int NA>
-__global__ void __launch_bounds__(kScanThreads) k_scan_reduce(ScanArrays<NA> a, int n_host, const int *n_dev,
-                                                              int *__restrict__ sums, const int *base) {
+__global__ void __launch_bounds__(kScanThreads) k_scan_reduce(const int *__restrict__ in, int n,
+                                                              int *__restrict__ sums) {
   __shared__ int red[kScanThreads / 64];
-  const int n = n_dev ? *n_dev : n_host;
-  const int G = gridDim.x;
   int b0, e;
-  scan_range(n, G, b0, e);
+  scan_range(n, gridDim.x, b0, e);
+  int v = 0;
+  for (int t0 = b0; t0 < e; t0 += kScanTile) {
+    int x[kScanItems];
 #pragma unroll
-  for (int k = 0; k < NA; k++) {
-    int v = 0;
-    for (int t0 = b0; t0 < e; t0 += kScanTile) {
-      int x[kScanItems];
-#pragma unroll
-      for (int j = 0; j < kScanItems; j++) {
-        const int i = t0 + j * kScanThreads + threadIdx.x;
-        x[j] = i < e ? a.in[k][i] : 0;
-      }
-#pragma unroll
-      for (int j = 0; j < kScanItems; j++) v += x[j];
+    for (int j = 0; j < kScanItems; j++) {
+      const int i = t0 + j * kScanThreads + threadIdx.x;
+      x[j] = i < e ? in[i] : 0;
     }
-    v = block_sum(v, red);
-    if (threadIdx.x == 0) sums[blockIdx.x * NA + k] = v;
+#pragma unroll
+    for (int j = 0; j < kScanItems; j++) v += x[j];
   }
-  // keep the incoming running totals where the apply pass reads them
-  if (blockIdx.x == 0 && threadIdx.x < NA) sums[kScanMaxBlocks * NA + threadIdx.x] = base ? base[threadIdx.x] : 0;
+  v = block_sum(v, red);
+  if (threadIdx.x == 0) sums[blockIdx.x] = v;
 }
 
-template <int NA>
-__global__ void __launch_bounds__(kScanThreads) k_scan_apply(ScanArrays<NA> a, int n_host, const int *n_dev,
-                                                             const int *__restrict__ sums, int *total, int *base,
-                                                             const int64_t *cap, int *flag) {
+// sums: the workgroups' totals (null: one workgroup).
+__global__ void __launch_bounds__(kScanThreads) k_scan_apply(const int *in, int *out, int n,
+                                                             const int *__restrict__ sums) {
   __shared__ int red[kScanThreads / 64];
   __shared__ int wtot[kScanThreads / 64];
   __shared__ int sm[kScanTile + kScanTile / 32];
-  const int n = n_dev ? *n_dev : n_host;
-  const int G = gridDim.x;
   int b0, e;
-  scan_range(n, G, b0, e);
+  scan_range(n, gridDim.x, b0, e);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  int carry = 0;
+  if (sums) {
+    int v = 0;
+    for (int j = tid; j < int(blockIdx.x); j += kScanThreads) v += sums[j];
+    carry = block_sum(v, red);
+  }
+  for (int t0 = b0; t0 < e; t0 += kScanTile) {
+    int x[kScanItems];
 #pragma unroll
-  for (int k = 0; k < NA; k++) {
-    // one workgroup (sums == nullptr): no reduce pass, the running total
-    // comes straight from base
-    int carry = sums ? sums[kScanMaxBlocks * NA + k] : (base ? base[k] : 0);
-    if (sums) {
-      int v = 0;
-      for (int j = tid; j < blockIdx.x; j += kScanThreads) v += sums[j * NA + k];
-      carry += block_sum(v, red);
+    for (int j = 0; j < kScanItems; j++) {
+      const int i = t0 + j * kScanThreads + tid;
+      x[j] = i < e ? in[i] : 0;
     }
-    for (int t0 = b0; t0 < e; t0 += kScanTile) {
-      int x[kScanItems];
 #pragma unroll
-      for (int j = 0; j < kScanItems; j++) {
-        const int i = t0 + j * kScanThreads + tid;
-        x[j] = i < e ? a.in[k][i] : 0;
-      }
+    for (int j = 0; j < kScanItems; j++) sm[scan_pad(j * kScanThreads + tid)] = x[j];
+    __syncthreads();
+    // this thread's kScanItems consecutive elements
+    int run = 0;
 #pragma unroll
-      for (int j = 0; j < kScanItems; j++) sm[scan_pad(j * kScanThreads + tid)] = x[j];
-      __syncthreads();
-      // this thread's kScanItems consecutive elements
-      int run = 0;
-#pragma unroll
-      for (int j = 0; j < kScanItems; j++) {
-        x[j] = sm[scan_pad(tid * kScanItems + j)];
-        run += x[j];
-      }
-      int incl = run;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int u = __shfl_up(incl, d);
-        if (lane >= d) incl += u;
-      }
-      if (lane == 63) wtot[w] = incl;
-      __syncthreads();
-      int before = carry, tile = 0;
-      for (int q = 0; q < kScanThreads / 64; q++) {
-        if (q < w) before += wtot[q];
-        tile += wtot[q];
-      }
-      before += incl - run;
-#pragma unroll
-      for (int j = 0; j < kScanItems; j++) {
-        sm[scan_pad(tid * kScanItems + j)] = before;
-        before += x[j];
-      }
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < kScanItems; j++) {
-        const int i = t0 + j * kScanThreads + tid;
-        if (i < e) a.out[k][i] = sm[scan_pad(j * kScanThreads + tid)];
-      }
-      carry += tile;
-      __syncthreads();
+    for (int j = 0; j < kScanItems; j++) {
+      x[j] = sm[scan_pad(tid * kScanItems + j)];
+      run += x[j];
     }
-    __syncthreads();  // every thread has read base[k] before it is overwritten
-    if (blockIdx.x == G - 1 && tid == 0) {
-      if (total) total[k] = carry;
-      if (base) base[k] = carry;
-      if (cap && flag && carry > cap[k]) atomicOr(flag, 1);
+    int incl = run;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int u = __shfl_up(incl, d);
+      if (lane >= d) incl += u;
     }
+    if (lane == 63) wtot[w] = incl;
+    __syncthreads();
+    int before = carry, tile = 0;
+    for (int q = 0; q < kScanThreads / 64; q++) {
+      if (q < w) before += wtot[q];
+      tile += wtot[q];
+    }
+    before += incl - run;
+#pragma unroll
+    for (int j = 0; j < kScanItems; j++) {
+      sm[scan_pad(tid * kScanItems + j)] = before;
+      before += x[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kScanItems; j++) {
+      const int i = t0 + j * kScanThreads + tid;
+      if (i < e) out[i] = sm[scan_pad(j * kScanThreads + tid)];
+    }
+    carry += tile;
+    __syncthreads();
   }
 }
 
-template <int NA>
-static void scan_launch(const ScanArrays<NA> &a, int n_host, const int *n_dev, int n_bound, int *total, int *base,
-                        const int64_t *cap, int *flag, Buf<int> &scratch, hipStream_t s) {
-  const int G = std::max(1, std::min(kScanMaxBlocks, ceil_div(std::max(n_bound, 1), 8 * kScanThreads)));
-  scratch.ensure(size_t(kScanMaxBlocks + 1) * NA);
+void scan_exclusive(const int *in, int *out, int count, Buf<int> &scratch, hipStream_t s) {
+  const int G = std::max(1, std::min(kScanMaxBlocks, ceil_div(std::max(count, 1), 8 * kScanThreads)));
+  scratch.ensure(kScanMaxBlocks);
   if (G > 1) {
-    hipLaunchKernelGGL(k_scan_reduce<NA>, dim3(G), dim3(kScanThreads), 0, s, a, n_host, n_dev, scratch.p,
-                       (const int *)base);
+    hipLaunchKernelGGL(k_scan_reduce, dim3(G), dim3(kScanThreads), 0, s, in, count, scratch.p);
     XF_LAUNCH();
   }
-  hipLaunchKernelGGL(k_scan_apply<NA>, dim3(G), dim3(kScanThreads), 0, s, a, n_host, n_dev,
-                     G > 1 ? (const int *)scratch.p : nullptr, total, base, cap, flag);
+  hipLaunchKernelGGL(k_scan_apply, dim3(G), dim3(kScanThreads), 0, s, in, out, count, G > 1 ? scratch.p : nullptr);
   XF_LAUNCH();
-}
-
-void scan_exclusive(const int *in, int *out, int count, int *total, Buf<int> &scratch, hipStream_t s) {
-  ScanArrays<1> a{{in}, {out}};
-  scan_launch<1>(a, count, nullptr, count, total, nullptr, nullptr, nullptr, scratch, s);
 }
 
 // ---------------------------------------------------------------- radix sort

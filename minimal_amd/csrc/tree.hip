@@ -885,7 +885,7 @@ void tree_build(Ctx &c) {
   if (Ds <= kHistLevels) {
     const int Dc = std::max(Ds, 3), bins = 1 << (3 * Dc);  // levels 1 and 2 are summed later
     t.cursor.ensure(bins);
-    scan_exclusive(t.hist.p + hist_off(Dc), t.cursor.p, bins, nullptr, t.scan_tmp, s);
+    scan_exclusive(t.hist.p + hist_off(Dc), t.cursor.p, bins, t.scan_tmp, s);
     hipLaunchKernelGGL(k_place, dim3(ceil_div(n, 256)), dim3(256), 0, s, k1, n, 3 * (kMaxLevel - Dc), t.cursor.p, k2,
                        v1);
     XF_LAUNCH();
