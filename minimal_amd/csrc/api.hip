@@ -197,7 +197,9 @@ void do_downward(Ctx &c) {
 // launches of 1.5M clustered bodies (90,000 cells) ended with it, 1.7 ms after
 // the lists, and the keyed GEMM waited for them (7.55 ms, 7.41 this way).  The
 // M2M of smaller trees is done sooner than that wait costs: 2^20 uniform bodies
-// (37,449 cells) 2.96 ms, 2.99 this way, 300,007 clustered 3.12 and 3.17.
+// (37,449 cells) 2.96 ms, 2.99 this way, 300,007 clustered 3.12 and 3.17.  The
+// line lies between those two sizes and the third, at a power of two; a tree
+// near it takes about the same time either way.
 constexpr int64_t kUpwardFirst = 65536;  // cells
 void run_passes(Ctx &c) {
   const bool upward_first = c.t.ncells >= kUpwardFirst;

@@ -89,6 +89,10 @@ __device__ inline unsigned mix32(unsigned h) {
   return h;
 }
 
+// Three hashes make the sort key 56 bits, seven radix passes where one hash took
+// three: a pass over the 37,449 cells of 2^20 uniform bodies takes 32 us beside P2P
+// (which hides it: P2P outlasts the tile build there), over the 19,199 of 300,007
+// clustered bodies 33 us.
 constexpr int kMinHashes = 3;
 constexpr int kGroupShift = 48, kSortBits = 56;
 
@@ -633,6 +637,12 @@ __device__ inline int op_run(int c, int nrt, int RT, int rt0) {
   return kk * RT + rt0 + rl;
 }
 
+// FP32 form: a workgroup per tile and row block, key slices where tiles are few,
+// every column multiplied (no subtile masks).  Against eight waves and tiles of one
+// level, whole evaluations: 10,000 / 10^5 / 10^6 uniform bodies, order 10: 929 -> 596
+// us, 1.39 -> 0.95 ms, 4.48 -> 4.13 ms; order 16: 2.86 -> 1.47, 4.67 -> 3.03, 18.2 ->
+// 16.1 ms; 500,000 clustered, order 14: 26.4 -> 24.8 ms; 50,000 periodic, order 10:
+// 5.14 -> 2.94 ms.
 template <int RH>
 __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RTB, int K4, int KP,
                                                           const int *__restrict__ tfirst,

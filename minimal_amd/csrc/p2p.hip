@@ -406,7 +406,7 @@ __device__ inline void p2p64_pair(double dx, double dy, double dz, double q, dou
 // FP64 P2P: a workgroup per target leaf, its waves taking the leaf's targets
 // in balanced blocks of at most kP2P64TC; as in the FP32 kernel a block's
 // targets are wave-uniform and the lanes take the staged entries' sources,
-// one load per source and block.  FP64 VALU bound (about 25 operations per
+// one load per source and block.  FP64 VALU bound (about 27 operations per
 // interaction).  67,984,904 interactions (30,000 bodies): 164 us; 903 us with
 // a thread per target walking its sources one by one through a divide and a
 // square root each.
@@ -541,7 +541,7 @@ void p2p_apply(Ctx &tc, const Ctx &sc, hipStream_t s, const int *list_flags) {
 // the same share (its lines then come from L2 once), or, with fewer than
 // four blocks, quarters of the share.  Each (share, target) partial is
 // stored and k_direct_sum adds a target's partials in a fixed order.  FP64
-// VALU bound.  1,000 targets x 2^20 sources: 0.85 ms; 2.83 ms with a workgroup
+// VALU bound.  1,000 targets x 2^20 sources: 0.92 ms; 2.83 ms with a workgroup
 // per target (every target streaming all sources, a divide and a root each).
 constexpr int kDirectTC = 8;
 constexpr int kDirectWaves = 4;
@@ -592,7 +592,10 @@ __global__ void __launch_bounds__(kDirectWaves *kWave) k_direct(const exafmm_bod
 // and adds its waves' sums itself, in one launch.  Up to kDirectOneMax
 // sources a wave has few enough rounds that the launch saved is worth more
 // than the even split: 1,000 x 8,000 in 23 us, 32 in two launches (and 2,000 x
-// 8,000 in 32 against 37); the gap closes beyond.
+// 8,000 in 32 against 37); the gap closes beyond.  Few targets leave most CUs idle
+// here and cross earlier: 1 to 100 x 8,192 in 21 - 22 us, 19 - 20 in two launches
+// (8,193 sources); the rule looks at the sources alone (a workgroup per target:
+// 23 - 24).
 constexpr int kDirectOneTC = 4, kDirectOneWaves = 16;
 constexpr int64_t kDirectOneMax = 8192;
 __global__ void __launch_bounds__(kDirectOneWaves *kWave) k_direct_one(exafmm_body *__restrict__ t, int64_t nt,

@@ -33,6 +33,10 @@ namespace xf {
 constexpr int kTravWaves = 8;
 // Pairs per target: the queue that fits beside the staged lists at 16 waves
 // per CU, and the one a pass is repeated with when a target overflows it.
+// The large one leaves room for one workgroup per CU instead of three; a context
+// that needed it (theta below about 0.3) keeps it.  30,000 uniform bodies, ncrit
+// 32: the lists take 298 us at theta 0.25 and 412 at 0.2, 391 and 721 as count,
+// scan and fill launches on that queue.
 constexpr int kQSmall = 768, kQCap = 2048;
 // list entries staged per target; a longer list is walked a second time,
 // straight into place
