@@ -389,7 +389,26 @@ __global__ void __launch_bounds__(256) k_place(const unsigned long long *__restr
   const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (i >= n) return;
   const unsigned long long k = key[i];
-  const int pos = atomicAdd(&cursor[int(k >> shift)], 1);
+  const int bin = int(k >> shift), lane = threadIdx.x & (kWave - 1);
+  // A run of equal prefixes among neighbouring lanes takes its places with one
+  // atomic: bodies that come in tree order (those of the step before) have
+  // nothing but such runs, and one atomic each made the lanes of a wave wait for
+  // one counter (10^6 uniform bodies in tree order, a build: ncrit 64 277 -> 191 us,
+  // ncrit 300 502 -> 209; 4 x 10^6 and ncrit 300 1,086 -> 515; bodies in random order
+  // the same).
+  const int prev = __shfl_up(bin, 1);
+  const unsigned long long here = __ballot(true), starts = __ballot(lane == 0 || prev != bin);
+  int pos;
+  if (starts == here) {  // uniform
+    pos = atomicAdd(&cursor[bin], 1);
+  } else {
+    const int first = 63 - __clzll((long long)(starts & (~0ull >> (63 - lane))));
+    const unsigned long long later = starts & ~(~0ull >> (63 - first));
+    const int end = later ? __ffsll((long long)later) - 1 : __popcll(here);
+    int at = 0;
+    if (lane == first) at = atomicAdd(&cursor[bin], end - first);
+    pos = __shfl(at, first) + lane - first;
+  }
   key_out[pos] = k;
   val_out[pos] = int(i);
 }
