@@ -127,7 +127,7 @@ struct HostBuf {
 // Slots of Ctx::pin_i (ints read back by the tree build, traversal and M2L plan)
 constexpr int kPinLevelMax = 0;   // 9: flags, largest prefix population of levels 1..8
 constexpr int kPinLevels = 16;    // kMaxLevel + 2 level sizes
-constexpr int kPinMisc = 48;      // 19: tree flags and counters
+constexpr int kPinMisc = 48;      // 21: tree flags and counters
 constexpr int kPinTot = 72;       // 8: list totals, key count and flags (Lists::tot)
 constexpr int kPinPlan = 80;      // 4: M2L slots, tiles, cells in tiles, key set differs from the operators'
 constexpr int kPinInts = 96;
@@ -138,7 +138,7 @@ constexpr int kListRetry = 1 | 8 | kListQueue;
 // ints of Lists::tot behind the three 64-bit totals
 constexpr int kTotKeys = 6, kTotFlags = 7;
 static_assert(kPinTot % 2 == 0, "64-bit totals");
-static_assert(kPinLevels + kMaxLevel + 2 <= kPinMisc && kPinMisc + 19 <= kPinTot, "pinned slots overlap");
+static_assert(kPinLevels + kMaxLevel + 2 <= kPinMisc && kPinMisc + 21 <= kPinTot, "pinned slots overlap");
 
 inline int ceil_div(int64_t a, int64_t b) { return int((a + b - 1) / b); }
 
@@ -193,6 +193,7 @@ struct Tree {
   double X0[3] = {0, 0, 0}, R0 = 0;
   int lroot = 0;                 // level of the (problem) roots: kForestLevel in a forest
   int ds_hint = -1;              // sort depth of the last build (-1: none yet)
+  bool in_order = false;         // the last build's bodies came in tree order
 
   Buf<double4> cx;     // centre xyz, radius R
   Buf<int> cbeg, ccnt; // body range in tree order

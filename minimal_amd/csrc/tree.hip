@@ -219,14 +219,19 @@ __global__ void __launch_bounds__(64) k_forest_roots(const int64_t *__restrict__
 // deep trees are sorted by radix anyway, and their crowded prefixes (a Plummer
 // core) make the XCDs' atomics pass the same counters around (1.5M clustered
 // bodies: 243 us, even with each workgroup's bodies counted in LDS first; 32 us
-// without, and 12 for k_hist_sorted).
+// without, and 12 for k_hist_sorted).  One wave in kOrderSample adds the number of
+// runs of equal level-4 prefixes among its lanes to order[0], its lanes to order[1]
+// (above the leaves of the sets it is looked at for: below them the order is the
+// caller's).
+constexpr int kOrderSample = 64;
 constexpr int kKeysThreads = 256;
 template <bool HIST>
 __global__ void __launch_bounds__(kKeysThreads) k_keys(const exafmm_body *__restrict__ b, int64_t n,
                                                        const double *__restrict__ root,
                                                        unsigned long long *__restrict__ key, int *__restrict__ val,
                                                        int *__restrict__ hist7, const double4 *__restrict__ froots,
-                                                       const int64_t *__restrict__ off, int nprob) {
+                                                       const int64_t *__restrict__ off, int nprob,
+                                                       int *__restrict__ order) {
   const int64_t i = int64_t(blockIdx.x) * kKeysThreads + threadIdx.x;
   if (i >= n) return;
   const double x = b[i].X[0], y = b[i].X[1], z = b[i].X[2];
@@ -263,6 +268,16 @@ __global__ void __launch_bounds__(kKeysThreads) k_keys(const exafmm_body *__rest
   }
   key[i] = k;
   val[i] = int(i);
+  if (i / kWave % kOrderSample == 0) {  // uniform
+    const unsigned p4 = unsigned(k >> (3 * (kMaxLevel - 4)));
+    const unsigned prev = __shfl_up(p4, 1);
+    const int lane = threadIdx.x & (kWave - 1);
+    const int runs = __popcll(__ballot(lane == 0 || prev != p4)), lanes = __popcll(__ballot(true));
+    if (lane == 0) {
+      atomicAdd(order, runs);
+      atomicAdd(order + 1, lanes);
+    }
+  }
   if (HIST) atomicAdd(&hist7[unsigned(k >> (3 * (kMaxLevel - kHistLevels)))], 1);
 }
 
@@ -412,6 +427,10 @@ __global__ void __launch_bounds__(256) k_place(const unsigned long long *__restr
   key_out[pos] = k;
   val_out[pos] = int(i);
 }
+
+// Bodies up to which a counting sort is taken whatever their order (tree_build):
+// two radix passes instead (up to five levels), three (six and seven).
+constexpr int64_t kPlaceMax5 = 750000, kPlaceMax7 = 1500000;
 
 // ---------------------------------------------------------------- levels
 // Node t of level l: if it holds more than ncrit bodies, find the body
@@ -748,7 +767,7 @@ __global__ void __launch_bounds__(64) k_leaf_gather(const int *__restrict__ leav
     auto put = [](auto *p, auto v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
     const int t = threadIdx.x;
     if (t < kMaxLevel + 2) put(rep.host_levels + t, rep.lcount[t]);
-    if (t < 19) put(rep.host_misc + t, rep.misc[t]);
+    if (t < 21) put(rep.host_misc + t, rep.misc[t]);
     if (t < 4) put(rep.host_root + t, rep.root[t]);
   }
   const int nl = *nleaves;
@@ -813,7 +832,7 @@ void tree_build(Ctx &c) {
   if (n > (int64_t(1) << 30)) fail(EXAFMM_ERR_ARG, "N above 2^30 is not supported");
 
   // misc layout (ints): [0] flags, [1..8] level max, [17] leaves, [18] cells
-  // that split, [24 + l] look-back tickets of level l's split, [46] of k_leaves
+  // that split, [19, 20] runs and lanes sampled by k_keys, [24 + l] look-back tickets of level l's split, [46] of k_leaves
   t.misc.ensure(kMiscInts);
   t.bounds_part.ensure(kBoundsBlocks * kBoundsInts + 8);
   double *root = t.bounds_part.p + kBoundsBlocks * kBoundsInts;
@@ -877,7 +896,7 @@ void tree_build(Ctx &c) {
   const bool sorted_hist = speculate && Ds > kHistLevels;
   hipLaunchKernelGGL(sorted_hist ? k_keys<false> : k_keys<true>, dim3(ceil_div(n, kKeysThreads)), dim3(kKeysThreads), 0,
                      s, c.bodies, n, root, t.key.p, t.val.p, t.hist.p + hist_off(kHistLevels), froots,
-                     forest ? c.forest_off.p : nullptr, c.forest_n);
+                     forest ? c.forest_off.p : nullptr, c.forest_n, t.misc.p + 19);
   XF_LAUNCH();
   // one block per level-3 prefix (4096 level-7 bins each)
   t.hist_bmax.ensure(8 << (3 * 3));
@@ -906,12 +925,20 @@ void tree_build(Ctx &c) {
     Ds = sort_depth(hm, n, ncrit, forest, lforce);
   }
 
-  // bodies in the order of their top Ds octant digits: a counting sort on the
+  // Bodies in the order of their top Ds octant digits: a counting sort on the
   // histogram up to its depth (2 - 3 launches where the radix sort takes three
-  // per eight bits), the stable radix sort below
+  // per eight bits), the stable radix sort below.  Bodies in random order cost the
+  // counting sort an atomic and a scattered write each, about 82 us per 10^6, a
+  // radix pass 24: many of them take the radix sort as well, unless the last
+  // build's came in tree order.  Builds of uniform bodies, counting / radix, random
+  // order and tree order: 500,000 ncrit 64 (5 levels) 198 / 202 and 161 / 183 us, 10^6
+  // ncrit 300 (5) 295 / 269 and 207 / 241, 4 x 10^6 ncrit 300 (5) 915 / 782 and 503 /
+  // 595, 1.5 x 10^6 ncrit 64 (6) 386 / 383 and 266 / 297, 4 x 10^6 ncrit 64 (6) 945 /
+  // 894 and 553 / 694.
+  const bool place = Ds <= kHistLevels && (t.in_order || n < (Ds <= 5 ? kPlaceMax5 : kPlaceMax7));
   unsigned long long *k1 = t.key.p, *k2 = t.key2.p;
   int *v1 = t.val.p, *v2 = t.val2.p;
-  if (Ds <= kHistLevels) {
+  if (place) {
     const int Dc = std::max(Ds, 3), bins = 1 << (3 * Dc);  // levels 1 and 2 are summed later
     t.cursor.ensure(bins);
     scan_exclusive(t.hist.p + hist_off(Dc), t.cursor.p, bins, t.scan_tmp, s);
@@ -1005,6 +1032,7 @@ void tree_build(Ctx &c) {
     t.lstart.push_back(t.lstart.back() + lc[l]);
   }
   t.depth = depth;
+  t.in_order = fl[20] >= 8 * int64_t(fl[19]);  // (random order: runs of one or two)
   t.ds_hint = need <= kHistLevels ? need : std::min(kMaxLevel, depth + 1);
   t.ncells = t.lstart.back();
   const int nc = int(t.ncells);

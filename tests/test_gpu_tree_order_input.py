@@ -38,3 +38,25 @@ def test_tree_order(gpu, orc, kind, n, ncrit):
         c, r = f.cells(), s.cells()
         for k in ("nchild", "nbody", "child", "body", "X", "R"):
             assert np.array_equal(c[k], r[k]), k
+
+
+@pytest.mark.parametrize("n,ncrit", [(760001, 300), (1600000, 64)])
+def test_large_sets_by_either_sort(gpu, orc, n, ncrit):
+    """Sizes that are sorted by radix or by counting, by the order in which the
+    last build's bodies came: random, tree order twice (the second by counting),
+    random on a hint of tree order, random again.  A tree built on its own order
+    leaves the bodies where they are."""
+    b0 = uniform_cube(n, 9, "sym")
+    s = orc.session(2, ncrit, 0.4)
+    ref = b0.copy()
+    s.build_tree(ref)
+    r = s.cells()
+    f = fmm.FMM(P=2, ncrit=ncrit, theta=0.4)
+    b = None
+    for fresh in (True, False, False, True, True):
+        b = b0.copy() if fresh else b
+        f.build_tree(b)
+        assert np.array_equal(b["X"], ref["X"]) and np.array_equal(b["q"], ref["q"])
+        c = f.cells()
+        for k in ("nchild", "nbody", "child", "body", "X", "R"):
+            assert np.array_equal(c[k], r[k]), k
