@@ -1384,9 +1384,10 @@ static void batch_forests(exafmm_ctx *ctx, const exafmm_problem *problems, int c
   // forest that fails leaves the others copying into the callers' bodies.
   struct Drain {
     std::vector<exafmm_ctx *> &forests;
+    bool pending = true;
     ~Drain() {
       for (exafmm_ctx *f : forests)
-        if (f)
+        if (f && pending)
           for (hipStream_t s : {f->c.s2, f->c.s1, f->c.s0})
             if (s) (void)hipStreamSynchronize(s);
     }
@@ -1441,6 +1442,7 @@ static void batch_forests(exafmm_ctx *ctx, const exafmm_problem *problems, int c
     XF_HIP(hipStreamSynchronize(f->c.s1));
     XF_HIP(hipStreamSynchronize(f->c.s0));
   }
+  drain.pending = false;
 }
 
 int exafmm_evaluate_batch(exafmm_ctx *ctx, const exafmm_problem *problems, int count, int flags) {
