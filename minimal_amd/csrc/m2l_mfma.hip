@@ -637,12 +637,17 @@ __device__ inline int op_run(int c, int nrt, int RT, int rt0) {
   return kk * RT + rt0 + rl;
 }
 
-// FP32 form: a workgroup per tile and row block, key slices where tiles are few,
-// every column multiplied (no subtile masks).  Against eight waves and tiles of one
-// level, whole evaluations: 10,000 / 10^5 / 10^6 uniform bodies, order 10: 929 -> 596
-// us, 1.39 -> 0.95 ms, 4.48 -> 4.13 ms; order 16: 2.86 -> 1.47, 4.67 -> 3.03, 18.2 ->
-// 16.1 ms; 500,000 clustered, order 14: 26.4 -> 24.8 ms; 50,000 periodic, order 10:
-// 5.14 -> 2.94 ms.
+// FP32 form: a workgroup per tile and row block, key slices where tiles are few;
+// subtiles without a pair of a key are not multiplied (tiles that mix levels have
+// larger key unions).  A k-step's operator rows are read together, ahead of the
+// branches on the subtile bits.  Kernel alone, us, against tiles of one level and
+// every column multiplied: 131,626 uniform bodies, ncrit 32, theta 0.3, order 6 /
+// 9 / 13: 1,443 / 5,045 / 16,102 -> 1,429 / 4,702 / 16,271; theta 0.4, order 9:
+// 2,391 -> 2,190; 30,000, ncrit 16, order 9: 2,531 -> 1,362; 20,000, order 16: 16,733
+// -> 6,461; 500,000, ncrit 64, order 8: 2,437 -> 2,571; 10^6, theta 0.5, order 8: 819
+// -> 698; 131,626 clustered, order 9: 13,956 -> 7,020; 50,000 periodic, order 9:
+// 4,378 -> 3,972.  (Mixed levels with every column multiplied: 6,831 where 5,045 is
+// given, 20,607 for 16,102.)
 template <int RH>
 __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RTB, int K4, int KP,
                                                           const int *__restrict__ tfirst,
@@ -651,6 +656,7 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RT
                                                           const int *__restrict__ sorted,
                                                           const int *__restrict__ tkeys,
                                                           const int *__restrict__ tmat,
+                                                          const unsigned long long *__restrict__ tmask,
                                                           const float *__restrict__ op32,
                                                           const float *__restrict__ mt,
                                                           const unsigned char *__restrict__ tkp, int kr,
@@ -719,12 +725,18 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RT
 #pragma unroll
       for (int ct = 0; ct < kCT; ct++) bv[ct] = mt[int64_t(sc[ct] >= 0 && k < kc ? sc[ct] : ncells) * KP + k];
     };
+    // bit ct: this wave's column tile ct holds a pair of key u (u < U)
+    auto mask_of = [&](int u) {
+      const unsigned long long m = uniform_load(tmask + base + u) >> (8 * (w >> 2) + (w & 3));
+      return int((m & 1) | ((m >> 31) & 2));
+    };
     stage_ops(0);
     stage_src(0);
     if (R > 1) stage_src(1);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     int src[kCT], nsrc[kCT];
+    int m = mask_of(0);
     float bcur[kCT], bnext[kCT];
     col_src(0, src);
     int kc = kcols(0);
@@ -741,6 +753,7 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RT
         const int kc_next = u + 1 < U ? kcols(u + 1) : 0;
         const bool next = u + 1 < U && ksteps(kc_next) > 0;
         if (u + 1 < U) col_src(u + 1, nsrc);
+        const int m_next = mask_of(min(u + 1, U - 1));
         for (int kk = 0; kk < ks; kk++) {
 #pragma unroll
           for (int ct = 0; ct < kCT; ct++) bcur[ct] = bnext[ct];
@@ -751,14 +764,18 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RT
             load_b(nsrc, 0, kc_next, bnext);
             b_after = true;
           }
+          if (m == 0) continue;  // uniform, as the subtile bits below
+          const float *Ak = Acur + kk * nrt * 64 + lane;
+          float a[RH];
 #pragma unroll
-          for (int r2 = 0; r2 < RH; r2++) {
-            if (r2 >= nr) break;
-            const float a = Acur[(kk * nrt + r2) * 64 + lane];
+          for (int r2 = 0; r2 < RH; r2++) a[r2] = Ak[min(r2, nr - 1) * 64];
 #pragma unroll
-            for (int ct = 0; ct < kCT; ct++)
-              acc[r2][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bcur[ct], acc[r2][ct], 0, 0, 0);
-          }
+          for (int ct = 0; ct < kCT; ct++)
+            if (m & (1 << ct)) {
+#pragma unroll
+              for (int r2 = 0; r2 < RH; r2++)
+                if (r2 < nr) acc[r2][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r2], bcur[ct], acc[r2][ct], 0, 0, 0);
+            }
         }
         if (ks <= 0 && next) {
           load_b(nsrc, 0, kc_next, bnext);
@@ -767,6 +784,7 @@ __global__ void __launch_bounds__(kGemmThreads) k_m2l_f32(int PP, int RT, int RT
 #pragma unroll
         for (int ct = 0; ct < kCT; ct++) src[ct] = nsrc[ct];
         kc = kc_next;
+        m = m_next;
       }
       // staging of this round's start landed (only the kCT loads of the last
       // B prefetch are younger); then every wave is done with this round
@@ -1439,7 +1457,7 @@ static void launch_f32(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, int KP,
   gemm_attr(&k_m2l_f32<RH>);
   hipLaunchKernelGGL((k_m2l_f32<RH>), dim3(ntiles, ceil_div(g.R, sh.rtb), sh.ksplit), dim3(kGemmThreads), lds, c.s0,
                      g.PP, g.R, sh.rtb, g.K4, KP, t, t + ts, t + 2 * ts, t + 3 * ts, t + 4 * ts, c.tile_keys.p,
-                     c.tile_mat.p, c.ops32.p, sc.mt32.p, c.learned ? c.tile_p.p : nullptr, sh.kr,
+                     c.tile_mat.p, c.tile_mask.p, c.ops32.p, sc.mt32.p, c.learned ? c.tile_p.p : nullptr, sh.kr,
                      int64_t(c.t.ncells), sh.ksplit > 1 ? Lpart : nullptr, Lout);
   XF_LAUNCH();
 }
@@ -1526,10 +1544,12 @@ static GemmShape gemm_shape(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, bo
   std::vector<GemmShape> cand;
   auto slices = [&](int rtb, int kr, int nb) {
     cand.push_back(GemmShape{rtb, kr, 1});
-    // key slices only where the workgroups would not fill the device
+    // key slices only where the workgroups would not fill the device (the FP32
+    // form, which has no stream-K, also in thirds and sixths: 80 tiles in three
+    // slices are one round of workgroups)
     const int wg = ntiles * nb;
-    for (const int ks : {2, 4, 8})
-      if (wg * ks <= 2048 && c.m2l_totalU >= 8 * ks * ntiles) cand.push_back(GemmShape{rtb, kr, ks});
+    for (const int ks : {2, 3, 4, 6, 8})
+      if ((bf16 ? ks != 3 && ks != 6 && wg * ks <= 2048 : wg * ks <= 4096) && c.m2l_totalU >= 8 * ks * ntiles) cand.push_back(GemmShape{rtb, kr, ks});
   };
   if (bf16) {
     for (const int G : gemm_rounds(go, c.cfg.device)) {
@@ -1538,9 +1558,10 @@ static GemmShape gemm_shape(Ctx &c, const Ctx &sc, const Geom &g, int ntiles, bo
       if (std::getenv("EXAFMM_GEMM_NO_SK") == nullptr) cand.push_back(GemmShape{r, G, 1, 1});
     }
   } else {
-    // low orders: short keys, so more of them per LDS round
-    const int krmax = go.P <= 10 ? 5 : 3;
-    for (int kr = 1; kr <= krmax; kr++) {
+    // low orders: short keys, so more of them per LDS round (481,932 clustered bodies,
+    // theta 0.3, order 4: rounds of 8 or 12 instead of up to 5, whole step 1.07 -> 0.99 of what tiles of one level took)
+    const int krmax = go.P <= 5 ? 12 : go.P <= 10 ? 5 : 3;
+    for (int kr = 1; kr <= krmax; kr += kr < 5 ? 1 : 3 + (kr > 5)) {
       const int rmax = rows_per_block(go, false, c.cfg.device, kr);
       if (rmax < 1) continue;
       int last = -1;
