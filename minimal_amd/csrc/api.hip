@@ -171,11 +171,18 @@ void do_horizontal(Ctx &tc, const Ctx &sc) {
   do_far(tc, sc);
 }
 
+// Locals to the bodies.  Without M2L pairs and far images they are all zero
+// (problems of a few leaves): nothing to pass down.
+void pass_locals(Ctx &c) {
+  if (c.lists.nm2l == 0 && c.cfg.images < 2) return;
+  l2l_pass(c);
+  l2p_pass(c);
+}
+
 void do_downward(Ctx &c) {
   if (!c.have_L) fail(EXAFMM_ERR_STATE, "downward pass before horizontal pass");
   rec(c, 10, c.s0);
-  l2l_pass(c);
-  l2p_pass(c);
+  pass_locals(c);
   rec(c, 8, c.s0);
 }
 
@@ -840,8 +847,7 @@ void replay(Ctx &c, hipStream_t s) {
     upward(c, s);
     p2p_apply(c, c, s);
     m2l_apply(c, c);
-    l2l_pass(c);
-    l2p_pass(c);
+    pass_locals(c);
   } catch (...) {
     c.s0 = a;
     c.s1 = b;

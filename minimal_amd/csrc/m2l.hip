@@ -305,7 +305,10 @@ __global__ void __launch_bounds__(256) k_m2l_fp64_sum(int64_t n, int shares, con
 // differ in length several times over (hundreds of image translations per
 // cell at the top of a periodic tree), and a batch of pairs is a long chain
 // (list, cell, harmonics, sums), so below 8,192 cells the lists are shared
-// out over up to 16 workgroups each.
+// out over up to 16 workgroups each -- as many as the mean list has batches: a tree
+// of a few cells with short lists is not worth the second launch (60 problems of
+// 60 bodies each, re-evaluated by a graph: 1,822 -> 1,440 us; most have no pairs, and
+// m2l_apply leaves before this).
 static void m2l_fp64(Ctx &tc, const Ctx &sc, int ncells, double cycle) {
   join_upward(tc);
   const int P = tc.P, PP = P * P;
@@ -313,7 +316,8 @@ static void m2l_fp64(Ctx &tc, const Ctx &sc, int ncells, double cycle) {
   const M2L64Plan pl = m2l64_plan(P, fillP);
   const size_t lds = std::max(sizeof(double2) * size_t(pl.batch) * (m2l64_stride(fillP) + m2l64_stride(P)),
                               sizeof(double2) * 2 * kM2L64Threads);  // (the last sums)
-  const int shares = std::max(1, std::min(16, 8192 / std::max(ncells, 1)));
+  const int64_t mean = ceil_div(tc.lists.nm2l, int64_t(pl.batch) * std::max(ncells, 1));
+  const int shares = int(std::max<int64_t>(1, std::min<int64_t>({16, 8192 / std::max(ncells, 1), mean})));
   double *part = nullptr;
   if (shares > 1) {
     tc.m2l_part64.ensure(size_t(shares) * ncells * PP);
@@ -365,6 +369,10 @@ int m2l_fp64_levels(const Ctx &c) { return c.cfg.images > 0 ? std::min(3, c.t.de
 void m2l_apply(Ctx &tc, const Ctx &sc) {
   Tree &t = tc.t;
   const double cyc = tc.cfg.images > 0 ? tc.cfg.cycle : 0.0;
+  if (tc.lists.nm2l == 0) {  // the locals are zero already
+    join_upward(tc);
+    return;
+  }
   if (tc.cfg.m2l_precision != EXAFMM_PREC_FP64 && tc.lists.nkeys > 0) {
     const int lf = m2l_fp64_levels(tc);
     if (lf > 0) m2l_fp64(tc, sc, t.lstart[lf], cyc);  // cells of levels < lf come first in breadth-first order

@@ -596,31 +596,39 @@ __global__ void __launch_bounds__(kDirectWaves *kWave) k_direct(const exafmm_bod
 // here and cross earlier: 1 to 100 x 8,192 in 21 - 22 us, 19 - 20 in two launches
 // (8,193 sources); the rule looks at the sources alone (a workgroup per target:
 // 23 - 24).
-constexpr int kDirectOneTC = 4, kDirectOneWaves = 16;
-constexpr int64_t kDirectOneMax = 8192;
-__global__ void __launch_bounds__(kDirectOneWaves *kWave) k_direct_one(exafmm_body *__restrict__ t, int64_t nt,
-                                                                       const exafmm_body *__restrict__ s, int64_t ns) {
+//
+// Sixteen waves shorten a workgroup's chain of rounds where the workgroups do not
+// fill the device.  Up to kDirectFewSources sources there are no rounds to share,
+// and from kDirectManyTargets targets on the device is full of workgroups anyway:
+// four waves, which start and meet sooner.  Sixteen / four waves, us: 200 x 264 15.0 /
+// 14.8, 1,000 x 2,000 16.9 / 17.7, 2,000 x 8,192 33.9 / 33.9, 10,000 x 2,000 49.9 / 34.8,
+// 100,000 x 264 192 / 72, 100,000 x 8,192 859 / 732.
+constexpr int kDirectOneTC = 4;
+constexpr int64_t kDirectOneMax = 8192, kDirectFewSources = 512, kDirectManyTargets = 2000;
+template <int W>
+__global__ void __launch_bounds__(W *kWave) k_direct_one(exafmm_body *__restrict__ t, int64_t nt,
+                                                         const exafmm_body *__restrict__ s, int64_t ns) {
   constexpr int kLow = kWave / kDirectOneTC;
-  __shared__ double red[kDirectOneWaves][kDirectOneTC * 4];
+  __shared__ double red[W][kDirectOneTC * 4];
   const int lane = threadIdx.x & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int64_t t0 = int64_t(blockIdx.x) * kDirectOneTC;
   const int tc = int(min(int64_t(kDirectOneTC), nt - t0));
-  const double v = direct_block<kDirectOneTC>(t + t0, tc, s, w * kWave, ns, kDirectOneWaves * kWave, lane);
+  const double v = direct_block<kDirectOneTC>(t + t0, tc, s, w * kWave, ns, W * kWave, lane);
   if (lane % kLow < 4) red[w][lane / kLow * 4 + lane % kLow] = v;
   __syncthreads();
   const int i = threadIdx.x / 4, comp = threadIdx.x % 4;
   if (i >= tc) return;
   // the waves' sums pairwise: one after the other their roundings add up (500 to
   // 8,192 sources of one sign: p off by 1.0 - 1.2e-16 rms, 0.7 this way)
-  double v16[kDirectOneWaves];
+  double ws[W];
 #pragma unroll
-  for (int k = 0; k < kDirectOneWaves; k++) v16[k] = red[k][threadIdx.x];
+  for (int k = 0; k < W; k++) ws[k] = red[k][threadIdx.x];
 #pragma unroll
-  for (int o = kDirectOneWaves / 2; o > 0; o /= 2)
+  for (int o = W / 2; o > 0; o /= 2)
 #pragma unroll
-    for (int k = 0; k < o; k++) v16[k] += v16[k + o];
-  const double sum = v16[0];
+    for (int k = 0; k < o; k++) ws[k] += ws[k + o];
+  const double sum = ws[0];
   if (comp == 0)
     t[t0 + i].p += sum;
   else
@@ -649,8 +657,9 @@ __global__ void __launch_bounds__(256) k_direct_sum(exafmm_body *__restrict__ t,
 void direct_sum(Ctx &c, exafmm_body *t, int64_t nt, const exafmm_body *s, int64_t ns) {
   if (nt <= 0 || ns <= 0) return;
   if (ns <= kDirectOneMax) {
-    hipLaunchKernelGGL(k_direct_one, dim3(ceil_div(nt, kDirectOneTC)), dim3(kDirectOneWaves * kWave), 0, c.s0, t, nt, s,
-                       ns);
+    const int waves = ns <= kDirectFewSources || nt >= kDirectManyTargets ? 4 : 16;
+    hipLaunchKernelGGL(waves == 4 ? k_direct_one<4> : k_direct_one<16>, dim3(ceil_div(nt, kDirectOneTC)),
+                       dim3(waves * kWave), 0, c.s0, t, nt, s, ns);
     XF_LAUNCH();
     return;
   }

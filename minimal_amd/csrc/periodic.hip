@@ -357,7 +357,7 @@ __device__ inline void ewald_pair(double x2, double &pot, double &grad) {
   grad = ex * (y * y) * (M_2_SQRTPI + hy);
 }
 
-// Two targets per workgroup, its eight waves sharing the waves and the
+// Two targets per workgroup, whose waves share the Ewald waves and the
 // sources.  A loaded source is tested against both targets; the pairs inside
 // the cutoff (about half at cutoff = cycle / 2) go into a queue per wave and
 // target in LDS, and a queue is evaluated a full wave at a time, so no lane
@@ -365,16 +365,25 @@ __device__ inline void ewald_pair(double x2, double &pot, double &grad) {
 // (140 registers would leave two).  1,000 targets x 100,003 sources: 400 us;
 // 743 us with a workgroup per target and every lane branching over its own
 // pair.
+//
+// Eight waves per workgroup while two workgroups per CU (all that their queues
+// leave room for) take every target: up to kEwaldManyTargets.  Beyond, four, and one
+// where there is a round or two of work (kEwaldFew sources and waves).  Eight /
+// four / one, us: 1,000 targets x 20,000 sources, ksize 6, 124 / 139 / 271; 2,238 x
+// 300, ksize 4, 35.6 / 30.3 / 28.0; 2,238 x 20,000 214 / 220 / 362; 20,000 x 256 132 /
+// - / 51; 20,000 x 1,000, ksize 3, 160 / 114 / 94; 20,000 x 20,000 1,301 / 1,243 / 1,279.
 constexpr int kEwaldTargets = 2;
+constexpr int64_t kEwaldManyTargets = 1024, kEwaldFew = 256;
 struct EwaldQueue {
   double x[2 * kWave], y[2 * kWave], z[2 * kWave], q[2 * kWave];
 };
-__global__ void __launch_bounds__(kEwaldThreads) __attribute__((amdgpu_waves_per_eu(4))) k_ewald_target(int nw, const Wave *__restrict__ waves,
-                                                                exafmm_body *__restrict__ t, int64_t nt,
-                                                                const exafmm_body *__restrict__ s, int64_t ns,
-                                                                double alpha, double cutoff, double cyc) {
+template <int W>
+__global__ void __launch_bounds__(W *kWave) __attribute__((amdgpu_waves_per_eu(4)))
+    k_ewald_target(int nw, const Wave *__restrict__ waves, exafmm_body *__restrict__ t, int64_t nt,
+                   const exafmm_body *__restrict__ s, int64_t ns, double alpha, double cutoff, double cyc) {
+  constexpr int NT = W * kWave;
   extern __shared__ EwaldQueue queues[];  // [wave][target]
-  __shared__ double red[kEwaldWaves][kEwaldTargets][4];
+  __shared__ double red[W][kEwaldTargets][4];
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int64_t t0 = int64_t(blockIdx.x) * kEwaldTargets;
@@ -389,7 +398,7 @@ __global__ void __launch_bounds__(kEwaldThreads) __attribute__((amdgpu_waves_per
   }
   // wave part (3dp/ewald.h:36-51), phases in half turns
   const double u = 2.0 / cyc, scale = M_PI * u;
-  for (int i = tid; i < nw; i += kEwaldThreads) {
+  for (int i = tid; i < nw; i += NT) {
     const Wave wv = waves[i];
 #pragma unroll
     for (int k = 0; k < kEwaldTargets; k++) {
@@ -416,9 +425,9 @@ __global__ void __launch_bounds__(kEwaldThreads) __attribute__((amdgpu_waves_per
     acc[k][2] -= dy * f;
     acc[k][3] -= dz * f;
   };
-  const int64_t rounds = (ns + kEwaldThreads - 1) / kEwaldThreads;
+  const int64_t rounds = (ns + NT - 1) / NT;
   for (int64_t r = 0; r < rounds; r++) {
-    const int64_t j = r * kEwaldThreads + tid;
+    const int64_t j = r * NT + tid;
     const bool in = j < ns;
     const exafmm_body *b = s + (in ? j : 0);
     const double sx = b->X[0], sy = b->X[1], sz = b->X[2], q = b->q;
@@ -467,7 +476,7 @@ __global__ void __launch_bounds__(kEwaldThreads) __attribute__((amdgpu_waves_per
   const int k = tid / 4, c = tid % 4;
   if (t0 + k >= nt) return;
   double v = 0.0;
-  for (int i = 0; i < kEwaldWaves; i++) v += red[i][k][c];
+  for (int i = 0; i < W; i++) v += red[i][k][c];
   exafmm_body *b = t + t0 + k;
   if (c == 0)
     b->p += v - M_2_SQRTPI * b->q * alpha;  // self term (3dp/ewald.h:146-150)
@@ -485,11 +494,12 @@ static void ewald_launch(Ctx &c, Wave *w, int nw, int ksize, exafmm_body *t, int
     XF_LAUNCH();
   }
   if (nt) {
-    const size_t lds = sizeof(EwaldQueue) * kEwaldWaves * kEwaldTargets;
-    XF_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_ewald_target),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-    hipLaunchKernelGGL(k_ewald_target, dim3(ceil_div(nt, kEwaldTargets)), dim3(kEwaldThreads), lds, c.s0, nw, w, t, nt,
-                       s, ns, alpha, cutoff, cyc);
+    const int waves = nt <= kEwaldManyTargets ? 8 : std::max<int64_t>(ns, nw) > kEwaldFew ? 4 : 1;
+    auto *k = waves == 8 ? &k_ewald_target<8> : waves == 4 ? &k_ewald_target<4> : &k_ewald_target<1>;
+    const size_t lds = sizeof(EwaldQueue) * waves * kEwaldTargets;
+    XF_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+    hipLaunchKernelGGL(k, dim3(ceil_div(nt, kEwaldTargets)), dim3(waves * kWave), lds, c.s0, nw, w, t, nt, s, ns, alpha,
+                       cutoff, cyc);
     XF_LAUNCH();
   }
   XF_HIP(hipStreamSynchronize(c.s0));
