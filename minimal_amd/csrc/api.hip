@@ -871,7 +871,7 @@ struct exafmm_graph {
   xf::Buf<xf::GroupLevel> lv;
   xf::Buf<int> starts;
   Stage pro, p2p, l2p;
-  std::map<int, Stage> p2m;  // by order
+  std::map<int, Stage> p2m;  // by order; 0: all of them
   std::vector<Stage> m2m_levels, l2l_levels;  // M2M bottom-up, L2L top-down
   std::vector<std::unique_ptr<xf::GemmGroupPlan>> gemm;  // one per order
   std::vector<int> level_soff_m2m, level_soff_l2l;       // start-array offsets of the level stages
@@ -906,6 +906,9 @@ void graph_release(exafmm_graph *g) {
   }
   delete g;
 }
+
+// Workgroups of a batch's P2M up to which the orders share a launch: one per CU.
+constexpr int kP2MOneLaunch = 256;
 
 // Descriptor tables of a grouped graph (host-built, copied once).
 void grouped_tables(exafmm_graph *g) {
@@ -958,11 +961,15 @@ void grouped_tables(exafmm_graph *g) {
     return int64_t(ceil_div(c.t.n, 256)) + ceil_div(c.t.ncells * c.P * c.P, 256);
   });
   per_problem(g->l2p, [](const Ctx &c) { return int64_t(ceil_div(c.t.n, kWave)); });
-  // one launch per order: the problems of another order have no blocks in it
+  // one launch per order (the problems of another order have no blocks in it),
+  // or one for all of a small batch, as order 0
   g->p2m.clear();
+  per_problem(g->p2m[0], [](const Ctx &c) { return int64_t(p2m_group_blocks(c.t.nleaves)); });
+  const bool small = g->p2m[0].blocks <= kP2MOneLaunch;
+  if (!small) g->p2m.clear();
   for (const exafmm_ctx *x : g->ctxs) {
     const int P = x->c.P;
-    if (g->p2m.count(P)) continue;
+    if (small || g->p2m.count(P)) continue;
     per_problem(g->p2m[P], [P](const Ctx &c) { return c.P == P ? int64_t(p2m_group_blocks(c.t.nleaves)) : 0; });
   }
   per_problem(g->p2p, [](const Ctx &c) { return int64_t(p2p_group_blocks(c.t.nleaves)); });
@@ -1034,7 +1041,11 @@ void grouped_record(exafmm_graph *g, hipStream_t sa, hipStream_t sb, hipEvent_t 
   XF_HIP(hipStreamWaitEvent(sb, fork, 0));
   if (g->p2p.blocks) p2p_grouped(g->gt.p, st + g->p2p.off, n, g->p2p.blocks, sb);
   XF_HIP(hipEventRecord(join, sb));
-  for (const auto &kv : g->p2m) p2m_grouped(kv.first, g->gt.p, st + kv.second.off, n, kv.second.blocks, sa);
+  for (const auto &kv : g->p2m)
+    if (kv.first == 0)
+      p2m_orders(g->gt.p, st + kv.second.off, n, kv.second.blocks, sa);
+    else
+      p2m_grouped(kv.first, g->gt.p, st + kv.second.off, n, kv.second.blocks, sa);
   for (size_t k = 0; k < g->m2m_levels.size(); k++) {
     const auto &sg = g->m2m_levels[k];
     if (sg.blocks) m2m_grouped(g->gt.p, g->lv.p + sg.off, st + g->level_soff_m2m[k], sg.n, sg.blocks, sa);

@@ -73,6 +73,7 @@ template <int P>
 struct P2MShape {
   static constexpr int J = (P + 1) / 2, G = kWave / J, T = P + 1;
   static constexpr int S = kWave + J;  // LDS row: lanes reading (term, column) pairs in turn hit distinct banks
+  using Lds = double[kP2MWaves][T * S];
 };
 
 template <int P>
@@ -82,10 +83,10 @@ __device__ __attribute__((always_inline)) inline void p2m_body(int bx, const int
                                                                const int *__restrict__ ccnt,
                                                                const double4 *__restrict__ cx,
                                                                const double4 *__restrict__ xs,
-                                                               double *__restrict__ M) {
+                                                               double *__restrict__ M,
+                                                               typename P2MShape<P>::Lds &red) {
   using Sh = P2MShape<P>;
   constexpr int J = Sh::J, G = Sh::G, T = Sh::T, S = Sh::S;
-  __shared__ double red[kP2MWaves][T * S];
   const int lane = threadIdx.x % kWave, w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int li = bx * kP2MWaves + w;
   if (li >= *nleaves) return;  // whole wave; wave-level syncs only below
@@ -188,7 +189,8 @@ __global__ void __launch_bounds__(kP2MWaves *kWave) k_p2m(const int *__restrict_
                                                           const int *__restrict__ cbeg, const int *__restrict__ ccnt,
                                                           const double4 *__restrict__ cx,
                                                           const double4 *__restrict__ xs, double *__restrict__ M) {
-  p2m_body<P>(blockIdx.x, leaves, nleaves, cbeg, ccnt, cx, xs, M);
+  __shared__ typename P2MShape<P>::Lds red;
+  p2m_body<P>(blockIdx.x, leaves, nleaves, cbeg, ccnt, cx, xs, M, red);
 }
 
 // The problems of one order of a batch in one launch (block -> problem through start[]).
@@ -197,7 +199,25 @@ __global__ void __launch_bounds__(kP2MWaves *kWave) k_p2m_grouped(const GroupTre
                                                                   const int *__restrict__ start, int nprob) {
   const int b = blockIdx.x, i = group_of(start, nprob, b);
   const GroupTree &t = g[i];
-  p2m_body<P>(b - start[i], t.leaves, t.nleaves, t.cbeg, t.ccnt, t.cx, t.xs, t.M);
+  __shared__ typename P2MShape<P>::Lds red;
+  p2m_body<P>(b - start[i], t.leaves, t.nleaves, t.cbeg, t.ccnt, t.cx, t.xs, t.M, red);
+}
+
+// All problems of a small batch in one launch, each workgroup by its problem's
+// order: the registers and LDS of the highest order leave room for few workgroups,
+// and a launch less per order is worth more (grouped_record).
+__global__ void __launch_bounds__(kP2MWaves *kWave) k_p2m_orders(const GroupTree *__restrict__ g,
+                                                                 const int *__restrict__ start, int nprob) {
+  __shared__ typename P2MShape<kMaxP>::Lds lds;  // every order's fits
+  const int b = blockIdx.x, i = group_of(start, nprob, b);
+  const GroupTree &t = g[i];
+  auto run = [&](auto p) {
+    p2m_body<p()>(b - start[i], t.leaves, t.nleaves, t.cbeg, t.ccnt, t.cx, t.xs, t.M,
+                  reinterpret_cast<typename P2MShape<p()>::Lds &>(lds));
+  };
+  switch (t.P) {
+    XF_ORDER_CASES(run)
+  }
 }
 
 
@@ -809,6 +829,10 @@ int p2m_group_blocks(int64_t nleaves) { return ceil_div(nleaves, kP2MWaves); }
 int shift_group_rows(int P) { return ceil_div(P * P, 16 * kShiftWaves); }
 int m2m_group_rows(int P) { return ceil_div(P * P, 16); }
 
+void p2m_orders(const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s) {
+  hipLaunchKernelGGL(k_p2m_orders, dim3(nblocks), dim3(kP2MWaves * kWave), 0, s, g, start, nprob);
+  XF_LAUNCH();
+}
 void p2m_grouped(int P, const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s) {
   by_order(P, [&](auto p) {
     hipLaunchKernelGGL((k_p2m_grouped<p()>), dim3(nblocks), dim3(kP2MWaves * kWave), 0, s, g, start, nprob);

@@ -373,6 +373,7 @@ int p2m_group_blocks(int64_t nleaves);
 int shift_group_rows(int P);
 int m2m_group_rows(int P);
 int p2p_group_blocks(int64_t nleaves);
+void p2m_orders(const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s);
 void p2m_grouped(int P, const GroupTree *g, const int *start, int nprob, int nblocks, hipStream_t s);
 void m2m_grouped(const GroupTree *g, const GroupLevel *lv, const int *start, int n, int nblocks, hipStream_t s);
 void l2l_grouped(const GroupTree *g, const GroupLevel *lv, const int *start, int n, int nblocks, hipStream_t s);
