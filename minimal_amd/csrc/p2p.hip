@@ -406,8 +406,8 @@ __device__ inline void p2p64_pair(double dx, double dy, double dz, double q, dou
 // FP64 P2P: a workgroup per target leaf, its waves taking the leaf's targets
 // in balanced blocks of at most kP2P64TC; as in the FP32 kernel a block's
 // targets are wave-uniform and the lanes take the staged entries' sources,
-// one load per source and block.  FP64 VALU bound (about 27 operations per
-// interaction).  67,984,904 interactions (30,000 bodies): 164 us; 903 us with
+// one load per source and block.  FP64 VALU bound (25 instructions per
+// interaction, 26 with image shifts).  67,984,904 interactions (30,000 bodies): 169 us; 903 us with
 // a thread per target walking its sources one by one through a divide and a
 // square root each.
 constexpr int kP2P64TC = 8;
